@@ -122,15 +122,15 @@ QUAD_OK = {'gdn': [
 def quad_variants(fam, c):
     """[(row blocks per wavefront, value heads per workgroup, wavefronts per SIMD the register allocation aims
     for)], widest head group first, of the workgroup-per-key-head kernels (sq_quad.cuh) for a case; empty where only
-    the one-wavefront kernels (sq_tile.cuh) serve it: value-axis groups, the float state, rows that are not a power
-    of two in size, d_k above 128, more than four scale groups per row."""
+    the one-wavefront kernels (sq_tile.cuh) serve it: value-axis groups other than 32 rows, the float state, rows that
+    are not a power of two in size, d_k above 128, more than four scale groups per row."""
     bits, dk, dv, group, qbuf, mmax, axv = c
-    if fam not in QUAD_FAMILIES or axv or bits not in (4, 8):
+    if fam not in QUAD_FAMILIES or bits not in (4, 8) or (axv and group != 32):
         return []
     rb = dk * bits // 8
     if rb & (rb - 1) or not 32 <= rb <= 128 or dk > 128 or dv % 32 or (bits == 4 and dk % 64):
         return []
-    if -(-dk // group) > 4:
+    if not axv and -(-dk // group) > 4:
         return []
     nrb = dv // 32
     nb = 2 if nrb % 2 == 0 else 1
@@ -141,12 +141,15 @@ def quad_variants(fam, c):
         if nw > 16:
             continue
         lds = gh * dv * rb + mmax * dk * be + gh * mmax * dv * be + 2 * dk * 4 + dk * 8 + 512
+        if axv:                                          # a plane set per wavefront
+            lds += nw * dk * 6 - dk * 8
         wgs = min(160 * 1024 // lds, 32 // nw)
         if wgs < 1:
             continue
-        # register target: as many wavefronts per SIMD as LDS lets workgroups in, up to 6 (5 with the 16-token buffer);
-        # asked for 7, the int4 kernels spill into scratch memory inside the fold (measured: +60 % bytes written)
-        wpe = max(1, min(6 if mmax <= 8 else 5, -(-wgs * nw // 4)))
+        # register target: as many wavefronts per SIMD as LDS lets workgroups in, up to 6 (5 with the 16-token buffer and
+        # for value-axis groups, which spill 10 registers at 80); asked for 7, the int4 kernels spill into scratch
+        # memory inside the fold (measured: +60 % bytes written)
+        wpe = max(1, min(6 if mmax <= 8 and not axv else 5, -(-wgs * nw // 4)))
         # the serving cases compiled in (SPEC of the kernels) for the default buffer: int8, 8 tokens
         for spec in SPECS[fam] if (qbuf and mmax == 8) else (0,):
             out.append((nb, gh, wpe, spec))

@@ -60,6 +60,7 @@ __device__ __forceinline__ float vec_elem(const uint32_t (&w)[NE], int dt, int t
 template <class T, class Q>
 struct GdnLoads {
     uint16_t sc[Q::NB][T::NG];             // scales of rows (block bi, lane % 32)
+    uint32_t scv[Q::NB];                   // value-axis groups: the block's scales of columns NE lane ..
     Raw4<T::QBUF> uraw[Q::UT], kraw[Q::KT];
     uint16_t kbs[Q::KT], ubs;
     float gbl, gcur;
@@ -184,9 +185,14 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     F.gcur = *A.gcp;
     {
 #pragma unroll
-        for (int bi = 0; bi < NB; ++bi)
+        for (int bi = 0; bi < NB; ++bi) {
+            if constexpr (T::AXV) {
+                F.scv[bi] = quad_load_colscales<NE>(A.SCh + (wh * NB + bi) * DK, lane);
+            } else {
 #pragma unroll
-            for (int g = 0; g < NG; ++g) F.sc[bi][g] = stream_load(A.SCh + uint32_t(((wh * NB + bi) * T::MR + n32) * NG + g));
+                for (int g = 0; g < NG; ++g) F.sc[bi][g] = stream_load(A.SCh + uint32_t(((wh * NB + bi) * T::MR + n32) * NG + g));
+            }
+        }
         // the buffer, live slots only (the others repeat the last live one: no new memory traffic); the fill count,
         // requested ahead of the row blocks, is here by now
         quad_dma_counter_wait(F.np);
@@ -232,7 +238,7 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
         if constexpr (NE == 1) lds_xn[v * DK + lane] = xe[0];
         else if constexpr (NE == 2) *reinterpret_cast<float2*>(lds_xn + v * DK + 2 * lane) = make_float2(xe[0], xe[1]);
         else *reinterpret_cast<float4*>(lds_xn + v * DK + 4 * lane) = make_float4(xe[0], xe[1], xe[2], xe[3]);
-        quad_stage_planes<T, NE>(xe, v, lane, lds_pl, lds_xs);
+        if constexpr (!T::AXV) quad_stage_planes<Q, T, NE>(xe, v, lane, lds_pl, lds_xs);
     };
     if constexpr (RQ == RK) {
         if (w == RQ) {
@@ -267,12 +273,15 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     const uint32_t vr = F.vr;
     uint16_t scw[NB][NG];
 #pragma unroll
-    for (int bi = 0; bi < NB; ++bi)
+    for (int bi = 0; bi < NB; ++bi) {
+        if constexpr (!T::AXV) {
 #pragma unroll
-        for (int g = 0; g < NG; ++g) {
-            scw[bi][g] = F.sc[bi][g];
-            if (kb == 0) lds_sc[((wh * NB + bi) * T::MR + n32) * NG + g] = F.sc[bi][g];
+            for (int g = 0; g < NG; ++g) {
+                scw[bi][g] = F.sc[bi][g];
+                if (kb == 0) lds_sc[((wh * NB + bi) * T::MR + n32) * NG + g] = F.sc[bi][g];
+            }
         }
+    }
 #pragma unroll
     for (int t = 0; t < Q::UT; ++t) {
         const int i = lane / Q::LU + Q::SU * t;
@@ -299,18 +308,25 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     // ---- every wavefront: state pass over its row blocks ----
     float sq, sk;                                    // (S0 q)[row], (S0 k)[row], scales applied
     {
-        v4i aop[T::NKS];
-        quad_fetch_planes<T, 2>(lds_pl, lane, aop);
-        float xs[NG];
-#pragma unroll
-        for (int g = 0; g < NG; ++g) xs[g] = lds_xs[kb * NG + g];
         float own[NB];
+        if constexpr (T::AXV) {
 #pragma unroll
-        for (int bi = 0; bi < NB; ++bi) {
-            float sc[NG];
+            for (int bi = 0; bi < NB; ++bi)
+                own[bi] = quad_block_pass_v<Q, T, 2>(my_codes + bi * Q::BLK, lds_xn, F.scv[bi], lds_pl + w * L::PL_BYTES,
+                                                     lds_xs + w * (L::XS_BYTES / 4), lane);
+        } else {
+            v4i aop[T::NKS];
+            quad_fetch_planes<Q, T, 2>(lds_pl, lane, aop);
+            float xs[NG];
 #pragma unroll
-            for (int g = 0; g < NG; ++g) sc[g] = f16_to_f32(scw[bi][g]);
-            own[bi] = quad_block_pass<Q, T>(my_codes + bi * Q::BLK, aop, xs, sc, lane);
+            for (int g = 0; g < NG; ++g) xs[g] = lds_xs[kb * NG + g];
+#pragma unroll
+            for (int bi = 0; bi < NB; ++bi) {
+                float sc[NG];
+#pragma unroll
+                for (int g = 0; g < NG; ++g) sc[g] = f16_to_f32(scw[bi][g]);
+                own[bi] = quad_block_pass<Q, T>(my_codes + bi * Q::BLK, aop, xs, sc, lane);
+            }
         }
         if constexpr (NB == 2) {                     // lane (n, kb) takes over row n of block kb: both sums
             const auto r = __builtin_amdgcn_permlane32_swap(as_u32(own[0]), as_u32(own[1]), false, false);
@@ -478,48 +494,89 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     // ---- fold ----
     if (full) {
         lds_barrier();                               // `full` is the same in every head of a slot
-        constexpr int MT4 = (MM + 3) / 4, CL = DK / 4;
         // what the fold derives from the lane id it derives anew (from a copy the compiler cannot trace back): offsets
         // formed at the top of the kernel would otherwise be kept in registers all the way to here
         int lf = lane;
         asm volatile("" : "+v"(lf));
-        const int fn = lf & 15, fq = lf >> 4;
         const int swzf = swz<Q>(lf / Q::CPR, lf % Q::CPR);
-        // decay ratios a_m / a_i of the lane's slots 4 t + q (this token: 1)
-        float decf[MT4];
-#pragma unroll
-        for (int t = 0; t < MT4; ++t) {
-            const int sl = 4 * t + fq;
-            decf[t] = sl < m - 1 ? expf(gnew - lds_gbf[sl < m - 1 ? sl : 0]) : 1.0f;
-        }
         const float cmul = expf(gnew);
-        const int fg = (fq * CL) / T::KGROUP;
-        FoldKeys<T> kop;
-        quad_fold_keys<T>(lds_kbr, lds_kbsf, m, lf, kop);
+        if constexpr (T::AXV) {
+            constexpr int MT = (MM + 1) / 2;
+            const int fj = lf & 31, fkb = lf >> 5;
+            float decf[MT];                          // decay ratios a_m / a_i of the lane's slots 2 t + kb (this token: 1)
 #pragma unroll
-        for (int bi = 0; bi < NB; ++bi) {
-            uint8_t* blk = my_codes + bi * Q::BLK;
+            for (int t = 0; t < MT; ++t) {
+                const int sl = 2 * t + fkb;
+                decf[t] = sl < m - 1 ? expf(gnew - lds_gbf[sl < m - 1 ? sl : 0]) : 1.0f;
+            }
+            auto key = [&](int sl, int col) {
+                const int sc_ = sl < m ? sl : 0;
+                float kv = lds_raw<T::QBUF>(lds_kbr, sc_ * DK + col);
+                if constexpr (T::QBUF) kv = kv * lds_kbsf[sc_];
+                return sl < m ? kv : 0.0f;
+            };
 #pragma unroll
-            for (int hf = 0; hf < 2; ++hf) {
-                const int frow = (wh * NB + bi) * T::MR + 16 * hf + fn;
-                float bop[MT4];
+            for (int bi = 0; bi < NB; ++bi) {
+                uint8_t* blk = my_codes + bi * Q::BLK;
+                const int grp = wh * NB + bi;
+                uint16_t* old = reinterpret_cast<uint16_t*>(lds_pl + w * L::PL_BYTES);      // the planes are done with
+                quad_store_colscales<NE>(old, lf, F.scv[bi]);
+                wave_sync();
+                float dop[MT];
 #pragma unroll
-                for (int t = 0; t < MT4; ++t) {
-                    const int sl = 4 * t + fq;
+                for (int t = 0; t < MT; ++t) {
+                    const int sl = 2 * t + fkb;
                     const int sc_ = sl < m ? sl : 0;
-                    float uv = lds_raw<T::QBUF>(lds_ubr, sc_ * DV + frow);
+                    float uv = lds_raw<T::QBUF>(lds_ubr, sc_ * DV + grp * T::MR + fj);
                     if constexpr (T::QBUF) uv = uv * lds_ubsf[sc_];
                     uv = decf[t] * uv;
-                    bop[t] = sl < m ? uv : 0.0f;
+                    dop[t] = sl < m ? uv : 0.0f;
                 }
-                quad_fold_half<Q, T>(blk, hf, kop, bop, cmul, f16_to_f32(lds_sc[frow * NG + fg]),
-                                            A.SCh + frow * NG + fg, lf);
-            }
-            wave_sync();
+                quad_fold_block_v<Q, T>(blk, key, dop, [&](int) { return cmul; }, cmul == 1.0f, old,
+                                        A.SCh + grp * DK, lf);
 #pragma unroll
-            for (int t = 0; t < Q::NLD; ++t)
-                stream_store(reinterpret_cast<v4u*>(A.Sh + (wh * NB + bi) * Q::BLK + t * 1024 + lf * 16),
-                             *reinterpret_cast<const v4u*>(blk + t * 1024 + swzf));
+                for (int t = 0; t < Q::NLD; ++t)
+                    stream_store(reinterpret_cast<v4u*>(A.Sh + grp * Q::BLK + t * 1024 + lf * 16),
+                                 *reinterpret_cast<const v4u*>(blk + t * 1024 + swzf));
+            }
+        } else {
+            constexpr int MT4 = (MM + 3) / 4, CL = DK / 4;
+            const int fn = lf & 15, fq = lf >> 4;
+            // decay ratios a_m / a_i of the lane's slots 4 t + q (this token: 1)
+            float decf[MT4];
+#pragma unroll
+            for (int t = 0; t < MT4; ++t) {
+                const int sl = 4 * t + fq;
+                decf[t] = sl < m - 1 ? expf(gnew - lds_gbf[sl < m - 1 ? sl : 0]) : 1.0f;
+            }
+            const int fg = (fq * CL) / T::KGROUP;
+            FoldKeys<T> kop;
+            quad_fold_keys<T>(lds_kbr, lds_kbsf, m, lf, kop);
+#pragma unroll
+            for (int bi = 0; bi < NB; ++bi) {
+                uint8_t* blk = my_codes + bi * Q::BLK;
+#pragma unroll
+                for (int hf = 0; hf < 2; ++hf) {
+                    const int frow = (wh * NB + bi) * T::MR + 16 * hf + fn;
+                    float bop[MT4];
+#pragma unroll
+                    for (int t = 0; t < MT4; ++t) {
+                        const int sl = 4 * t + fq;
+                        const int sc_ = sl < m ? sl : 0;
+                        float uv = lds_raw<T::QBUF>(lds_ubr, sc_ * DV + frow);
+                        if constexpr (T::QBUF) uv = uv * lds_ubsf[sc_];
+                        uv = decf[t] * uv;
+                        bop[t] = sl < m ? uv : 0.0f;
+                    }
+                    quad_fold_half<Q, T>(blk, hf, kop, bop, cmul, f16_to_f32(lds_sc[frow * NG + fg]),
+                                                A.SCh + frow * NG + fg, lf);
+                }
+                wave_sync();
+#pragma unroll
+                for (int t = 0; t < Q::NLD; ++t)
+                    stream_store(reinterpret_cast<v4u*>(A.Sh + (wh * NB + bi) * Q::BLK + t * 1024 + lf * 16),
+                                 *reinterpret_cast<const v4u*>(blk + t * 1024 + swzf));
+            }
         }
     }
     SQ_MARK(14);                                                  // fold done and stored (if any)

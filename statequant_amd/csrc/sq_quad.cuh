@@ -1,6 +1,6 @@
 // The state tile of one (sequence, value head) shared by the wavefronts of one workgroup: every wavefront owns NB of
 // the tile's 32-row blocks.  Shared by the Gated DeltaNet and Mamba2 workgroup-per-key-head step kernels (int4 / int8
-// codes with key-axis scale groups and a power-of-two row size).
+// codes with key-axis scale groups, or value-axis groups of one row block, and a power-of-two row size).
 //
 // What this buys over one wavefront per tile (sq_tile.cuh, kept for the other formats):
 //   * a tile's life is a quarter as long, so the launch's ramp-up and tail shrink and the dispatcher balances the
@@ -77,7 +77,8 @@ __device__ __forceinline__ void quad_start_wait(uint32_t ramp) {
 
 template <class T, int NB_, int GH_ = 1>
 struct Quad {
-    static_assert(!T::FLT && !T::AXV && !T::RAGV, "int4 / int8 codes with key-axis groups, whole row blocks");
+    static_assert(!T::FLT && !T::RAGV, "int4 / int8 codes, whole row blocks");
+    static_assert(!T::AXV || T::GROUP == T::MR, "value-axis groups: one row block each");
     static constexpr int NB = NB_;                         // row blocks per wavefront
     static constexpr int GH = GH_;                         // value heads of one key head per workgroup
     static_assert(T::NRB % NB == 0 && (NB == 1 || NB == 2), "one or two row blocks per wavefront");
@@ -95,6 +96,7 @@ struct Quad {
     static constexpr int NLD = BLK / 1024;                 // wavefront loads per row block
     static constexpr int SWM = CPR < 8 ? CPR : 8;          // swizzle: chunk c of row r sits at chunk c ^ ((r / SWD) % SWM)
     static constexpr int SWD = 8 / SWM;
+    static constexpr int PLS = T::AXV ? 6 : 8;             // digit-plane slots per 16-column piece
     static_assert(T::NG <= 4, "at most four scale groups per row (result rows 8 g + 4 v + d)");
     // a d_k vector in a wavefront: lane l holds the NE consecutive elements NE l ..
     static constexpr int NE = T::DK / WAVE;
@@ -115,27 +117,31 @@ __device__ __forceinline__ int swz(int r, int c) { return r * Q::RB + ((c ^ ((r 
 template <class T, int NB, int GH, int NX, int NV>
 struct QuadLds {
     using Q = Quad<T, NB, GH>;
+    // digit planes and their factors: one set for the workgroup; value-axis groups: one per wavefront, rebuilt for
+    // each of its row blocks (the block's scales ride on the read-out vectors)
+    static constexpr int SETS = T::AXV ? Q::NW : 1;
+    static constexpr int PL_BYTES = T::DK / CPL * Q::PLS * 16, XS_BYTES = round_up(NV * T::NG * 4, 16);
     static constexpr int CODES = 0;                                    // [GH][DV] rows, swizzled
     static constexpr int KBR = CODES + GH * Q::HEAD;                   // buffered keys, raw [m][DK]
     static constexpr int UBR = KBR + T::MMAX * T::DK * T::BE;          // buffered values, raw [GH][m][DV]
     static constexpr int XN = UBR + GH * T::MMAX * T::DV * T::BE;      // read-out vectors, fp32 [NX][DK]
-    static constexpr int PL = XN + NX * T::DK * 4;                     // digit planes [k-step][half][8][16]
-    static constexpr int XS = PL + T::DK * 8;                          // [NV][NG] exponent factors
-    static constexpr int DOTS = XS + round_up(NV * T::NG * 4, 16);     // [NV][MMAX] K_i . x
+    static constexpr int PL = XN + NX * T::DK * 4;                     // digit planes [k-step][half][PLS][16]
+    static constexpr int XS = PL + SETS * PL_BYTES;                    // [NV][NG] exponent factors
+    static constexpr int DOTS = XS + SETS * XS_BYTES;                  // [NV][MMAX] K_i . x
     static constexpr int KBSF = DOTS + NV * T::MMAX * 4;               // [MMAX] key scales as fp32
     static constexpr int UBSF = KBSF + T::MMAX * 4;                    // [GH][MMAX] value scales as fp32
     static constexpr int SCAL = UBSF + GH * T::MMAX * 4;               // [GH][8] scalars of a head + [8] of the group
     static constexpr int RED = SCAL + (GH + 1) * 32;                   // one float per wavefront
     static constexpr int GBF = RED + round_up(Q::NW * 4, 16);          // [GH][MMAX] cumulative decays of the slots
-    static constexpr int SC = GBF + GH * T::MMAX * 4;                  // [GH][DV][NG] fp16 scales of the rows
-    static constexpr int BYTES = SC + round_up(GH * T::DV * T::NG * 2, 16);
+    static constexpr int SC = GBF + GH * T::MMAX * 4;                  // [GH][DV][NG] fp16 scales of the rows (value-axis
+    static constexpr int BYTES = SC + (T::AXV ? 0 : round_up(GH * T::DV * T::NG * 2, 16));   // scales stay in registers)
 };
 
 // Where column e of a read-out vector goes in the digit-plane region: the (k-step, lane half, byte) at which the
 // matrix core meets it with the codes.  int8: k-step ks, half kb carry columns 32 ks + 16 kb + [0, 16).  int4: a lane
 // reads whole 16-byte chunks (32 columns) and feeds them as two k-steps, so k-step ks, half kb carry columns
 // 32 (2 (ks / 2) + kb) + 16 (ks % 2) + [0, 16), in the nibble-split order of `operand`.
-template <class T>
+template <class Q, class T>
 __device__ __forceinline__ int plane_addr(int e, int pl) {
     int ks, kb, pos;
     if constexpr (T::BITS == 8) {
@@ -144,7 +150,7 @@ __device__ __forceinline__ int plane_addr(int e, int pl) {
         const int p = e / 32;
         kb = p % 2; ks = 2 * (p / 2) + (e % 32) / 16; pos = operand_pos<4>(e % 16);
     }
-    return ((ks * 2 + kb) * 8 + pl) * 16 + pos;
+    return ((ks * 2 + kb) * Q::PLS + pl) * 16 + pos;
 }
 template <class T>
 __device__ __forceinline__ constexpr int op_colbase(int ks, int kb) {
@@ -180,7 +186,7 @@ __device__ __forceinline__ float lanes_max(float v) {
 // One read-out vector -> its three digit planes (plane slots 3 v .. 3 v + 2) and its exponent factors; xe[t] =
 // element NE lane + t.  Arithmetic as `stage_planes` in sq_tile.cuh: per scale group e = exponent of the largest
 // |x|, q = rint(x 2^(22 - e)) cut into three signed 8-bit digits.
-template <class T, int NE>
+template <class Q, class T, int NE>
 __device__ __forceinline__ void quad_stage_planes(const float (&xe)[NE], int v, int lane, uint8_t* lds_pl,
                                                   float* lds_xs) {
     float mx = 0.0f;
@@ -200,14 +206,14 @@ __device__ __forceinline__ void quad_stage_planes(const float (&xe)[NE], int v, 
     }
     const int e0 = NE * lane;
     if constexpr (T::BITS == 8 && NE == 2) {                 // neighbouring columns are neighbouring operand bytes
-        uint8_t* at = lds_pl + plane_addr<T>(e0, 3 * v);
+        uint8_t* at = lds_pl + plane_addr<Q, T>(e0, 3 * v);
         *reinterpret_cast<uint16_t*>(at) = uint16_t((d[0] & 0xFFu) | ((d[1] & 0xFFu) << 8));
         *reinterpret_cast<uint16_t*>(at + 16) = uint16_t(((d[0] >> 8) & 0xFFu) | (d[1] & 0xFF00u));
         *reinterpret_cast<uint16_t*>(at + 32) = uint16_t(((d[0] >> 16) & 0xFFu) | ((d[1] >> 8) & 0xFF00u));
     } else {
 #pragma unroll
         for (int t = 0; t < NE; ++t) {
-            uint8_t* at = lds_pl + plane_addr<T>(e0 + t, 3 * v);
+            uint8_t* at = lds_pl + plane_addr<Q, T>(e0 + t, 3 * v);
             at[0] = uint8_t(d[t]);
             at[16] = uint8_t(d[t] >> 8);
             at[32] = uint8_t(d[t] >> 16);
@@ -219,14 +225,14 @@ __device__ __forceinline__ void quad_stage_planes(const float (&xe)[NE], int v, 
 // The digit planes as the matrix core's first operand, per k-step: lane (i, kb) carries result row i = 8 g + 4 v + d,
 // i.e. digit d of vector v -- on the k-steps whose columns belong to scale group g, zero elsewhere (and zero in the
 // unused rows), so that ONE accumulation over all k-steps leaves every group's sums in its own result rows.
-template <class T, int NV>
+template <class Q, class T, int NV>
 __device__ __forceinline__ void quad_fetch_planes(const uint8_t* lds_pl, int lane, v4i (&aop)[T::NKS]) {
     const int i = lane & 31, kb = lane >> 5;
     const int g = i >> 3, v = (i >> 2) & 1, d = i & 3;
     const bool used = d < 3 && g < T::NG && v < NV;
 #pragma unroll
     for (int ks = 0; ks < T::NKS; ++ks) {
-        const v4i x = *reinterpret_cast<const v4i*>(lds_pl + ((ks * 2 + kb) * 8 + 3 * v + (d < 3 ? d : 0)) * 16);
+        const v4i x = *reinterpret_cast<const v4i*>(lds_pl + ((ks * 2 + kb) * Q::PLS + 3 * (v < NV ? v : 0) + (d < 3 ? d : 0)) * 16);
         const bool mine = used && (kb == 0 ? op_colbase<T>(ks, 0) : op_colbase<T>(ks, 1)) / T::KGROUP == g;
         aop[ks] = mine ? x : v4i{0, 0, 0, 0};
     }
@@ -580,6 +586,164 @@ __device__ __forceinline__ void quad_fold_half(uint8_t* blk, int hf, const FoldK
     if (exact) requantize(std::true_type{}, std::true_type{});
     else if (__builtin_amdgcn_ballot_w64(sc < 6.103515625e-05f) != 0) requantize(std::true_type{}, std::false_type{});
     else requantize(std::false_type{}, std::false_type{});
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// value-axis scale groups of one row block (32 rows x one key column share a scale)
+//
+// A group lies inside one wavefront's rows, so nothing of it crosses wavefronts; what the workgroup shape buys over one
+// wavefront per head is the length of a head's life (bound by latency and by the vector ALU, not by memory, at every
+// batch size: the fold of a head is half of it) -- two wavefronts per head and the front end shared by the heads of a
+// key head.  us per launch with sequences out of step, one wavefront per head -> this (32 / 16 heads of 128 x 128):
+// int4 1 sequence 9.9 -> 6.0, 16: 19.3 -> 10.5, 100: 32.0 -> 23.0, 256: 37.7 -> 32.3; int8 1: 9.3 -> 5.7,
+// 32: 20.8 -> 14.5, 256: 44.6 -> 38.1; Mamba2 (128 heads of 128 x 64) int4 16: 15.4 -> 13.9.
+// ---------------------------------------------------------------------------------------------------------------
+// A lane's scales of one row block: columns NE lane .. (the columns it holds of a read-out vector), NE fp16 numbers.
+template <int NE>
+__device__ __forceinline__ uint32_t quad_load_colscales(const uint16_t* sc, int lane) {
+    if constexpr (NE == 1) return stream_load(sc + lane);
+    else return stream_load(reinterpret_cast<const uint32_t*>(sc) + lane);
+}
+template <int NE>
+__device__ __forceinline__ void quad_store_colscales(uint16_t* lds_sc, int lane, uint32_t s) {
+    if constexpr (NE == 1) lds_sc[lane] = uint16_t(s);
+    else reinterpret_cast<uint32_t*>(lds_sc)[lane] = s;
+}
+// The row sums of one block: the scales belong to (block, column), so they ride on the read-out vectors (x'_k = x_k
+// s_k, `lds_x` [NV][DK] fp32) and the digit planes are rebuilt per block, in this wavefront's own plane set.  Lane
+// (n, kb) returns (S0 x_kb)[row n of the block].
+template <class Q, class T, int NV>
+__device__ __forceinline__ float quad_block_pass_v(const uint8_t* blk, const float* lds_x, uint32_t colscales,
+                                                   uint8_t* lds_pl, float* lds_xs, int lane) {
+    constexpr int NE = Q::NE;
+    static_assert(NE <= 2, "two fp16 scales per lane");
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+        float xe[NE];
+#pragma unroll
+        for (int t = 0; t < NE; ++t)
+            xe[t] = lds_x[v * T::DK + NE * lane + t] * f16_to_f32(uint16_t(colscales >> (16 * t)));
+        quad_stage_planes<Q, T, NE>(xe, v, lane, lds_pl, lds_xs);
+    }
+    wave_sync();
+    v4i aop[T::NKS];
+    quad_fetch_planes<Q, T, NV>(lds_pl, lane, aop);
+    const float xs[1] = {lds_xs[(lane >> 5) < NV ? lane >> 5 : 0]};
+    const float one[1] = {1.0f};
+    const float s = quad_block_pass<Q, T>(blk, aop, xs, one, lane);
+    wave_sync();                                             // the planes are rebuilt for the next block
+    return s;
+}
+
+// The low bytes of four words as one word.
+__device__ __forceinline__ uint32_t pack_low_bytes(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+    const uint32_t lo = __builtin_amdgcn_perm(b, a, 0x0c0c0400u), hi = __builtin_amdgcn_perm(d, c, 0x0c0c0400u);
+    return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+}
+
+// The fold of one row block with value-axis scales, out of its LDS image and back into it.  32 columns at a time, held
+// "columns across lanes": lane (j, kb) owns column 32 cs + j and, in accumulator element 4 a + b, row 8 a + 4 kb + b, so
+// a column's absmax is a per-lane maximum and one lane exchange.  The codes arrive in that shape through the matrix
+// core (operand-shaped block x 32 x 32 identity), the m rank-1 updates run on v_mfma_f32_32x32x2_f32 (values feed the
+// rows, keys the columns, two slots per issue in slot order) as in `fold_tile_v`.  One column step at a time needs 32
+// result registers instead of the 64 of a whole block, and its loop is not unrolled (the fold is run by one workgroup in m).
+// The new codes go back to rows across lanes through the matrix core too and enter LDS in words: written byte by byte
+// from the column shape (16 one-byte stores per column step, each with its own address) the fold took half again as
+// long (int4, 100 sequences 27.8 -> 23.0 us per launch with this).
+//   key(slot, col)  the folded key's element as fp32 (0 for slots >= m)
+//   dop[t]          the lane's folded value: slot 2 t + kb, row j of the block
+//   cm(col)         the factor on the old state's column
+//   sc_old / sc_out the block's old scales (LDS) / where the new ones go (memory), [DK]
+template <class Q, class T, class KeyF, class ColF>
+__device__ __forceinline__ void quad_fold_block_v(uint8_t* blk, KeyF&& key, const float (&dop)[(T::MMAX + 1) / 2],
+                                                  ColF&& cm, bool frozen, const uint16_t* sc_old, uint16_t* sc_out,
+                                                  int lane) {
+    constexpr int MT = (T::MMAX + 1) / 2;
+    constexpr float MAGIC = 12582912.0f + (T::BITS == 4 ? 8.0f : 0.0f);
+    const int j = lane & 31, kb = lane >> 5;
+    v4i ident;                                               // byte t is 1 where operand position (kb, t) carries column j
+    {
+        const int t = operand_pos<T::BITS>(j % CPL);
+        const int one = (j / CPL == kb) ? (1 << (8 * (t % 4))) : 0;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) ident[d] = t / 4 == d ? one : 0;
+    }
+    v4i ident_t;                                             // byte t is 1 where (kb, t) carries row j: t = 4 (j / 8) + j % 4
+    {
+        const int one = ((j >> 2) & 1) == kb ? 1 << (8 * (j & 3)) : 0;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) ident_t[d] = (j >> 3) == d ? one : 0;
+    }
+    constexpr int LB = T::LANE_BYTES;                        // bytes of a lane's 16 columns
+#pragma unroll 1
+    for (int cs = 0; cs < T::NKS; ++cs) {
+        const int col = 32 * cs + j;
+        const uint16_t so = sc_old[col];
+        const int piece = 2 * cs + kb;                       // the lane's 16 columns of its row (operand shape: row j)
+        const RawRow<T::BITS> r = load_row<T::BITS>(blk + swz<Q>(j, piece * LB / 16) + (piece * LB) % 16);
+        float kop[MT];
+#pragma unroll
+        for (int t = 0; t < MT; ++t) kop[t] = key(2 * t + kb, col);
+        const v16i ci = __builtin_amdgcn_mfma_i32_32x32x32_i8(operand<T::BITS>(r), ident, v16i{0}, 0, 0, 0);
+        // exact quotients where the old state is empty or undecayed, as in `fold_tile_v`
+        const bool exact = __builtin_amdgcn_ballot_w64(frozen || so <= 1) != 0;
+        const float se = f16_to_f32(so) * DECODE_UNIT<T::BITS>, c = cm(col);
+        v16f acc;
+#pragma unroll
+        for (int e = 0; e < CPL; ++e) acc[e] = float(ci[e]) * (se * c);
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(dop[t], kop[t], acc, 0, 0, 0);
+        float mx = 0.0f;
+#pragma unroll
+        for (int e = 0; e < CPL; e += 2) mx = fmaxf(fmaxf(mx, fabsf(acc[e])), fabsf(acc[e + 1]));
+        const Pair pm = pair32(mx);
+        const float sc = fp16_scale(fmaxf(pm.lo, pm.hi), T::QMAX);
+        const Divisor d = scale_divisor(sc);
+        if (kb == 0) sc_out[col] = f32_to_f16(sc);
+        // codes, four rows to a word: byte b of word a is row 8 a + 4 kb + b of the lane's column
+        uint32_t cw[4];
+        auto requantize = [&](auto clamp, auto exactly) {
+            uint32_t u[CPL];
+#pragma unroll
+            for (int e = 0; e < CPL; ++e) {
+                float f;
+                if constexpr (decltype(exactly)::value) f = div_rc(acc[e], d.d, d.rc) + MAGIC;
+                else f = __builtin_fmaf(acc[e], d.rc, MAGIC);
+                if constexpr (decltype(clamp)::value) f = __builtin_amdgcn_fmed3f(f, MAGIC - T::QMAX, MAGIC + T::QMAX);
+                u[e] = as_u32(f);
+            }
+#pragma unroll
+            for (int a = 0; a < 4; ++a) cw[a] = pack_low_bytes(u[4 * a], u[4 * a + 1], u[4 * a + 2], u[4 * a + 3]);
+        };
+        // the clamp only where a scale is subnormal (as in `quad_fold_half`)
+        if (exact) requantize(std::true_type{}, std::true_type{});
+        else if (__builtin_amdgcn_ballot_w64(sc < 6.103515625e-05f) != 0) requantize(std::true_type{}, std::false_type{});
+        else requantize(std::false_type{}, std::false_type{});
+        if constexpr (T::BITS == 4) {                        // code + 8 of columns j, j + 1 (j even) as one stored byte
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+                const uint32_t other = as_u32(partner<0>(as_f32(cw[a])));
+                cw[a] = (cw[a] & 0x0F0F0F0Fu) | ((other << 4) & 0xF0F0F0F0u);
+            }
+        }
+        // back to "rows across lanes" through the matrix core: element 4 a + b of lane (n, kb) is row n, column
+        // 32 cs + 8 a + 4 kb + b, so the codes go to LDS in words (int4: half words) instead of single bytes
+        const v16i co = __builtin_amdgcn_mfma_i32_32x32x32_i8(v4i{int(cw[0]), int(cw[1]), int(cw[2]), int(cw[3])}, ident_t,
+                                                              v16i{0}, 0, 0, 0);
+        wave_sync();                                         // every lane has its codes of these columns
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            const int byte = (32 * cs + 8 * a + 4 * kb) * T::BITS / 8;
+            uint8_t* at = blk + swz<Q>(j, byte / 16) + byte % 16;
+            if constexpr (T::BITS == 8)
+                *reinterpret_cast<uint32_t*>(at) = pack_low_bytes(uint32_t(co[4 * a]), uint32_t(co[4 * a + 1]),
+                                                                  uint32_t(co[4 * a + 2]), uint32_t(co[4 * a + 3]));
+            else
+                *reinterpret_cast<uint16_t*>(at) = uint16_t(__builtin_amdgcn_perm(uint32_t(co[4 * a + 2]), uint32_t(co[4 * a]),
+                                                                                  0x0c0c0400u));
+        }
+        wave_sync();
+    }
 }
 
 }  // namespace sq

@@ -1,0 +1,99 @@
+"""The workgroup step kernels against the one-wavefront kernels on the same state, token by token, for the formats and
+shapes at the edges of what the workgroup kernels serve.  Both kinds are held to the oracle elsewhere; here every step
+of one starts from the other's state, so a difference is one step's.
+
+Bounds: the two kinds add the same fp32 products in another order -- outputs within d_k 2^-24 of the largest one (1e-5
+for d_k = 128); a stored or buffered value may come out one step off where it lies within that of a rounding boundary,
+a scale one fp16 number off likewise (1e-4 of them, and the entries of a re-scaled vector)."""
+import pytest
+import torch
+
+import statequant_amd as sq
+from _util import code_diff
+from statequant_amd.kernels import Mamba2SlotLayout, SlotLayout, _hip
+
+pytestmark = pytest.mark.gpu
+DEV = 'cuda'
+
+CASES = [
+    # value-axis groups of one row block: one / two row blocks per wavefront, both buffers, short and long periods
+    ('gdn', (4, 'v', 32), (4, 2, 128, 128), 8, 8), ('gdn', (8, 'v', 32), (4, 2, 128, 128), 8, 8),
+    ('gdn', (4, 'v', 32), (3, 3, 128, 128), 1, 16), ('gdn', (8, 'v', 32), (6, 2, 64, 64), 16, 16),
+    ('gdn', (4, 'v', 32), (4, 2, 64, 64), 4, 8), ('gdn', (8, 'v', 32), (2, 1, 128, 256), 2, 8),
+    ('mamba2', (4, 'v', 32), (8, 2, 128, 64), 8, 8), ('mamba2', (8, 'v', 32), (6, 2, 128, 64), 4, 16),
+    ('mamba2', (8, 'v', 32), (4, 1, 128, 128), 16, 8), ('mamba2', (4, 'v', 32), (3, 3, 64, 64), 1, 8),
+]
+
+
+def _layout(family, fmt, shape, m, bb):
+    hv, hk, dk, dv = shape
+    fmt = fmt if isinstance(fmt, str) else sq.Quantizer(*fmt)
+    cls = {'gdn': SlotLayout, 'mamba2': Mamba2SlotLayout}[family]
+    return cls(fmt, hv, hk, dk, dv, m=m, buffer_bits=bb)
+
+
+def _token(family, gen, rows, shape):
+    hv, hk, dk, dv = shape
+    r = lambda *s: torch.randn(*s, generator=gen).to(DEV)          # noqa: E731
+    if family == 'mamba2':
+        return dict(x=r(rows, hv, dv), dt=r(rows, hv), B=r(rows, hk, dk), C=r(rows, hk, dk))
+    return dict(q=r(rows, hk, dk), k=r(rows, hk, dk), v=r(rows, hv, dv), g=-torch.nn.functional.softplus(r(rows, hv)),
+                beta=torch.sigmoid(r(rows, hv)))
+
+
+def _step(family, lay, V, idx, t, out, model):
+    if family == 'mamba2':
+        lay.step(V, idx, t['x'], t['dt'], t['B'], t['C'], out, *model)
+    else:
+        lay.step(V, idx, t['q'], t['k'], t['v'], out, lay.DK ** -0.5, g=t['g'], beta=t['beta'])
+
+
+@pytest.mark.parametrize('family,fmt,shape,m,bb', CASES)
+def test_group_kernel_matches_the_one_wavefront_kernel(family, fmt, shape, m, bb):
+    hv, hk, dk, dv = shape
+    lay = _layout(family, fmt, shape, m, bb)
+    gen = torch.Generator().manual_seed(5)
+    rows = 7
+    idx = torch.tensor([3, 1, 0, 9, 4, -1, 6], dtype=torch.int32, device=DEV)
+    live = idx > 0
+    blob = lay.alloc(10, DEV)
+    V = lay.views(blob)
+    S0 = torch.randn(rows, hv, dv, dk, generator=gen).to(DEV) * 0.4
+    S0[0] = 0.0                                                     # a fresh sequence: its first fold is the exact one
+    lay.write(V, idx, S0)
+    r = lambda *s: torch.randn(*s, generator=gen).to(DEV)          # noqa: E731
+    model = (-torch.exp(r(hv)), r(hv), r(hv)) if family == 'mamba2' else None
+    codes = off = entries = flips = scales = scales_off = 0
+    for step in range(2 * m + 3):
+        if step == 1 and m > 1:                                     # from here on the sequences are out of step
+            lay.write(V, idx[3:5], S0[3:5])
+        t = _token(family, gen, rows, shape)
+        twin = blob.clone()
+        W = lay.views(twin)
+        outs = [torch.full((rows, hv, dv), 3.0, device=DEV) for _ in range(2)]
+        _step(family, lay, V, idx, t, outs[0], model)
+        _hip.select_instances(no_group_kernel=True)
+        try:
+            _step(family, lay, W, idx, t, outs[1], model)
+        finally:
+            _hip.select_instances()
+        assert torch.equal(outs[0][~live], torch.zeros_like(outs[0][~live]))
+        assert ((outs[0] - outs[1]).abs().max() / outs[1].abs().max()).item() <= 1e-5, step
+        for name in V:
+            a, b = V[name], W[name]
+            if name == 'NPTR':
+                assert torch.equal(a, b)
+            elif name == 'S':
+                mism, far, n = code_diff(a.cpu(), b.cpu(), lay.bits)
+                assert far == 0
+                codes, off = codes + n, off + mism
+            elif name in ('SC', 'KBS', 'UBS'):
+                d = (a.view(torch.int16).int() - b.view(torch.int16).int()).abs()
+                assert d.max().item() <= 1
+                scales, scales_off = scales + d.numel(), scales_off + int((d > 0).sum())
+            elif name in ('KB', 'UB'):
+                entries, flips = entries + a.numel(), flips + int((a != b).sum())
+            else:
+                assert torch.allclose(a, b, rtol=1e-6, atol=1e-7), name
+    assert off <= 1e-4 * codes and scales_off <= 1e-4 * scales + 2, (off, codes, scales_off, scales)
+    assert flips <= 1e-4 * entries + 2 * max(dk, dv), (flips, entries)
