@@ -1,12 +1,12 @@
 #!/usr/bin/env python3
 """Where the life of a workgroup goes: a timeline of one launch of the Gated DeltaNet workgroup-per-key-head step or
-of the KDA one-wavefront step.
+of the KDA step.
 
     python -m statequant_amd.csrc.build --timeline        # once, here: writes statequant_amd/libsqhip_timeline.so
     python profile_timeline.py [--workload gdn-int8-g128 | kda-int4-g32] [--steps 3,7] [--out profiles]
 
 The timeline library is the product library with marks compiled into `gdn_quad_kernel` (sq_gdn_quad.cuh) and
-`kda_step_kernel` (sq_kda.cuh) by -DSQ_TIMELINE (sq_timeline.cuh): every wavefront stores the GPU's 100 MHz
+`kda_quad_kernel` (sq_kda_quad.cuh) by -DSQ_TIMELINE (sq_timeline.cuh): every wavefront stores the GPU's 100 MHz
 real-time counter at 15 (KDA: 9) points of its life.  This script
 builds bench.py's workload, runs whole fold periods back to back (eager launches, the 24 layer states in turn, as
 bench.py does without a graph), and for each requested step of the fold period (0 .. m - 1; the last one folds) has
@@ -44,7 +44,7 @@ def timeline(workload, step, dev, m=8):
     fam, lay, views, idx = bench.build(workload, m, dev)
     inputs, extra = bench.make_inputs(fam, lay, slots, layers, m, dev)
     out = torch.zeros(slots, hv, dv, device=dev, dtype=torch.bfloat16)
-    waves = 4 if fam == 'gdn' else 1                         # GDN: two value heads x two wavefronts; KDA: one per head
+    waves = 4                                                # GDN: two value heads x two wavefronts; KDA: four per head
     nwg = slots * hv // 2 if fam == 'gdn' else slots * hv
     buf = torch.zeros(nwg * waves * 16, dtype=torch.int64, device=dev)
 
@@ -68,7 +68,7 @@ def timeline(workload, step, dev, m=8):
     if not (t[:, :, 0] > 0).all():
         sys.exit(f'profile_timeline.py: {workload} did not run on an instrumented kernel (gdn_quad_kernel serves '
                  'Gated DeltaNet int4 / int8 states with key-axis groups, two value heads per key head; '
-                 'kda_step_kernel every KDA state)')
+                 'kda_quad_kernel int4 / int8 KDA states)')
     return t, nwg, fam
 
 
@@ -94,8 +94,8 @@ def report(workload, step, t, nwg, fam, m=8):
         lines.append('  from the start: ' + ' '.join(f'{d[first][:, :, k].mean():5.2f}' for k in range(last)))
         lines.append('  the others:     ' + ' '.join(f'{d[~first][:, :, k].mean():5.2f}' for k in range(last)))
     if waves > 1:
-        lines.append('mean of each interval by wavefront of the workgroup (1 and 3: q and k vectors; 0 and 2: gates; '
-                     '2: key append):')
+        lines.append('mean of each interval by wavefront of the workgroup (1 and 3: q and k vectors; 0 and 2: gates, KDA '
+                     '0: decays; 2: key append):')
         for w in range(waves):
             lines.append(f'  wavefront {w}: ' + ' '.join(f'{d[:, w, k].mean():5.2f}' for k in range(last)))
     st, en = T[:, 0, 0], T[:, :, last].max(axis=1)

@@ -73,7 +73,7 @@ CASES = _cases()
 GGA_SHAPES = [(128, 128), (64, 64)]                  # (d_k, d_v) of the mixed-width GGA / STEP slot (sq_gga.cuh)
 PARAMS = {'gdn': 'GdnParams', 'kda': 'KdaParams', 'mamba2': 'Mamba2Params'}
 # families with a workgroup-per-key-head kernel (sq_<family>_quad.cuh) -> value heads per workgroup that are built
-QUAD_FAMILIES = {'gdn': (2, 1), 'mamba2': (4, 2, 1)}
+QUAD_FAMILIES = {'gdn': (2, 1), 'mamba2': (4, 2, 1), 'kda': (1,)}
 # compile-time specialisations of the step kernels (SPEC, sq_params.h), most specific first; 0: everything read from
 # the arguments.  Built for the default buffer (int8, 8 tokens) only.
 SPECS = {'gdn': (1, 2, 0), 'kda': (1, 0), 'mamba2': (1, 0)}
@@ -116,6 +116,14 @@ QUAD_OK = {'gdn': [
     '        return reinterpret_cast<uintptr_t>(ptr) % 16 == 0 && (uint64_t(stride) * (dt == 0 ? 4 : 2)) % 16 == 0;',
     '    };',
     '    return ok(p.B, p.s_B, p.B_dt) && ok(p.C, p.s_C, p.C_dt);',
+    '}'],
+    'kda': [
+    '// q, k, g rows that 16-byte vector loads can address',
+    'static bool kda_quad_ok(const KdaParams& p) {',
+    '    auto ok = [](const void* ptr, uint32_t stride, int dt) {',
+    '        return reinterpret_cast<uintptr_t>(ptr) % 16 == 0 && (uint64_t(stride) * (dt == 0 ? 4 : 2)) % 16 == 0;',
+    '    };',
+    '    return ok(p.q, p.s_q, p.q_dt) && ok(p.k, p.s_k, p.k_dt) && ok(p.g, p.s_g, p.g_dt);',
     '}']}
 
 
@@ -133,7 +141,7 @@ def quad_variants(fam, c):
     if not axv and -(-dk // group) > 4:
         return []
     nrb = dv // 32
-    nb = 2 if nrb % 2 == 0 else 1
+    nb = 2 if nrb % 2 == 0 and fam != 'kda' else 1
     be = 1 if qbuf else 2
     out = []
     for gh in QUAD_FAMILIES[fam]:
@@ -141,6 +149,8 @@ def quad_variants(fam, c):
         if nw > 16:
             continue
         lds = gh * dv * rb + mmax * dk * be + gh * mmax * dv * be + 2 * dk * 4 + dk * 8 + 512
+        if fam == 'kda':                                 # keys x decay ratio in fp32 (the raw ones stay in registers), decays
+            lds += mmax * dk * 4 + 2 * dk * 4 + (2 * dk * 4 if axv else 0)
         if axv:                                          # a plane set per wavefront
             lds += nw * dk * 6 - dk * 8
         wgs = min(160 * 1024 // lds, 32 // nw)

@@ -1,0 +1,472 @@
+// KDA packed decode step, one workgroup per (batch row, head): every wavefront owns NB 32-row blocks of the head's state
+// (int4 / int8 codes, key-axis groups or value-axis groups of one row block; geometry and building blocks in
+// sq_quad.cuh).
+//
+// Same arithmetic as the one-wavefront kernel of sq_kda.cuh (the reference's `_kda_step`,
+// /root/reference/src/statequant/kernels/_kda_triton.py:38-149), with A = exp(G_n), G_n = G_{n-1} + g_n per channel:
+//   c_x[i] = sum_j k_i[j] exp(G_n[j] - G_i[j]) x[j];   u = beta (v - S0^T (A k) - sum_i c_k[i] u_i);
+//   o = S0^T (A q) + sum_i c_q[i] u_i + (k.q) u;   fold: S = S0 diag(A) + sum_i u_i (exp(G_n - G_i) k_i)^T
+// KDA has no grouped keys, so a head is a workgroup.  What its one-wavefront kernel does in sequence is dealt out:
+//   issue            every wavefront: its row blocks, scales, its rows of v and of the buffered values, its share of the
+//                    buffered keys with their decays; one wavefront each q and k, both with g and the running decay
+//   roles            q / k normalised, A q / A k as digit planes; G_n and A for all                       [barrier]
+//   per wavefront    its row blocks' read-outs; c_q, c_k of its share of the slots                        [barrier]
+//                    buffer term, u, o of its rows; max |u|; one wavefront each: the key, the decays      [barrier]
+//                    append;  with a full buffer: fold of its row blocks out of LDS (one read of the codes)
+// One row block per wavefront (NB = 1, four wavefronts for d_v 128): two per wavefront measured the same at 128
+// sequences and 3 % faster at 256 (int4), but a third slower at 16 and slower everywhere on int8.
+// us per launch, one wavefront per head -> this (32 heads of 128 x 128, sequences out of step): int4 g32 1 sequence
+// 6.7 -> 4.5, 16: 16.7 -> 7.8, 128: 25.5 -> 20.6, 256: 36.6 -> 35.8; int8 g32 1: 7.8 -> 4.6, 256: 59.0 -> 43.4;
+// value-axis int4 128: 33.6 -> 22.1, int8 256: 60.0 -> 45.0.  Bound at small batches by the chain of a head's life, at
+// large ones by the vector ALU (491 instructions per wavefront, 13 of 20.6 us of issue at 128 sequences, int4).
+#pragma once
+#include "sq_gdn_quad.cuh"
+#include "sq_kda.cuh"
+
+namespace sq {
+
+template <class T, class Q>
+struct KdaLoads {
+    uint16_t sc[Q::NB][T::NG];             // scales of rows (block bi, lane % 32)
+    uint32_t scv[Q::NB];                   // value-axis groups: the block's scales of columns NE lane ..
+    Raw4<T::QBUF> uraw[Q::UT], kraw[Q::KT];
+    float4 gb[Q::KT];                      // cumulative decays beside kraw
+    uint16_t kbs[Q::KT], ubs;
+    int np;
+    uint32_t xr[Q::NE], xr2[Q::NE], gr[Q::NE], beta, vr;
+    float gc[Q::NE];
+};
+
+template <class T, int NB>
+struct KdaLds {
+    using Q = Quad<T, NB, 1>;
+    using B = QuadLds<T, NB, 1, 2, 2>;                               // read-out vectors: q, k (normalised)
+    static constexpr int GN = B::BYTES;                              // [DK] G_n
+    static constexpr int CM = GN + T::DK * 4;                        // [DK] A = exp(G_n)
+    static constexpr int XA = CM + T::DK * 4;                        // [2][DK] A q, A k (value-axis groups: planes per block)
+    static constexpr int KD = XA + (T::AXV ? 2 * T::DK * 4 : 0);     // [m][DK] buffered keys x decay ratio, fp32
+    static constexpr int BYTES = KD + T::MMAX * T::DK * 4;
+};
+
+// SPEC = 1: the serving case compiled in -- bf16 q / k / v / out, fp32 g and beta, a power-of-two head count.
+template <class T, int NB, int WPE, int SPEC>
+__global__ __launch_bounds__((Quad<T, NB, 1>::THREADS), WPE)
+void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict__ order, int per_xcd, int hv, int hv_shift,
+                     const uint8_t* codes, uint32_t codes_stride, const int32_t* counters, uint32_t counters_stride,
+                     uint32_t start_ramp, SQ_TL_PARAM const KdaParams p) {
+    SQ_MARK(0);                                                   // entry
+    constexpr bool FIX = SPEC > 0;
+    const int q_dt = FIX ? int(BF16) : p.q_dt, k_dt = FIX ? int(BF16) : p.k_dt, v_dt = FIX ? int(BF16) : p.v_dt;
+    const int out_dt = FIX ? int(BF16) : p.out_dt, g_dt = FIX ? int(F32) : p.g_dt, beta_dt = FIX ? int(F32) : p.beta_dt;
+    using Q = Quad<T, NB, 1>;
+    using L = QuadLds<T, NB, 1, 2, 2>;
+    using K = KdaLds<T, NB>;
+    constexpr int DK = T::DK, DV = T::DV, NW = Q::NW, MM = T::MMAX, NE = Q::NE, NG = T::NG;
+    constexpr int RQ = 1 % NW, RK = 3 % NW, RX = 2 % NW, RG = 0;  // which wavefront plays which shared role
+    __shared__ __attribute__((aligned(16))) uint8_t lds[K::BYTES];
+    float* lds_xn = reinterpret_cast<float*>(lds + L::XN);
+    uint8_t* lds_pl = lds + L::PL;
+    float* lds_xs = reinterpret_cast<float*>(lds + L::XS);
+    float* lds_dots = reinterpret_cast<float*>(lds + L::DOTS);
+    float* lds_red = reinterpret_cast<float*>(lds + L::RED);
+    float* lds_scal = reinterpret_cast<float*>(lds + L::SCAL);
+    uint8_t* lds_ubr = lds + L::UBR;
+    float* lds_ubsf = reinterpret_cast<float*>(lds + L::UBSF);
+    uint16_t* lds_sc = reinterpret_cast<uint16_t*>(lds + L::SC);
+    float* lds_gn = reinterpret_cast<float*>(lds + K::GN);
+    float* lds_cm = reinterpret_cast<float*>(lds + K::CM);
+    float* lds_xa = reinterpret_cast<float*>(lds + K::XA);
+    float* lds_kd = reinterpret_cast<float*>(lds + K::KD);
+
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+    const int m = p.m;
+    const uint32_t um = m;
+    uint8_t* my_codes = lds + L::CODES + w * NB * Q::BLK;
+    static_assert((WAVE / Q::CPR) % (Q::SWD * Q::SWM) == 0 || Q::NLD == 1, "swizzle period");
+
+    const TileId tid = tile_id_lead<SPEC>(order, per_xcd, hv, hv_shift);
+    const uint32_t b = tid.b, h = tid.h;
+    const int32_t slot = idx ? idx[b] : int32_t(b);
+    const int n32 = lane & 31, kb = lane >> 5;
+    // the row of the head this lane finishes after the pass (NB = 2: the wavefront's halves take a block each)
+    const int row = (w * NB + (NB == 2 ? kb : 0)) * T::MR + n32;
+
+    KdaLoads<T, Q> F;
+    // ---- issue every load: first the token's own operands (their addresses need the batch row only) ...
+    if (w == RQ)
+        load_vec<NE>(advance(p.q, q_dt, uint64_t(b) * p.s_q + h * DK), q_dt, lane, F.xr);
+    if (w == RK)
+        load_vec<NE>(advance(p.k, k_dt, uint64_t(b) * p.s_k + h * DK), k_dt, lane, RQ == RK ? F.xr2 : F.xr);
+    if (w == RQ || w == RK) load_vec<NE>(advance(p.g, g_dt, uint64_t(b) * p.s_g + h * DK), g_dt, lane, F.gr);
+    F.beta = load_raw_uniform(p.beta, beta_dt, uint64_t(b) * p.s_beta + h);
+    F.vr = load_raw(advance(p.v, v_dt, uint64_t(b) * p.s_v + h * DV), v_dt, uint32_t(row));
+    void* const outp = advance(p.out, out_dt, uint64_t(b) * p.s_out + h * DV);
+    if (idx && slot <= 0) {                              // padding row: zero output, touch nothing of a slot
+        for (int r = w * WAVE + lane; r < DV; r += NW * WAVE) store_f(outp, out_dt, r, 0.0f);
+        return;
+    }
+    SQ_MARK(1);                                                   // slot known, the token's loads issued
+    const uint32_t seq = slot;
+    float* const gch = field(p.st.GCUR, seq, p.st.sGC, h * DK);
+    if (w == RQ || w == RK) {                            // the running decay, ahead of the row blocks: the roles wait for it
+#pragma unroll
+        for (int t = 0; t < NE; ++t) F.gc[t] = gch[NE * lane + t];
+    }
+    // ... then the row blocks, straight into their LDS image, and the fill counter (a scalar load; sq_quad.cuh) ...
+    quad_start_wait<Q, WPE>(start_ramp);
+    quad_dma_blocks<Q, NB>(field(codes, seq, codes_stride, h * (DV * T::ROW_BYTES)) + w * NB * Q::BLK, my_codes, lane);
+    F.np = quad_dma_counter(field(counters, seq, counters_stride, h));
+    __builtin_amdgcn_sched_barrier(0);
+    // ... and the rest of the slot: scales and -- once the fill counter is here -- the live part of the decode buffer
+    uint8_t* const Sh = field(p.st.S, seq, p.st.sS, h * (DV * T::ROW_BYTES));
+    uint16_t* const SCh = field(p.st.SC, seq, p.st.sSC, h * T::SC_ELEMS);
+    BufAddr<T> buf;
+    buf.KB = p.st.KB + (uint64_t(seq) * p.st.sKB + h * um * DK) * T::BE;
+    buf.UB = p.st.UB + (uint64_t(seq) * p.st.sUB + h * um * DV) * T::BE;
+    buf.KBS = field(p.st.KBS, seq, p.st.sKBS, h * um);
+    buf.UBS = field(p.st.UBS, seq, p.st.sUBS, h * um);
+    float* const GBh = field(p.st.GB, seq, p.st.sGB, h * um * DK);
+#pragma unroll
+    for (int bi = 0; bi < NB; ++bi) {
+        if constexpr (T::AXV) {
+            F.scv[bi] = quad_load_colscales<NE>(SCh + (w * NB + bi) * DK, lane);
+        } else {
+#pragma unroll
+            for (int g = 0; g < NG; ++g) F.sc[bi][g] = stream_load(SCh + uint32_t(((w * NB + bi) * T::MR + n32) * NG + g));
+        }
+    }
+    quad_dma_counter_wait(F.np);
+    const uint32_t nfill = uint32_t(F.np & (m - 1));
+    const uint32_t nl = nfill > 0 ? nfill : 1u;
+#pragma unroll
+    for (int t = 0; t < Q::UT; ++t) {                    // lane (slot = lane / LU + SU t, rows 4 (lane % LU) ..)
+        const uint32_t i = lane / Q::LU + Q::SU * t;
+        const uint32_t ic = i < nl ? i : nl - 1;
+        F.uraw[t] = stream_raw4<T::QBUF>(buf.UB + (ic * DV + w * Q::RW + 4 * (lane % Q::LU)) * T::BE);
+    }
+#pragma unroll
+    for (int t = 0; t < Q::KT; ++t) {                    // lane (slot = SPP (NW t + w) + lane / LPS, columns 4 (lane % LPS) ..)
+        const uint32_t i = Q::SPP * (NW * t + w) + lane / Q::LPS;
+        const uint32_t ic = i < nl ? i : nl - 1;
+        F.kraw[t] = stream_raw4<T::QBUF>(buf.KB + (ic * DK + 4 * (lane % Q::LPS)) * T::BE);
+        typedef float v4fl __attribute__((ext_vector_type(4)));
+        const v4fl g4 = stream_load(reinterpret_cast<const v4fl*>(GBh + ic * DK + 4 * (lane % Q::LPS)));
+        F.gb[t] = make_float4(g4.x, g4.y, g4.z, g4.w);
+        F.kbs[t] = T::QBUF ? buf.KBS[ic] : uint16_t(0);
+    }
+    F.ubs = T::QBUF ? buf.UBS[uint32_t(lane) < nl ? lane : 0] : uint16_t(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    SQ_MARK(2);                                                   // fill count here, every load issued
+
+    // ---- roles: q and k normalised, times A the read-out vectors of the stored state; G_n, A ----
+    auto role_vector = [&](const uint32_t (&raw)[NE], int dt, float post, int v) {
+        float xe[NE], xa[NE], ss = 0.0f;
+#pragma unroll
+        for (int t = 0; t < NE; ++t) {
+            xe[t] = vec_elem<NE>(raw, dt, t);
+            ss = __builtin_fmaf(xe[t], xe[t], ss);
+        }
+        const float nrm = sqrtf(lanes_sum<WAVE>(ss) + 1e-6f);
+#pragma unroll
+        for (int t = 0; t < NE; ++t) {
+            xe[t] = xe[t] / nrm * post;
+            const float gn = F.gc[t] + vec_elem<NE>(F.gr, g_dt, t);
+            const float A = kda_exp(gn);
+            xa[t] = A * xe[t];
+            lds_xn[v * DK + NE * lane + t] = xe[t];
+            if (v == 0) {
+                lds_gn[NE * lane + t] = gn;
+                lds_cm[NE * lane + t] = A;
+            }
+            if constexpr (T::AXV) lds_xa[v * DK + NE * lane + t] = xa[t];
+        }
+        if constexpr (!T::AXV) quad_stage_planes<Q, T, NE>(xa, v, lane, lds_pl, lds_xs);
+    };
+    if (w == RQ) role_vector(F.xr, q_dt, p.scale, 0);
+    if (w == RK) role_vector(RQ == RK ? F.xr2 : F.xr, k_dt, 1.0f, 1);
+    // ---- the loads land ----
+    const int n = F.np & (m - 1);
+    const bool full = n == m - 1;
+    uint16_t scw[NB][NG];
+#pragma unroll
+    for (int bi = 0; bi < NB; ++bi) {
+        if constexpr (!T::AXV) {
+#pragma unroll
+            for (int g = 0; g < NG; ++g) {
+                scw[bi][g] = F.sc[bi][g];
+                if (kb == 0) lds_sc[((w * NB + bi) * T::MR + n32) * NG + g] = F.sc[bi][g];
+            }
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < Q::UT; ++t) {
+        const int i = lane / Q::LU + Q::SU * t;
+        if (i < m) store_raw4<T::QBUF>(lds_ubr + (i * DV + w * Q::RW + 4 * (lane % Q::LU)) * T::BE, F.uraw[t]);
+    }
+    if (w == RG && T::QBUF && lane < m) lds_ubsf[lane] = f16_to_f32(F.ubs);
+    quad_dma_landed();                                             // the row blocks are in LDS
+    SQ_MARK(3);                                                   // vectors, scales, buffered values here and staged
+    lds_barrier();
+
+    // ---- c_q, c_k of this wavefront's share of the slots: the decay ratio rides on the key ----
+    {
+        float x[2][4], gn[4];
+        const int c4 = 4 * (lane % Q::LPS);
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+            const float4 f = *reinterpret_cast<const float4*>(lds_xn + v * DK + c4);
+            x[v][0] = f.x; x[v][1] = f.y; x[v][2] = f.z; x[v][3] = f.w;
+        }
+        {
+            const float4 f = *reinterpret_cast<const float4*>(lds_gn + c4);
+            gn[0] = f.x; gn[1] = f.y; gn[2] = f.z; gn[3] = f.w;
+        }
+#pragma unroll
+        for (int t = 0; t < Q::KT; ++t) {
+            const int i = Q::SPP * (NW * t + w) + lane / Q::LPS;
+            const bool alive = i < n;                              // dead slots may hold anything: discard
+            float kf[4];
+            decode_raw4<T::QBUF>(F.kraw[t], kf);
+            const float ks = f16_to_f32(F.kbs[t]);
+            const float gi[4] = {F.gb[t].x, F.gb[t].y, F.gb[t].z, F.gb[t].w};
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                if constexpr (T::QBUF) kf[c] = kf[c] * ks;
+                kf[c] = alive ? kf[c] * kda_exp(gn[c] - gi[c]) : 0.0f;
+            }
+            if (full && i < n) *reinterpret_cast<float4*>(lds_kd + i * DK + c4) = make_float4(kf[0], kf[1], kf[2], kf[3]);
+#pragma unroll
+            for (int v = 0; v < 2; ++v) {
+                float pr = kf[0] * x[v][0];
+#pragma unroll
+                for (int c = 1; c < 4; ++c) pr = __builtin_fmaf(kf[c], x[v][c], pr);
+                pr = lanes_sum<Q::LPS>(pr);
+                if (lane % Q::LPS == 0 && i < MM) lds_dots[v * MM + i] = pr;
+            }
+        }
+    }
+    if (w == RK) {                                                // k . q
+        float kqp = 0.0f;
+#pragma unroll
+        for (int t = 0; t < NE; ++t) kqp = __builtin_fmaf(lds_xn[DK + NE * lane + t], lds_xn[NE * lane + t], kqp);
+        kqp = lanes_sum<WAVE>(kqp);
+        if (lane == 0) lds_scal[0] = kqp;
+    }
+    SQ_MARK(4);                                                   // buffered keys and decays here, coefficients done
+    // ---- state pass against A q, A k ----
+    float sq, sk;
+    {
+        float own[NB];
+        if constexpr (T::AXV) {
+#pragma unroll
+            for (int bi = 0; bi < NB; ++bi)
+                own[bi] = quad_block_pass_v<Q, T, 2>(my_codes + bi * Q::BLK, lds_xa, F.scv[bi], lds_pl + w * L::PL_BYTES,
+                                                     lds_xs + w * (L::XS_BYTES / 4), lane);
+        } else {
+            v4i aop[T::NKS];
+            quad_fetch_planes<Q, T, 2>(lds_pl, lane, aop);
+            float xs[NG];
+#pragma unroll
+            for (int g = 0; g < NG; ++g) xs[g] = lds_xs[kb * NG + g];
+#pragma unroll
+            for (int bi = 0; bi < NB; ++bi) {
+                float sc[NG];
+#pragma unroll
+                for (int g = 0; g < NG; ++g) sc[g] = f16_to_f32(scw[bi][g]);
+                own[bi] = quad_block_pass<Q, T>(my_codes + bi * Q::BLK, aop, xs, sc, lane);
+            }
+        }
+        if constexpr (NB == 2) {                         // lane (n, kb) takes over row n of block kb: both sums
+            const auto r = __builtin_amdgcn_permlane32_swap(as_u32(own[0]), as_u32(own[1]), false, false);
+            sq = as_f32(r[0]);
+            sk = as_f32(r[1]);
+        } else {
+            const Pair qk = pair32(own[0]);
+            sq = qk.lo;
+            sk = qk.hi;
+        }
+    }
+    SQ_MARK(5);                                                   // state pass done
+    lds_barrier();
+
+    // ---- append the key (its decay ratio within this buffer is 1) and the decays ----
+    if (w == RX) {
+        float kxe[NE], kmax = 0.0f;
+#pragma unroll
+        for (int t = 0; t < NE; ++t) {
+            kxe[t] = lds_xn[DK + NE * lane + t];
+            kmax = fmaxf(kmax, fabsf(kxe[t]));
+        }
+        float ks = 1.0f;
+        if constexpr (T::QBUF) ks = fp16_scale(lanes_max<WAVE>(kmax), 127.0f);
+        if (T::QBUF && lane == 0) buf.KBS[n] = f32_to_f16(ks);
+        uint32_t pk = 0;
+#pragma unroll
+        for (int t = 0; t < NE; ++t) {
+            float kr;
+            if constexpr (T::QBUF) {
+                const float c = round_buf(kxe[t], ks);
+                kr = c * ks;
+                pk |= (uint32_t(int(c)) & 0xFFu) << (8 * t);
+            } else {
+                const uint16_t hb = f32_to_bf16(kxe[t]);
+                kr = bf16_to_f32(hb);
+                reinterpret_cast<uint16_t*>(buf.KB)[n * DK + NE * lane + t] = hb;
+            }
+            if (full) lds_kd[n * DK + NE * lane + t] = kr;
+        }
+        if constexpr (T::QBUF) {
+            uint8_t* dg = buf.KB + n * DK + NE * lane;
+            if constexpr (NE == 1) *dg = uint8_t(pk);
+            else if constexpr (NE == 2) *reinterpret_cast<uint16_t*>(dg) = uint16_t(pk);
+            else *reinterpret_cast<uint32_t*>(dg) = pk;
+        }
+    }
+    if (w == RG) {
+#pragma unroll
+        for (int t = 0; t < NE; ++t) {
+            const float gn = lds_gn[NE * lane + t];
+            GBh[n * DK + NE * lane + t] = gn;
+            gch[NE * lane + t] = full ? 0.0f : gn;
+        }
+    }
+    // ---- this wavefront's rows: buffer term, u, o ----
+    const float kq = lds_scal[0], beta = raw_to_f(F.beta, beta_dt);
+    float cq, ck;
+    {
+        const int li = lane < m ? lane : 0;
+        const float us_i = T::QBUF ? lds_ubsf[li] : 1.0f;
+        const float dq = lds_dots[li], dk_ = lds_dots[MM + li];
+        const bool alive = lane < n;
+        cq = alive ? (T::QBUF ? dq * us_i : dq) : 0.0f;
+        ck = alive ? (T::QBUF ? dk_ * us_i : dk_) : 0.0f;
+    }
+    float uv[MM];
+#pragma unroll
+    for (int i = 0; i < MM; ++i) uv[i] = lds_raw<T::QBUF>(lds_ubr, (i < m ? i : 0) * DV + row);
+    float accq = sq, acck = sk;
+#pragma unroll
+    for (int i = 0; i < MM; ++i) {
+        const float u_i = T::QBUF ? uv[i] : (i < n ? uv[i] : 0.0f);
+        accq = __builtin_fmaf(u_i, lane_bcast(cq, i), accq);
+        acck = __builtin_fmaf(u_i, lane_bcast(ck, i), acck);
+    }
+    const float u = beta * (raw_to_f(F.vr, v_dt) - acck);
+    const float o = __builtin_fmaf(kq, u, accq);
+    if (NB == 2 || kb == 0) store_f(outp, out_dt, row, o);
+    SQ_MARK(6);                                                   // outputs stored
+    float us = 1.0f;
+    if constexpr (T::QBUF) {
+        float amax = lanes_max<WAVE>(fabsf(u));
+        if constexpr (NW > 1) {
+            if (lane == 0) lds_red[w] = amax;
+            lds_barrier();
+#pragma unroll
+            for (int ww = 0; ww < NW; ++ww) amax = fmaxf(amax, lds_red[ww]);
+        }
+        us = fp16_scale(amax, 127.0f);
+        if (w == RG && lane == 0) { buf.UBS[n] = f32_to_f16(us); lds_ubsf[n] = us; }
+    }
+    if (NB == 2 || kb == 0) {
+        if constexpr (T::QBUF) {
+            const int8_t c = int8_t(int(round_buf(u, us)));
+            reinterpret_cast<int8_t*>(buf.UB)[n * DV + row] = c;
+            reinterpret_cast<int8_t*>(lds_ubr)[n * DV + row] = c;
+        } else {
+            const uint16_t hb = f32_to_bf16(u);
+            reinterpret_cast<uint16_t*>(buf.UB)[n * DV + row] = hb;
+            reinterpret_cast<uint16_t*>(lds_ubr)[n * DV + row] = hb;
+        }
+    }
+    if (w == RG && lane == 0) *field(p.st.NPTR, seq, p.st.sN, h) = full ? 0 : n + 1;
+    SQ_MARK(7);                                                   // appended, counter advanced
+    // ---- fold ----
+    if (full) {
+        lds_barrier();
+        int lf = lane;                                   // (offsets derived anew: see the GDN kernel)
+        asm volatile("" : "+v"(lf));
+        const int swzf = swz<Q>(lf / Q::CPR, lf % Q::CPR);
+        if constexpr (T::AXV) {
+            constexpr int MT = (MM + 1) / 2;
+            const int fj = lf & 31, fkb = lf >> 5;
+            auto key = [&](int sl, int col) {
+                const float kv = lds_kd[(sl < m ? sl : 0) * DK + col];
+                return sl < m ? kv : 0.0f;
+            };
+            auto cm = [&](int col) { return lds_cm[col]; };
+#pragma unroll
+            for (int bi = 0; bi < NB; ++bi) {
+                uint8_t* blk = my_codes + bi * Q::BLK;
+                const int grp = w * NB + bi;
+                uint16_t* old = reinterpret_cast<uint16_t*>(lds_pl + w * L::PL_BYTES);      // the planes are done with
+                quad_store_colscales<NE>(old, lf, F.scv[bi]);
+                wave_sync();
+                float dop[MT];
+#pragma unroll
+                for (int t = 0; t < MT; ++t) {
+                    const int sl = 2 * t + fkb;
+                    const int sc_ = sl < m ? sl : 0;
+                    float uv_ = lds_raw<T::QBUF>(lds_ubr, sc_ * DV + grp * T::MR + fj);
+                    if constexpr (T::QBUF) uv_ = uv_ * lds_ubsf[sc_];
+                    dop[t] = sl < m ? uv_ : 0.0f;
+                }
+                quad_fold_block_v<Q, T>(blk, key, dop, cm, false, old, SCh + grp * DK, lf);
+#pragma unroll
+                for (int t = 0; t < Q::NLD; ++t)
+                    stream_store(reinterpret_cast<v4u*>(Sh + grp * Q::BLK + t * 1024 + lf * 16),
+                                 *reinterpret_cast<const v4u*>(blk + t * 1024 + swzf));
+            }
+        } else {
+            constexpr int MT4 = (MM + 3) / 4, CL = DK / 4;
+            const int fn = lf & 15, fq = lf >> 4;
+            const int fg = (fq * CL) / T::KGROUP;
+            FoldKeys<T, true> kop;
+            quad_fold_keys_f32<T>(lds_kd, m, lf, kop);
+#pragma unroll
+            for (int bi = 0; bi < NB; ++bi) {
+                uint8_t* blk = my_codes + bi * Q::BLK;
+#pragma unroll
+                for (int hf = 0; hf < 2; ++hf) {
+                    const int frow = (w * NB + bi) * T::MR + 16 * hf + fn;
+                    float bop[MT4];
+#pragma unroll
+                    for (int t = 0; t < MT4; ++t) {
+                        const int sl = 4 * t + fq;
+                        const int sc_ = sl < m ? sl : 0;
+                        float uv_ = lds_raw<T::QBUF>(lds_ubr, sc_ * DV + frow);
+                        if constexpr (T::QBUF) uv_ = uv_ * lds_ubsf[sc_];
+                        bop[t] = sl < m ? uv_ : 0.0f;
+                    }
+                    quad_fold_half<Q, T, true>(blk, hf, kop, bop, 1.0f, f16_to_f32(lds_sc[frow * NG + fg]),
+                                               SCh + frow * NG + fg, lf, lds_cm);
+                }
+                wave_sync();
+#pragma unroll
+                for (int t = 0; t < Q::NLD; ++t)
+                    stream_store(reinterpret_cast<v4u*>(Sh + (w * NB + bi) * Q::BLK + t * 1024 + lf * 16),
+                                 *reinterpret_cast<const v4u*>(blk + t * 1024 + swzf));
+            }
+        }
+    }
+    SQ_MARK(8);                                                   // folded (a full buffer)
+}
+
+template <class T, int NB, int GH, int WPE, int SPEC>
+int launch_kda_quad(const KdaParams& p, hipStream_t stream) {
+    static_assert(GH == 1, "no grouped keys");
+    const uint32_t grid = uint32_t(p.rows) * uint32_t(p.hv);
+    using Q = Quad<T, NB, 1>;
+#ifdef SQ_TIMELINE
+    const SqTimelineBuf tl = sq_timeline_buffer();
+    hipLaunchKernelGGL((kda_quad_kernel<T, NB, WPE, SPEC>), dim3(grid), dim3(Q::THREADS), quad_lds_pad(), stream, p.idx,
+                       p.order, p.per_xcd, p.hv, p.hv_shift, p.st.S, p.st.sS, p.st.NPTR, p.st.sN, 0u, tl.p, tl.cap, p);
+#else
+    hipLaunchKernelGGL((kda_quad_kernel<T, NB, WPE, SPEC>), dim3(grid), dim3(Q::THREADS), quad_lds_pad(), stream, p.idx,
+                       p.order, p.per_xcd, p.hv, p.hv_shift, p.st.S, p.st.sS, p.st.NPTR, p.st.sN, 0u, p);
+#endif
+    return int(hipGetLastError());
+}
+
+}  // namespace sq

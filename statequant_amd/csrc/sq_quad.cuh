@@ -398,10 +398,11 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 // int4 states with the int8 buffer, whose kernels run at 80 registers where 16 more long-lived ones made the compiler
 // shuffle and spill -- as the raw bytes (biased to unsigned, four per register) with the slot's scale, expanded where
 // they are used: (byte - 128) x scale in one conversion and one fma, the same number as the product it replaces.
-template <class T>
+// F32: the keys are not the buffered ones (KDA folds a decay per column into them) and come as fp32.
+template <class T, bool F32 = false>
 struct FoldKeys {
     static constexpr int MT4 = (T::MMAX + 3) / 4, NT = T::DK / 16;
-    static constexpr bool PACKED = T::BITS == 4 && T::QBUF && NT % 4 == 0;
+    static constexpr bool PACKED = !F32 && T::BITS == 4 && T::QBUF && NT % 4 == 0;
     float f[PACKED ? 1 : NT][PACKED ? 1 : MT4];
     uint32_t raw[PACKED ? MT4 : 1][PACKED ? NT / 4 : 1];
     float ks[PACKED ? MT4 : 1], off[PACKED ? MT4 : 1];
@@ -444,10 +445,28 @@ __device__ __forceinline__ void quad_fold_keys(const uint8_t* lds_kbr, const flo
     }
 }
 
-template <class Q, class T>
-__device__ __forceinline__ void quad_fold_half(uint8_t* blk, int hf, const FoldKeys<T>& kop,
+// The same from fp32 keys in LDS, [m][DK].
+template <class T>
+__device__ __forceinline__ void quad_fold_keys_f32(const float* lds_kd, int m, int lane, FoldKeys<T, true>& kop) {
+    constexpr int MT4 = (T::MMAX + 3) / 4, CL = T::DK / 4, NT = CL / 4;
+    const int n = lane & 15, q = lane >> 4;
+    const int kcol = (n >> 2) * CL + (n & 3);
+#pragma unroll
+    for (int t = 0; t < MT4; ++t) {
+        const int slot = 4 * t + q;
+#pragma unroll
+        for (int ct = 0; ct < NT; ++ct) {
+            const float kv = lds_kd[(slot < m ? slot : 0) * T::DK + kcol + 4 * ct];
+            kop.f[ct][t] = slot < m ? kv : 0.0f;
+        }
+    }
+}
+
+// COLVEC: the old state decays per column -- `lds_cm` [DK] fp32 in the place of the scalar `cmul`.
+template <class Q, class T, bool COLVEC = false>
+__device__ __forceinline__ void quad_fold_half(uint8_t* blk, int hf, const FoldKeys<T, COLVEC>& kop,
                                                const float (&bop)[(T::MMAX + 3) / 4], float cmul, float s_old,
-                                               uint16_t* sc_out, int lane) {
+                                               uint16_t* sc_out, int lane, const float* lds_cm = nullptr) {
     constexpr int MT4 = (T::MMAX + 3) / 4;
     constexpr int CL = T::DK / 4;                            // columns per lane
     constexpr int NT = CL / 4;                               // accumulator tiles per lane
@@ -475,7 +494,7 @@ __device__ __forceinline__ void quad_fold_half(uint8_t* blk, int hf, const FoldK
     }
     // dequantize: (code x scale) x factor, one conversion + one fma per code
     const float s = T::BITS == 8 ? s_old : s_old * 0.0625f;
-    const float sm = s * cmul;
+    const float sm = COLVEC ? s : s * cmul;
     const float off = -128.0f * sm;
     v4f acc[NT];
     // int8 with one scale group per row: the whole half block is folded in units of the row's old scale x decay
@@ -483,12 +502,12 @@ __device__ __forceinline__ void quad_fold_half(uint8_t* blk, int hf, const FoldK
     // ALU -- they enter the accumulators through the matrix core: each byte, biased to unsigned, becomes the fp16
     // number 1024 + byte by a byte permute (exponent byte 0x64 on top), and one v_mfma_f32_16x16x16_f16 against the
     // 16 x 16 identity hands every lane its own four numbers back as fp32 on top of the constant -1152 (exact).
-    constexpr bool UNITS = T::BITS == 8 && T::NG == 1;
+    constexpr bool UNITS = T::BITS == 8 && T::NG == 1 && !COLVEC;
     // An old scale at its floor is an empty group (or one too small to matter), and a decay of exactly 1 leaves the
     // stored codes times their scale as they are: what is quantized then is a sum of a few products of low-precision
     // numbers, whose quotients by the new scale are exact half-integers by the thousand -- the codes are taken as
     // rint of the IEEE quotient there (quantize_row<.., EXACT>), which sends them to even as the reference's do.
-    const bool exact = __builtin_amdgcn_ballot_w64(s_old <= FP16_TINY || cmul == 1.0f) != 0;
+    const bool exact = __builtin_amdgcn_ballot_w64(s_old <= FP16_TINY || (!COLVEC && cmul == 1.0f)) != 0;
     float unit = 1.0f;                                       // what one accumulator unit is worth
     if constexpr (UNITS) {
         typedef _Float16 v4h __attribute__((ext_vector_type(4)));
@@ -531,6 +550,14 @@ __device__ __forceinline__ void quad_fold_half(uint8_t* blk, int hf, const FoldK
             acc[2 * d][2] = ubyte_fma<1>(lo, sm, off); acc[2 * d][3] = ubyte_fma<1>(hi, sm, off);
             acc[2 * d + 1][0] = ubyte_fma<2>(lo, sm, off); acc[2 * d + 1][1] = ubyte_fma<2>(hi, sm, off);
             acc[2 * d + 1][2] = ubyte_fma<3>(lo, sm, off); acc[2 * d + 1][3] = ubyte_fma<3>(hi, sm, off);
+        }
+    }
+    if constexpr (COLVEC) {
+#pragma unroll
+        for (int ct = 0; ct < NT; ++ct) {
+            const float4 c = *reinterpret_cast<const float4*>(lds_cm + q * CL + 4 * ct);
+            acc[ct][0] = acc[ct][0] * c.x; acc[ct][1] = acc[ct][1] * c.y;
+            acc[ct][2] = acc[ct][2] * c.z; acc[ct][3] = acc[ct][3] * c.w;
         }
     }
     // the m rank-1 updates: first operand = keys (result row i = 4 q' + b <-> column q' CL + 4 ct + b), second = values

@@ -10,7 +10,7 @@ import torch
 
 import statequant_amd as sq
 from _util import code_diff
-from statequant_amd.kernels import Mamba2SlotLayout, SlotLayout, _hip
+from statequant_amd.kernels import KDASlotLayout, Mamba2SlotLayout, SlotLayout, _hip
 
 pytestmark = pytest.mark.gpu
 DEV = 'cuda'
@@ -22,12 +22,19 @@ CASES = [
     ('gdn', (4, 'v', 32), (4, 2, 64, 64), 4, 8), ('gdn', (8, 'v', 32), (2, 1, 128, 256), 2, 8),
     ('mamba2', (4, 'v', 32), (8, 2, 128, 64), 8, 8), ('mamba2', (8, 'v', 32), (6, 2, 128, 64), 4, 16),
     ('mamba2', (8, 'v', 32), (4, 1, 128, 128), 16, 8), ('mamba2', (4, 'v', 32), (3, 3, 64, 64), 1, 8),
+    # KDA: one to eight wavefronts per head, key- and value-axis groups
+    ('kda', (4, 'k', 32), (3, 3, 128, 128), 8, 8), ('kda', (8, 'k', 128), (2, 2, 128, 128), 8, 16),
+    ('kda', (8, 'k', 32), (5, 5, 64, 32), 4, 8), ('kda', (4, 'k', 64), (2, 2, 64, 64), 16, 16),
+    ('kda', (8, 'k', 64), (2, 2, 128, 256), 1, 8), ('kda', (4, 'v', 32), (3, 3, 128, 128), 8, 8),
+    ('kda', (8, 'v', 32), (2, 2, 128, 128), 16, 16), ('kda', (8, 'v', 32), (3, 3, 64, 32), 2, 8),
 ]
 
 
 def _layout(family, fmt, shape, m, bb):
     hv, hk, dk, dv = shape
     fmt = fmt if isinstance(fmt, str) else sq.Quantizer(*fmt)
+    if family == 'kda':
+        return KDASlotLayout(fmt, hv, dk, dv, m=m, buffer_bits=bb)
     cls = {'gdn': SlotLayout, 'mamba2': Mamba2SlotLayout}[family]
     return cls(fmt, hv, hk, dk, dv, m=m, buffer_bits=bb)
 
@@ -37,13 +44,16 @@ def _token(family, gen, rows, shape):
     r = lambda *s: torch.randn(*s, generator=gen).to(DEV)          # noqa: E731
     if family == 'mamba2':
         return dict(x=r(rows, hv, dv), dt=r(rows, hv), B=r(rows, hk, dk), C=r(rows, hk, dk))
-    return dict(q=r(rows, hk, dk), k=r(rows, hk, dk), v=r(rows, hv, dv), g=-torch.nn.functional.softplus(r(rows, hv)),
+    g = r(rows, hv, dk) if family == 'kda' else r(rows, hv)
+    return dict(q=r(rows, hk, dk), k=r(rows, hk, dk), v=r(rows, hv, dv), g=-torch.nn.functional.softplus(g),
                 beta=torch.sigmoid(r(rows, hv)))
 
 
 def _step(family, lay, V, idx, t, out, model):
     if family == 'mamba2':
         lay.step(V, idx, t['x'], t['dt'], t['B'], t['C'], out, *model)
+    elif family == 'kda':
+        lay.step(V, idx, t['q'], t['k'], t['v'], t['g'], t['beta'], out)
     else:
         lay.step(V, idx, t['q'], t['k'], t['v'], out, lay.DK ** -0.5, g=t['g'], beta=t['beta'])
 
