@@ -22,6 +22,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
 OUT = os.path.join(HERE, 'build')
 LIB = os.path.join(PKG, 'libsqhip.so')
+HOST = os.path.join(PKG, '_sqhost.so')
 ARCH = 'gfx950'
 
 # -ffp-contract=off: every fused multiply-add in the kernels is written explicitly, as in the reference's kernels.
@@ -291,7 +292,7 @@ def _stamp():
     """Hash of every source that goes into the library (to skip a rebuild when nothing changed)."""
     h = hashlib.sha256()
     for name in sorted(os.listdir(HERE)):
-        if name.endswith(('.cuh', '.h', '.hip', '.py')):
+        if name.endswith(('.cuh', '.h', '.hip', '.cpp', '.py')):
             h.update(open(os.path.join(HERE, name), 'rb').read())
     h.update(open(os.path.join(os.path.dirname(PKG), 'include', 'statequant_hip.h'), 'rb').read())
     h.update(' '.join(HIPCC_FLAGS).encode())
@@ -393,13 +394,32 @@ def _compile(src, force=False):
     return obj
 
 
+def build_host():
+    """Compile the Python extension of the step wrappers (sq_host.cpp: host code only, against this interpreter's and
+    this torch's headers) next to the library."""
+    import sysconfig
+    import torch
+    from torch.utils import cpp_extension
+    lib_dirs = cpp_extension.library_paths()
+    cmd = ['g++', '-O2', '-std=c++17', '-fPIC', '-shared', '-D__HIP_PLATFORM_AMD__=1', '-DUSE_ROCM=1',
+           f'-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}',
+           *(f'-I{p}' for p in cpp_extension.include_paths()), '-I' + sysconfig.get_paths()['include'],
+           '-I' + os.path.join(os.environ.get('ROCM_PATH', '/opt/rocm'), 'include'),
+           os.path.join(HERE, 'sq_host.cpp'), '-o', HOST, *(f'-L{p}' for p in lib_dirs),
+           *(f'-Wl,-rpath,{p}' for p in lib_dirs), '-ltorch_python', '-ltorch_cpu', '-lc10', '-lc10_hip']
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode:
+        raise RuntimeError(f'{" ".join(cmd)}\n{r.stdout}\n{r.stderr}')
+    return HOST
+
+
 def build(jobs=None, force=False, verbose=True):
     """Compile and link; returns the path of the library."""
     jobs = jobs or min(16, os.cpu_count() or 4)
     units = generate()
     stamp_path = os.path.join(OUT, 'stamp')
     stamp = _stamp()
-    if not force and os.path.exists(LIB) and os.path.exists(stamp_path) and open(stamp_path).read() == stamp:
+    if not force and os.path.exists(LIB) and os.path.exists(HOST) and os.path.exists(stamp_path) and open(stamp_path).read() == stamp:
         if verbose:
             print(f'[build] {LIB} is up to date')
         return LIB
@@ -412,6 +432,7 @@ def build(jobs=None, force=False, verbose=True):
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode:
         raise RuntimeError(f'{" ".join(cmd)}\n{r.stdout}\n{r.stderr}')
+    build_host()
     with open(stamp_path, 'w') as f:
         f.write(stamp)
     if verbose:

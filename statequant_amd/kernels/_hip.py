@@ -13,6 +13,7 @@ import torch
 
 _PKG = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB_PATH = os.path.join(_PKG, 'libsqhip.so')
+HOST_PATH = os.path.join(_PKG, '_sqhost.so')
 ABI_VERSION = 6
 
 F32, BF16, F16 = 0, 1, 2
@@ -108,6 +109,7 @@ class SqGgaArgs(C.Structure):
 
 
 _lib = None
+_host = None
 
 
 def lib():
@@ -145,6 +147,23 @@ def lib():
             raise RuntimeError(f'{LIB_PATH}: ABI version {L.sq_abi_version()}, this package expects {ABI_VERSION}')
         _lib = L
     return _lib
+
+
+def host():
+    """The native side of the step and hand-over wrappers (``csrc/sq_host.cpp``): checks, argument structs and the
+    launch of one ordinary call in about a microsecond of host time.  Each of its functions returns the library's status,
+    or None for a call that is not of the ordinary form, which the Python code then does (or refuses) itself."""
+    global _host
+    if _host is None:
+        L = lib()
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError(f'{HOST_PATH} is missing: build it with `python -m statequant_amd.csrc.build`')
+        from .. import _sqhost
+        addr = lambda f: C.cast(f, C.c_void_p).value                            # noqa: E731
+        _sqhost.init(addr(L.sq_gdn_step), addr(L.sq_kda_step), addr(L.sq_mamba2_step), addr(L.sq_gga_step),
+                     addr(L.sq_pack_vk), addr(L.sq_read))
+        _host = _sqhost
+    return _host
 
 
 def dtype_code(t):

@@ -227,6 +227,10 @@ class PackedGDNState(LockstepState):
         return unpack(self.codes, self.scales, self.fmt, self.DK)
 
     def step(self, q, k, v, g, beta, scale):
+        rc = _hip.host().gdn_lockstep(self._lay, self._T, self._strides, self.B, q, k, v, g, beta, self.O, scale)
+        if rc is not None:                                # the ordinary call, done in native code
+            _hip.check(rc)
+            return self.O
         BH, HV, HK = self.BH, self.HV, self.HK
         per_key = q.shape[0] != BH
         if per_key:

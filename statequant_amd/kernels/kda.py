@@ -112,6 +112,11 @@ class PackedKDAState(LockstepState):
 
     def step(self, q, k, v, g, beta, scale=None):
         Bn, HV, DK, DV = self.B, self.HV, self.DK, self.DV
+        rc = _hip.host().kda_lockstep(self._lay, self.T, self._strides, Bn, q, k, v, g, beta, self.O,
+                                      DK ** -0.5 if scale is None else scale)
+        if rc is not None:                                # the ordinary call, done in native code
+            _hip.check(rc)
+            return self.O
         q, k = q.reshape(Bn, HV, DK), k.reshape(Bn, HV, DK)
         v, g, beta = v.reshape(Bn, HV, DV), g.reshape(Bn, HV, DK), beta.reshape(Bn, HV)
         return _launch(self, self._lay, Bn, q, k, v, g, beta, self.O, DK ** -0.5 if scale is None else scale, None,
@@ -148,6 +153,12 @@ class KDASlotLayout(SlotLayout):
         q, k [rows, H, d_k] raw, v [rows, H, d_v], g [rows, H, d_k] log decay, beta [rows, H] (after sigmoid): any
         row stride, contiguous rows; out [rows, H, d_v] (row stride free).  ``order``: optional dispatch order of the
         rows (``fold_order``; not in the reference).  One launch, no host syncs."""
+        if self._lay is not None:                         # the ordinary call, in native code
+            rc = _hip.host().kda_step(self._lay, views, idx, q, k, v, g, beta, out,
+                                      self.DK ** -0.5 if scale is None else scale, order)
+            if rc is not None:
+                _hip.check(rc)
+                return out
         rows = idx.shape[0]
         if rows == 0:
             return out
@@ -156,13 +167,14 @@ class KDASlotLayout(SlotLayout):
         return _launch(self, self._layout_struct(), rows, q, k, v, g, beta, out,
                        self.DK ** -0.5 if scale is None else scale, idx, T, strides, sN, order)
 
-    @torch.no_grad()
     def read(self, views, idx):
         """The current state of slots ``idx`` as fp32 [P, H, d_v, d_k]: diag(alpha_n) S_0 +
         sum_{i<n} diag(alpha_n / alpha_i) k_i u_i^T (value-major) (kda.py:351-372)."""
         out = self._read_hip(views, idx, kda=True)
-        if out is not None:
-            return out
+        return self._read_torch(views, idx) if out is None else out
+
+    @torch.no_grad()
+    def _read_torch(self, views, idx):
         idx = idx.long()
         m = self.m
         S0 = self._stored(views, idx)

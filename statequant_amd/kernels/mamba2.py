@@ -128,6 +128,11 @@ class PackedMamba2State(LockstepState):
 
     def step(self, x, dt, B, C, A, D=None, dt_bias=None, dt_softplus=False, dt_limit=None):
         Bn, HV, HK = self.B, self.HV, self.HK
+        rc = _hip.host().mamba2_lockstep(self._lay, self.T, self._strides, Bn, x, dt, B, C, self.O, A, D, dt_bias,
+                                         dt_softplus, dt_limit)
+        if rc is not None:                                # the ordinary call, done in native code
+            _hip.check(rc)
+            return self.O
         x = x.reshape(Bn, HV, self.DV)
         dt = dt.reshape(Bn, HV)
         B = B.reshape(Bn, HK, self.DK)
@@ -166,6 +171,12 @@ class Mamba2SlotLayout(SlotLayout):
         x [rows, H, d_v], dt [rows, H] (raw: + dt_bias, softplus, clamp in the kernel), B / C [rows, G, d_k]: any row
         stride, contiguous rows; out [rows, H, d_v] (row stride free); A [H] (= -exp(A_log)), D, dt_bias [H] or None.
         ``order``: optional dispatch order of the rows (``fold_order``; not in the reference)."""
+        if self._lay is not None:                         # the ordinary call, in native code
+            rc = _hip.host().mamba2_step(self._lay, views, idx, x, dt, B, C, out, A, D, dt_bias, dt_softplus, dt_limit,
+                                         order)
+            if rc is not None:
+                _hip.check(rc)
+                return out
         rows = idx.shape[0]
         if rows == 0:
             return out

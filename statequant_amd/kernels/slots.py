@@ -112,6 +112,7 @@ class SlotLayout:
         self._lay = None
 
     _family = 'gdn'
+    _conv = None                    # the layout struct of `read` and `write` (which need no step kernel)
 
     def __repr__(self):
         f = ('bf16' if self.state_dtype == torch.bfloat16 else 'fp32') if self.fmt is None else \
@@ -168,6 +169,11 @@ class SlotLayout:
         One kernel launch on the current stream, no allocation, no host synchronization: graph-capturable.  Each
         row's buffer counter advances; rows whose buffer fills are folded and re-rounded in place.
         """
+        if self._lay is not None:                         # the ordinary call, in native code
+            rc = _hip.host().gdn_step(self._lay, views, idx, q, k, v, out, scale, g, beta, gate, order)
+            if rc is not None:
+                _hip.check(rc)
+                return out
         B = idx.shape[0]
         if B == 0:
             return out
@@ -229,24 +235,31 @@ class SlotLayout:
     def _read_hip(self, views, idx, kda):
         """``sq_read`` for a blob on the GPU (``idx`` may live anywhere, as in the reference's indexing; rows with
         ``idx <= 0`` are padding and come back as zeros), None for a CPU blob."""
+        if self._conv is not None:                        # the ordinary call, in native code
+            done = _hip.host().read(self._conv, views, idx, kda)
+            if done is not None:
+                _hip.check(done[0])
+                return done[1]
         if not self._hip_format(views) or idx.shape[0] == 0:
             return None
         dev = views['S'].device
         P = idx.shape[0]
         out = torch.empty(P, self.HV, self.DV, self.DK, device=dev, dtype=torch.float32)
         T, strides, sN = slot_state(views)
-        _hip.read_state(_hip.make_layout(self), T, strides, sN, idx.to(device=dev, dtype=torch.int32).contiguous(),
+        self._conv = _hip.make_layout(self)
+        _hip.read_state(self._conv, T, strides, sN, idx.to(device=dev, dtype=torch.int32).contiguous(),
                         out, kda)
         return out
 
-    @torch.no_grad()
     def read(self, views, idx):
         """The current state of slots ``idx`` as fp32 [P, HV, d_v, d_k]: the stored state advanced across its
         pending buffer, S_n = a_n S_0 + sum_{i<n} (a_n/a_i) u_i k_i^T (slots.py:210-233).  Entries of dead buffer
         slots are discarded with ``where`` (they may hold anything)."""
         out = self._read_hip(views, idx, kda=False)
-        if out is not None:
-            return out
+        return self._read_torch(views, idx) if out is None else out
+
+    @torch.no_grad()
+    def _read_torch(self, views, idx):
         idx = idx.long()
         m = self.m
         S0 = self._stored(views, idx)
@@ -260,11 +273,18 @@ class SlotLayout:
         Kx = Kb.repeat_interleave(self.gqa, dim=1)                                    # [P, HV, m, DK]
         return torch.exp(gcur)[..., None, None] * S0 + torch.einsum('phmv,phmk->phvk', Ub * dec[..., None], Kx)
 
-    @torch.no_grad()
     def write(self, views, idx, S):
         """Store states S [P, HV, d_v, d_k] (value-major) packed into slots ``idx`` and empty their buffers
         (n = 0, running decay 0) (slots.py:236-252).  On the GPU rows with ``idx <= 0`` are padding and store nothing
         (slot 0 is the engine's null slot); the CPU formulation indexes like the reference."""
+        if self._conv is not None:                        # the ordinary call, in native code
+            rc = _hip.host().write(self._conv, views, idx, S)
+            if rc is not None:
+                return _hip.check(rc)
+        self._write_general(views, idx, S)
+
+    @torch.no_grad()
+    def _write_general(self, views, idx, S):
         P = idx.shape[0]
         V = views
         if self._hip_format(views):
@@ -274,7 +294,8 @@ class SlotLayout:
             src = S.reshape(P, self.HV, self.DV, self.DK).to(device=dev, dtype=torch.float32).contiguous()
             gc = V['GCUR']
             sc = V.get('SC')
-            _hip.pack_into(_hip.make_layout(self), src, V['S'], V['S'].stride(0), sc,
+            self._conv = _hip.make_layout(self)
+            _hip.pack_into(self._conv, src, V['S'], V['S'].stride(0), sc,
                            sc.stride(0) if sc is not None else 0,
                            idx=idx.to(device=dev, dtype=torch.int32).contiguous(), GCUR=gc, sGC=gc.stride(0),
                            gcur_per_head=gc[0].numel() // self.HV, NPTR=V['NPTR'], sN=V['NPTR'].stride(0))
