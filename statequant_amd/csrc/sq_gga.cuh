@@ -16,9 +16,17 @@
 //
 // A workgroup of four wavefronts holds the head's [d_k, d_v] tile in registers.  Wavefront w owns a quarter of the
 // columns and all rows: lane (tr, q) = (lane / 4, lane % 4) owns the columns tc CT .. tc CT + CT - 1 (tc = 4 w + q,
-// CT = d_v / 16) of the rows s 16 + tr.  Sums along d_k -- the step and the fit take six of them per column -- stay
-// inside a wavefront (two DPP row rotations and two lane swaps, no LDS, no barrier); the one sum along d_v (the row
-// factors of the fit) is a quad reduction plus one exchange of per-wavefront partials through LDS.
+// CT = d_v / 16) of the rows s 16 + tr.  Sums along d_k -- the step and the fit take five of them per column -- stay
+// inside a wavefront and end SPREAD over it: each of the four 16-lane rows keeps a quarter of its lanes' columns
+// (gga_col_reduce), does what is to be done per column for those alone, and hands only the results that every lane
+// needs back (gga_col_gather).  The one sum along d_v (the row factors of the fit) is a quad reduction plus an exchange
+// of per-wavefront partials through LDS, where one thread per row then forms that row's factors for everybody.
+//
+// What bounds the step is the vector ALU: every head is unpacked, updated, fitted and packed at every token (some 20
+// instructions per state value), while its bytes would take a tenth of the time.  So what counts is instructions, and
+// enough wavefronts to hide the serial stretches between them: the fit keeps ONE copy of the tile and divides by the
+// row factors again where it needs the quotients (three instructions a value), which leaves registers for four
+// wavefronts per SIMD where values and quotients side by side left them for two.
 #pragma once
 #include "sq_device.cuh"
 #include "sq_params.h"
@@ -34,6 +42,7 @@ template <int DK_, int DV_>
 struct GgaTile {
     static constexpr int DK = DK_, DV = DV_;
     static constexpr int CT = DV / 16;                  // columns per thread
+    static constexpr int CO = CT / 4;                   // columns a lane keeps of a sum along d_k
     static constexpr int RPT = DK / 16;                 // rows per thread
     static constexpr int NE = DK / WAVE;                // a key vector's elements per lane (one wavefront per vector)
     static constexpr int NV = DV / WAVE;
@@ -43,14 +52,19 @@ struct GgaTile {
 
 struct GgaThread {
     int tid, lane, wave, tc, tr;
+    int own;                                            // first of the lane's kept columns, of its CT, in quarters of CT
 };
 __device__ __forceinline__ GgaThread gga_thread() {
     GgaThread t;
     t.tid = threadIdx.x;
+    // from a copy the compiler cannot trace back: called anew in front of a phase, what it derives does not stay in
+    // registers from the kernel's top on
+    asm volatile("" : "+v"(t.tid));
     t.lane = t.tid & (WAVE - 1);
     t.wave = t.tid >> 6;
     t.tc = t.wave * 4 + (t.lane & 3);
     t.tr = t.lane >> 2;
+    t.own = 2 * ((t.lane >> 4) & 1) + (t.lane >> 5);
     return t;
 }
 
@@ -66,38 +80,64 @@ __device__ __forceinline__ float gga_div(float x, float d, float rc) { return di
 __device__ __forceinline__ float gga_rcp_f16(float d) { return rcp_f16(d); }
 
 // ---------------------------------------------------------------------------------------------------------------
-// sums / maxima along d_k: every thread ends with the totals of its CT columns (the same value in all row groups)
+// sums / maxima along d_k
 // ---------------------------------------------------------------------------------------------------------------
-// The partner's value across 16 / 32 lanes and the lane's own, as one VALU swap each (v_permlane16_swap exchanges the
-// odd 16-lane rows of its first operand with the even rows of its second, v_permlane32_swap the upper half of the
-// first with the lower half of the second; fed the same register twice they leave both values of a pair in both of
-// its lanes, in the same order, so the combined value is bit-identical across the pair).
-template <bool MAX>
-__device__ __forceinline__ float gga_pair16(float v) {
-    const auto r = __builtin_amdgcn_permlane16_swap(as_u32(v), as_u32(v), false, false);
-    return MAX ? fmaxf(as_f32(r[0]), as_f32(r[1])) : as_f32(r[0]) + as_f32(r[1]);
-}
-template <bool MAX>
-__device__ __forceinline__ float gga_pair32(float v) {
-    const auto r = __builtin_amdgcn_permlane32_swap(as_u32(v), as_u32(v), false, false);
-    return MAX ? fmaxf(as_f32(r[0]), as_f32(r[1])) : as_f32(r[0]) + as_f32(r[1]);
-}
-
 constexpr int DPP_ROR4 = 0x124, DPP_ROR8 = 0x128;      // row_ror: lane i of a 16-lane row reads lane (i + n) % 16
 
-// Sum / maximum over the 16 row groups of a wavefront (lanes with the same lane % 4): every lane ends with the total
-// of its CT columns, bit-identical across the lanes of a column (each step combines a pair symmetrically).
+template <bool MAX>
+__device__ __forceinline__ float gga_combine(float a, float b) { return MAX ? fmaxf(a, b) : a + b; }
+
+// Totals over the 16 row groups of a wavefront (lanes with the same lane % 4) of the CT columns of a lane, spread: the
+// lane keeps the CO = CT / 4 columns from CO own on.  A lane swap takes two columns at once -- v_permlane16_swap(a, b)
+// leaves {a's even 16-lane rows | b's even rows} and {a's odd rows | b's odd rows}, whose sum is column a's in the even
+// rows and column b's in the odd ones, v_permlane32_swap the same for the halves -- so the swaps of eight columns cost 12
+// instructions where handing every lane all of them costs 56.  The four lanes that keep a column hold the same bits.
+// (Sums: lanes 8 and 4 apart first, then 16, then 32 -- the order decides the last bit of a sum and with it, now and
+// then, which side of an fp16 rounding threshold a column factor falls on.)
 template <class T, int K, bool MAX>
-__device__ __forceinline__ void gga_col_allreduce(float (&p)[K][T::CT]) {
+__device__ __forceinline__ void gga_col_reduce(float (&p)[K][T::CT], float (&own)[K][T::CO]) {
+    constexpr int CT = T::CT, CO = T::CO;
+    auto rows = [](float v) {
+        v = gga_combine<MAX>(v, dpp<DPP_ROR8>(v));
+        return gga_combine<MAX>(v, dpp<DPP_ROR4>(v));
+    };
 #pragma unroll
-    for (int k = 0; k < K; ++k)
+    for (int k = 0; k < K; ++k) {
+        if constexpr (!MAX) {
 #pragma unroll
-        for (int e = 0; e < T::CT; ++e) {
-            float v = p[k][e];
-            v = MAX ? fmaxf(v, dpp<DPP_ROR8>(v)) : v + dpp<DPP_ROR8>(v);
-            v = MAX ? fmaxf(v, dpp<DPP_ROR4>(v)) : v + dpp<DPP_ROR4>(v);
-            p[k][e] = gga_pair32<MAX>(gga_pair16<MAX>(v));
+            for (int e = 0; e < CT; ++e) p[k][e] = rows(p[k][e]);
         }
+        float half[CT / 2];
+#pragma unroll
+        for (int e = 0; e < CT / 2; ++e) {
+            const auto r = __builtin_amdgcn_permlane16_swap(as_u32(p[k][e]), as_u32(p[k][e + CT / 2]), false, false);
+            half[e] = gga_combine<MAX>(as_f32(r[0]), as_f32(r[1]));
+        }
+#pragma unroll
+        for (int e = 0; e < CO; ++e) {
+            const auto r = __builtin_amdgcn_permlane32_swap(as_u32(half[e]), as_u32(half[e + CO]), false, false);
+            own[k][e] = gga_combine<MAX>(as_f32(r[0]), as_f32(r[1]));
+            if constexpr (MAX) own[k][e] = rows(own[k][e]);
+        }
+    }
+}
+// Every lane's CT columns from the kept ones.
+template <class T>
+__device__ __forceinline__ void gga_col_gather(const float (&own)[T::CO], float (&all)[T::CT]) {
+    constexpr int CT = T::CT, CO = T::CO;
+    float half[CT / 2];
+#pragma unroll
+    for (int e = 0; e < CO; ++e) {
+        const auto r = __builtin_amdgcn_permlane32_swap(as_u32(own[e]), as_u32(own[e]), false, false);
+        half[e] = as_f32(r[0]);
+        half[e + CO] = as_f32(r[1]);
+    }
+#pragma unroll
+    for (int e = 0; e < CT / 2; ++e) {
+        const auto r = __builtin_amdgcn_permlane16_swap(as_u32(half[e]), as_u32(half[e]), false, false);
+        all[e] = as_f32(r[0]);
+        all[e + CT / 2] = as_f32(r[1]);
+    }
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -145,6 +185,23 @@ __device__ __forceinline__ void gga_store_bytes(uint8_t* p, uint64_t v) {
     }
 }
 
+// Code e of a row piece as its signed value z times 2^up(e).  The code's bits are left where they are, in the mantissa
+// of 2^23: masked in, 2^23 + (bias + z) 2^up comes out as a float without a shift or a conversion, and one exact
+// subtraction leaves z 2^up.  The power of two goes into the column factor (exact).  PER codes fit a mantissa at a time.
+template <int B>
+struct GgaCode {
+    static constexpr int LOW = B == 2 ? 1 : 0;                             // two bits: z = 2 u - 3, from a word shifted by 1
+    static constexpr int PER = B == 8 ? 2 : B == 6 ? 3 : B == 4 ? 4 : 8;
+    __device__ static constexpr int up(int e) { return (e % PER) * B; }
+    __device__ __forceinline__ static float value(uint64_t raw, int e) {
+        const int at = (e / PER) * PER * B;
+        const uint32_t w = LOW ? uint32_t(raw) << 1 : uint32_t(raw >> at);
+        const uint32_t mask = ((1u << B) - 1) << (up(e) + LOW);
+        const float bias = 8388608.0f + float((B == 2 ? 3 : gga_qmax(B)) << up(e));
+        return as_f32((w & mask) | 0x4B000000u) - bias;
+    }
+};
+
 // Head state of width B at S -> the thread's x[s][e] (reference: `_load_head`, _gga_triton.py:131-143).
 template <class T, int B>
 __device__ __forceinline__ void gga_load_head(const uint8_t* S, const GgaThread& t, float (&x)[T::RPT][T::CT]) {
@@ -176,36 +233,56 @@ __device__ __forceinline__ void gga_load_head(const uint8_t* S, const GgaThread&
             raw[s] = gga_load_bytes<NB>(S + i * RB + t.tc * NB);
             rr[s] = B == 2 ? R[i * T::NG + (t.tc * CT) / GGA_GROUP] : R[i];
         }
-        float c[CT];
+        float c[CT];                                                       // column factors, over the code's scale
+        {
+            uint32_t cw[CT / 2];
+            if constexpr (CT == 8) {
+                const uint4 v = *reinterpret_cast<const uint4*>(C + t.tc * CT);
+                cw[0] = v.x; cw[1] = v.y; cw[2] = v.z; cw[3] = v.w;
+            } else {
+                const uint2 v = *reinterpret_cast<const uint2*>(C + t.tc * CT);
+                cw[0] = v.x; cw[1] = v.y;
+            }
 #pragma unroll
-        for (int e = 0; e < CT; ++e) c[e] = f16_to_f32(C[t.tc * CT + e]);
+            for (int e = 0; e < CT; ++e)
+                c[e] = f16_to_f32(uint16_t(cw[e / 2] >> (16 * (e % 2)))) * (1.0f / float(1u << GgaCode<B>::up(e)));
+        }
 #pragma unroll
         for (int s = 0; s < RPT; ++s) {
             const float r = f16_to_f32(rr[s]);
 #pragma unroll
-            for (int e = 0; e < CT; ++e) {
-                const int u = int((raw[s] >> (e * B)) & ((1u << B) - 1));
-                const float z = B == 2 ? float(2 * u - 3) : float(u - gga_qmax(B));
-                x[s][e] = (r * c[e]) * z;
-            }
+            for (int e = 0; e < CT; ++e) x[s][e] = (r * c[e]) * GgaCode<B>::value(raw[s], e);
+            __builtin_amdgcn_sched_barrier(0);              // a row at a time: rows side by side would not fit the registers
         }
     }
 }
 
-template <int B>
-__device__ __forceinline__ float gga_encode(float y) {
-    if constexpr (B == 2) return (y >= 0.0f ? 1.0f : -1.0f) * (fabsf(y) >= 2.0f ? 3.0f : 1.0f);
-    else return fminf(fmaxf(rintf(y), -float(gga_qmax(B))), float(gga_qmax(B)));
+// LDS of the fit: per-wavefront partial row sums, and every row's factors {r, 1 / r, w^2} (two-bit heads: per group
+// of value columns).
+template <class T>
+struct GgaFitLds {
+    float4 row[T::NG][T::DK];
+    float sum[GGA_WAVES * T::DK];
+};
+
+constexpr float GGA_MAGIC = 12582912.0f;               // 1.5 2^23 (even: ties go to even): adding it rounds to an integer, left
+                                                       // in the low mantissa bits
+
+// A row's factor from its mean |x| a: {r, 1 / r, w^2}.  The division and the square root are IEEE.
+__device__ __forceinline__ float4 gga_row_factor(float a, float w) {
+    const float r = gga_half(sqrtf(fmaxf(a, 1e-20f) / w));
+    return make_float4(r, gga_rcp_f16(r), w * w, 0.0f);
 }
 
 // STEP's dual-axis fit of the thread block's tile x at width B, packed at S (reference: `_store_head` ->
 // `_fit_parts`): row factors r = half(sqrt(max(mean_j |x|, 1e-20) / w)), column factors c = half(max_i |x / r| /
 // qmax), codes, one w^2-weighted least-squares refit of c with the codes fixed, codes again.  Divisions and the
-// square root are IEEE, as in torch.  `wrow[s]` = w of the thread's rows.
+// square root are IEEE, as in torch (quotients are exact half-integers often enough -- one 8-bit head in eight -- that
+// rounding y times a reciprocal would store other codes).  `w` = the head's row weights.
 template <class T, int B>
-__device__ __forceinline__ void gga_fit_store(uint8_t* S, float (&x)[T::RPT][T::CT], const float (&wrow)[T::RPT],
-                                              float* red, const GgaThread& t) {
-    constexpr int CT = T::CT, RPT = T::RPT, DK = T::DK, DV = T::DV;
+__device__ __forceinline__ void gga_fit_store(uint8_t* S, float (&x)[T::RPT][T::CT], const float* w,
+                                              GgaFitLds<T>& L, const GgaThread& t) {
+    constexpr int CT = T::CT, CO = T::CO, RPT = T::RPT, DK = T::DK, DV = T::DV;
     if constexpr (B == 16) {
         uint16_t* H = reinterpret_cast<uint16_t*>(S);
 #pragma unroll
@@ -223,92 +300,142 @@ __device__ __forceinline__ void gga_fit_store(uint8_t* S, float (&x)[T::RPT][T::
         constexpr int NB = CT * B / 8;
         constexpr int RB = DV * B / 8;
         constexpr float QMAX = float(gga_qmax(B));
-        constexpr int RN = B == 2 ? GGA_GROUP / CT : 16;                    // threads sharing one row factor
+        constexpr int COLS = B == 2 ? GGA_GROUP : DV;                       // columns sharing one row factor
         uint16_t* R = reinterpret_cast<uint16_t*>(S + gga_code_bytes(B, DK, DV));
         uint16_t* C = R + (B == 2 ? DK * T::NG : DK);
-        float rf[RPT], asum[RPT];
-        float y0[RPT][CT];
-        float cmax[1][CT];
-#pragma unroll
-        for (int e = 0; e < CT; ++e) cmax[0][e] = 0.0f;
+        // ---- row factors ----
+        constexpr bool OWN = B == 2 && 4 * CT >= GGA_GROUP;       // a two-bit group lies inside one wavefront's columns
+        const int grp = B == 2 ? (t.wave * 4 * CT) / GGA_GROUP : 0;
 #pragma unroll
         for (int s = 0; s < RPT; ++s) {
             float a = 0.0f;
 #pragma unroll
             for (int e = 0; e < CT; ++e) a = a + fabsf(x[s][e]);
-            asum[s] = block_sum<4>(a);                      // over the wavefront's 4 CT columns
+            a = block_sum<4>(a);                            // over the wavefront's 4 CT columns
+            __builtin_amdgcn_sched_barrier(0);
+            if ((t.lane & 3) == 0) L.sum[OWN ? t.wave * DK + s * 16 + t.tr : (s * 16 + t.tr) * GGA_WAVES + t.wave] = a;
         }
-        constexpr bool OWN = B == 2 && 4 * CT >= GGA_GROUP;       // a two-bit group lies inside one wavefront's columns
-        if constexpr (!OWN) {
-            if ((t.lane & 3) == 0) {
+        if constexpr (OWN) {
+            wave_sync();
 #pragma unroll
-                for (int s = 0; s < RPT; ++s) red[(s * 16 + t.tr) * GGA_WAVES + t.wave] = asum[s];
+            for (int i = t.lane; i < DK; i += WAVE) {
+                const float4 f = gga_row_factor(L.sum[t.wave * DK + i] * (1.0f / float(COLS)), w[i]);
+                L.row[grp][i] = f;
+                R[i * T::NG + grp] = f32_to_f16(f.x);
+            }
+            wave_sync();
+        } else {
+            constexpr int GROUPS = B == 2 ? T::NG : 1;
+            static_assert(GROUPS * DK <= GGA_THREADS, "a thread per row factor");
+            __syncthreads();
+            if (t.tid < GROUPS * DK) {
+                const int i = t.tid % DK, g = t.tid / DK;
+                const float4 w4 = *reinterpret_cast<const float4*>(L.sum + i * GGA_WAVES);
+                float a = (w4.x + w4.y) + (w4.z + w4.w);
+                if constexpr (B == 2) a = g == 0 ? w4.x + w4.y : w4.z + w4.w;         // d_v = 64: two wavefronts
+                const float4 f = gga_row_factor(a * (1.0f / float(COLS)), w[i]);
+                L.row[g][i] = f;
+                R[B == 2 ? i * T::NG + g : i] = f32_to_f16(f.x);
             }
             __syncthreads();
-#pragma unroll
-            for (int s = 0; s < RPT; ++s) {
-                const float4 w4 = *reinterpret_cast<const float4*>(red + (s * 16 + t.tr) * GGA_WAVES);
-                if constexpr (B == 2) asum[s] = t.wave < 2 ? w4.x + w4.y : w4.z + w4.w;     // d_v = 64: two wavefronts
-                else asum[s] = (w4.x + w4.y) + (w4.z + w4.w);
-            }
         }
+        // ---- the columns' first factors, from the quotients y by the row factors ----
+        float cmax[1][CT], cm[1][CO];
+#pragma unroll
+        for (int e = 0; e < CT; ++e) cmax[0][e] = 0.0f;
 #pragma unroll
         for (int s = 0; s < RPT; ++s) {
-            const float a = asum[s] * (1.0f / float(RN * CT));
-            rf[s] = gga_half(sqrtf(fmaxf(a, 1e-20f) / wrow[s]));
-            const float rrc = gga_rcp_f16(rf[s]);
+            const float2 f = *reinterpret_cast<const float2*>(&L.row[grp][s * 16 + t.tr]);
+#pragma unroll
+            for (int e = 0; e < CT; ++e) cmax[0][e] = fmaxf(cmax[0][e], fabsf(gga_div(x[s][e], f.x, f.y)));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        gga_col_reduce<T, 1, true>(cmax, cm);
+        // what a code is formed with, per column: its factor and the reciprocal; two bits: twice the factor
+        float c[CO], k[CT], crc[CT];
+        auto against = [&]() {
+            float f[CO];
+#pragma unroll
+            for (int e = 0; e < CO; ++e) f[e] = B == 2 ? 2.0f * c[e] : c[e];
+            gga_col_gather<T>(f, k);
+            if constexpr (B != 2) {
+#pragma unroll
+                for (int e = 0; e < CO; ++e) f[e] = gga_rcp_f16(c[e]);
+                gga_col_gather<T>(f, crc);
+            }
+        };
+        // rint(y / c), clamped, as GGA_MAGIC + z, of value v in a row of factors {r, 1 / r}
+        auto code = [&](float v, const float4& f, int e) {
+            return __builtin_amdgcn_fmed3f(gga_div(gga_div(v, f.x, f.y), k[e], crc[e]) + GGA_MAGIC, GGA_MAGIC - QMAX,
+                                           GGA_MAGIC + QMAX);
+        };
+        // two bits: |z| is 3 where y / c >= 2, which -- rounded quotients or not -- is exactly where |x| >= r 2 c: the
+        // product of two fp16 numbers is exact, and the next float below it is further off than the quotients' rounding
+        auto big = [&](float v, const float4& f, int e) { return fabsf(v) >= f.x * k[e]; };
+#pragma unroll
+        for (int e = 0; e < CO; ++e)                        // max_i (|y| / qmax) = (max_i |y|) / qmax: division is monotonic
+            c[e] = gga_half(gga_div(cm[0][e], QMAX, 1.0f / QMAX));
+        against();
+        // ---- codes, and the least-squares column factors for them ----
+        float nd[2][CT], so[2][CO];
+#pragma unroll
+        for (int e = 0; e < CT; ++e) nd[0][e] = nd[1][e] = 0.0f;
+#pragma unroll
+        for (int s = 0; s < RPT; ++s) {
+            const float4 f = L.row[grp][s * 16 + t.tr];
 #pragma unroll
             for (int e = 0; e < CT; ++e) {
-                y0[s][e] = gga_div(x[s][e], rf[s], rrc);
-                cmax[0][e] = fmaxf(cmax[0][e], fabsf(y0[s][e]));
+                float z;
+                if constexpr (B == 2) {
+                    const float mag = big(x[s][e], f, e) ? 3.0f : 1.0f;
+                    z = x[s][e] >= 0.0f ? mag : -mag;
+                } else {
+                    z = code(x[s][e], f, e) - GGA_MAGIC;
+                }
+                const float vv = f.x * z;
+                nd[0][e] = __builtin_fmaf(f.z * vv, x[s][e], nd[0][e]);
+                nd[1][e] = __builtin_fmaf(f.z, vv * vv, nd[1][e]);
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
-        gga_col_allreduce<T, 1, true>(cmax);
-        float c[CT], crc[CT];
-        float nd[2][CT];
+        gga_col_reduce<T, 2, false>(nd, so);
 #pragma unroll
-        for (int e = 0; e < CT; ++e) {
-            // max_i (|y| / qmax) = (max_i |y|) / qmax: division is monotonic
-            c[e] = gga_half(gga_div(cmax[0][e], QMAX, 1.0f / QMAX));
-            crc[e] = gga_rcp_f16(c[e]);
-            nd[0][e] = nd[1][e] = 0.0f;
-        }
+        for (int e = 0; e < CO; ++e)
+            c[e] = gga_half(so[1][e] > 0.0f ? so[0][e] / fmaxf(so[1][e], 1e-30f) : c[e]);
+        against();
+        // ---- codes again, packed: u = z + qmax (two bits: (z + 3) / 2) ----
 #pragma unroll
         for (int s = 0; s < RPT; ++s) {
-            const float ww = wrow[s] * wrow[s];
-#pragma unroll
-            for (int e = 0; e < CT; ++e) {
-                const float vv = rf[s] * gga_encode<B>(gga_div(y0[s][e], c[e], crc[e]));
-                nd[0][e] = __builtin_fmaf(ww * vv, x[s][e], nd[0][e]);
-                nd[1][e] = __builtin_fmaf(ww, vv * vv, nd[1][e]);
-            }
-        }
-        gga_col_allreduce<T, 2, false>(nd);
-#pragma unroll
-        for (int e = 0; e < CT; ++e) {
-            c[e] = gga_half(nd[1][e] > 0.0f ? nd[0][e] / fmaxf(nd[1][e], 1e-30f) : c[e]);
-            crc[e] = gga_rcp_f16(c[e]);
-        }
-#pragma unroll
-        for (int s = 0; s < RPT; ++s) {
-            const int i = s * 16 + t.tr;
+            constexpr int WB = B == 6 ? 4 : 32 / B;         // codes per word (six bits: 24 of its bits)
+            constexpr int WORDS = (CT + WB - 1) / WB;
+            const float4 f = L.row[grp][s * 16 + t.tr];
             uint64_t bits = 0;
 #pragma unroll
-            for (int e = 0; e < CT; ++e) {
-                const float z = gga_encode<B>(gga_div(y0[s][e], c[e], crc[e]));
-                const int u = B == 2 ? (int(z) + 3) >> 1 : int(z) + gga_qmax(B);
-                bits |= uint64_t(uint32_t(u)) << (e * B);
-            }
-            gga_store_bytes<NB>(S + i * RB + t.tc * NB, bits);
-            if (B == 2) {
-                if ((t.tc & (RN - 1)) == 0) R[i * T::NG + (t.tc * CT) / GGA_GROUP] = f32_to_f16(rf[s]);
-            } else if (t.tc == 0) {
-                R[i] = f32_to_f16(rf[s]);
-            }
-        }
-        if (t.tr == 0) {
+            for (int d = WORDS - 1; d >= 0; --d) {
+                uint32_t acc = 0, magic = 0;
 #pragma unroll
-            for (int e = 0; e < CT; ++e) C[t.tc * CT + e] = f32_to_f16(c[e]);
+                for (int j = WB - 1; j >= 0; --j) {
+                    const int e = d * WB + j;
+                    if (e >= CT) continue;
+                    uint32_t u;
+                    if constexpr (B == 2) {
+                        const bool b3 = big(x[s][e], f, e);
+                        u = x[s][e] >= 0.0f ? (b3 ? 3u : 2u) : (b3 ? 0u : 1u);
+                    } else {                                // z on top of constant bits, which add up to a constant
+                        u = as_u32(code(x[s][e], f, e));
+                        magic = (magic << B) + (0x4B400000u - uint32_t(gga_qmax(B)));
+                    }
+                    acc = (acc << B) + u;
+                }
+                bits = (bits << (B * WB % 64)) | uint64_t(acc - magic);
+            }
+            gga_store_bytes<NB>(S + (s * 16 + t.tr) * RB + t.tc * NB, bits);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if ((t.lane & 12) == 0) {                           // one of the four lanes that keep these columns
+            uint16_t* at = C + t.tc * CT + t.own * CO;
+            if constexpr (CO == 2) *reinterpret_cast<uint32_t*>(at) = uint32_t(f32_to_f16(c[0])) | (uint32_t(f32_to_f16(c[1])) << 16);
+            else *at = f32_to_f16(c[0]);
         }
     }
 }
@@ -322,13 +449,14 @@ __device__ __forceinline__ void gga_load_any(const uint8_t* S, int bits, const G
     else gga_load_head<T, 2>(S, t, x);
 }
 template <class T>
-__device__ __forceinline__ void gga_store_any(uint8_t* S, int bits, float (&x)[T::RPT][T::CT], const float (&wrow)[T::RPT],
-                                              float* red, const GgaThread& t) {
-    if (bits == 16) gga_fit_store<T, 16>(S, x, wrow, red, t);
-    else if (bits == 8) gga_fit_store<T, 8>(S, x, wrow, red, t);
-    else if (bits == 6) gga_fit_store<T, 6>(S, x, wrow, red, t);
-    else if (bits == 4) gga_fit_store<T, 4>(S, x, wrow, red, t);
-    else gga_fit_store<T, 2>(S, x, wrow, red, t);
+__device__ __forceinline__ void gga_store_any(uint8_t* S, int bits, float (&x)[T::RPT][T::CT], const float* w,
+                                              GgaFitLds<T>& L) {
+    const GgaThread t = gga_thread();
+    if (bits == 16) gga_fit_store<T, 16>(S, x, w, L, t);
+    else if (bits == 8) gga_fit_store<T, 8>(S, x, w, L, t);
+    else if (bits == 6) gga_fit_store<T, 6>(S, x, w, L, t);
+    else if (bits == 4) gga_fit_store<T, 4>(S, x, w, L, t);
+    else gga_fit_store<T, 2>(S, x, w, L, t);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -375,14 +503,19 @@ __device__ __forceinline__ void fp8_load(const uint8_t* p, int lane, uint32_t (&
 // ---------------------------------------------------------------------------------------------------------------
 template <class T>
 struct GgaLds {
-    float kn[T::DK], qn[T::DK], r0[T::DK];
+    float2 kq[T::DK];                             // k, q normalised
+    float r0[T::DK];                              // left factor of the write that enters the state
     float coef[GGA_MMAX];
-    float red[GGA_WAVES * T::DK];                 // the fit's row sums: one partial per wavefront and row
+    GgaFitLds<T> fit;
 };
 
+// Four wavefronts per SIMD (128 registers, 11 of them spilled): the launch of 32 sequences x 32 heads of 128 x 128 then
+// runs in one round of workgroups.  us per launch there, mixed widths: 44.0 with values and quotients side by side (225
+// registers, two wavefronts per SIMD) -> 34.6 at three -> 32.4 at four; 4151 -> 3415 vector instructions per wavefront,
+// which is 23 us of issue.
 template <class T>
-__global__ __launch_bounds__(GGA_THREADS, 2) void gga_step_kernel(const GgaParams p) {
-    constexpr int CT = T::CT, RPT = T::RPT, DK = T::DK, DV = T::DV, NE = T::NE, NV = T::NV;
+__global__ __launch_bounds__(GGA_THREADS, 4) void gga_step_kernel(const GgaParams p) {
+    constexpr int CT = T::CT, CO = T::CO, RPT = T::RPT, DK = T::DK, DV = T::DV, NE = T::NE, NV = T::NV;
     __shared__ __attribute__((aligned(16))) GgaLds<T> L;
     const GgaThread t = gga_thread();
     // head-major order: workgroups that run together work on the same head, hence on the same width, and share the
@@ -427,27 +560,30 @@ __global__ __launch_bounds__(GGA_THREADS, 2) void gga_step_kernel(const GgaParam
     const uint32_t btr = load_raw_uniform(p.bt, p.bt_dt, uint64_t(b) * p.s_bt + h);
     const uint32_t alr = load_raw_uniform(p.A_log, p.A_log_dt, h);
     const uint32_t dbr = load_raw_uniform(p.dt_bias, p.dt_bias_dt, h);
-    // the thread's columns of v, and of the queued right factors
+    // the lane's kept columns of v and of the queued right factors (for the output), and all its columns of the write
+    // that enters the state: the oldest pair of a full window, v itself without a window
+    const bool full = window && n == m, enters = full || !window;
     const void* vp = advance(p.v, p.v_dt, uint64_t(b) * p.s_v + h * DV);
-    uint32_t vr[CT];
+    const int c0 = t.tc * CT, oc = c0 + t.own * CO;
+    uint32_t vo[CO], v0q[CT / 4];
 #pragma unroll
-    for (int e = 0; e < CT; ++e) vr[e] = load_raw(vp, p.v_dt, t.tc * CT + e);
-    uint32_t vq[GGA_MMAX][CT / 4];
-    float vs[GGA_MMAX];
+    for (int e = 0; e < CO; ++e) vo[e] = load_raw(vp, p.v_dt, oc + e);
+    uint32_t vq[GGA_MMAX];
+    float vsl = 0.0f;                                   // lane oi: the scale of the oi-th oldest right factor
     if (window) {
+        if (t.lane < n) vsl = VS[hd + t.lane < m ? hd + t.lane : hd + t.lane - m];
 #pragma unroll
         for (int oi = 0; oi < GGA_MMAX; ++oi) {
-            const int jj = (hd + oi) % m;
+            const int jj = hd + oi < m ? hd + oi : hd + oi - m;
             const bool live = oi < n;
+            if constexpr (CO == 2) vq[oi] = live ? *reinterpret_cast<const uint16_t*>(VP + jj * DV + oc) : 0u;
+            else vq[oi] = live ? VP[jj * DV + oc] : 0u;
+        }
+        if (full) {
 #pragma unroll
-            for (int w4 = 0; w4 < CT / 4; ++w4)
-                vq[oi][w4] = live ? reinterpret_cast<const uint32_t*>(VP + jj * DV + t.tc * CT)[w4] : 0u;
-            vs[oi] = live ? VS[jj] : 0.0f;
+            for (int w4 = 0; w4 < CT / 4; ++w4) v0q[w4] = reinterpret_cast<const uint32_t*>(VP + hd * DV + c0)[w4];
         }
     }
-    float wrow[RPT];
-#pragma unroll
-    for (int s = 0; s < RPT; ++s) wrow[s] = p.w[h * DK + s * 16 + t.tr];
 
     float x[RPT][CT];
     gga_load_any<T>(S, bits, t, x);
@@ -484,16 +620,15 @@ __global__ __launch_bounds__(GGA_THREADS, 2) void gga_step_kernel(const GgaParam
     if (t.wave == 0) {
 #pragma unroll
         for (int e = 0; e < NE; ++e) {
-            L.kn[t.lane * NE + e] = ke[e];
-            L.qn[t.lane * NE + e] = qe[e];
+            L.kq[t.lane * NE + e] = make_float2(ke[e], qe[e]);
+            if (!window) L.r0[t.lane * NE + e] = bke[e];
         }
     }
 
     // ---- the queued left factors: propagate, re-encode, read out (wavefront w: entries w, w + 4) ----
-    const bool full = window && n == m;
     if (window) {
         for (int oi = t.wave; oi < n; oi += GGA_WAVES) {
-            const int jj = (hd + oi) % m;
+            const int jj = hd + oi < m ? hd + oi : hd + oi - m;
             uint32_t code[NE];
             fp8_load<NE>(PP + jj * DK, t.lane, code);
             const float ps = PS[jj];
@@ -525,91 +660,84 @@ __global__ __launch_bounds__(GGA_THREADS, 2) void gga_step_kernel(const GgaParam
     }
     __syncthreads();
 
-    // ---- O_pre = a (O - beta k (k^T O)), its read-out ----
-    float krow[RPT], qrow[RPT];
+    // ---- k^T O and q^T O; the output: q^T O_pre = a (q^T O - (beta k . q) k^T O), the queued pairs oldest first, and
+    //      this token's write -- for the lane's kept columns ----
+    float kO[CT], krow[RPT];
+    {
+        float acc[2][CT], own[2][CO], o[CO];
 #pragma unroll
-    for (int s = 0; s < RPT; ++s) {
-        krow[s] = L.kn[s * 16 + t.tr];
-        qrow[s] = L.qn[s * 16 + t.tr];
+        for (int e = 0; e < CT; ++e) acc[0][e] = acc[1][e] = 0.0f;
+#pragma unroll
+        for (int s = 0; s < RPT; ++s) {
+            const float2 kq = L.kq[s * 16 + t.tr];
+            krow[s] = kq.x;
+#pragma unroll
+            for (int e = 0; e < CT; ++e) {
+                acc[0][e] = __builtin_fmaf(kq.x, x[s][e], acc[0][e]);
+                acc[1][e] = __builtin_fmaf(kq.y, x[s][e], acc[1][e]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        gga_col_reduce<T, 2, false>(acc, own);
+        gga_col_gather<T>(own[0], kO);
+#pragma unroll
+        for (int e = 0; e < CO; ++e) {
+            o[e] = a * __builtin_fmaf(-bkq, own[0][e], own[1][e]);
+            o[e] = o[e] + bkq * raw_to_f(vo[e], p.v_dt);
+        }
+        if (window) {
+            const float cfl = t.lane < n ? L.coef[t.lane] * vsl : 0.0f;
+#pragma unroll
+            for (int oi = 0; oi < GGA_MMAX; ++oi) {
+                if (oi < n) {
+                    const float cf = lane_bcast(cfl, oi);
+#pragma unroll
+                    for (int e = 0; e < CO; ++e) o[e] = __builtin_fmaf(cf, fp8_to_f32((vq[oi] >> (8 * e)) & 0xFFu), o[e]);
+                }
+            }
+        }
+        if ((t.lane & 12) == 0) {                          // one of the four lanes that keep these columns
+#pragma unroll
+            for (int e = 0; e < CO; ++e) store_f(outp, p.out_dt, oc + e, o[e]);
+        }
     }
-    float acc[1][CT];
-#pragma unroll
-    for (int e = 0; e < CT; ++e) acc[0][e] = 0.0f;
-#pragma unroll
-    for (int s = 0; s < RPT; ++s)
-#pragma unroll
-        for (int e = 0; e < CT; ++e) acc[0][e] = __builtin_fmaf(krow[s], x[s][e], acc[0][e]);
-    gga_col_allreduce<T, 1, false>(acc);
-    float kO[CT];
-#pragma unroll
-    for (int e = 0; e < CT; ++e) {
-        kO[e] = acc[0][e];
-        acc[0][e] = 0.0f;
-    }
+
+    // ---- O_pre = a (O - beta k (k^T O)), and the write that enters the state: the pair that leaves a full window;
+    //      pivots and slots without a window take the new one ----
 #pragma unroll
     for (int s = 0; s < RPT; ++s) {
         const float bk = beta * krow[s];
 #pragma unroll
-        for (int e = 0; e < CT; ++e) {
-            x[s][e] = a * __builtin_fmaf(-bk, kO[e], x[s][e]);
-            acc[0][e] = __builtin_fmaf(x[s][e], qrow[s], acc[0][e]);
-        }
+        for (int e = 0; e < CT; ++e) x[s][e] = a * __builtin_fmaf(-bk, kO[e], x[s][e]);
     }
-    gga_col_allreduce<T, 1, false>(acc);
-    float ve[CT], o[CT];
-#pragma unroll
-    for (int e = 0; e < CT; ++e) {
-        ve[e] = raw_to_f(vr[e], p.v_dt);
-        o[e] = acc[0][e] + bkq * ve[e];
-    }
-
-    if (window) {
-        // read-out of the queued pairs (oldest first), the merge of the evicted one
-#pragma unroll
-        for (int oi = 0; oi < GGA_MMAX; ++oi) {
-            if (oi < n) {
-                const float cf = L.coef[oi];
-#pragma unroll
-                for (int e = 0; e < CT; ++e) {
-                    const float vt = fp8_to_f32((vq[oi][e / 4] >> (8 * (e % 4))) & 0xFFu) * vs[oi];
-                    o[e] = o[e] + cf * vt;
-                }
-            }
-        }
+    if (enters) {
+        float v0[CT];
         if (full) {
-            float v0[CT];
+            const float s0 = lane_bcast(vsl, 0);
 #pragma unroll
-            for (int e = 0; e < CT; ++e) v0[e] = fp8_to_f32((vq[0][e / 4] >> (8 * (e % 4))) & 0xFFu) * vs[0];
+            for (int e = 0; e < CT; ++e) v0[e] = fp8_to_f32((v0q[e / 4] >> (8 * (e % 4))) & 0xFFu) * s0;
+        } else {
 #pragma unroll
-            for (int s = 0; s < RPT; ++s) {
-                const float r0 = L.r0[s * 16 + t.tr];
-#pragma unroll
-                for (int e = 0; e < CT; ++e) x[s][e] = __builtin_fmaf(r0, v0[e], x[s][e]);
-            }
+            for (int e = 0; e < CT; ++e) v0[e] = raw_to_f(load_raw(vp, p.v_dt, c0 + e), p.v_dt);
         }
-    } else {
-        // pivots and slots without a window: the new write goes into the state
 #pragma unroll
         for (int s = 0; s < RPT; ++s) {
-            const float bk = beta * krow[s];
+            const float r0 = L.r0[s * 16 + t.tr];
 #pragma unroll
-            for (int e = 0; e < CT; ++e) x[s][e] = __builtin_fmaf(bk, ve[e], x[s][e]);
+            for (int e = 0; e < CT; ++e) x[s][e] = __builtin_fmaf(r0, v0[e], x[s][e]);
         }
-    }
-    if (t.tr == 0) {
-#pragma unroll
-        for (int e = 0; e < CT; ++e) store_f(outp, p.out_dt, t.tc * CT + e, o[e]);
     }
 
     // ---- re-fit and re-pack in place ----
-    gga_store_any<T>(S, bits, x, wrow, L.red, t);
+    gga_store_any<T>(S, bits, x, p.w + h * DK, L.fit);
 
     // ---- queue (R(beta k), R(v)).  A full window's new pair replaces the oldest one, whose right factor every
     // wavefront has read for the merge: the barrier puts the store behind all of those reads (each wavefront used its
     // copy before it got here).
     if (window) {
+        const GgaThread t = gga_thread();
         __syncthreads();
-        const int jn = n < m ? (hd + n) % m : hd;
+        const int jn = n == m ? hd : hd + n < m ? hd + n : hd + n - m;
         if (t.wave == 0) {
             uint32_t code[NE];
             float rec[NE];
@@ -646,7 +774,7 @@ __global__ void gga_advance_kernel(uint8_t* blob, uint64_t slot_stride, const in
 template <class T>
 __global__ __launch_bounds__(GGA_THREADS, 2) void gga_store_kernel(const GgaParams p) {
     constexpr int CT = T::CT, RPT = T::RPT, DK = T::DK, DV = T::DV;
-    __shared__ __attribute__((aligned(16))) float red[GGA_WAVES * DK];
+    __shared__ __attribute__((aligned(16))) GgaFitLds<T> L;
     const GgaThread t = gga_thread();
     // head-major order: workgroups that run together work on the same head, hence on the same width, and share the
     // instructions of one of the five width paths (each path is ~40 KB of straight-line code)
@@ -656,18 +784,17 @@ __global__ __launch_bounds__(GGA_THREADS, 2) void gga_store_kernel(const GgaPara
     if (seq <= 0) return;
     uint8_t* const base = p.blob + uint64_t(seq) * p.slot_stride;
     const float* X = p.X + uint64_t(bh) * (DK * DV);
-    float x[RPT][CT], wrow[RPT];
+    float x[RPT][CT];
 #pragma unroll
     for (int s = 0; s < RPT; ++s) {
         const int i = s * 16 + t.tr;
-        wrow[s] = p.w[h * DK + i];
 #pragma unroll
         for (int e4 = 0; e4 < CT; e4 += 4) {
             const float4 v = *reinterpret_cast<const float4*>(X + i * DV + t.tc * CT + e4);
             x[s][e4] = v.x; x[s][e4 + 1] = v.y; x[s][e4 + 2] = v.z; x[s][e4 + 3] = v.w;
         }
     }
-    gga_store_any<T>(base + p.offs[h], p.bits[h], x, wrow, red, t);
+    gga_store_any<T>(base + p.offs[h], p.bits[h], x, p.w + h * DK, L);
     if (h == 0 && t.tid < 2) reinterpret_cast<int32_t*>(base)[t.tid] = 0;
 }
 
