@@ -4,8 +4,8 @@
 //   read   the stored state advanced across its pending buffer, as fp32 value-major
 //          S_n = a_n S_0 + sum_{i<n} (a_n / a_i) u_i k_i^T;  KDA: decays per key channel
 //          (reference: kernels/slots.py:210-233, kernels/kda.py:351-372)
-// Both are plain streaming kernels, one wavefront per (sequence, value head): rows in the row shape of the fold
-// (LPRP lanes per row, 16 columns per lane), d_v and m taken at run time.  Value-axis scale groups (32 rows of one key
+// Both are plain streaming kernels, one wavefront per (sequence, value head, range of rows): rows in the row shape of the
+// fold (LPRP lanes per row, 16 columns per lane), d_v and m taken at run time.  Value-axis scale groups (32 rows of one key
 // column share a scale) pack with a column shape instead (a lane owns two neighbouring columns of a 32-row block);
 // the unquantized state (bf16 / fp32) packs as a cast.  They are bound by the fp32 side of the
 // transfer (pack reads 4 bytes per code it writes, read writes 4 bytes per code it reads).
@@ -18,6 +18,22 @@ namespace sq {
 // geometry carrier: only the d_k-shaped members of Tile are used here
 template <int BITS, int DK, int GROUP, bool QBUF, bool AXV = false>
 using RowTile = Tile<BITS, DK, 128, GROUP, QBUF, 16, AXV>;
+
+// How many wavefronts share a head's rows, and how many rows each takes (a multiple of `step`, what a wavefront's pass
+// covers).  A hand-over concerns the few sequences that begin or end a prefill chunk: one wavefront per head leaves most
+// of the chip idle and walks the rows one memory round trip after the other, so heads are split until there are some
+// 4096 wavefronts (16 per compute unit, what full batches give by themselves and what keeps memory busy).  6 sequences
+// of 32 heads of 128 x 128, int8 g32: write 11.9 -> 4.7 us per launch, read 14.8 -> 7.0 (256 sequences, one wavefront
+// per head as before: 142 and 149).
+struct RowSplit {
+    uint32_t parts, rows;
+};
+inline RowSplit split_rows(uint32_t heads, uint32_t dv, uint32_t step) {
+    uint32_t parts = 1;
+    while (heads * parts < 4096 && parts * step < dv) parts *= 2;
+    const uint32_t rows = ((dv + parts - 1) / parts + step - 1) / step * step;
+    return RowSplit{(dv + rows - 1) / rows, rows};
+}
 
 // Empty a sequence's buffer: this head's counter copy and running decay.
 __device__ __forceinline__ void reset_counters(const PackParams& p, uint32_t seq, uint32_t h, int lane) {
@@ -32,7 +48,7 @@ __device__ __forceinline__ void reset_counters(const PackParams& p, uint32_t seq
 }
 
 template <int BITS, int DK, int GROUP>
-__global__ __launch_bounds__(WAVE) void pack_kernel(const PackParams p) {
+__global__ __launch_bounds__(WAVE) void pack_kernel(const PackParams p, uint32_t part_rows) {
     using T = RowTile<BITS, DK, GROUP, true>;
     const LaneId l = lane_id<T>();
     const uint32_t b = blockIdx.x / uint32_t(p.hv), h = blockIdx.x - b * uint32_t(p.hv);
@@ -48,7 +64,8 @@ __global__ __launch_bounds__(WAVE) void pack_kernel(const PackParams p) {
     const bool has_group = gi < T::NG;
     gi = has_group ? gi : T::NG - 1;
     const bool lead = live && (l.cg % T::LPG) == 0 && has_group;
-    for (uint32_t r0 = 0; r0 < dv; r0 += T::RG) {
+    const uint32_t r_begin = blockIdx.y * part_rows, r_end = min(dv, r_begin + part_rows);
+    for (uint32_t r0 = r_begin; r0 < r_end; r0 += T::RG) {
         const uint32_t row = r0 + l.rg;
         const bool in = row < dv;
         const float4* s4 = reinterpret_cast<const float4*>(src + (in ? row : dv - 1) * DK + cc * CPL);
@@ -70,13 +87,13 @@ __global__ __launch_bounds__(WAVE) void pack_kernel(const PackParams p) {
         if (in && live) store_row<BITS>(Sh + row * T::ROW_BYTES + l.cg * T::LANE_BYTES, encode_row<BITS>(q));
         if (in && lead) SCh[row * T::NG + gi] = f32_to_f16(s);
     }
-    reset_counters(p, seq, h, l.lane);
+    if (blockIdx.y == 0) reset_counters(p, seq, h, l.lane);
 }
 
 // Value-axis groups of G rows (fold.py:139-146): scales [dv / G][DK].  A lane owns columns 2 lane, 2 lane + 1 and
 // walks the G rows of a group twice (absmax, then codes) with the group's 2 G values in registers.
 template <int BITS, int DK, int G>
-__global__ __launch_bounds__(WAVE) void pack_v_kernel(const PackParams p) {
+__global__ __launch_bounds__(WAVE) void pack_v_kernel(const PackParams p, uint32_t part_rows) {
     constexpr float QMAX = float((1 << (BITS - 1)) - 1);
     constexpr int ROW_BYTES = DK * BITS / 8;
     static_assert(DK % 2 == 0 && DK <= 2 * WAVE, "two columns per lane");
@@ -90,7 +107,8 @@ __global__ __launch_bounds__(WAVE) void pack_v_kernel(const PackParams p) {
     uint16_t* SCh = field(p.SC, seq, p.sSC, h * ((dv / G) * DK));
     const bool live = 2 * lane < DK;
     const int c0 = live ? 2 * lane : DK - 2;
-    for (uint32_t r0 = 0; r0 < dv; r0 += G) {
+    const uint32_t r_begin = blockIdx.y * part_rows, r_end = min(dv, r_begin + part_rows);
+    for (uint32_t r0 = r_begin; r0 < r_end; r0 += G) {
         float2 x[G];
 #pragma unroll
         for (int r = 0; r < G; ++r) x[r] = *reinterpret_cast<const float2*>(src + (r0 + r) * DK + c0);
@@ -114,12 +132,12 @@ __global__ __launch_bounds__(WAVE) void pack_v_kernel(const PackParams p) {
             }
         }
     }
-    reset_counters(p, seq, h, lane);
+    if (blockIdx.y == 0) reset_counters(p, seq, h, lane);
 }
 
 // The unquantized state: a cast to bf16 (round to nearest even) or a copy (fp32), [dv][DK] per head.
 template <int BITS, int DK>
-__global__ __launch_bounds__(WAVE) void pack_f_kernel(const PackParams p) {
+__global__ __launch_bounds__(WAVE) void pack_f_kernel(const PackParams p, uint32_t part_rows) {
     static_assert(DK % 4 == 0, "four columns per lane and step");
     const int lane = threadIdx.x;
     const uint32_t b = blockIdx.x / uint32_t(p.hv), h = blockIdx.x - b * uint32_t(p.hv);
@@ -128,7 +146,8 @@ __global__ __launch_bounds__(WAVE) void pack_f_kernel(const PackParams p) {
     const uint32_t seq = slot, n = p.dv * DK;
     const float* src = p.src + (uint64_t(b) * p.s_src + uint64_t(h) * n);
     uint8_t* Sh = field(p.S, seq, p.sS, h * (n * (BITS / 8)));
-    for (uint32_t e = 4 * lane; e < n; e += 4 * WAVE) {
+    const uint32_t e_begin = blockIdx.y * part_rows * DK, e_end = min(n, e_begin + part_rows * DK);
+    for (uint32_t e = e_begin + 4 * lane; e < e_end; e += 4 * WAVE) {
         const float4 f = *reinterpret_cast<const float4*>(src + e);
         if constexpr (BITS == 16)
             *reinterpret_cast<uint2*>(Sh + 2 * e) =
@@ -137,24 +156,32 @@ __global__ __launch_bounds__(WAVE) void pack_f_kernel(const PackParams p) {
         else
             *reinterpret_cast<float4*>(Sh + 4 * e) = f;
     }
-    reset_counters(p, seq, h, lane);
+    if (blockIdx.y == 0) reset_counters(p, seq, h, lane);
 }
 
 // AXV: value-axis groups of GROUP rows; BITS 16 / 32: the unquantized state (GROUP = DK).
 template <int BITS, int DK, int GROUP, bool AXV>
 int launch_pack(const PackParams& p, hipStream_t stream) {
-    if constexpr (BITS >= 16) hipLaunchKernelGGL((pack_f_kernel<BITS, DK>), dim3(p.rows * p.hv), dim3(WAVE), 0, stream, p);
-    else if constexpr (AXV) hipLaunchKernelGGL((pack_v_kernel<BITS, DK, GROUP>), dim3(p.rows * p.hv), dim3(WAVE), 0, stream, p);
-    else hipLaunchKernelGGL((pack_kernel<BITS, DK, GROUP>), dim3(p.rows * p.hv), dim3(WAVE), 0, stream, p);
+    const uint32_t heads = uint32_t(p.rows) * uint32_t(p.hv);
+    if constexpr (BITS >= 16) {
+        const RowSplit sp = split_rows(heads, p.dv, 8);
+        hipLaunchKernelGGL((pack_f_kernel<BITS, DK>), dim3(heads, sp.parts), dim3(WAVE), 0, stream, p, sp.rows);
+    } else if constexpr (AXV) {
+        const RowSplit sp = split_rows(heads, p.dv, GROUP);
+        hipLaunchKernelGGL((pack_v_kernel<BITS, DK, GROUP>), dim3(heads, sp.parts), dim3(WAVE), 0, stream, p, sp.rows);
+    } else {
+        const RowSplit sp = split_rows(heads, p.dv, RowTile<BITS, DK, GROUP, true>::RG);
+        hipLaunchKernelGGL((pack_kernel<BITS, DK, GROUP>), dim3(heads, sp.parts), dim3(WAVE), 0, stream, p, sp.rows);
+    }
     return int(hipGetLastError());
 }
 
-// LDS (dynamic): keys x decay ratio [m][DK] fp32, values [m][dv] fp32.
+// LDS (dynamic): keys x decay ratio [m][DK] fp32, values [m][rows of the part] fp32.
 // Column split of the output pass: a lane takes NCH chunks of 4 columns, chunk t = columns 4 LPR t + 4 cg .. + 3, so
 // that the LPR lanes of a row write 16 LPR consecutive bytes with every store instruction (whole 128-byte lines for
 // d_k = 128) -- with 16 consecutive columns per lane each store would scatter 16-byte pieces 64 bytes apart.
 template <int BITS, int DK, int GROUP, bool QBUF, bool KDA, bool AXV>
-__global__ __launch_bounds__(WAVE) void read_kernel(const ReadParams p) {
+__global__ __launch_bounds__(WAVE) void read_kernel(const ReadParams p, uint32_t part_rows) {
     using T = RowTile<BITS, DK, GROUP, QBUF, AXV>;
     constexpr int NCH = CPL / 4;
     constexpr int CSTEP = 4 * T::LPR;                             // columns between a lane's chunks
@@ -167,10 +194,11 @@ __global__ __launch_bounds__(WAVE) void read_kernel(const ReadParams p) {
     const uint32_t b = blockIdx.x / uint32_t(p.hv), h = blockIdx.x - b * uint32_t(p.hv);
     const uint32_t hk = h / uint32_t(p.gqa);
     float* out = p.out + (uint64_t(b) * p.s_out + uint64_t(h) * dv * DK);
+    const uint32_t r_begin = blockIdx.y * part_rows, r_end = min(dv, r_begin + part_rows), nrows = r_end - r_begin;
     const int32_t slot = p.idx ? p.idx[b] : int32_t(b);
     if (p.idx && slot <= 0) {                                      // padding row: a zero state, nothing of a slot read
-        float4* o4 = reinterpret_cast<float4*>(out);
-        for (uint32_t e = l.lane; e < dv * DK / 4; e += WAVE) o4[e] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        float4* o4 = reinterpret_cast<float4*>(out + r_begin * DK);
+        for (uint32_t e = l.lane; e < nrows * DK / 4; e += WAVE) o4[e] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         return;
     }
     const uint32_t seq = slot;
@@ -206,11 +234,11 @@ __global__ __launch_bounds__(WAVE) void read_kernel(const ReadParams p) {
             for (int c = 0; c < CPL / 4; ++c) d4[c] = make_float4(kb[4 * c], kb[4 * c + 1], kb[4 * c + 2], kb[4 * c + 3]);
         }
     }
-    for (uint32_t e = l.lane; e < uint32_t(n) * dv; e += WAVE) {
-        const uint32_t i = e / dv;
+    for (uint32_t e = l.lane; e < uint32_t(n) * nrows; e += WAVE) {
+        const uint32_t i = e / nrows, at = i * dv + r_begin + (e - i * nrows);
         float u;
-        if constexpr (QBUF) u = float(reinterpret_cast<const int8_t*>(UB)[e]) * f16_to_f32(UBS[i]);
-        else u = bf16_to_f32(reinterpret_cast<const uint16_t*>(UB)[e]);
+        if constexpr (QBUF) u = float(reinterpret_cast<const int8_t*>(UB)[at]) * f16_to_f32(UBS[i]);
+        else u = bf16_to_f32(reinterpret_cast<const uint16_t*>(UB)[at]);
         lds_u[e] = u;
     }
     float alpha_p[NCH][4];                                        // a_n at this lane's columns
@@ -221,13 +249,13 @@ __global__ __launch_bounds__(WAVE) void read_kernel(const ReadParams p) {
     __syncthreads();
 
     constexpr int RR = 2;                                         // rows per pass over the buffered keys
-    for (uint32_t r0 = 0; r0 < dv; r0 += RR * T::RG) {
+    for (uint32_t r0 = r_begin; r0 < r_end; r0 += RR * T::RG) {
         uint32_t row[RR], rc[RR];
         float acc[RR][NCH][4];
 #pragma unroll
         for (int k = 0; k < RR; ++k) {
             row[k] = r0 + k * T::RG + l.rg;
-            rc[k] = row[k] < dv ? row[k] : dv - 1;
+            rc[k] = row[k] < r_end ? row[k] : r_end - 1;
 #pragma unroll
             for (int t = 0; t < NCH; ++t) {
                 const int col = t * CSTEP + 4 * cc;
@@ -270,7 +298,7 @@ __global__ __launch_bounds__(WAVE) void read_kernel(const ReadParams p) {
             for (int t = 0; t < NCH; ++t) kx[t] = *reinterpret_cast<const float4*>(lds_k + i * DK + t * CSTEP + 4 * cc);
 #pragma unroll
             for (int k = 0; k < RR; ++k) {
-                const float du = lds_u[i * dv + rc[k]];
+                const float du = lds_u[i * nrows + rc[k] - r_begin];
 #pragma unroll
                 for (int t = 0; t < NCH; ++t) {
                     acc[k][t][0] = __builtin_fmaf(du, kx[t].x, acc[k][t][0]);
@@ -282,7 +310,7 @@ __global__ __launch_bounds__(WAVE) void read_kernel(const ReadParams p) {
         }
 #pragma unroll
         for (int k = 0; k < RR; ++k)
-            if (row[k] < dv && live) {
+            if (row[k] < r_end && live) {
 #pragma unroll
                 for (int t = 0; t < NCH; ++t)
                     *reinterpret_cast<float4*>(out + row[k] * DK + t * CSTEP + 4 * l.cg) =
@@ -293,8 +321,11 @@ __global__ __launch_bounds__(WAVE) void read_kernel(const ReadParams p) {
 
 template <int BITS, int DK, int GROUP, bool QBUF, bool KDA, bool AXV>
 int launch_read(const ReadParams& p, hipStream_t stream) {
-    const size_t lds = size_t(p.m) * (DK + p.dv) * sizeof(float);
-    hipLaunchKernelGGL((read_kernel<BITS, DK, GROUP, QBUF, KDA, AXV>), dim3(p.rows * p.hv), dim3(WAVE), lds, stream, p);
+    const uint32_t heads = uint32_t(p.rows) * uint32_t(p.hv);
+    const RowSplit sp = split_rows(heads, p.dv, 2 * RowTile<BITS, DK, GROUP, QBUF, AXV>::RG);
+    const size_t lds = size_t(p.m) * (DK + sp.rows) * sizeof(float);
+    hipLaunchKernelGGL((read_kernel<BITS, DK, GROUP, QBUF, KDA, AXV>), dim3(heads, sp.parts), dim3(WAVE), lds, stream, p,
+                       sp.rows);
     return int(hipGetLastError());
 }
 
