@@ -77,7 +77,7 @@ PARAMS = {'gdn': 'GdnParams', 'kda': 'KdaParams', 'mamba2': 'Mamba2Params'}
 QUAD_FAMILIES = {'gdn': (2, 1), 'mamba2': (4, 2, 1), 'kda': (1,)}
 # compile-time specialisations of the step kernels (SPEC, sq_params.h), most specific first; 0: everything read from
 # the arguments.  Built for the default buffer (int8, 8 tokens) only.
-SPECS = {'gdn': (1, 2, 0), 'kda': (1, 0), 'mamba2': (1, 0)}
+SPECS = {'gdn': (1, 2, 0), 'kda': (1, 0), 'mamba2': (1, 2, 0)}
 
 
 def specs_of(fam, c, quad):
@@ -131,29 +131,35 @@ QUAD_OK = {'gdn': [
 def quad_variants(fam, c):
     """[(row blocks per wavefront, value heads per workgroup, wavefronts per SIMD the register allocation aims
     for)], widest head group first, of the workgroup-per-key-head kernels (sq_quad.cuh) for a case; empty where only
-    the one-wavefront kernels (sq_tile.cuh) serve it: value-axis groups other than 32 rows, the float state, rows that
-    are not a power of two in size, d_k above 128, more than four scale groups per row."""
+    the one-wavefront kernels (sq_tile.cuh) serve it: value-axis groups other than 32 rows, the fp32 state, d_v that is no
+    multiple of 32, d_k above 128, more than four scale groups per row, states beyond 64 KB."""
     bits, dk, dv, group, qbuf, mmax, axv = c
-    if fam not in QUAD_FAMILIES or bits not in (4, 8) or (axv and group != 32):
+    if fam not in QUAD_FAMILIES or bits not in (4, 8, 16) or (axv and group != 32):
         return []
-    rb = dk * bits // 8
-    if rb & (rb - 1) or not 32 <= rb <= 128 or dk > 128 or dv % 32 or (bits == 4 and dk % 64):
+    flt = bits == 16
+    dkp = 1 << (dk - 1).bit_length()
+    rb = 1 << (dk * bits // 8 - 1).bit_length()              # LDS row: the next power of two
+    if (dk * bits // 8) % 16 or not 32 <= rb <= 256 or dk > 128 or dv % 32:
         return []
-    if not axv and -(-dk // group) > 4:
+    if not axv and not flt and -(-dk // group) > 4:
         return []
     nrb = dv // 32
-    nb = 2 if nrb % 2 == 0 and fam != 'kda' else 1
+    # row blocks per wavefront: one for the bf16 state, whose blocks are 8 KB each (a head of 128 x 128 on two wavefronts
+    # leaves eight per compute unit)
+    nb = 2 if nrb % 2 == 0 and fam != 'kda' and not flt else 1
     be = 1 if qbuf else 2
     out = []
     for gh in QUAD_FAMILIES[fam]:
         nw = gh * nrb // nb
         if nw > 16:
             continue
-        lds = gh * dv * rb + mmax * dk * be + gh * mmax * dv * be + 2 * dk * 4 + dk * 8 + 512
+        lds = gh * dv * rb + mmax * dkp * be + gh * mmax * dv * be + 2 * dkp * 4 + (0 if flt else dkp * 8) + 512
         if fam == 'kda':                                 # keys x decay ratio in fp32 (the raw ones stay in registers), decays
-            lds += mmax * dk * 4 + 2 * dk * 4 + (2 * dk * 4 if axv else 0)
+            lds += mmax * dkp * 4 + 2 * dkp * 4 + (2 * dkp * 4 if axv or flt else 0)
         if axv:                                          # a plane set per wavefront
-            lds += nw * dk * 6 - dk * 8
+            lds += nw * dkp * 6 - dkp * 8
+        if lds > (40 * 1024 if flt and gh > 1 else 63 * 1024):      # heads share a workgroup only while four of them fit
+            continue
         wgs = min(160 * 1024 // lds, 32 // nw)
         if wgs < 1:
             continue

@@ -152,7 +152,7 @@ void gdn_step_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     constexpr int KT = KeyBuf<T>::KT;
     const bool own_key = !p.qk_per_key_head && gqa > 1;
     const LaneId l = lane_id<T>();
-    TileId tid = tile_id_lead<SPEC>(order, per_xcd, hv, hv_shift);          // from the leading arguments
+    TileId tid = tile_id_lead<(SPEC > 0 && heads_pow2(T::DK))>(order, per_xcd, hv, hv_shift);          // from the leading arguments
     const int32_t slot = idx ? idx[tid.b] : tid.b;               // scalar load: on its way while the inputs are issued
     tid.hk = p.gqa_shift >= 0 ? tid.h >> p.gqa_shift : tid.h / p.gqa;
     GdnFront<T> F;

@@ -69,8 +69,8 @@ struct GdnLoads {
 };
 
 // SPEC > 0 compiles the serving cases in, so that dtypes and options cost no scalar branches on the way to the first
-// load (measured on the 128 x 128 int8 step: 35.4 -> 34.2 us per launch): bf16 q / k / v / out,
-// head counts that are powers of two, and  1: g and beta given as fp32;  2: the gate formed in the kernel from bf16
+// load (measured on the 128 x 128 int8 step: 35.4 -> 34.2 us per launch): bf16 q / k / v / out, head
+// counts that are powers of two where d_k is one, and  1: g and beta given as fp32;  2: the gate formed in the kernel from bf16
 // a, b and fp32 A_log, dt_bias.  SPEC = 0 reads all of it from the arguments.
 template <class T, int NB, int GH, int WPE, int SPEC>
 __global__ __launch_bounds__((Quad<T, NB, GH>::THREADS), WPE)
@@ -82,7 +82,7 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     // the leading arguments (copies of fields of `p`) are what the slot index load, the fill counter and the row blocks
     // need: as separate scalar arguments they are preloaded into registers at wave launch, so those requests go out
     // without waiting for the argument block
-    constexpr bool FIX = SPEC > 0;
+    constexpr bool FIX = SPEC > 0, POW2 = FIX && heads_pow2(T::DK);
     const int q_dt = FIX ? int(BF16) : p.q_dt, k_dt = FIX ? int(BF16) : p.k_dt, v_dt = FIX ? int(BF16) : p.v_dt;
     const int out_dt = FIX ? int(BF16) : p.out_dt;
     const int a_dt = SPEC == 1 ? int(F32) : SPEC == 2 ? int(BF16) : p.a_dt;
@@ -91,7 +91,7 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     const bool gate = SPEC == 1 ? false : SPEC == 2 ? true : p.gate != 0;
     using Q = Quad<T, NB, GH>;
     using L = QuadLds<T, NB, GH, 2, 2>;
-    constexpr int DK = T::DK, DV = T::DV, NW = Q::NW, NWH = Q::NWH, MM = T::MMAX, NE = Q::NE, NG = T::NG;
+    constexpr int DK = T::DK, DV = T::DV, NW = Q::NW, NWH = Q::NWH, MM = T::MMAX, NE = Q::NE, NG = T::NG, DKP = Q::DKP;
     constexpr int RQ = 1 % NW, RK = 3 % NW, RX = 2 % NW;          // which wavefront plays which shared role
     __shared__ __attribute__((aligned(16))) uint8_t lds[L::BYTES];
     uint8_t* lds_kbr = lds + L::KBR;
@@ -113,7 +113,6 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     float* lds_gbf = reinterpret_cast<float*>(lds + L::GBF) + hl * MM;
     uint16_t* lds_sc = reinterpret_cast<uint16_t*>(lds + L::SC) + hl * (DV * NG);
     uint8_t* my_codes = lds + L::CODES + hl * Q::HEAD + wh * NB * Q::BLK;
-    static_assert((WAVE / Q::CPR) % (Q::SWD * Q::SWM) == 0 || Q::NLD == 1, "swizzle period");
 
     // ---- this workgroup's item: (batch row, head group), dealt so that every XCD walks a contiguous range ----
     const int ngrp = hv / GH;                                     // head groups per batch row
@@ -122,12 +121,12 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     {
         const int wg = blockIdx.x;
         const int item = per_xcd ? (wg & 7) * per_xcd + (wg >> 3) : wg;
-        tid.b = (FIX || hv_shift >= 0) ? item >> (hv_shift - ilog2(GH)) : item / ngrp;
+        tid.b = (POW2 || hv_shift >= 0) ? item >> (hv_shift - ilog2(GH)) : item / ngrp;
         tid.h = (item - tid.b * ngrp) * GH + hl;
         if (order) tid.b = order[tid.b];            // the caller's dispatch order: position -> batch row
         SQ_MARK(1);                                               // item known (the leading arguments are here)
         slot = idx ? idx[tid.b] : tid.b;
-        tid.hk = (FIX || p.gqa_shift >= 0) ? tid.h >> p.gqa_shift : tid.h / p.gqa;
+        tid.hk = (POW2 || p.gqa_shift >= 0) ? tid.h >> p.gqa_shift : tid.h / p.gqa;
     }
     const int lane = lane0;
     const int n32 = lane & 31, kb = lane >> 5;
@@ -135,20 +134,21 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     const int row = (wh * NB + (NB == 2 ? kb : 0)) * T::MR + n32;
 
     GdnLoads<T, Q> F;
+    const int vl = Q::vec_lane(lane);                             // whose elements of a d_k vector this lane loads
     // ---- issue every load: first the token's own operands (their addresses need the batch row only: they go out
     //      while the slot index is on its way, and being older than the row blocks they are back before them) ...
     {
         const uint32_t b = tid.b, h = tid.h;
         if constexpr (RQ == RK) {                                 // a single wavefront carries both vectors
             if (w == RQ) {
-                load_vec<NE>(advance(p.q, q_dt, uint64_t(b) * p.s_q + uint32_t(tid.hk) * DK), q_dt, lane, F.xr);
-                load_vec<NE>(advance(p.k, k_dt, uint64_t(b) * p.s_k + uint32_t(tid.hk) * DK), k_dt, lane, F.xr2);
+                load_vec<NE>(advance(p.q, q_dt, uint64_t(b) * p.s_q + uint32_t(tid.hk) * DK), q_dt, vl, F.xr);
+                load_vec<NE>(advance(p.k, k_dt, uint64_t(b) * p.s_k + uint32_t(tid.hk) * DK), k_dt, vl, F.xr2);
             }
         } else if (w == RQ || w == RK) {
             const bool isq = w == RQ;
             const void* base = isq ? advance(p.q, q_dt, uint64_t(b) * p.s_q + uint32_t(tid.hk) * DK)
                                    : advance(p.k, k_dt, uint64_t(b) * p.s_k + uint32_t(tid.hk) * DK);
-            load_vec<NE>(base, isq ? q_dt : k_dt, lane, F.xr);
+            load_vec<NE>(base, isq ? q_dt : k_dt, vl, F.xr);
         }
         if (wh == 0) {
             F.g0 = load_raw_uniform(p.a, a_dt, uint64_t(b) * p.s_a + h);
@@ -172,7 +172,7 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     // and the fill counter (a scalar load; sq_quad.cuh) -- behind the row blocks, because the first wait for any
     // scalar load, the argument block's included, waits for it as well ...
     quad_start_wait<Q, WPE>(start_ramp);                  // the launch's first workgroups: spread over a ramp
-    quad_dma_blocks<Q, NB>(field(codes, uint32_t(slot), codes_stride, uint32_t(tid.h) * (DV * T::ROW_BYTES)) + wh * NB * Q::BLK,
+    quad_dma_blocks<Q, NB>(field(codes, uint32_t(slot), codes_stride, uint32_t(tid.h) * (DV * T::ROW_BYTES)) + wh * NB * Q::GBLK,
                            my_codes, lane);
     SQ_MARK(3);                                                   // row blocks issued
     F.np = quad_dma_counter(field(counters, uint32_t(slot), counters_stride, uint32_t(tid.h)));
@@ -187,8 +187,8 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
 #pragma unroll
         for (int bi = 0; bi < NB; ++bi) {
             if constexpr (T::AXV) {
-                F.scv[bi] = quad_load_colscales<NE>(A.SCh + (wh * NB + bi) * DK, lane);
-            } else {
+                F.scv[bi] = quad_load_colscales<NE>(A.SCh + (wh * NB + bi) * DK, vl);
+            } else if constexpr (!T::FLT) {
 #pragma unroll
                 for (int g = 0; g < NG; ++g) F.sc[bi][g] = stream_load(A.SCh + uint32_t(((wh * NB + bi) * T::MR + n32) * NG + g));
             }
@@ -210,7 +210,7 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
         for (int t = 0; t < Q::KT; ++t) {
             const uint32_t i = Q::SPP * (NW * t + w) + lane / Q::LPS;
             const uint32_t ic = i < nl ? i : nl - 1;
-            F.kraw[t] = stream_raw4<T::QBUF>(A.buf.KB + (ic * DK + 4 * (lane % Q::LPS)) * T::BE);
+            F.kraw[t] = stream_raw4<T::QBUF>(A.buf.KB + (ic * DK + Q::key_col(lane)) * T::BE);
             F.kbs[t] = T::QBUF ? A.buf.KBS[ic] : uint16_t(0);
         }
         // per slot of this head, lane i: cumulative decay and value scale
@@ -229,16 +229,16 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
         float xe[NE], ss = 0.0f;
 #pragma unroll
         for (int t = 0; t < NE; ++t) {
-            xe[t] = vec_elem<NE>(raw, dt, t);
+            xe[t] = Q::vec_live(lane) ? vec_elem<NE>(raw, dt, t) : 0.0f;
             ss = __builtin_fmaf(xe[t], xe[t], ss);
         }
         const float nrm = sqrtf(lanes_sum<WAVE>(ss) + 1e-6f);
 #pragma unroll
         for (int t = 0; t < NE; ++t) xe[t] = xe[t] / nrm * post;
-        if constexpr (NE == 1) lds_xn[v * DK + lane] = xe[0];
-        else if constexpr (NE == 2) *reinterpret_cast<float2*>(lds_xn + v * DK + 2 * lane) = make_float2(xe[0], xe[1]);
-        else *reinterpret_cast<float4*>(lds_xn + v * DK + 4 * lane) = make_float4(xe[0], xe[1], xe[2], xe[3]);
-        if constexpr (!T::AXV) quad_stage_planes<Q, T, NE>(xe, v, lane, lds_pl, lds_xs);
+        if constexpr (NE == 1) lds_xn[v * DKP + lane] = xe[0];
+        else if constexpr (NE == 2) *reinterpret_cast<float2*>(lds_xn + v * DKP + 2 * lane) = make_float2(xe[0], xe[1]);
+        else *reinterpret_cast<float4*>(lds_xn + v * DKP + 4 * lane) = make_float4(xe[0], xe[1], xe[2], xe[3]);
+        if constexpr (!T::AXV && !T::FLT) quad_stage_planes<Q, T, NE>(xe, v, lane, lds_pl, lds_xs);
     };
     if constexpr (RQ == RK) {
         if (w == RQ) {
@@ -274,7 +274,7 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     uint16_t scw[NB][NG];
 #pragma unroll
     for (int bi = 0; bi < NB; ++bi) {
-        if constexpr (!T::AXV) {
+        if constexpr (!T::AXV && !T::FLT) {
 #pragma unroll
             for (int g = 0; g < NG; ++g) {
                 scw[bi][g] = F.sc[bi][g];
@@ -291,7 +291,7 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     for (int t = 0; t < Q::KT; ++t) {
         const int i = Q::SPP * (NW * t + w) + lane / Q::LPS;
         if (i < m) {
-            store_raw4<T::QBUF>(lds_kbr + (i * DK + 4 * (lane % Q::LPS)) * T::BE, F.kraw[t]);
+            store_raw4<T::QBUF>(lds_kbr + (i * DKP + 4 * (lane % Q::LPS)) * T::BE, F.kraw[t]);
             if (T::QBUF && lane % Q::LPS == 0) lds_kbsf[i] = f16_to_f32(F.kbs[t]);
         }
     }
@@ -314,8 +314,11 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
             for (int bi = 0; bi < NB; ++bi)
                 own[bi] = quad_block_pass_v<Q, T, 2>(my_codes + bi * Q::BLK, lds_xn, F.scv[bi], lds_pl + w * L::PL_BYTES,
                                                      lds_xs + w * (L::XS_BYTES / 4), lane);
+        } else if constexpr (T::FLT) {
+#pragma unroll
+            for (int bi = 0; bi < NB; ++bi) own[bi] = quad_block_pass_f<Q, T, 2>(my_codes + bi * Q::BLK, lds_xn, lane);
         } else {
-            v4i aop[T::NKS];
+            v4i aop[Q::NKS];
             quad_fetch_planes<Q, T, 2>(lds_pl, lane, aop);
             float xs[NG];
 #pragma unroll
@@ -347,7 +350,7 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
         float x[2][4];
 #pragma unroll
         for (int v = 0; v < 2; ++v) {
-            const float4 f = *reinterpret_cast<const float4*>(lds_xn + v * DK + 4 * (lane % Q::LPS));
+            const float4 f = *reinterpret_cast<const float4*>(lds_xn + v * DKP + 4 * (lane % Q::LPS));
             x[v][0] = f.x; x[v][1] = f.y; x[v][2] = f.z; x[v][3] = f.w;
         }
 #pragma unroll
@@ -355,7 +358,7 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
             const int i = Q::SPP * (NW * t + w) + lane / Q::LPS;
             const int ic = i < m ? i : m - 1;
             float kf[4];
-            decode_raw4<T::QBUF>(load_raw4<T::QBUF>(lds_kbr + (ic * DK + 4 * (lane % Q::LPS)) * T::BE), kf);
+            decode_raw4<T::QBUF>(load_raw4<T::QBUF>(lds_kbr + (ic * DKP + 4 * (lane % Q::LPS)) * T::BE), kf);
             if constexpr (T::QBUF) {
                 const float s = lds_kbsf[ic];
 #pragma unroll
@@ -375,7 +378,7 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     if (w == RK) {
         float kqp = 0.0f;
 #pragma unroll
-        for (int t = 0; t < NE; ++t) kqp = __builtin_fmaf(lds_xn[DK + NE * lane + t], lds_xn[NE * lane + t], kqp);
+        for (int t = 0; t < NE; ++t) kqp = __builtin_fmaf(lds_xn[DKP + NE * lane + t], lds_xn[NE * lane + t], kqp);
         kqp = lanes_sum<WAVE>(kqp);
         if (lane == 0) lds_gsc[0] = kqp;
     }
@@ -389,12 +392,12 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
         float kxe[NE], kmax = 0.0f;
 #pragma unroll
         for (int t = 0; t < NE; ++t) {
-            kxe[t] = lds_xn[DK + NE * lane + t];
+            kxe[t] = lds_xn[DKP + NE * lane + t];
             kmax = fmaxf(kmax, fabsf(kxe[t]));
         }
         float ks = 1.0f;
         if constexpr (T::QBUF) ks = fp16_scale(lanes_max<WAVE>(kmax), 127.0f);
-        const bool write = tid.h - hl == tid.hk * p.gqa;
+        const bool live = Q::vec_live(lane), write = live && tid.h - hl == tid.hk * p.gqa;
         if (T::QBUF && lane == 0) {
             lds_kbsf[n] = ks;
             if (write) A.buf.KBS[n] = f32_to_f16(ks);
@@ -403,7 +406,7 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
             uint32_t pk = 0;
 #pragma unroll
             for (int t = 0; t < NE; ++t) pk |= (uint32_t(int(round_buf(kxe[t], ks))) & 0xFFu) << (8 * t);
-            uint8_t* dl = lds_kbr + n * DK + NE * lane;
+            uint8_t* dl = lds_kbr + n * DKP + NE * lane;
             uint8_t* dg = A.buf.KB + n * DK + NE * lane;
             if constexpr (NE == 1) { *dl = uint8_t(pk); if (write) *dg = uint8_t(pk); }
             else if constexpr (NE == 2) {
@@ -417,7 +420,7 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
 #pragma unroll
             for (int t = 0; t < NE; ++t) {
                 const uint16_t hb = f32_to_bf16(kxe[t]);
-                reinterpret_cast<uint16_t*>(lds_kbr)[n * DK + NE * lane + t] = hb;
+                reinterpret_cast<uint16_t*>(lds_kbr)[n * DKP + NE * lane + t] = hb;
                 if (write) reinterpret_cast<uint16_t*>(A.buf.KB)[n * DK + NE * lane + t] = hb;
             }
         }
@@ -498,7 +501,6 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
         // formed at the top of the kernel would otherwise be kept in registers all the way to here
         int lf = lane;
         asm volatile("" : "+v"(lf));
-        const int swzf = swz<Q>(lf / Q::CPR, lf % Q::CPR);
         const float cmul = expf(gnew);
         if constexpr (T::AXV) {
             constexpr int MT = (MM + 1) / 2;
@@ -511,7 +513,7 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
             }
             auto key = [&](int sl, int col) {
                 const int sc_ = sl < m ? sl : 0;
-                float kv = lds_raw<T::QBUF>(lds_kbr, sc_ * DK + col);
+                float kv = lds_raw<T::QBUF>(lds_kbr, sc_ * DKP + col);
                 if constexpr (T::QBUF) kv = kv * lds_kbsf[sc_];
                 return sl < m ? kv : 0.0f;
             };
@@ -534,13 +536,10 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
                 }
                 quad_fold_block_v<Q, T>(blk, key, dop, [&](int) { return cmul; }, cmul == 1.0f, old,
                                         A.SCh + grp * DK, lf);
-#pragma unroll
-                for (int t = 0; t < Q::NLD; ++t)
-                    stream_store(reinterpret_cast<v4u*>(A.Sh + grp * Q::BLK + t * 1024 + lf * 16),
-                                 *reinterpret_cast<const v4u*>(blk + t * 1024 + swzf));
+                quad_store_block<Q>(A.Sh + grp * Q::GBLK, blk, lf);
             }
         } else {
-            constexpr int MT4 = (MM + 3) / 4, CL = DK / 4;
+            constexpr int MT4 = (MM + 3) / 4, CL = DKP / 4;
             const int fn = lf & 15, fq = lf >> 4;
             // decay ratios a_m / a_i of the lane's slots 4 t + q (this token: 1)
             float decf[MT4];
@@ -549,7 +548,7 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
                 const int sl = 4 * t + fq;
                 decf[t] = sl < m - 1 ? expf(gnew - lds_gbf[sl < m - 1 ? sl : 0]) : 1.0f;
             }
-            const int fg = (fq * CL) / T::KGROUP;
+            const int fg = min((fq * CL) / T::KGROUP, NG - 1);
             FoldKeys<T> kop;
             quad_fold_keys<T>(lds_kbr, lds_kbsf, m, lf, kop);
 #pragma unroll
@@ -568,14 +567,14 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
                         uv = decf[t] * uv;
                         bop[t] = sl < m ? uv : 0.0f;
                     }
-                    quad_fold_half<Q, T>(blk, hf, kop, bop, cmul, f16_to_f32(lds_sc[frow * NG + fg]),
+                    if constexpr (T::FLT)
+                        quad_fold_half_f<Q, T>(blk, hf, kop, bop, cmul, lf);
+                    else
+                        quad_fold_half<Q, T>(blk, hf, kop, bop, cmul, f16_to_f32(lds_sc[frow * NG + fg]),
                                                 A.SCh + frow * NG + fg, lf);
                 }
                 wave_sync();
-#pragma unroll
-                for (int t = 0; t < Q::NLD; ++t)
-                    stream_store(reinterpret_cast<v4u*>(A.Sh + (wh * NB + bi) * Q::BLK + t * 1024 + lf * 16),
-                                 *reinterpret_cast<const v4u*>(blk + t * 1024 + swzf));
+                quad_store_block<Q>(A.Sh + (wh * NB + bi) * Q::GBLK, blk, lf);
             }
         }
     }

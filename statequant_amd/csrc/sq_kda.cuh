@@ -43,7 +43,7 @@ void kda_step_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     float* lds_c = reinterpret_cast<float*>(lds + L::FC);
 
     const LaneId l = lane_id<T>();
-    const TileId tid = tile_id_lead<SPEC>(order, per_xcd, hv, hv_shift);   // from the leading arguments
+    const TileId tid = tile_id_lead<(SPEC > 0 && heads_pow2(T::DK))>(order, per_xcd, hv, hv_shift);   // from the leading arguments
     const uint32_t b = tid.b, h = tid.h;
     const int m = p.m;
     const uint32_t um = m;

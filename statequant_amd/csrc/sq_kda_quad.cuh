@@ -41,14 +41,15 @@ template <class T, int NB>
 struct KdaLds {
     using Q = Quad<T, NB, 1>;
     using B = QuadLds<T, NB, 1, 2, 2>;                               // read-out vectors: q, k (normalised)
-    static constexpr int GN = B::BYTES;                              // [DK] G_n
-    static constexpr int CM = GN + T::DK * 4;                        // [DK] A = exp(G_n)
-    static constexpr int XA = CM + T::DK * 4;                        // [2][DK] A q, A k (value-axis groups: planes per block)
-    static constexpr int KD = XA + (T::AXV ? 2 * T::DK * 4 : 0);     // [m][DK] buffered keys x decay ratio, fp32
-    static constexpr int BYTES = KD + T::MMAX * T::DK * 4;
+    static constexpr int GN = B::BYTES;                              // [DKP] G_n
+    static constexpr int CM = GN + Q::DKP * 4;                       // [DKP] A = exp(G_n)
+    static constexpr int XA = CM + Q::DKP * 4;                       // [2][DKP] A q, A k (value-axis groups: planes per block)
+    static constexpr int KD = XA + (T::AXV || T::FLT ? 2 * Q::DKP * 4 : 0);  // [m][DKP] buffered keys x decay ratio, fp32
+    static constexpr int BYTES = KD + T::MMAX * Q::DKP * 4;
 };
 
-// SPEC = 1: the serving case compiled in -- bf16 q / k / v / out, fp32 g and beta, a power-of-two head count.
+// SPEC = 1: the serving case compiled in -- bf16 q / k / v / out, fp32 g and beta, a power-of-two
+// head count where d_k is one too.
 template <class T, int NB, int WPE, int SPEC>
 __global__ __launch_bounds__((Quad<T, NB, 1>::THREADS), WPE)
 void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict__ order, int per_xcd, int hv, int hv_shift,
@@ -61,7 +62,7 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     using Q = Quad<T, NB, 1>;
     using L = QuadLds<T, NB, 1, 2, 2>;
     using K = KdaLds<T, NB>;
-    constexpr int DK = T::DK, DV = T::DV, NW = Q::NW, MM = T::MMAX, NE = Q::NE, NG = T::NG;
+    constexpr int DK = T::DK, DV = T::DV, NW = Q::NW, MM = T::MMAX, NE = Q::NE, NG = T::NG, DKP = Q::DKP;
     constexpr int RQ = 1 % NW, RK = 3 % NW, RX = 2 % NW, RG = 0;  // which wavefront plays which shared role
     __shared__ __attribute__((aligned(16))) uint8_t lds[K::BYTES];
     float* lds_xn = reinterpret_cast<float*>(lds + L::XN);
@@ -83,9 +84,8 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     const int m = p.m;
     const uint32_t um = m;
     uint8_t* my_codes = lds + L::CODES + w * NB * Q::BLK;
-    static_assert((WAVE / Q::CPR) % (Q::SWD * Q::SWM) == 0 || Q::NLD == 1, "swizzle period");
 
-    const TileId tid = tile_id_lead<SPEC>(order, per_xcd, hv, hv_shift);
+    const TileId tid = tile_id_lead<(FIX && heads_pow2(T::DK))>(order, per_xcd, hv, hv_shift);
     const uint32_t b = tid.b, h = tid.h;
     const int32_t slot = idx ? idx[b] : int32_t(b);
     const int n32 = lane & 31, kb = lane >> 5;
@@ -93,12 +93,13 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     const int row = (w * NB + (NB == 2 ? kb : 0)) * T::MR + n32;
 
     KdaLoads<T, Q> F;
+    const int vl = Q::vec_lane(lane);                             // whose elements of a d_k vector this lane loads
     // ---- issue every load: first the token's own operands (their addresses need the batch row only) ...
     if (w == RQ)
-        load_vec<NE>(advance(p.q, q_dt, uint64_t(b) * p.s_q + h * DK), q_dt, lane, F.xr);
+        load_vec<NE>(advance(p.q, q_dt, uint64_t(b) * p.s_q + h * DK), q_dt, vl, F.xr);
     if (w == RK)
-        load_vec<NE>(advance(p.k, k_dt, uint64_t(b) * p.s_k + h * DK), k_dt, lane, RQ == RK ? F.xr2 : F.xr);
-    if (w == RQ || w == RK) load_vec<NE>(advance(p.g, g_dt, uint64_t(b) * p.s_g + h * DK), g_dt, lane, F.gr);
+        load_vec<NE>(advance(p.k, k_dt, uint64_t(b) * p.s_k + h * DK), k_dt, vl, RQ == RK ? F.xr2 : F.xr);
+    if (w == RQ || w == RK) load_vec<NE>(advance(p.g, g_dt, uint64_t(b) * p.s_g + h * DK), g_dt, vl, F.gr);
     F.beta = load_raw_uniform(p.beta, beta_dt, uint64_t(b) * p.s_beta + h);
     F.vr = load_raw(advance(p.v, v_dt, uint64_t(b) * p.s_v + h * DV), v_dt, uint32_t(row));
     void* const outp = advance(p.out, out_dt, uint64_t(b) * p.s_out + h * DV);
@@ -111,11 +112,11 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     float* const gch = field(p.st.GCUR, seq, p.st.sGC, h * DK);
     if (w == RQ || w == RK) {                            // the running decay, ahead of the row blocks: the roles wait for it
 #pragma unroll
-        for (int t = 0; t < NE; ++t) F.gc[t] = gch[NE * lane + t];
+        for (int t = 0; t < NE; ++t) F.gc[t] = gch[NE * vl + t];
     }
     // ... then the row blocks, straight into their LDS image, and the fill counter (a scalar load; sq_quad.cuh) ...
     quad_start_wait<Q, WPE>(start_ramp);
-    quad_dma_blocks<Q, NB>(field(codes, seq, codes_stride, h * (DV * T::ROW_BYTES)) + w * NB * Q::BLK, my_codes, lane);
+    quad_dma_blocks<Q, NB>(field(codes, seq, codes_stride, h * (DV * T::ROW_BYTES)) + w * NB * Q::GBLK, my_codes, lane);
     F.np = quad_dma_counter(field(counters, seq, counters_stride, h));
     __builtin_amdgcn_sched_barrier(0);
     // ... and the rest of the slot: scales and -- once the fill counter is here -- the live part of the decode buffer
@@ -130,8 +131,8 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
 #pragma unroll
     for (int bi = 0; bi < NB; ++bi) {
         if constexpr (T::AXV) {
-            F.scv[bi] = quad_load_colscales<NE>(SCh + (w * NB + bi) * DK, lane);
-        } else {
+            F.scv[bi] = quad_load_colscales<NE>(SCh + (w * NB + bi) * DK, vl);
+        } else if constexpr (!T::FLT) {
 #pragma unroll
             for (int g = 0; g < NG; ++g) F.sc[bi][g] = stream_load(SCh + uint32_t(((w * NB + bi) * T::MR + n32) * NG + g));
         }
@@ -149,9 +150,9 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     for (int t = 0; t < Q::KT; ++t) {                    // lane (slot = SPP (NW t + w) + lane / LPS, columns 4 (lane % LPS) ..)
         const uint32_t i = Q::SPP * (NW * t + w) + lane / Q::LPS;
         const uint32_t ic = i < nl ? i : nl - 1;
-        F.kraw[t] = stream_raw4<T::QBUF>(buf.KB + (ic * DK + 4 * (lane % Q::LPS)) * T::BE);
+        F.kraw[t] = stream_raw4<T::QBUF>(buf.KB + (ic * DK + Q::key_col(lane)) * T::BE);
         typedef float v4fl __attribute__((ext_vector_type(4)));
-        const v4fl g4 = stream_load(reinterpret_cast<const v4fl*>(GBh + ic * DK + 4 * (lane % Q::LPS)));
+        const v4fl g4 = stream_load(reinterpret_cast<const v4fl*>(GBh + ic * DK + Q::key_col(lane)));
         F.gb[t] = make_float4(g4.x, g4.y, g4.z, g4.w);
         F.kbs[t] = T::QBUF ? buf.KBS[ic] : uint16_t(0);
     }
@@ -165,7 +166,7 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
         float xe[NE], xa[NE], ss = 0.0f;
 #pragma unroll
         for (int t = 0; t < NE; ++t) {
-            xe[t] = vec_elem<NE>(raw, dt, t);
+            xe[t] = Q::vec_live(lane) ? vec_elem<NE>(raw, dt, t) : 0.0f;
             ss = __builtin_fmaf(xe[t], xe[t], ss);
         }
         const float nrm = sqrtf(lanes_sum<WAVE>(ss) + 1e-6f);
@@ -175,14 +176,14 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
             const float gn = F.gc[t] + vec_elem<NE>(F.gr, g_dt, t);
             const float A = kda_exp(gn);
             xa[t] = A * xe[t];
-            lds_xn[v * DK + NE * lane + t] = xe[t];
+            lds_xn[v * DKP + NE * lane + t] = xe[t];
             if (v == 0) {
                 lds_gn[NE * lane + t] = gn;
                 lds_cm[NE * lane + t] = A;
             }
-            if constexpr (T::AXV) lds_xa[v * DK + NE * lane + t] = xa[t];
+            if constexpr (T::AXV || T::FLT) lds_xa[v * DKP + NE * lane + t] = xa[t];
         }
-        if constexpr (!T::AXV) quad_stage_planes<Q, T, NE>(xa, v, lane, lds_pl, lds_xs);
+        if constexpr (!T::AXV && !T::FLT) quad_stage_planes<Q, T, NE>(xa, v, lane, lds_pl, lds_xs);
     };
     if (w == RQ) role_vector(F.xr, q_dt, p.scale, 0);
     if (w == RK) role_vector(RQ == RK ? F.xr2 : F.xr, k_dt, 1.0f, 1);
@@ -192,7 +193,7 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     uint16_t scw[NB][NG];
 #pragma unroll
     for (int bi = 0; bi < NB; ++bi) {
-        if constexpr (!T::AXV) {
+        if constexpr (!T::AXV && !T::FLT) {
 #pragma unroll
             for (int g = 0; g < NG; ++g) {
                 scw[bi][g] = F.sc[bi][g];
@@ -216,7 +217,7 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
         const int c4 = 4 * (lane % Q::LPS);
 #pragma unroll
         for (int v = 0; v < 2; ++v) {
-            const float4 f = *reinterpret_cast<const float4*>(lds_xn + v * DK + c4);
+            const float4 f = *reinterpret_cast<const float4*>(lds_xn + v * DKP + c4);
             x[v][0] = f.x; x[v][1] = f.y; x[v][2] = f.z; x[v][3] = f.w;
         }
         {
@@ -236,7 +237,7 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
                 if constexpr (T::QBUF) kf[c] = kf[c] * ks;
                 kf[c] = alive ? kf[c] * kda_exp(gn[c] - gi[c]) : 0.0f;
             }
-            if (full && i < n) *reinterpret_cast<float4*>(lds_kd + i * DK + c4) = make_float4(kf[0], kf[1], kf[2], kf[3]);
+            if (full && i < n) *reinterpret_cast<float4*>(lds_kd + i * DKP + c4) = make_float4(kf[0], kf[1], kf[2], kf[3]);
 #pragma unroll
             for (int v = 0; v < 2; ++v) {
                 float pr = kf[0] * x[v][0];
@@ -250,7 +251,7 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     if (w == RK) {                                                // k . q
         float kqp = 0.0f;
 #pragma unroll
-        for (int t = 0; t < NE; ++t) kqp = __builtin_fmaf(lds_xn[DK + NE * lane + t], lds_xn[NE * lane + t], kqp);
+        for (int t = 0; t < NE; ++t) kqp = __builtin_fmaf(lds_xn[DKP + NE * lane + t], lds_xn[NE * lane + t], kqp);
         kqp = lanes_sum<WAVE>(kqp);
         if (lane == 0) lds_scal[0] = kqp;
     }
@@ -264,8 +265,11 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
             for (int bi = 0; bi < NB; ++bi)
                 own[bi] = quad_block_pass_v<Q, T, 2>(my_codes + bi * Q::BLK, lds_xa, F.scv[bi], lds_pl + w * L::PL_BYTES,
                                                      lds_xs + w * (L::XS_BYTES / 4), lane);
+        } else if constexpr (T::FLT) {
+#pragma unroll
+            for (int bi = 0; bi < NB; ++bi) own[bi] = quad_block_pass_f<Q, T, 2>(my_codes + bi * Q::BLK, lds_xa, lane);
         } else {
-            v4i aop[T::NKS];
+            v4i aop[Q::NKS];
             quad_fetch_planes<Q, T, 2>(lds_pl, lane, aop);
             float xs[NG];
 #pragma unroll
@@ -296,7 +300,7 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
         float kxe[NE], kmax = 0.0f;
 #pragma unroll
         for (int t = 0; t < NE; ++t) {
-            kxe[t] = lds_xn[DK + NE * lane + t];
+            kxe[t] = lds_xn[DKP + NE * lane + t];
             kmax = fmaxf(kmax, fabsf(kxe[t]));
         }
         float ks = 1.0f;
@@ -313,18 +317,18 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
             } else {
                 const uint16_t hb = f32_to_bf16(kxe[t]);
                 kr = bf16_to_f32(hb);
-                reinterpret_cast<uint16_t*>(buf.KB)[n * DK + NE * lane + t] = hb;
+                if (Q::vec_live(lane)) reinterpret_cast<uint16_t*>(buf.KB)[n * DK + NE * lane + t] = hb;
             }
-            if (full) lds_kd[n * DK + NE * lane + t] = kr;
+            if (full) lds_kd[n * DKP + NE * lane + t] = kr;
         }
-        if constexpr (T::QBUF) {
+        if (T::QBUF && Q::vec_live(lane)) {
             uint8_t* dg = buf.KB + n * DK + NE * lane;
             if constexpr (NE == 1) *dg = uint8_t(pk);
             else if constexpr (NE == 2) *reinterpret_cast<uint16_t*>(dg) = uint16_t(pk);
             else *reinterpret_cast<uint32_t*>(dg) = pk;
         }
     }
-    if (w == RG) {
+    if (w == RG && Q::vec_live(lane)) {
 #pragma unroll
         for (int t = 0; t < NE; ++t) {
             const float gn = lds_gn[NE * lane + t];
@@ -387,12 +391,11 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
         lds_barrier();
         int lf = lane;                                   // (offsets derived anew: see the GDN kernel)
         asm volatile("" : "+v"(lf));
-        const int swzf = swz<Q>(lf / Q::CPR, lf % Q::CPR);
         if constexpr (T::AXV) {
             constexpr int MT = (MM + 1) / 2;
             const int fj = lf & 31, fkb = lf >> 5;
             auto key = [&](int sl, int col) {
-                const float kv = lds_kd[(sl < m ? sl : 0) * DK + col];
+                const float kv = lds_kd[(sl < m ? sl : 0) * DKP + col];
                 return sl < m ? kv : 0.0f;
             };
             auto cm = [&](int col) { return lds_cm[col]; };
@@ -413,15 +416,12 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
                     dop[t] = sl < m ? uv_ : 0.0f;
                 }
                 quad_fold_block_v<Q, T>(blk, key, dop, cm, false, old, SCh + grp * DK, lf);
-#pragma unroll
-                for (int t = 0; t < Q::NLD; ++t)
-                    stream_store(reinterpret_cast<v4u*>(Sh + grp * Q::BLK + t * 1024 + lf * 16),
-                                 *reinterpret_cast<const v4u*>(blk + t * 1024 + swzf));
+                quad_store_block<Q>(Sh + grp * Q::GBLK, blk, lf);
             }
         } else {
-            constexpr int MT4 = (MM + 3) / 4, CL = DK / 4;
+            constexpr int MT4 = (MM + 3) / 4, CL = DKP / 4;
             const int fn = lf & 15, fq = lf >> 4;
-            const int fg = (fq * CL) / T::KGROUP;
+            const int fg = min((fq * CL) / T::KGROUP, NG - 1);
             FoldKeys<T, true> kop;
             quad_fold_keys_f32<T>(lds_kd, m, lf, kop);
 #pragma unroll
@@ -439,14 +439,14 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
                         if constexpr (T::QBUF) uv_ = uv_ * lds_ubsf[sc_];
                         bop[t] = sl < m ? uv_ : 0.0f;
                     }
-                    quad_fold_half<Q, T, true>(blk, hf, kop, bop, 1.0f, f16_to_f32(lds_sc[frow * NG + fg]),
+                    if constexpr (T::FLT)
+                        quad_fold_half_f<Q, T, true>(blk, hf, kop, bop, 1.0f, lf, lds_cm);
+                    else
+                        quad_fold_half<Q, T, true>(blk, hf, kop, bop, 1.0f, f16_to_f32(lds_sc[frow * NG + fg]),
                                                SCh + frow * NG + fg, lf, lds_cm);
                 }
                 wave_sync();
-#pragma unroll
-                for (int t = 0; t < Q::NLD; ++t)
-                    stream_store(reinterpret_cast<v4u*>(Sh + (w * NB + bi) * Q::BLK + t * 1024 + lf * 16),
-                                 *reinterpret_cast<const v4u*>(blk + t * 1024 + swzf));
+                quad_store_block<Q>(Sh + (w * NB + bi) * Q::GBLK, blk, lf);
             }
         }
     }

@@ -26,21 +26,22 @@ struct Mamba2Loads {
     uint32_t xr[Q::NE], xr2[Q::NE], g0, g1, g2, g3, vr;
 };
 
-// SPEC = 1 compiles the serving case in (as in the Gated DeltaNet kernel): bf16 x / B / C / out, fp32 dt, A, D and
-// dt_bias, head counts that are powers of two.  SPEC = 0 reads all of it from the arguments.
+// SPEC > 0 compiles the serving case in (as in the Gated DeltaNet kernel): bf16 x / B / C / out, fp32 A, D and
+// dt_bias (dt comes as fp32 or bf16: one scalar load); 1: head counts that are powers of two (128 heads 36.0 -> 33.9 us
+// per launch against SPEC 0), 2: others.  SPEC = 0 reads all of it from the arguments.
 template <class T, int NB, int GH, int WPE, int SPEC>
 __global__ __launch_bounds__((Quad<T, NB, GH>::THREADS), WPE)
 void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict__ order, int per_xcd, int hv, int hv_shift,
                      const uint8_t* codes,
                         uint32_t codes_stride, const int32_t* counters, uint32_t counters_stride, uint32_t start_ramp,
                         const Mamba2Params p) {
-    constexpr bool FIX = SPEC > 0;
+    constexpr bool FIX = SPEC > 0, POW2 = SPEC == 1;
     const int x_dt = FIX ? int(BF16) : p.x_dt, B_dt = FIX ? int(BF16) : p.B_dt, C_dt = FIX ? int(BF16) : p.C_dt;
-    const int out_dt = FIX ? int(BF16) : p.out_dt, dt_dt = FIX ? int(F32) : p.dt_dt, A_dt = FIX ? int(F32) : p.A_dt;
+    const int out_dt = FIX ? int(BF16) : p.out_dt, dt_dt = p.dt_dt, A_dt = FIX ? int(F32) : p.A_dt;
     const int D_dt = FIX ? int(F32) : p.D_dt, dt_bias_dt = FIX ? int(F32) : p.dt_bias_dt;
     using Q = Quad<T, NB, GH>;
     using L = QuadLds<T, NB, GH, 2, 1>;
-    constexpr int DK = T::DK, DV = T::DV, NW = Q::NW, NWH = Q::NWH, MM = T::MMAX, NE = Q::NE, NG = T::NG;
+    constexpr int DK = T::DK, DV = T::DV, NW = Q::NW, NWH = Q::NWH, MM = T::MMAX, NE = Q::NE, NG = T::NG, DKP = Q::DKP;
     constexpr int RQ = 1 % NW, RK = 3 % NW, RX = 2 % NW;          // which wavefront plays which shared role
     __shared__ __attribute__((aligned(16))) uint8_t lds[L::BYTES];
     uint8_t* lds_kbr = lds + L::KBR;
@@ -62,7 +63,6 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
     float* lds_gbf = reinterpret_cast<float*>(lds + L::GBF) + hl * MM;
     uint16_t* lds_sc = reinterpret_cast<uint16_t*>(lds + L::SC) + hl * (DV * NG);
     uint8_t* my_codes = lds + L::CODES + hl * Q::HEAD + wh * NB * Q::BLK;
-    static_assert((WAVE / Q::CPR) % (Q::SWD * Q::SWM) == 0 || Q::NLD == 1, "swizzle period");
 
     // ---- this workgroup's item: (batch row, head group), dealt so that every XCD walks a contiguous range ----
     const int ngrp = hv / GH;
@@ -70,13 +70,13 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
     {
         const int wg = blockIdx.x;
         const int item = per_xcd ? (wg & 7) * per_xcd + (wg >> 3) : wg;
-        b = (FIX || hv_shift >= 0) ? item >> (hv_shift - ilog2(GH)) : item / ngrp;
+        b = (POW2 || hv_shift >= 0) ? item >> (hv_shift - ilog2(GH)) : item / ngrp;
         grp = item - b * ngrp;
         if (order) b = order[b];                    // the caller's dispatch order: position -> batch row
         slot = idx ? idx[b] : b;
     }
     const uint32_t h = grp * GH + hl;
-    const uint32_t hk = (FIX || p.gqa_shift >= 0) ? h >> p.gqa_shift : h / uint32_t(p.gqa);
+    const uint32_t hk = (POW2 || p.gqa_shift >= 0) ? h >> p.gqa_shift : h / uint32_t(p.gqa);
 
     const int lane = lane0;
     const int n32 = lane & 31, kb = lane >> 5;
@@ -84,18 +84,19 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
     const int row = (wh * NB + (NB == 2 ? kb : 0)) * T::MR + n32;
 
     Mamba2Loads<T, Q> F;
+    const int vl = Q::vec_lane(lane);                             // whose elements of a d_k vector this lane loads
     // ---- issue every load: first the token's own operands (their addresses need the batch row only; being older
     //      than the row blocks they are back before them) ...
     if constexpr (RQ == RK) {                                     // a single wavefront carries both vectors
         if (w == RQ) {
-            load_vec<NE>(advance(p.C, C_dt, uint64_t(uint32_t(b)) * p.s_C + hk * DK), C_dt, lane, F.xr);
-            load_vec<NE>(advance(p.B, B_dt, uint64_t(uint32_t(b)) * p.s_B + hk * DK), B_dt, lane, F.xr2);
+            load_vec<NE>(advance(p.C, C_dt, uint64_t(uint32_t(b)) * p.s_C + hk * DK), C_dt, vl, F.xr);
+            load_vec<NE>(advance(p.B, B_dt, uint64_t(uint32_t(b)) * p.s_B + hk * DK), B_dt, vl, F.xr2);
         }
     } else if (w == RQ || w == RK) {
         const bool isq = w == RQ;
         const void* base = isq ? advance(p.C, C_dt, uint64_t(uint32_t(b)) * p.s_C + hk * DK)
                                : advance(p.B, B_dt, uint64_t(uint32_t(b)) * p.s_B + hk * DK);
-        load_vec<NE>(base, isq ? C_dt : B_dt, lane, F.xr);
+        load_vec<NE>(base, isq ? C_dt : B_dt, vl, F.xr);
     }
     if (wh == 0) {
         F.g0 = load_raw_uniform(p.dt, dt_dt, uint64_t(uint32_t(b)) * p.s_dt + h);
@@ -112,7 +113,7 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
     // ... then the slot's big side, from the preloaded leading arguments alone: the row blocks, straight into their
     // LDS image, and the fill counter (a scalar load; sq_quad.cuh) behind them ...
     quad_start_wait<Q, WPE>(start_ramp);                  // the launch's first workgroups: spread over a ramp
-    quad_dma_blocks<Q, NB>(field(codes, uint32_t(slot), codes_stride, h * (DV * T::ROW_BYTES)) + wh * NB * Q::BLK, my_codes, lane);
+    quad_dma_blocks<Q, NB>(field(codes, uint32_t(slot), codes_stride, h * (DV * T::ROW_BYTES)) + wh * NB * Q::GBLK, my_codes, lane);
     F.np = quad_dma_counter(field(counters, uint32_t(slot), counters_stride, h));
     __builtin_amdgcn_sched_barrier(0);
     // ... and the rest of the slot
@@ -130,8 +131,8 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
 #pragma unroll
     for (int bi = 0; bi < NB; ++bi) {
         if constexpr (T::AXV) {
-            F.scv[bi] = quad_load_colscales<NE>(SCh + (wh * NB + bi) * DK, lane);
-        } else {
+            F.scv[bi] = quad_load_colscales<NE>(SCh + (wh * NB + bi) * DK, vl);
+        } else if constexpr (!T::FLT) {
 #pragma unroll
             for (int g = 0; g < NG; ++g) F.sc[bi][g] = stream_load(SCh + uint32_t(((wh * NB + bi) * T::MR + n32) * NG + g));
         }
@@ -153,7 +154,7 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
     for (int t = 0; t < Q::KT; ++t) {
         const uint32_t i = Q::SPP * (NW * t + w) + lane / Q::LPS;
         const uint32_t ic = i < nl ? i : nl - 1;
-        F.kraw[t] = stream_raw4<T::QBUF>(KBp + (ic * DK + 4 * (lane % Q::LPS)) * T::BE);
+        F.kraw[t] = stream_raw4<T::QBUF>(KBp + (ic * DK + Q::key_col(lane)) * T::BE);
         F.kbs[t] = T::QBUF ? KBSp[ic] : uint16_t(0);
     }
     {   // per slot of this head, lane i: cumulative decay and value scale
@@ -170,11 +171,13 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
     auto role_vector = [&](const uint32_t (&raw)[NE], int dt, int v) {
         float xe[NE];
 #pragma unroll
-        for (int t = 0; t < NE; ++t) xe[t] = vec_elem<NE>(raw, dt, t);
-        if constexpr (NE == 1) lds_xn[v * DK + lane] = xe[0];
-        else if constexpr (NE == 2) *reinterpret_cast<float2*>(lds_xn + v * DK + 2 * lane) = make_float2(xe[0], xe[1]);
-        else *reinterpret_cast<float4*>(lds_xn + v * DK + 4 * lane) = make_float4(xe[0], xe[1], xe[2], xe[3]);
-        if (!T::AXV && v == 0) quad_stage_planes<Q, T, NE>(xe, 0, lane, lds_pl, lds_xs);
+        for (int t = 0; t < NE; ++t) xe[t] = Q::vec_live(lane) ? vec_elem<NE>(raw, dt, t) : 0.0f;
+        if constexpr (NE == 1) lds_xn[v * DKP + lane] = xe[0];
+        else if constexpr (NE == 2) *reinterpret_cast<float2*>(lds_xn + v * DKP + 2 * lane) = make_float2(xe[0], xe[1]);
+        else *reinterpret_cast<float4*>(lds_xn + v * DKP + 4 * lane) = make_float4(xe[0], xe[1], xe[2], xe[3]);
+        if constexpr (!T::AXV && !T::FLT) {
+            if (v == 0) quad_stage_planes<Q, T, NE>(xe, 0, lane, lds_pl, lds_xs);
+        }
     };
     if constexpr (RQ == RK) {
         if (w == RQ) {
@@ -206,7 +209,7 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
     uint16_t scw[NB][NG];
 #pragma unroll
     for (int bi = 0; bi < NB; ++bi) {
-        if constexpr (!T::AXV) {
+        if constexpr (!T::AXV && !T::FLT) {
 #pragma unroll
             for (int g = 0; g < NG; ++g) {
                 scw[bi][g] = F.sc[bi][g];
@@ -223,7 +226,7 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
     for (int t = 0; t < Q::KT; ++t) {
         const int i = Q::SPP * (NW * t + w) + lane / Q::LPS;
         if (i < m) {
-            store_raw4<T::QBUF>(lds_kbr + (i * DK + 4 * (lane % Q::LPS)) * T::BE, F.kraw[t]);
+            store_raw4<T::QBUF>(lds_kbr + (i * DKP + 4 * (lane % Q::LPS)) * T::BE, F.kraw[t]);
             if (T::QBUF && lane % Q::LPS == 0) lds_kbsf[i] = f16_to_f32(F.kbs[t]);
         }
     }
@@ -244,8 +247,11 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
             for (int bi = 0; bi < NB; ++bi)
                 own[bi] = quad_block_pass_v<Q, T, 1>(my_codes + bi * Q::BLK, lds_xn, F.scv[bi], lds_pl + w * L::PL_BYTES,
                                                      lds_xs + w * (L::XS_BYTES / 4), lane);
+        } else if constexpr (T::FLT) {
+#pragma unroll
+            for (int bi = 0; bi < NB; ++bi) own[bi] = quad_block_pass_f<Q, T, 1>(my_codes + bi * Q::BLK, lds_xn, lane);
         } else {
-            v4i aop[T::NKS];
+            v4i aop[Q::NKS];
             quad_fetch_planes<Q, T, 1>(lds_pl, lane, aop);
             float xs[NG];
 #pragma unroll
@@ -277,7 +283,7 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
             const int i = Q::SPP * (NW * t + w) + lane / Q::LPS;
             const int ic = i < m ? i : m - 1;
             float kf[4];
-            decode_raw4<T::QBUF>(load_raw4<T::QBUF>(lds_kbr + (ic * DK + 4 * (lane % Q::LPS)) * T::BE), kf);
+            decode_raw4<T::QBUF>(load_raw4<T::QBUF>(lds_kbr + (ic * DKP + 4 * (lane % Q::LPS)) * T::BE), kf);
             if constexpr (T::QBUF) {
                 const float s = lds_kbsf[ic];
 #pragma unroll
@@ -294,7 +300,7 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
     if (w == RK) {
         float bcp = 0.0f;
 #pragma unroll
-        for (int t = 0; t < NE; ++t) bcp = __builtin_fmaf(lds_xn[DK + NE * lane + t], lds_xn[NE * lane + t], bcp);
+        for (int t = 0; t < NE; ++t) bcp = __builtin_fmaf(lds_xn[DKP + NE * lane + t], lds_xn[NE * lane + t], bcp);
         bcp = lanes_sum<WAVE>(bcp);
         if (lane == 0) lds_gsc[0] = bcp;
     }
@@ -306,12 +312,12 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
         float kxe[NE], kmax = 0.0f;
 #pragma unroll
         for (int t = 0; t < NE; ++t) {
-            kxe[t] = lds_xn[DK + NE * lane + t];
+            kxe[t] = lds_xn[DKP + NE * lane + t];
             kmax = fmaxf(kmax, fabsf(kxe[t]));
         }
         float ks = 1.0f;
         if constexpr (T::QBUF) ks = fp16_scale(lanes_max<WAVE>(kmax), 127.0f);
-        const bool write = h - hl == hk * uint32_t(p.gqa);
+        const bool live = Q::vec_live(lane), write = live && h - hl == hk * uint32_t(p.gqa);
         if (T::QBUF && lane == 0) {
             lds_kbsf[n] = ks;
             if (write) KBSp[n] = f32_to_f16(ks);
@@ -320,7 +326,7 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
             uint32_t pk = 0;
 #pragma unroll
             for (int t = 0; t < NE; ++t) pk |= (uint32_t(int(round_buf(kxe[t], ks))) & 0xFFu) << (8 * t);
-            uint8_t* dl = lds_kbr + n * DK + NE * lane;
+            uint8_t* dl = lds_kbr + n * DKP + NE * lane;
             uint8_t* dg = KBp + n * DK + NE * lane;
             if constexpr (NE == 1) { *dl = uint8_t(pk); if (write) *dg = uint8_t(pk); }
             else if constexpr (NE == 2) {
@@ -334,7 +340,7 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
 #pragma unroll
             for (int t = 0; t < NE; ++t) {
                 const uint16_t hb = f32_to_bf16(kxe[t]);
-                reinterpret_cast<uint16_t*>(lds_kbr)[n * DK + NE * lane + t] = hb;
+                reinterpret_cast<uint16_t*>(lds_kbr)[n * DKP + NE * lane + t] = hb;
                 if (write) reinterpret_cast<uint16_t*>(KBp)[n * DK + NE * lane + t] = hb;
             }
         }
@@ -405,7 +411,6 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
         // formed at the top of the kernel are not kept in registers all the way to here
         int lf = lane;
         asm volatile("" : "+v"(lf));
-        const int swzf = swz<Q>(lf / Q::CPR, lf % Q::CPR);
         const float cmul = expf(gnew);
         if constexpr (T::AXV) {
             constexpr int MT = (MM + 1) / 2;
@@ -418,7 +423,7 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
             }
             auto key = [&](int sl, int col) {
                 const int sc_ = sl < m ? sl : 0;
-                float kv = lds_raw<T::QBUF>(lds_kbr, sc_ * DK + col);
+                float kv = lds_raw<T::QBUF>(lds_kbr, sc_ * DKP + col);
                 if constexpr (T::QBUF) kv = kv * lds_kbsf[sc_];
                 return sl < m ? kv : 0.0f;
             };
@@ -441,13 +446,10 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
                 }
                 quad_fold_block_v<Q, T>(blk, key, dop, [&](int) { return cmul; }, cmul == 1.0f, old,
                                         SCh + grp * DK, lf);
-#pragma unroll
-                for (int t = 0; t < Q::NLD; ++t)
-                    stream_store(reinterpret_cast<v4u*>(Sh + grp * Q::BLK + t * 1024 + lf * 16),
-                                 *reinterpret_cast<const v4u*>(blk + t * 1024 + swzf));
+                quad_store_block<Q>(Sh + grp * Q::GBLK, blk, lf);
             }
         } else {
-            constexpr int MT4 = (MM + 3) / 4, CL = DK / 4;
+            constexpr int MT4 = (MM + 3) / 4, CL = DKP / 4;
             const int fn = lf & 15, fq = lf >> 4;
             float decf[MT4];                                 // decay ratios a_m / a_i of the lane's slots 4 t + q
 #pragma unroll
@@ -455,7 +457,7 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
                 const int sl = 4 * t + fq;
                 decf[t] = sl < m - 1 ? expf(gnew - lds_gbf[sl < m - 1 ? sl : 0]) : 1.0f;
             }
-            const int fg = (fq * CL) / T::KGROUP;
+            const int fg = min((fq * CL) / T::KGROUP, NG - 1);
             FoldKeys<T> kop;
             quad_fold_keys<T>(lds_kbr, lds_kbsf, m, lf, kop);
 #pragma unroll
@@ -474,14 +476,14 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
                         fv = decf[t] * fv;
                         bop[t] = sl < m ? fv : 0.0f;
                     }
-                    quad_fold_half<Q, T>(blk, hf, kop, bop, cmul, f16_to_f32(lds_sc[frow * NG + fg]),
+                    if constexpr (T::FLT)
+                        quad_fold_half_f<Q, T>(blk, hf, kop, bop, cmul, lf);
+                    else
+                        quad_fold_half<Q, T>(blk, hf, kop, bop, cmul, f16_to_f32(lds_sc[frow * NG + fg]),
                                                 SCh + frow * NG + fg, lf);
                 }
                 wave_sync();
-#pragma unroll
-                for (int t = 0; t < Q::NLD; ++t)
-                    stream_store(reinterpret_cast<v4u*>(Sh + (wh * NB + bi) * Q::BLK + t * 1024 + lf * 16),
-                                 *reinterpret_cast<const v4u*>(blk + t * 1024 + swzf));
+                quad_store_block<Q>(Sh + (wh * NB + bi) * Q::GBLK, blk, lf);
             }
         }
     }

@@ -1,6 +1,6 @@
 // The state tile of one (sequence, value head) shared by the wavefronts of one workgroup: every wavefront owns NB of
-// the tile's 32-row blocks.  Shared by the Gated DeltaNet and Mamba2 workgroup-per-key-head step kernels (int4 / int8
-// codes with key-axis scale groups, or value-axis groups of one row block, and a power-of-two row size).
+// the tile's 32-row blocks.  Shared by the Gated DeltaNet, KDA and Mamba2 workgroup step kernels (int4 / int8 codes with
+// key-axis scale groups, or value-axis groups of one row block, and the unquantized bf16 state).
 //
 // What this buys over one wavefront per tile (sq_tile.cuh, kept for the other formats):
 //   * a tile's life is a quarter as long, so the launch's ramp-up and tail shrink and the dispatcher balances the
@@ -18,7 +18,13 @@
 //
 // LDS image of a row block: the rows as stored, 16-byte chunks XOR-swizzled inside a row so that both the row-shaped
 // writes (lanes along a row) and the operand-shaped reads (lanes down a column of chunks) are conflict free without
-// padding.
+// padding.  A d_k that is no power of two (96) gets rows as long as the next one's in LDS -- the loads leave the unused
+// chunks alone, the read-out vectors are zero there -- so that every address stays shifts and masks.
+//
+// us per launch, sequences out of step, one wavefront per head -> this: 96 x 192 int4 g64 (30 heads, 64 sequences) 21.8 ->
+// 15.0; bf16 128 x 128 (32 heads, 40 sequences) 31.4 -> 17.0, where the one-wavefront kernel reads the state twice on a
+// fold and has five wavefronts per compute unit to wait with; four workgroups of 38 KB per compute unit are what LDS
+// admits there.
 #pragma once
 #include <stdlib.h>
 
@@ -77,7 +83,7 @@ __device__ __forceinline__ void quad_start_wait(uint32_t ramp) {
 
 template <class T, int NB_, int GH_ = 1>
 struct Quad {
-    static_assert(!T::FLT && !T::RAGV, "int4 / int8 codes, whole row blocks");
+    static_assert(T::BITS <= 16 && !T::RAGV, "int4 / int8 codes or a bf16 state, whole row blocks");
     static_assert(!T::AXV || T::GROUP == T::MR, "value-axis groups: one row block each");
     static constexpr int NB = NB_;                         // row blocks per wavefront
     static constexpr int GH = GH_;                         // value heads of one key head per workgroup
@@ -87,22 +93,34 @@ struct Quad {
     static constexpr int THREADS = NW * WAVE;
     static_assert(THREADS <= 1024, "workgroup size");
     static constexpr int RW = NB * T::MR;                  // rows per wavefront
-    static constexpr int RB = T::ROW_BYTES;
-    static_assert((RB & (RB - 1)) == 0 && RB >= 32 && RB <= 256, "row size: a power of two in 32..256 bytes");
-    static_assert(T::BITS == 8 || T::DK % 64 == 0, "int4: d_k a multiple of 64");
-    static constexpr int CPR = RB / 16;                    // 16-byte chunks per row
-    static constexpr int BLK = T::MR * RB;                 // bytes of a row block
-    static constexpr int HEAD = T::DV * RB;                // bytes of a head's codes
+    static constexpr int DKP = pow2_ceil(T::DK);           // columns of a row, a read-out vector and a buffered key in LDS
+    static constexpr bool PADK = DKP != T::DK;
+    static constexpr int RB = pow2_ceil(T::ROW_BYTES);     // bytes of a row in LDS
+    static_assert(T::ROW_BYTES % 16 == 0 && RB >= 32 && RB <= 256, "row size: whole 16-byte chunks, 32..256 bytes in LDS");
+    static constexpr int CPR = RB / 16;                    // 16-byte chunks per row in LDS
+    static constexpr int LIVE = T::ROW_BYTES / 16;         // ... of which hold columns
+    static constexpr int BLK = T::MR * RB;                 // bytes of a row block in LDS
+    static constexpr int GBLK = T::MR * T::ROW_BYTES;      // ... in memory
+    static constexpr int HEAD = T::DV * RB;                // bytes of a head's codes in LDS
+    static constexpr int NKS = T::BITS == 4 ? (T::NKS + 1) / 2 * 2 : T::NKS;    // column steps (int4: whole chunk pairs)
     static constexpr int NLD = BLK / 1024;                 // wavefront loads per row block
     static constexpr int SWM = CPR < 8 ? CPR : 8;          // swizzle: chunk c of row r sits at chunk c ^ ((r / SWD) % SWM)
     static constexpr int SWD = 8 / SWM;
     static constexpr int PLS = T::AXV ? 6 : 8;             // digit-plane slots per 16-column piece
     static_assert(T::NG <= 4, "at most four scale groups per row (result rows 8 g + 4 v + d)");
     // a d_k vector in a wavefront: lane l holds the NE consecutive elements NE l ..
-    static constexpr int NE = T::DK / WAVE;
-    static_assert(NE * WAVE == T::DK && NE >= 1 && NE <= 4, "d_k: 64, 128 or 256");
+    static constexpr int NE = DKP / WAVE;
+    static_assert(NE * WAVE == DKP && NE >= 1 && NE <= 4 && T::DK % NE == 0, "d_k: 64, 96, 128 or 256");
+    // the lane whose elements a lane loads (lanes beyond d_k repeat the last), and whether it has any of its own
+    __device__ static __forceinline__ int vec_lane(int lane) { return PADK && NE * lane >= T::DK ? T::DK / NE - 1 : lane; }
+    __device__ static __forceinline__ bool vec_live(int lane) { return !PADK || NE * lane < T::DK; }
+    // column 4 (lane % LPS) of a buffered key, inside d_k
+    __device__ static __forceinline__ int key_col(int lane) {
+        const int c = 4 * (lane % LPS);
+        return PADK && c >= T::DK ? T::DK - 4 : c;
+    }
     // buffer passes: keys 4 columns per lane (slots dealt over the workgroup's wavefronts), values 4 rows per lane
-    static constexpr int LPS = T::DK / 4;                  // lanes per buffered key
+    static constexpr int LPS = DKP / 4;                    // lanes per buffered key
     static constexpr int SPP = WAVE / LPS;                 // keys per wavefront and pass
     static constexpr int KT = (T::MMAX + NW * SPP - 1) / (NW * SPP);
     static constexpr int LU = RW / 4;                      // lanes per buffered value piece of this wavefront's rows
@@ -120,12 +138,12 @@ struct QuadLds {
     // digit planes and their factors: one set for the workgroup; value-axis groups: one per wavefront, rebuilt for
     // each of its row blocks (the block's scales ride on the read-out vectors)
     static constexpr int SETS = T::AXV ? Q::NW : 1;
-    static constexpr int PL_BYTES = T::DK / CPL * Q::PLS * 16, XS_BYTES = round_up(NV * T::NG * 4, 16);
+    static constexpr int PL_BYTES = T::FLT ? 0 : Q::DKP / CPL * Q::PLS * 16, XS_BYTES = round_up(NV * T::NG * 4, 16);
     static constexpr int CODES = 0;                                    // [GH][DV] rows, swizzled
-    static constexpr int KBR = CODES + GH * Q::HEAD;                   // buffered keys, raw [m][DK]
-    static constexpr int UBR = KBR + T::MMAX * T::DK * T::BE;          // buffered values, raw [GH][m][DV]
-    static constexpr int XN = UBR + GH * T::MMAX * T::DV * T::BE;      // read-out vectors, fp32 [NX][DK]
-    static constexpr int PL = XN + NX * T::DK * 4;                     // digit planes [k-step][half][PLS][16]
+    static constexpr int KBR = CODES + GH * Q::HEAD;                   // buffered keys, raw [m][DKP]
+    static constexpr int UBR = KBR + T::MMAX * Q::DKP * T::BE;         // buffered values, raw [GH][m][DV]
+    static constexpr int XN = UBR + GH * T::MMAX * T::DV * T::BE;      // read-out vectors, fp32 [NX][DKP]
+    static constexpr int PL = XN + NX * Q::DKP * 4;                    // digit planes [k-step][half][PLS][16]
     static constexpr int XS = PL + SETS * PL_BYTES;                    // [NV][NG] exponent factors
     static constexpr int DOTS = XS + SETS * XS_BYTES;                  // [NV][MMAX] K_i . x
     static constexpr int KBSF = DOTS + NV * T::MMAX * 4;               // [MMAX] key scales as fp32
@@ -134,7 +152,7 @@ struct QuadLds {
     static constexpr int RED = SCAL + (GH + 1) * 32;                   // one float per wavefront
     static constexpr int GBF = RED + round_up(Q::NW * 4, 16);          // [GH][MMAX] cumulative decays of the slots
     static constexpr int SC = GBF + GH * T::MMAX * 4;                  // [GH][DV][NG] fp16 scales of the rows (value-axis
-    static constexpr int BYTES = SC + (T::AXV ? 0 : round_up(GH * T::DV * T::NG * 2, 16));   // scales stay in registers)
+    static constexpr int BYTES = SC + (T::AXV || T::FLT ? 0 : round_up(GH * T::DV * T::NG * 2, 16));   // scales stay in registers)
 };
 
 // Where column e of a read-out vector goes in the digit-plane region: the (k-step, lane half, byte) at which the
@@ -219,19 +237,19 @@ __device__ __forceinline__ void quad_stage_planes(const float (&xe)[NE], int v, 
             at[32] = uint8_t(d[t] >> 16);
         }
     }
-    if (e0 % T::KGROUP == 0) lds_xs[v * T::NG + e0 / T::KGROUP] = __builtin_ldexpf(1.0f, ex - 22 - (T::BITS == 4 ? 4 : 0));
+    if (e0 % T::KGROUP == 0 && (!Q::PADK || e0 < T::DK)) lds_xs[v * T::NG + e0 / T::KGROUP] = __builtin_ldexpf(1.0f, ex - 22 - (T::BITS == 4 ? 4 : 0));
 }
 
 // The digit planes as the matrix core's first operand, per k-step: lane (i, kb) carries result row i = 8 g + 4 v + d,
 // i.e. digit d of vector v -- on the k-steps whose columns belong to scale group g, zero elsewhere (and zero in the
 // unused rows), so that ONE accumulation over all k-steps leaves every group's sums in its own result rows.
 template <class Q, class T, int NV>
-__device__ __forceinline__ void quad_fetch_planes(const uint8_t* lds_pl, int lane, v4i (&aop)[T::NKS]) {
+__device__ __forceinline__ void quad_fetch_planes(const uint8_t* lds_pl, int lane, v4i (&aop)[Q::NKS]) {
     const int i = lane & 31, kb = lane >> 5;
     const int g = i >> 3, v = (i >> 2) & 1, d = i & 3;
     const bool used = d < 3 && g < T::NG && v < NV;
 #pragma unroll
-    for (int ks = 0; ks < T::NKS; ++ks) {
+    for (int ks = 0; ks < Q::NKS; ++ks) {
         const v4i x = *reinterpret_cast<const v4i*>(lds_pl + ((ks * 2 + kb) * Q::PLS + 3 * (v < NV ? v : 0) + (d < 3 ? d : 0)) * 16);
         const bool mine = used && (kb == 0 ? op_colbase<T>(ks, 0) : op_colbase<T>(ks, 1)) / T::KGROUP == g;
         aop[ks] = mine ? x : v4i{0, 0, 0, 0};
@@ -242,7 +260,7 @@ __device__ __forceinline__ void quad_fetch_planes(const uint8_t* lds_pl, int lan
 // row's scales applied group by group, in order.  xs[g] = the exponent factor of vector kb, group g; sc[g] = the
 // row's scales.
 template <class Q, class T>
-__device__ __forceinline__ float quad_block_pass(const uint8_t* blk, const v4i (&aop)[T::NKS], const float (&xs)[T::NG],
+__device__ __forceinline__ float quad_block_pass(const uint8_t* blk, const v4i (&aop)[Q::NKS], const float (&xs)[T::NG],
                                                  const float (&sc)[T::NG], int lane) {
     const int n = lane & 31, kb = lane >> 5;
     v16i acc = {0};
@@ -254,7 +272,7 @@ __device__ __forceinline__ float quad_block_pass(const uint8_t* blk, const v4i (
         }
     } else {
 #pragma unroll
-        for (int kp = 0; kp < T::NKS / 2; ++kp) {
+        for (int kp = 0; kp < Q::NKS / 2; ++kp) {
             const uint4 c = *reinterpret_cast<const uint4*>(blk + swz<Q>(n, 2 * kp + kb));
             RawRow<4> lo, hi;
             lo.v = make_uint2(c.x, c.y);
@@ -274,6 +292,43 @@ __device__ __forceinline__ float quad_block_pass(const uint8_t* blk, const v4i (
     return s;
 }
 
+// The same for a bf16 state: fp32 multiply-adds on the vector ALU (the read-out vectors stay fp32, and an infinity in the
+// state stays one), `lds_x` [NV][DKP].  Lane (n, kb) walks half kb of row n against all NV vectors -- the vectors' pieces
+// are the same for half a wavefront, so LDS hands them out as broadcasts -- and one lane swap adds the halves.
+template <class Q, class T, int NV>
+__device__ __forceinline__ float quad_block_pass_f(const uint8_t* blk, const float* lds_x, int lane) {
+    const int n = lane & 31, kb = lane >> 5;
+    constexpr int HALF = Q::LIVE / 2;                        // chunks of 8 columns per lane
+    static_assert(Q::LIVE % 2 == 0 && (NV == 1 || NV == 2), "two halves, one or two vectors");
+    float s[NV][2];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) s[v][0] = s[v][1] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < HALF; ++j) {
+        const int c = kb * HALF + j;
+        const v4u r = *reinterpret_cast<const v4u*>(blk + swz<Q>(n, c));
+        const uint32_t w[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const float* x = lds_x + v * Q::DKP + 8 * c;
+            const float4 lo = *reinterpret_cast<const float4*>(x), hi = *reinterpret_cast<const float4*>(x + 4);
+            const float xe[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+                s[v][0] = __builtin_fmaf(as_f32(w[d] << 16), xe[2 * d], s[v][0]);
+                s[v][1] = __builtin_fmaf(as_f32(w[d] & 0xFFFF0000u), xe[2 * d + 1], s[v][1]);
+            }
+        }
+    }
+    const float a = s[0][0] + s[0][1];
+    if constexpr (NV == 1) {
+        const Pair p = pair32(a);
+        return p.lo + p.hi;
+    } else {
+        const auto r = __builtin_amdgcn_permlane32_swap(as_u32(a), as_u32(s[1][0] + s[1][1]), false, false);
+        return as_f32(r[0]) + as_f32(r[1]);
+    }
+}
 
 // ---------------------------------------------------------------------------------------------------------------
 // Row blocks loaded straight into their LDS image (global_load_lds_dwordx4: no pass through registers, no LDS store
@@ -316,12 +371,24 @@ __device__ __forceinline__ void quad_dma_blocks(const uint8_t* src, uint8_t* dst
         for (int t = 0; t < Q::NLD; ++t) {
             const int r = t * (1024 / Q::RB) + pr;
             const int c = pc ^ ((r / Q::SWD) % Q::SWM);
-            const uint8_t* g = src + bi * Q::BLK + r * Q::RB + (c << 4);
+            const uint8_t* g = src + bi * Q::GBLK + r * (Q::GBLK / 32) + (c << 4);
             const uint32_t at = uint32_t(reinterpret_cast<uintptr_t>(
                 (__attribute__((address_space(3))) uint8_t*)(dst + bi * Q::BLK + t * 1024)));
-            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt"
-                         :: "v"(g), "s"(at) : "memory", "m0");
+            if (!Q::PADK || c < Q::LIVE)                     // a lane that is switched off writes nothing
+                asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt"
+                             :: "v"(g), "s"(at) : "memory", "m0");
         }
+}
+// A row block's LDS image back to memory.
+template <class Q>
+__device__ __forceinline__ void quad_store_block(uint8_t* dst, const uint8_t* blk, int lane) {
+#pragma unroll
+    for (int t = 0; t < Q::NLD; ++t) {
+        const int r = t * (1024 / Q::RB) + lane / Q::CPR, c = lane % Q::CPR;
+        if (!Q::PADK || c < Q::LIVE)
+            stream_store(reinterpret_cast<v4u*>(dst + r * (Q::GBLK / 32) + (c << 4)),
+                         *reinterpret_cast<const v4u*>(blk + swz<Q>(r, c)));
+    }
 }
 __device__ __forceinline__ void quad_dma_landed() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
@@ -401,7 +468,7 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 // F32: the keys are not the buffered ones (KDA folds a decay per column into them) and come as fp32.
 template <class T, bool F32 = false>
 struct FoldKeys {
-    static constexpr int MT4 = (T::MMAX + 3) / 4, NT = T::DK / 16;
+    static constexpr int MT4 = (T::MMAX + 3) / 4, DKP = pow2_ceil(T::DK), NT = DKP / 16;
     static constexpr bool PACKED = !F32 && T::BITS == 4 && T::QBUF && NT % 4 == 0;
     float f[PACKED ? 1 : NT][PACKED ? 1 : MT4];
     uint32_t raw[PACKED ? MT4 : 1][PACKED ? NT / 4 : 1];
@@ -416,7 +483,7 @@ struct FoldKeys {
 template <class T>
 __device__ __forceinline__ void quad_fold_keys(const uint8_t* lds_kbr, const float* lds_kbsf, int m, int lane,
                                                FoldKeys<T>& kop) {
-    constexpr int MT4 = (T::MMAX + 3) / 4, CL = T::DK / 4, NT = CL / 4;
+    constexpr int MT4 = (T::MMAX + 3) / 4, DKP = pow2_ceil(T::DK), CL = DKP / 4, NT = CL / 4;
     const int n = lane & 15, q = lane >> 4;
     const int kcol = (n >> 2) * CL + (n & 3);
 #pragma unroll
@@ -429,7 +496,7 @@ __device__ __forceinline__ void quad_fold_keys(const uint8_t* lds_kbr, const flo
             for (int c4 = 0; c4 < NT / 4; ++c4) {
                 uint32_t w = 0;
 #pragma unroll
-                for (int b = 0; b < 4; ++b) w |= uint32_t(lds_kbr[sl * T::DK + kcol + 4 * (4 * c4 + b)]) << (8 * b);
+                for (int b = 0; b < 4; ++b) w |= uint32_t(lds_kbr[sl * DKP + kcol + 4 * (4 * c4 + b)]) << (8 * b);
                 kop.raw[t][c4] = w ^ 0x80808080u;
             }
             kop.ks[t] = slot < m ? ks : 0.0f;                 // a slot beyond m contributes nothing
@@ -437,7 +504,7 @@ __device__ __forceinline__ void quad_fold_keys(const uint8_t* lds_kbr, const flo
         } else {
 #pragma unroll
             for (int ct = 0; ct < NT; ++ct) {
-                float kv = lds_raw<T::QBUF>(lds_kbr, sl * T::DK + kcol + 4 * ct);
+                float kv = lds_raw<T::QBUF>(lds_kbr, sl * DKP + kcol + 4 * ct);
                 if constexpr (T::QBUF) kv = kv * ks;
                 kop.f[ct][t] = slot < m ? kv : 0.0f;
             }
@@ -445,10 +512,10 @@ __device__ __forceinline__ void quad_fold_keys(const uint8_t* lds_kbr, const flo
     }
 }
 
-// The same from fp32 keys in LDS, [m][DK].
+// The same from fp32 keys in LDS, [m][DKP].
 template <class T>
 __device__ __forceinline__ void quad_fold_keys_f32(const float* lds_kd, int m, int lane, FoldKeys<T, true>& kop) {
-    constexpr int MT4 = (T::MMAX + 3) / 4, CL = T::DK / 4, NT = CL / 4;
+    constexpr int MT4 = (T::MMAX + 3) / 4, DKP = pow2_ceil(T::DK), CL = DKP / 4, NT = CL / 4;
     const int n = lane & 15, q = lane >> 4;
     const int kcol = (n >> 2) * CL + (n & 3);
 #pragma unroll
@@ -456,25 +523,29 @@ __device__ __forceinline__ void quad_fold_keys_f32(const float* lds_kd, int m, i
         const int slot = 4 * t + q;
 #pragma unroll
         for (int ct = 0; ct < NT; ++ct) {
-            const float kv = lds_kd[(slot < m ? slot : 0) * T::DK + kcol + 4 * ct];
+            const float kv = lds_kd[(slot < m ? slot : 0) * DKP + kcol + 4 * ct];
             kop.f[ct][t] = slot < m ? kv : 0.0f;
         }
     }
 }
 
-// COLVEC: the old state decays per column -- `lds_cm` [DK] fp32 in the place of the scalar `cmul`.
+// COLVEC: the old state decays per column -- `lds_cm` [DKP] fp32 in the place of the scalar `cmul`.
+// A quarter that lies beyond d_k (the last one of 96 columns) computes on whatever its chunks hold and keeps it to
+// itself: it adds nothing to a group's maximum and stores no scale; its chunks never leave LDS.
 template <class Q, class T, bool COLVEC = false>
 __device__ __forceinline__ void quad_fold_half(uint8_t* blk, int hf, const FoldKeys<T, COLVEC>& kop,
                                                const float (&bop)[(T::MMAX + 3) / 4], float cmul, float s_old,
                                                uint16_t* sc_out, int lane, const float* lds_cm = nullptr) {
     constexpr int MT4 = (T::MMAX + 3) / 4;
-    constexpr int CL = T::DK / 4;                            // columns per lane
+    constexpr int CL = Q::DKP / 4;                           // columns per lane
+    static_assert(T::DK % CL == 0, "a quarter is inside d_k or outside");
     constexpr int NT = CL / 4;                               // accumulator tiles per lane
     constexpr int NBY = Q::RB / 4;                           // bytes per lane
     constexpr int NW32 = NBY / 4;                            // 32-bit words per lane
     static_assert(CL % 16 == 0 && T::KGROUP % CL == 0 && T::KGROUP / CL <= 4, "a scale group is 1, 2 or 4 lanes wide");
     constexpr int LPG = T::KGROUP / CL;
     const int n = lane & 15, q = lane >> 4;
+    const bool inside = !Q::PADK || q * CL < T::DK;
     const int row = 16 * hf + n;
     // where the lane's bytes of the row sit in the LDS image
     const int at = NBY >= 16 ? swz<Q>(row, q * (NBY / 16)) : swz<Q>(row, q >> 1) + 8 * (q & 1);
@@ -581,13 +652,14 @@ __device__ __forceinline__ void quad_fold_half(uint8_t* blk, int hf, const FoldK
         mx = fmaxf(fmaxf(mx, fabsf(acc[ct][0])), fabsf(acc[ct][1]));
         mx = fmaxf(fmaxf(mx, fabsf(acc[ct][2])), fabsf(acc[ct][3]));
     }
+    if (!inside) mx = 0.0f;
     if constexpr (LPG >= 2) { const Pair pm = pair16(mx); mx = fmaxf(pm.lo, pm.hi); }
     if constexpr (LPG >= 4) { const Pair pm = pair32(mx); mx = fmaxf(pm.lo, pm.hi); }
     const float sc = fp16_scale(UNITS ? mx * unit : mx, T::QMAX);
     const Divisor dsc = scale_divisor(sc);                   // sc is an fp16 value: the correctly rounded reciprocal
     const float rs = UNITS ? unit * dsc.rc : dsc.rc;         // (exact mode: unit is a power of two, both stay exact)
     const float ds = UNITS ? dsc.d * __builtin_amdgcn_rcpf(unit) : dsc.d;
-    if (q % LPG == 0) *sc_out = f32_to_f16(sc);
+    if (q % LPG == 0 && inside) *sc_out = f32_to_f16(sc);
     // new codes, back into the LDS image.  A scale in fp16's normal range cannot push a quotient past qmax + 1/2, so
     // the clamp is only compiled into the path taken when some lane's scale is subnormal (or at its floor).
     auto requantize = [&](auto clamp, auto exactly) {
@@ -615,6 +687,50 @@ __device__ __forceinline__ void quad_fold_half(uint8_t* blk, int hf, const FoldK
     else requantize(std::false_type{}, std::false_type{});
 }
 
+// The fold of half a row block of a bf16 state: the same matrix-core updates in the same order, rounded to bf16 (nearest
+// even) in place.
+template <class Q, class T, bool COLVEC = false>
+__device__ __forceinline__ void quad_fold_half_f(uint8_t* blk, int hf, const FoldKeys<T, COLVEC>& kop,
+                                                 const float (&bop)[(T::MMAX + 3) / 4], float cmul, int lane,
+                                                 const float* lds_cm = nullptr) {
+    constexpr int MT4 = (T::MMAX + 3) / 4, CL = Q::DKP / 4, NT = CL / 4;
+    constexpr int CHUNKS = CL / 8;                           // 16-byte chunks (8 columns, two tiles) per lane
+    static_assert(T::DK % CL == 0, "a quarter is inside d_k or outside");
+    const int n = lane & 15, q = lane >> 4;
+    v4f acc[NT];
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+        const v4u x = *reinterpret_cast<const v4u*>(blk + swz<Q>(16 * hf + n, q * CHUNKS + c));
+        const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            float f0 = cmul, f1 = cmul;
+            if constexpr (COLVEC) {
+                const float2 f = *reinterpret_cast<const float2*>(lds_cm + q * CL + 8 * c + 2 * d);
+                f0 = f.x; f1 = f.y;
+            }
+            acc[2 * c + d / 2][2 * (d % 2)] = as_f32(w[d] << 16) * f0;
+            acc[2 * c + d / 2][2 * (d % 2) + 1] = as_f32(w[d] & 0xFFFF0000u) * f1;
+        }
+    }
+    static_for<NT>([&](auto ct) {
+        static_for<MT4>([&](auto t) {
+            acc[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(kop.template get<decltype(ct)::value, decltype(t)::value>(), bop[t],
+                                                           acc[ct], 0, 0, 0);
+        });
+    });
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+        v4u o;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            const v4f a = acc[2 * c + d / 2];
+            o[d] = uint32_t(f32_to_bf16(a[2 * (d % 2)])) | (uint32_t(f32_to_bf16(a[2 * (d % 2) + 1])) << 16);
+        }
+        *reinterpret_cast<v4u*>(blk + swz<Q>(16 * hf + n, q * CHUNKS + c)) = o;
+    }
+}
+
 // ---------------------------------------------------------------------------------------------------------------
 // value-axis scale groups of one row block (32 rows x one key column share a scale)
 //
@@ -637,7 +753,7 @@ __device__ __forceinline__ void quad_store_colscales(uint16_t* lds_sc, int lane,
     else reinterpret_cast<uint32_t*>(lds_sc)[lane] = s;
 }
 // The row sums of one block: the scales belong to (block, column), so they ride on the read-out vectors (x'_k = x_k
-// s_k, `lds_x` [NV][DK] fp32) and the digit planes are rebuilt per block, in this wavefront's own plane set.  Lane
+// s_k, `lds_x` [NV][DKP] fp32) and the digit planes are rebuilt per block, in this wavefront's own plane set.  Lane
 // (n, kb) returns (S0 x_kb)[row n of the block].
 template <class Q, class T, int NV>
 __device__ __forceinline__ float quad_block_pass_v(const uint8_t* blk, const float* lds_x, uint32_t colscales,
@@ -649,11 +765,11 @@ __device__ __forceinline__ float quad_block_pass_v(const uint8_t* blk, const flo
         float xe[NE];
 #pragma unroll
         for (int t = 0; t < NE; ++t)
-            xe[t] = lds_x[v * T::DK + NE * lane + t] * f16_to_f32(uint16_t(colscales >> (16 * t)));
+            xe[t] = Q::vec_live(lane) ? lds_x[v * Q::DKP + NE * lane + t] * f16_to_f32(uint16_t(colscales >> (16 * t))) : 0.0f;
         quad_stage_planes<Q, T, NE>(xe, v, lane, lds_pl, lds_xs);
     }
     wave_sync();
-    v4i aop[T::NKS];
+    v4i aop[Q::NKS];
     quad_fetch_planes<Q, T, NV>(lds_pl, lane, aop);
     const float xs[1] = {lds_xs[(lane >> 5) < NV ? lane >> 5 : 0]};
     const float one[1] = {1.0f};
