@@ -23,7 +23,7 @@ using RowTile = Tile<BITS, DK, 128, GROUP, QBUF, 16, AXV>;
 // covers).  A hand-over concerns the few sequences that begin or end a prefill chunk: one wavefront per head leaves most
 // of the chip idle and walks the rows one memory round trip after the other, so heads are split until there are some
 // 4096 wavefronts (16 per compute unit, what full batches give by themselves and what keeps memory busy).  6 sequences
-// of 32 heads of 128 x 128, int8 g32: write 11.9 -> 4.7 us per launch, read 14.8 -> 7.0 (256 sequences, one wavefront
+// of 32 heads of 128 x 128, int8 g32: write 11.9 -> 4.7 us per launch, read 14.8 -> 6.2 (256 sequences, one wavefront
 // per head as before: 142 and 149).
 struct RowSplit {
     uint32_t parts, rows;
@@ -210,10 +210,47 @@ __global__ __launch_bounds__(WAVE) void read_kernel(const ReadParams p, uint32_t
     const uint16_t* UBS = field(p.st.UBS, seq, p.st.sUBS, h * um);
     const float* GBh = field(p.st.GB, seq, p.st.sGB, h * um * (KDA ? DK : 1));
     const float* gch = field(p.st.GCUR, seq, p.st.sGC, h * (KDA ? DK : 1));
-    const int n = *field(p.st.NPTR, seq, p.st.sN, 0u) & (m - 1);     // the first head's copy, as the reference reads it
     const bool live = l.cg < T::LPR;
     const int cc = live ? l.cg : T::LPR - 1;
 
+    constexpr int RR = 2;                                         // rows per pass over the buffered keys
+    constexpr int CW = BITS == 32 ? 4 : BITS == 16 ? 2 : 1;       // words of a 4-column chunk
+    // a pass's stored rows and scales as loaded; the first pass's are requested before anything that waits for the fill
+    // counter (6 sequences as above: 7.0 -> 6.2 us per launch)
+    uint32_t cw[RR][NCH][CW];
+    uint2 sw[RR][NCH];
+    auto request = [&](uint32_t r0) {
+#pragma unroll
+        for (int k = 0; k < RR; ++k) {
+            const uint32_t r = r0 + k * T::RG + l.rg, rc = r < r_end ? r : r_end - 1;
+#pragma unroll
+            for (int t = 0; t < NCH; ++t) {
+                const int col = t * CSTEP + 4 * cc;
+                if constexpr (T::FLT) {
+                } else if constexpr (AXV) {                       // one scale per (group of rows, column)
+                    sw[k][t] = *reinterpret_cast<const uint2*>(SCh + (rc / GROUP) * DK + col);
+                } else {
+                    sw[k][t].x = SCh[rc * T::NG + col / GROUP];
+                }
+                const uint8_t* at = Sh + rc * T::ROW_BYTES + col * BITS / 8;
+                if constexpr (BITS == 32) {
+                    const v4u w = *reinterpret_cast<const v4u*>(at);
+                    cw[k][t][0] = w.x; cw[k][t][1] = w.y; cw[k][t][2] = w.z; cw[k][t][3] = w.w;
+                } else if constexpr (BITS == 16) {
+                    const v2u w = *reinterpret_cast<const v2u*>(at);
+                    cw[k][t][0] = w.x; cw[k][t][1] = w.y;
+                } else if constexpr (BITS == 8) {
+                    cw[k][t][0] = *reinterpret_cast<const uint32_t*>(at);
+                } else {
+                    cw[k][t][0] = *reinterpret_cast<const uint16_t*>(at);
+                }
+            }
+        }
+    };
+    request(r_begin);
+    asm volatile("" ::: "memory");
+
+    const int n = *field(p.st.NPTR, seq, p.st.sN, 0u) & (m - 1);     // the first head's copy, as the reference reads it
     // keys of the live slots, times their decay ratio (slot = row group + RG x pass, 16 consecutive columns per lane)
     for (int i0 = 0; i0 < n; i0 += T::RG) {
         const int i = i0 + l.rg;
@@ -248,45 +285,41 @@ __global__ __launch_bounds__(WAVE) void read_kernel(const ReadParams p, uint32_t
         for (int c = 0; c < 4; ++c) alpha_p[t][c] = expf(KDA ? gch[t * CSTEP + 4 * cc + c] : gch[0]);
     __syncthreads();
 
-    constexpr int RR = 2;                                         // rows per pass over the buffered keys
     for (uint32_t r0 = r_begin; r0 < r_end; r0 += RR * T::RG) {
         uint32_t row[RR], rc[RR];
         float acc[RR][NCH][4];
+        if (r0 != r_begin) request(r0);
 #pragma unroll
         for (int k = 0; k < RR; ++k) {
             row[k] = r0 + k * T::RG + l.rg;
             rc[k] = row[k] < r_end ? row[k] : r_end - 1;
 #pragma unroll
             for (int t = 0; t < NCH; ++t) {
-                const int col = t * CSTEP + 4 * cc;
                 float s4[4], c4[4];
+                const uint2 w = sw[k][t];
                 if constexpr (T::FLT) {
 #pragma unroll
                     for (int c = 0; c < 4; ++c) s4[c] = 1.0f;
-                } else if constexpr (AXV) {                       // one scale per (group of rows, column)
-                    const uint2 w = *reinterpret_cast<const uint2*>(SCh + (rc[k] / GROUP) * DK + col);
+                } else if constexpr (AXV) {
                     s4[0] = f16_to_f32(uint16_t(w.x)); s4[1] = f16_to_f32(uint16_t(w.x >> 16));
                     s4[2] = f16_to_f32(uint16_t(w.y)); s4[3] = f16_to_f32(uint16_t(w.y >> 16));
                 } else {
-                    const float s = f16_to_f32(SCh[rc[k] * T::NG + col / GROUP]);
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) s4[c] = s;
+                    for (int c = 0; c < 4; ++c) s4[c] = f16_to_f32(uint16_t(w.x));
                 }
+                const uint32_t (&v)[CW] = cw[k][t];
                 if constexpr (BITS == 32) {
-                    const float4 w = *reinterpret_cast<const float4*>(Sh + rc[k] * T::ROW_BYTES + 4 * col);
-                    c4[0] = w.x; c4[1] = w.y; c4[2] = w.z; c4[3] = w.w;
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) c4[c] = as_f32(v[c]);
                 } else if constexpr (BITS == 16) {
-                    const uint2 w = *reinterpret_cast<const uint2*>(Sh + rc[k] * T::ROW_BYTES + 2 * col);
-                    c4[0] = as_f32(w.x << 16); c4[1] = as_f32(w.x & 0xFFFF0000u);
-                    c4[2] = as_f32(w.y << 16); c4[3] = as_f32(w.y & 0xFFFF0000u);
+                    c4[0] = as_f32(v[0] << 16); c4[1] = as_f32(v[0] & 0xFFFF0000u);
+                    c4[2] = as_f32(v[1] << 16); c4[3] = as_f32(v[1] & 0xFFFF0000u);
                 } else if constexpr (BITS == 8) {
-                    const uint32_t w = *reinterpret_cast<const uint32_t*>(Sh + rc[k] * T::ROW_BYTES + col);
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) c4[c] = s8_to_f(w, c);
+                    for (int c = 0; c < 4; ++c) c4[c] = s8_to_f(v[0], c);
                 } else {
-                    const uint32_t w = *reinterpret_cast<const uint16_t*>(Sh + rc[k] * T::ROW_BYTES + col / 2);
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) c4[c] = float(int32_t((w >> (4 * c)) & 0xFu) - 8);
+                    for (int c = 0; c < 4; ++c) c4[c] = float(int32_t((v[0] >> (4 * c)) & 0xFu) - 8);
                 }
 #pragma unroll
                 for (int c = 0; c < 4; ++c) acc[k][t][c] = alpha_p[t][c] * (c4[c] * s4[c]);
