@@ -132,28 +132,30 @@ def quad_variants(fam, c):
     """[(row blocks per wavefront, value heads per workgroup, wavefronts per SIMD the register allocation aims
     for)], widest head group first, of the workgroup-per-key-head kernels (sq_quad.cuh) for a case; empty where only
     the one-wavefront kernels (sq_tile.cuh) serve it: value-axis groups other than 32 rows, the fp32 state, d_v that is no
-    multiple of 32, d_k above 128, more than four scale groups per row, states beyond 64 KB."""
+    multiple of 32 (Mamba2: 16), d_k above 128, more than four scale groups per row, states beyond 64 KB."""
     bits, dk, dv, group, qbuf, mmax, axv = c
     if fam not in QUAD_FAMILIES or bits not in (4, 8, 16) or (axv and group != 32):
         return []
     flt = bits == 16
     dkp = 1 << (dk - 1).bit_length()
     rb = 1 << (dk * bits // 8 - 1).bit_length()              # LDS row: the next power of two
-    if (dk * bits // 8) % 16 or not 32 <= rb <= 256 or dk > 128 or dv % 32:
+    if (dk * bits // 8) % 16 or not 32 <= rb <= 256 or dk > 128 or dv % 32 and (fam != 'mamba2' or dv % 16 or axv):
         return []
     if not axv and not flt and -(-dk // group) > 4:
         return []
-    nrb = dv // 32
+    nrb = -(-dv // 32)                                       # the last one may be half empty (Mamba2)
     # row blocks per wavefront: one for the bf16 state, whose blocks are 8 KB each (a head of 128 x 128 on two wavefronts
     # leaves eight per compute unit)
     nb = 2 if nrb % 2 == 0 and fam != 'kda' and not flt else 1
     be = 1 if qbuf else 2
     out = []
     for gh in QUAD_FAMILIES[fam]:
+        if dv % 32 and gh > 1:                               # d_v 80: a head a workgroup (96 heads, int8 g32, 128 sequences:
+            continue                                         # 42.3 us per launch, two heads 53.5, four 44.5)
         nw = gh * nrb // nb
         if nw > 16:
             continue
-        lds = gh * dv * rb + mmax * dkp * be + gh * mmax * dv * be + 2 * dkp * 4 + (0 if flt else dkp * 8) + 512
+        lds = gh * nrb * 32 * rb + mmax * dkp * be + gh * mmax * dv * be + 2 * dkp * 4 + (0 if flt else dkp * 8) + 512
         if fam == 'kda':                                 # keys x decay ratio in fp32 (the raw ones stay in registers), decays
             lds += mmax * dkp * 4 + 2 * dkp * 4 + (2 * dkp * 4 if axv or flt else 0)
         if axv:                                          # a plane set per wavefront
@@ -171,6 +173,27 @@ def quad_variants(fam, c):
         for spec in SPECS[fam] if (qbuf and mmax == 8) else (0,):
             out.append((nb, gh, wpe, spec))
     return out
+
+
+# Heads per launch from which the one-wavefront kernel serves these cases again.  Their workgroups waste something -- lanes
+# and LDS on the columns between 96 and 128, a half empty row block (d_v 80) -- which does not matter while a launch is
+# short of wavefronts and does once it has several rounds of them.  us per launch, workgroup / one wavefront, sequences out
+# of step, just below and above: 96 x 192 (30 heads) int4 g64 128 sequences 25.1 / 27.7, 256 40.9 / 39.2; int8 g128 27.6 /
+# 30.3, 48.1 / 46.9; int8 value-axis 31.0 / 34.6, 192 sequences 43.2 / 42.1; KDA 96 x 96 (20 heads) int4 g32 192 sequences
+# 19.7 / 21.4, 256 24.0 / 23.5; Mamba2 128 x 80 (96 heads) int4 g64 48 sequences 23.3 / 25.5, 64 24.3 / 22.0, int8 g128
+# 24.2 / 27.1, 25.5 / 24.5.  Not for int4 value-axis groups (256 sequences 49.5 / 50.6), KDA's other formats (int8 g32 256
+# sequences 25.3 / 32.2) and the bf16 state (96 x 192, 128 sequences 52.1 / 62.1; Mamba2 128 x 80, 64: 36.8 / 38.7).
+GROUP_HEADS = 5120
+
+
+def group_limit(fam, c):
+    """Whether a case's workgroup kernels serve launches below GROUP_HEADS heads only."""
+    bits, dk, dv, group, qbuf, mmax, axv = c
+    if bits == 16 or (bits == 4 and axv):
+        return False
+    if fam == 'mamba2':
+        return dv % 32 != 0
+    return dk == 96 and (fam == 'gdn' or (bits == 4 and not axv))
 
 
 def _quad_name(fam, c, v):
@@ -255,7 +278,8 @@ def generate():
                     f'&& p.qbuf == {qbuf} && p.m <= {mmax}')
             for v in quad_variants(fam, c):
                 want = f'spec == {v[3]} && ' if v[3] else ''             # the general instance takes whatever is left
-                d.append(f'    if (quad && {want}p.gqa % {v[1]} == 0 && {v[1]} <= ghmax && {cond}) return run ? {_quad_name(fam, c, v)}(p, stream) : 0;')
+                few = f'(!run || int64_t(p.rows) * p.hv < {GROUP_HEADS}) && ' if group_limit(fam, c) else ''
+                d.append(f'    if (quad && {want}{few}p.gqa % {v[1]} == 0 && {v[1]} <= ghmax && {cond}) return run ? {_quad_name(fam, c, v)}(p, stream) : 0;')
             for sp in specs_of(fam, c, False):
                 want = f'spec == {sp} && ' if sp else ''
                 d.append(f'    if ({want}{cond}) return run ? launch_{fam}<{_tile(c)}, {sp}>(p, stream) : 0;')

@@ -81,7 +81,11 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
     const int lane = lane0;
     const int n32 = lane & 31, kb = lane >> 5;
     // the row of the head this lane finishes after the pass (NB = 2: the wavefront's halves take a block each)
-    const int row = (wh * NB + (NB == 2 ? kb : 0)) * T::MR + n32;
+    const int row_ = (wh * NB + (NB == 2 ? kb : 0)) * T::MR + n32;
+    // d_v may end inside the last row block (80): its lanes beyond repeat the last row and keep the result to themselves
+    const bool rlive = !T::RAGV || row_ < DV;
+    const int row = rlive ? row_ : DV - 1;
+    const int rows_left = DV - wh * NB * T::MR;                   // of this wavefront's blocks
 
     Mamba2Loads<T, Q> F;
     const int vl = Q::vec_lane(lane);                             // whose elements of a d_k vector this lane loads
@@ -113,7 +117,7 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
     // ... then the slot's big side, from the preloaded leading arguments alone: the row blocks, straight into their
     // LDS image, and the fill counter (a scalar load; sq_quad.cuh) behind them ...
     quad_start_wait<Q, WPE>(start_ramp);                  // the launch's first workgroups: spread over a ramp
-    quad_dma_blocks<Q, NB>(field(codes, uint32_t(slot), codes_stride, h * (DV * T::ROW_BYTES)) + wh * NB * Q::GBLK, my_codes, lane);
+    quad_dma_blocks<Q, NB, T::RAGV>(field(codes, uint32_t(slot), codes_stride, h * (DV * T::ROW_BYTES)) + wh * NB * Q::GBLK, my_codes, lane, rows_left);
     F.np = quad_dma_counter(field(counters, uint32_t(slot), counters_stride, h));
     __builtin_amdgcn_sched_barrier(0);
     // ... and the rest of the slot
@@ -134,7 +138,7 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
             F.scv[bi] = quad_load_colscales<NE>(SCh + (wh * NB + bi) * DK, vl);
         } else if constexpr (!T::FLT) {
 #pragma unroll
-            for (int g = 0; g < NG; ++g) F.sc[bi][g] = stream_load(SCh + uint32_t(((wh * NB + bi) * T::MR + n32) * NG + g));
+            for (int g = 0; g < NG; ++g) F.sc[bi][g] = stream_load(SCh + uint32_t((T::RAGV ? row : (wh * NB + bi) * T::MR + n32) * NG + g));
         }
     }
     // the buffer, live slots only (the others repeat the last live one: no new memory traffic); the fill count,
@@ -142,12 +146,13 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
     quad_dma_counter_wait(F.np);
     const uint32_t nfill = uint32_t(F.np & (m - 1));
     const uint32_t nl = nfill > 0 ? nfill : 1u;
+    const int ucol = T::RAGV ? min(4 * (lane % Q::LU), rows_left - 4) : 4 * (lane % Q::LU);
     // buffered values of this wavefront's rows: lane (slot = lane / LU + SU t, rows 4 (lane % LU) ..)
 #pragma unroll
     for (int t = 0; t < Q::UT; ++t) {
         const uint32_t i = lane / Q::LU + Q::SU * t;
         const uint32_t ic = i < nl ? i : nl - 1;
-        F.uraw[t] = stream_raw4<T::QBUF>(UBp + (ic * DV + wh * Q::RW + 4 * (lane % Q::LU)) * T::BE);
+        F.uraw[t] = stream_raw4<T::QBUF>(UBp + (ic * DV + wh * Q::RW + ucol) * T::BE);
     }
     // buffered keys, dealt over the workgroup: lane (slot = SPP (NW t + w) + lane / LPS, columns 4 (lane % LPS) ..)
 #pragma unroll
@@ -213,14 +218,14 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
 #pragma unroll
             for (int g = 0; g < NG; ++g) {
                 scw[bi][g] = F.sc[bi][g];
-                if (kb == 0) lds_sc[((wh * NB + bi) * T::MR + n32) * NG + g] = F.sc[bi][g];
+                if (kb == 0) lds_sc[(T::RAGV ? row : (wh * NB + bi) * T::MR + n32) * NG + g] = F.sc[bi][g];
             }
         }
     }
 #pragma unroll
     for (int t = 0; t < Q::UT; ++t) {
         const int i = lane / Q::LU + Q::SU * t;
-        if (i < m) store_raw4<T::QBUF>(lds_ubr + (i * DV + wh * Q::RW + 4 * (lane % Q::LU)) * T::BE, F.uraw[t]);
+        if (i < m) store_raw4<T::QBUF>(lds_ubr + (i * DV + wh * Q::RW + ucol) * T::BE, F.uraw[t]);
     }
 #pragma unroll
     for (int t = 0; t < Q::KT; ++t) {
@@ -369,10 +374,10 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
         accq = __builtin_fmaf(u_i, lane_bcast(cq, i), accq);
     }
     const float xt = raw_to_f(vr, x_dt);
-    const float u = dt * xt;
+    const float u = rlive ? dt * xt : 0.0f;
     float y = __builtin_fmaf(bc, u, a * accq);
     if (p.has_D) y = __builtin_fmaf(dd, xt, y);
-    if (NB == 2 || kb == 0) store_f(outp, out_dt, row, y);
+    if (rlive && (NB == 2 || kb == 0)) store_f(outp, out_dt, row, y);
 
     // ---- append ----
     float us = 1.0f;
@@ -387,7 +392,7 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
         us = fp16_scale(amax, 127.0f);
         if (wh == 0 && lane == 0) { UBSp[n] = f32_to_f16(us); lds_ubsf[n] = us; }
     }
-    if (NB == 2 || kb == 0) {
+    if (rlive && (NB == 2 || kb == 0)) {
         if constexpr (T::QBUF) {
             const int8_t c = int8_t(int(round_buf(u, us)));
             reinterpret_cast<int8_t*>(UBp)[n * DV + row] = c;
@@ -465,6 +470,7 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
                 uint8_t* blk = my_codes + bi * Q::BLK;
 #pragma unroll
                 for (int hf = 0; hf < 2; ++hf) {
+                    if (T::RAGV && 16 * hf >= rows_left) continue;
                     const int frow = (wh * NB + bi) * T::MR + 16 * hf + fn;
                     float bop[MT4];
 #pragma unroll
@@ -483,7 +489,7 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
                                                 SCh + frow * NG + fg, lf);
                 }
                 wave_sync();
-                quad_store_block<Q>(Sh + (wh * NB + bi) * Q::GBLK, blk, lf);
+                quad_store_block<Q, T::RAGV>(Sh + (wh * NB + bi) * Q::GBLK, blk, lf, rows_left);
             }
         }
     }

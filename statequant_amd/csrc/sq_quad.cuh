@@ -83,7 +83,8 @@ __device__ __forceinline__ void quad_start_wait(uint32_t ramp) {
 
 template <class T, int NB_, int GH_ = 1>
 struct Quad {
-    static_assert(T::BITS <= 16 && !T::RAGV, "int4 / int8 codes or a bf16 state, whole row blocks");
+    static_assert(T::BITS <= 16 && T::DV % 16 == 0, "int4 / int8 codes or a bf16 state, whole half row blocks");
+    static_assert(!T::RAGV || (NB_ == 1 && !T::AXV), "a half empty last row block: a wavefront of its own, key-axis groups");
     static_assert(!T::AXV || T::GROUP == T::MR, "value-axis groups: one row block each");
     static constexpr int NB = NB_;                         // row blocks per wavefront
     static constexpr int GH = GH_;                         // value heads of one key head per workgroup
@@ -101,7 +102,7 @@ struct Quad {
     static constexpr int LIVE = T::ROW_BYTES / 16;         // ... of which hold columns
     static constexpr int BLK = T::MR * RB;                 // bytes of a row block in LDS
     static constexpr int GBLK = T::MR * T::ROW_BYTES;      // ... in memory
-    static constexpr int HEAD = T::DV * RB;                // bytes of a head's codes in LDS
+    static constexpr int HEAD = T::NRB * BLK;              // bytes of a head's codes in LDS
     static constexpr int NKS = T::BITS == 4 ? (T::NKS + 1) / 2 * 2 : T::NKS;    // column steps (int4: whole chunk pairs)
     static constexpr int NLD = BLK / 1024;                 // wavefront loads per row block
     static constexpr int SWM = CPR < 8 ? CPR : 8;          // swizzle: chunk c of row r sits at chunk c ^ ((r / SWD) % SWM)
@@ -362,8 +363,9 @@ __device__ __forceinline__ void quad_dma_counter_wait(int& counter) {
 // its own address pair and LDS base on purpose: the four pieces of a block behind one address with the instruction's
 // immediate offsets (which advance both addresses) issue back to back and measured slower (headline 33.1 against
 // 32.7 us per launch, Mamba2 32.1 against 31.1) -- the address arithmetic in between spaces a wavefront's requests.
-template <class Q, int NBLK>
-__device__ __forceinline__ void quad_dma_blocks(const uint8_t* src, uint8_t* dst, int lane) {
+// `rows`: how many of them exist (d_v that ends inside a block; the rest of the image is left alone).
+template <class Q, int NBLK, bool RAGV = false>
+__device__ __forceinline__ void quad_dma_blocks(const uint8_t* src, uint8_t* dst, int lane, int rows = 0) {
     const int pr = lane / Q::CPR, pc = lane % Q::CPR;
 #pragma unroll
     for (int bi = 0; bi < NBLK; ++bi)
@@ -374,20 +376,23 @@ __device__ __forceinline__ void quad_dma_blocks(const uint8_t* src, uint8_t* dst
             const uint8_t* g = src + bi * Q::GBLK + r * (Q::GBLK / 32) + (c << 4);
             const uint32_t at = uint32_t(reinterpret_cast<uintptr_t>(
                 (__attribute__((address_space(3))) uint8_t*)(dst + bi * Q::BLK + t * 1024)));
-            if (!Q::PADK || c < Q::LIVE)                     // a lane that is switched off writes nothing
+            if ((!Q::PADK || c < Q::LIVE) && (!RAGV || r < rows))    // a lane that is switched off writes nothing
                 asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt"
                              :: "v"(g), "s"(at) : "memory", "m0");
         }
 }
 // A row block's LDS image back to memory.
-template <class Q>
-__device__ __forceinline__ void quad_store_block(uint8_t* dst, const uint8_t* blk, int lane) {
+template <class Q, bool RAGV = false>
+__device__ __forceinline__ void quad_store_block(uint8_t* dst, const uint8_t* blk, int lane, int rows = 0) {
+    const uint32_t rp = uint32_t(lane) / Q::CPR, c = uint32_t(lane) % Q::CPR;
+    constexpr bool PERIOD = (WAVE / Q::CPR) % (Q::SWD * Q::SWM) == 0;       // the swizzle repeats from load to load
 #pragma unroll
     for (int t = 0; t < Q::NLD; ++t) {
-        const int r = t * (1024 / Q::RB) + lane / Q::CPR, c = lane % Q::CPR;
-        if (!Q::PADK || c < Q::LIVE)
-            stream_store(reinterpret_cast<v4u*>(dst + r * (Q::GBLK / 32) + (c << 4)),
-                         *reinterpret_cast<const v4u*>(blk + swz<Q>(r, c)));
+        const int r = t * (1024 / Q::RB) + rp;
+        const uint32_t at = Q::PADK ? r * (Q::GBLK / 32) + (c << 4) : t * 1024 + uint32_t(lane) * 16;
+        const int image = PERIOD ? t * 1024 + swz<Q>(rp, c) : swz<Q>(r, c);
+        if ((!Q::PADK || c < uint32_t(Q::LIVE)) && (!RAGV || r < rows))
+            stream_store(reinterpret_cast<v4u*>(dst + at), *reinterpret_cast<const v4u*>(blk + image));
     }
 }
 __device__ __forceinline__ void quad_dma_landed() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }

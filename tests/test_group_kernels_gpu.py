@@ -39,6 +39,10 @@ CASES = [
     ('gdn', 'bf16', (2, 1, 96, 96), 1, 16), ('kda', 'bf16', (3, 3, 128, 128), 8, 8), ('kda', 'bf16', (2, 2, 96, 96), 4, 16),
     ('kda', 'bf16', (5, 5, 64, 32), 8, 8), ('mamba2', 'bf16', (8, 2, 128, 64), 8, 8),
     ('mamba2', 'bf16', (4, 1, 128, 128), 16, 16), ('mamba2', 'bf16', (6, 6, 64, 64), 2, 8),
+    # d_v 80: the last row block half empty
+    ('mamba2', (8, 'k', 128), (6, 2, 128, 80), 8, 8), ('mamba2', (4, 'k', 64), (4, 1, 128, 80), 16, 16),
+    ('mamba2', (8, 'k', 32), (12, 4, 96, 80), 4, 8), ('mamba2', (4, 'k', 32), (3, 3, 96, 80), 1, 8),
+    ('mamba2', 'bf16', (4, 1, 128, 80), 8, 8), ('mamba2', 'bf16', (6, 6, 96, 80), 2, 16),
 ]
 
 
@@ -125,3 +129,28 @@ def test_group_kernel_matches_the_one_wavefront_kernel(family, fmt, shape, m, bb
     # bf16 steps are 2^-8 of a value; the two sums of up to 17 terms differ by some 2^-23 of it, and by more where they cancel
     assert off <= (2e-3 if lay.bits == 16 else 1e-4) * codes and scales_off <= 1e-4 * scales + 2, (off, codes, scales_off, scales)
     assert flips <= 1e-4 * entries + 2 * max(dk, dv), (flips, entries)
+
+
+@pytest.mark.parametrize('family,fmt,shape', [('gdn', (4, 'k', 64), (40, 40, 96, 96)), ('kda', (4, 'k', 32), (40, 40, 96, 96)),
+                                              ('mamba2', (8, 'k', 32), (40, 8, 128, 80))])
+def test_launches_either_side_of_the_head_count_agree(family, fmt, shape):
+    """5120 heads go to the one-wavefront kernel, one sequence less to the workgroup kernel (bounds as above)."""
+    hv, hk, dk, dv = shape
+    rows = 128
+    lay = _layout(family, fmt, shape, 4, 8)
+    gen = torch.Generator().manual_seed(6)
+    blobs = [lay.alloc(rows + 1, DEV) for _ in range(2)]
+    V = [lay.views(b) for b in blobs]
+    idx = torch.arange(1, rows + 1, dtype=torch.int32, device=DEV)
+    lay.write(V[0], idx, torch.randn(rows, hv, dv, dk, generator=gen).to(DEV) * 0.4)
+    r = lambda *s: torch.randn(*s, generator=gen).to(DEV)          # noqa: E731
+    model = (-torch.exp(r(hv)), r(hv), r(hv)) if family == 'mamba2' else None
+    for step in range(5):
+        blobs[1].copy_(blobs[0])
+        t = _token(family, gen, rows, shape)
+        outs = [torch.zeros(rows, hv, dv, device=DEV) for _ in range(2)]
+        _step(family, lay, V[0], idx, t, outs[0], model)
+        _step(family, lay, V[1], idx[:-1], {k: x[:-1] for k, x in t.items()}, outs[1], model)
+        assert ((outs[0] - outs[1])[:-1].abs().max() / outs[0].abs().max()).item() <= 1e-5, step
+        mism, far, n = code_diff(V[0]['S'][1:rows].cpu(), V[1]['S'][1:rows].cpu(), lay.bits)
+        assert far == 0 and mism <= 1e-4 * n
