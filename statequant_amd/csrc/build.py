@@ -129,9 +129,9 @@ QUAD_OK = {'gdn': [
 
 
 def quad_variants(fam, c):
-    """[(row blocks per wavefront, value heads per workgroup, wavefronts per SIMD the register allocation aims
-    for)], widest head group first, of the workgroup-per-key-head kernels (sq_quad.cuh) for a case; empty where only
-    the one-wavefront kernels (sq_tile.cuh) serve it: value-axis groups other than 32 rows, the fp32 state, d_v that is no
+    """[(row blocks per wavefront, value heads per workgroup, wavefronts per SIMD the register allocation aims for,
+    serving case, heads per launch it is for -- 0: any)], small launches' first, then widest head group first, of the
+    workgroup kernels (sq_quad.cuh) for a case; empty where only the one-wavefront kernels (sq_tile.cuh) serve it: value-axis groups other than 32 rows, the fp32 state, d_v that is no
     multiple of 32 (Mamba2: 16), d_k above 128, more than four scale groups per row, states beyond 64 KB."""
     bits, dk, dv, group, qbuf, mmax, axv = c
     if fam not in QUAD_FAMILIES or bits not in (4, 8, 16) or (axv and group != 32):
@@ -171,8 +171,22 @@ def quad_variants(fam, c):
         wpe = max(1, min(6 if mmax <= 8 and not axv else 5, -(-wgs * nw // 4)))
         # the serving cases compiled in (SPEC of the kernels) for the default buffer: int8, 8 tokens
         for spec in SPECS[fam] if (qbuf and mmax == 8) else (0,):
-            out.append((nb, gh, wpe, spec))
+            out.append((nb, gh, wpe, spec, 0))
+    small = SMALL_LAUNCH.get((fam, dk, dv, axv)) if not flt and qbuf and mmax == 8 else None
+    if small:                                            # the one-head entries again, a row block per wavefront
+        out = [(1, 1, 6 if not axv else 5, spec, small) for spec in SPECS[fam]] + out
     return out
+
+
+# Launches below so many heads take one row block per wavefront and one head per workgroup: twice the wavefronts on up to
+# four times the compute units, so that a head's life -- which is all such a launch consists of, the fold's four half
+# blocks in sequence above all -- gets shorter.  (One block per wavefront with two heads per workgroup gains nothing:
+# the wavefronts then share the SIMDs they had.)  us per launch, two blocks and two heads / this, sequences out of step:
+# GDN 128 x 128 (32 heads) int8 g32 1 sequence 5.22 / 4.77, 16: 9.8 / 8.0, 56: 15.4 / 14.8, 64: 14.3 / 14.7; int4 g64 16:
+# 9.4 / 7.7, 56: 13.7 / 13.4, 64: 12.2 / 13.3; value-axis int4 1: 6.2 / 5.3, 16: 12.4 / 9.1, 64: 15.0 / 14.0, 100: 24.0 /
+# 23.3; 96 x 192 int4 g64 (30 heads) 8: 7.8 / 6.9, 24: 12.3 / 11.8, 28: 12.6 / 13.9; Mamba2 128 x 64 (128 heads) int8 g128
+# 1: 5.07 / 4.54, 6: 7.16 / 7.09, 8: 7.89 / 8.01.
+SMALL_LAUNCH = {('gdn', 128, 128, 0): 2048, ('gdn', 128, 128, 1): 3072, ('gdn', 96, 192, 0): 768, ('mamba2', 128, 64, 0): 768}
 
 
 # Heads per launch from which the one-wavefront kernel serves these cases again.  Their workgroups waste something -- lanes
@@ -197,7 +211,7 @@ def group_limit(fam, c):
 
 
 def _quad_name(fam, c, v):
-    nb, gh, wpe, spec = v
+    nb, gh, wpe, spec, _ = v
     return f'launch_{fam}_quad<{_tile(c)}, {nb}, {gh}, {wpe}, {spec}>'
 
 
@@ -278,7 +292,8 @@ def generate():
                     f'&& p.qbuf == {qbuf} && p.m <= {mmax}')
             for v in quad_variants(fam, c):
                 want = f'spec == {v[3]} && ' if v[3] else ''             # the general instance takes whatever is left
-                few = f'(!run || int64_t(p.rows) * p.hv < {GROUP_HEADS}) && ' if group_limit(fam, c) else ''
+                limit = v[4] or (GROUP_HEADS if group_limit(fam, c) else 0)
+                few = f'(!run || int64_t(p.rows) * p.hv < {limit}) && ' if limit else ''
                 d.append(f'    if (quad && {want}{few}p.gqa % {v[1]} == 0 && {v[1]} <= ghmax && {cond}) return run ? {_quad_name(fam, c, v)}(p, stream) : 0;')
             for sp in specs_of(fam, c, False):
                 want = f'spec == {sp} && ' if sp else ''

@@ -131,12 +131,19 @@ def test_group_kernel_matches_the_one_wavefront_kernel(family, fmt, shape, m, bb
     assert flips <= 1e-4 * entries + 2 * max(dk, dv), (flips, entries)
 
 
-@pytest.mark.parametrize('family,fmt,shape', [('gdn', (4, 'k', 64), (40, 40, 96, 96)), ('kda', (4, 'k', 32), (40, 40, 96, 96)),
-                                              ('mamba2', (8, 'k', 32), (40, 8, 128, 80))])
-def test_launches_either_side_of_the_head_count_agree(family, fmt, shape):
-    """5120 heads go to the one-wavefront kernel, one sequence less to the workgroup kernel (bounds as above)."""
+@pytest.mark.parametrize('family,fmt,shape,rows', [
+    # workgroup / one-wavefront kernel
+    ('gdn', (4, 'k', 64), (40, 40, 96, 96), 128), ('kda', (4, 'k', 32), (40, 40, 96, 96), 128),
+    ('mamba2', (8, 'k', 32), (40, 8, 128, 80), 128),
+    # one / two row blocks per wavefront
+    ('gdn', (8, 'k', 32), (32, 16, 128, 128), 64), ('gdn', (4, 'k', 64), (32, 16, 128, 128), 64),
+    ('gdn', (8, 'k', 128), (32, 8, 128, 128), 64), ('gdn', (4, 'v', 32), (32, 16, 128, 128), 96),
+    ('gdn', (8, 'v', 32), (24, 24, 128, 128), 128), ('gdn', (8, 'k', 64), (30, 30, 96, 192), 26),
+    ('mamba2', (8, 'k', 128), (128, 8, 128, 64), 6), ('mamba2', (4, 'k', 32), (96, 8, 128, 64), 8)])
+def test_launches_either_side_of_a_head_count_agree(family, fmt, shape, rows):
+    """A launch at the number of heads where another kernel takes over, and the same launch one sequence shorter (bounds
+    as above)."""
     hv, hk, dk, dv = shape
-    rows = 128
     lay = _layout(family, fmt, shape, 4, 8)
     gen = torch.Generator().manual_seed(6)
     blobs = [lay.alloc(rows + 1, DEV) for _ in range(2)]
