@@ -1,6 +1,7 @@
 // Gated DeltaNet packed decode step, one workgroup per (batch row, key head): the GH value heads of the key head
 // share q, k, the buffered keys and everything computed from them; every wavefront owns NB 32-row blocks of one
-// value head's state (int4 / int8 codes, key-axis scale groups; geometry and building blocks in sq_quad.cuh).
+// value head's state (int4 / int8 codes with key-axis or 32-row value-axis groups, or bf16; geometry and building blocks
+// in sq_quad.cuh).
 //
 // Same arithmetic per head as the one-wavefront kernel of sq_gdn.cuh (the reference's fused Triton step,
 // /root/reference/src/statequant/kernels/_fused_triton.py:48-190).  Division of labour inside the workgroup:

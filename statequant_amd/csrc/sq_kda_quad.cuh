@@ -1,5 +1,5 @@
 // KDA packed decode step, one workgroup per (batch row, head): every wavefront owns NB 32-row blocks of the head's state
-// (int4 / int8 codes, key-axis groups or value-axis groups of one row block; geometry and building blocks in
+// (int4 / int8 codes, key-axis groups or value-axis groups of one row block, or bf16; geometry and building blocks in
 // sq_quad.cuh).
 //
 // Same arithmetic as the one-wavefront kernel of sq_kda.cuh (the reference's `_kda_step`,

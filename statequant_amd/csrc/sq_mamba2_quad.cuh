@@ -1,7 +1,7 @@
 // Mamba2 / SSD packed decode step, one workgroup per (batch row, GH heads of one B / C group): the heads share C
 // (the read-out vector, its digit planes), B (this token's key, its rounded copy for the buffer) and every product
-// with the buffered keys; every wavefront owns NB 32-row blocks of one head's state (int4 / int8 codes, key-axis
-// scale groups; geometry and building blocks in sq_quad.cuh).
+// with the buffered keys; every wavefront owns NB 32-row blocks of one head's state (int4 / int8 codes with key-axis or
+// 32-row value-axis groups, or bf16; geometry and building blocks in sq_quad.cuh).
 //
 // Same arithmetic per head as the one-wavefront kernel of sq_mamba2.cuh (the reference's `_m2_step`,
 // /root/reference/src/statequant/kernels/_mamba2_triton.py:48-197):
