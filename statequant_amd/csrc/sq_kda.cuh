@@ -183,7 +183,9 @@ void kda_step_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
             const int i = l.rg + T::RG * t;
             float kb[CPL];
             decode_kpiece<T>(kbuf.piece[t], f16_to_f32(kbuf.kbs[t]), l, kb);
-            const bool alive = i < n;                             // dead slots may hold anything: discard
+            // dead slots may hold anything, and idle lanes hold another piece's G_i beside a zero G_n, a ratio that can
+            // overflow: discard both (an infinity times the idle lanes' zero keys would be a NaN in the sums)
+            const bool alive = i < n && l.cg < T::LPR;
             float pq = 0.0f, pk = 0.0f;
 #pragma unroll
             for (int k = 0; k < CPL / 4; ++k) {

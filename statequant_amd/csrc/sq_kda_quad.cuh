@@ -227,7 +227,9 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
 #pragma unroll
         for (int t = 0; t < Q::KT; ++t) {
             const int i = Q::SPP * (NW * t + w) + lane / Q::LPS;
-            const bool alive = i < n;                              // dead slots may hold anything: discard
+            // dead slots may hold anything, and the columns beyond d_k pair one channel's G_n with another's G_i, a ratio
+            // that can overflow: discard both (an infinity times the vectors' zeros there would be a NaN in the sums)
+            const bool alive = i < n && (!Q::PADK || c4 < DK);
             float kf[4];
             decode_raw4<T::QBUF>(F.kraw[t], kf);
             const float ks = f16_to_f32(F.kbs[t]);

@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from oracle import states as ST
-from statequant_amd.kernels import KDASlotLayout, PackedKDAState, kda_recurrence
+from statequant_amd.kernels import KDASlotLayout, PackedKDAState, _hip, kda_recurrence
 from tests._util import Tally, buffer_entry, quantizer, unpack_nib
 
 pytestmark = pytest.mark.gpu
@@ -149,6 +149,25 @@ def test_strong_per_channel_decays(fmt, m, bb):
     T = 2 * m + 3
     tal = run_decode(fmt, m, bb, T=T, shape_token=shape_token)
     check(tal, f'kda strong decays {fmt} m={m} buf{bb}', T, m)
+
+
+@pytest.mark.parametrize('group_kernel', [True, False])
+@pytest.mark.parametrize('fmt,m,bb', [((4, 'k', 32), 8, 8), ((8, 'k', 32), 16, 16), ((4, 'v', 32), 8, 8), ('bf16', 8, 8)])
+def test_padded_columns_stay_out_of_strong_decays(fmt, m, bb, group_kernel):
+    """d_k 96: a quarter of the channels decays by e^-40 a token beside channels that do not decay at all.  Both kernels
+    hold a row in 128 columns, and the 32 beyond d_k pair the decays of different channels: their ratios overflow fp32
+    from the third buffered token on (exp(120)), which no coefficient may see."""
+    def shape_token(q, k, v, g, beta):
+        g[..., 0::4] = -40.0
+        g[..., 1::2] = 0.0
+
+    T = 2 * m + 3
+    _hip.select_instances(no_group_kernel=not group_kernel)
+    try:
+        tal = run_decode(fmt, m, bb, H=3, DK=96, DV=96, T=T, shape_token=shape_token)
+    finally:
+        _hip.select_instances()
+    check(tal, f'kda d_k 96, strong decays {fmt} m={m} buf{bb}', T, m)
 
 
 def test_bf16_inputs():
