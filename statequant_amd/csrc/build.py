@@ -17,12 +17,13 @@ import os
 import re
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
 OUT = os.path.join(HERE, 'build')
 LIB = os.path.join(PKG, 'libsqhip.so')
-HOST = os.path.join(PKG, '_sqhost.so')
+HOST = os.path.join(PKG, '_sqhost' + sysconfig.get_config_var('EXT_SUFFIX'))
 ARCH = 'gfx950'
 
 # -ffp-contract=off: every fused multiply-add in the kernels is written explicitly, as in the reference's kernels.
@@ -337,7 +338,7 @@ def _stamp():
     """Hash of every source that goes into the library (to skip a rebuild when nothing changed)."""
     h = hashlib.sha256()
     for name in sorted(os.listdir(HERE)):
-        if name.endswith(('.cuh', '.h', '.hip', '.cpp', '.py')):
+        if name.endswith(('.cuh', '.h', '.hip', '.py')):
             h.update(open(os.path.join(HERE, name), 'rb').read())
     h.update(open(os.path.join(os.path.dirname(PKG), 'include', 'statequant_hip.h'), 'rb').read())
     h.update(' '.join(HIPCC_FLAGS).encode())
@@ -439,15 +440,27 @@ def _compile(src, force=False):
     return obj
 
 
-def build_host():
+def _host_stamp():
+    """What the extension depends on: its source, the C ABI, and the interpreter and torch whose headers it includes."""
+    import torch
+    h = hashlib.sha256()
+    for path in (os.path.join(HERE, 'sq_host.cpp'), os.path.join(os.path.dirname(PKG), 'include', 'statequant_hip.h')):
+        h.update(open(path, 'rb').read())
+    h.update(repr((torch.__version__, torch._C._GLIBCXX_USE_CXX11_ABI, os.path.basename(HOST))).encode())
+    return h.hexdigest()
+
+
+def build_host(force=False):
     """Compile the Python extension of the step wrappers (sq_host.cpp: host code only, against this interpreter's and
-    this torch's headers) next to the library."""
-    import sysconfig
+    this torch's headers) next to the library, unless it is current."""
     import torch
     from torch.utils import cpp_extension
+    stamp_path, stamp = os.path.join(OUT, 'host_stamp'), _host_stamp()
+    if not force and os.path.exists(HOST) and os.path.exists(stamp_path) and open(stamp_path).read() == stamp:
+        return HOST
     lib_dirs = cpp_extension.library_paths()
     cmd = ['g++', '-O2', '-std=c++17', '-fPIC', '-shared', '-D__HIP_PLATFORM_AMD__=1', '-DUSE_ROCM=1',
-           f'-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}',
+           f'-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}', f'-DSQ_TORCH="{torch.__version__}"',
            *(f'-I{p}' for p in cpp_extension.include_paths()), '-I' + sysconfig.get_paths()['include'],
            '-I' + os.path.join(os.environ.get('ROCM_PATH', '/opt/rocm'), 'include'),
            os.path.join(HERE, 'sq_host.cpp'), '-o', HOST, *(f'-L{p}' for p in lib_dirs),
@@ -455,6 +468,8 @@ def build_host():
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode:
         raise RuntimeError(f'{" ".join(cmd)}\n{r.stdout}\n{r.stderr}')
+    with open(stamp_path, 'w') as f:
+        f.write(stamp)
     return HOST
 
 
@@ -464,7 +479,8 @@ def build(jobs=None, force=False, verbose=True):
     units = generate()
     stamp_path = os.path.join(OUT, 'stamp')
     stamp = _stamp()
-    if not force and os.path.exists(LIB) and os.path.exists(HOST) and os.path.exists(stamp_path) and open(stamp_path).read() == stamp:
+    build_host(force)
+    if not force and os.path.exists(LIB) and os.path.exists(stamp_path) and open(stamp_path).read() == stamp:
         if verbose:
             print(f'[build] {LIB} is up to date')
         return LIB
@@ -477,7 +493,6 @@ def build(jobs=None, force=False, verbose=True):
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode:
         raise RuntimeError(f'{" ".join(cmd)}\n{r.stdout}\n{r.stderr}')
-    build_host()
     with open(stamp_path, 'w') as f:
         f.write(stamp)
     if verbose:

@@ -10,6 +10,9 @@
 // tensors on one GPU, the documented shapes -- and answers None to anything else (another tensor class, a tensor under a
 // function transform, a CPU tensor, a wrong dtype or stride, a dict entry that is missing): the Python code then does the
 // whole call itself, so what is refused, and with which message, is decided in one place.  Nothing is kept between calls.
+//
+// The extension uses torch's C++ classes, so it belongs to the torch it was built against: SQ_TORCH, the module's TORCH,
+// names that version, and the Python side leaves a module of another one alone (every call then goes the Python way).
 #include <torch/csrc/autograd/python_variable.h>
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
@@ -548,5 +551,10 @@ PyMODINIT_FUNC PyInit__sqhost() {
     for (int f = 0; f < F_COUNT; ++f)
         if (!(field_name[f] = PyUnicode_InternFromString(FIELD_NAMES[f]))) return nullptr;
     if (!(blob_name = PyUnicode_InternFromString("blob"))) return nullptr;
-    return PyModule_Create(&module);
+    PyObject* const m = PyModule_Create(&module);
+    if (m && PyModule_AddStringConstant(m, "TORCH", SQ_TORCH) != 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
 }

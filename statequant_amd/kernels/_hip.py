@@ -8,12 +8,12 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import warnings
 
 import torch
 
 _PKG = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB_PATH = os.path.join(_PKG, 'libsqhip.so')
-HOST_PATH = os.path.join(_PKG, '_sqhost.so')
 ABI_VERSION = 6
 
 F32, BF16, F16 = 0, 1, 2
@@ -149,20 +149,35 @@ def lib():
     return _lib
 
 
+class _PythonOnly:
+    """In the place of the native call path where there is none: every call is declined."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 def host():
     """The native side of the step and hand-over wrappers (``csrc/sq_host.cpp``): checks, argument structs and the
-    launch of one ordinary call in about a microsecond of host time.  Each of its functions returns the library's status,
-    or None for a call that is not of the ordinary form, which the Python code then does (or refuses) itself."""
+    launch of one ordinary call without Python in between.  Each of its functions returns the library's status, or None
+    for a call that is not of the ordinary form, which the Python code then does (or refuses) itself -- as it does every
+    call where the extension is missing or was built against another torch (it uses torch's C++ classes; the library
+    itself has no torch types)."""
     global _host
     if _host is None:
         L = lib()
-        if not os.path.exists(HOST_PATH):
-            raise RuntimeError(f'{HOST_PATH} is missing: build it with `python -m statequant_amd.csrc.build`')
-        from .. import _sqhost
+        try:
+            from .. import _sqhost as h
+            if h.TORCH != str(torch.__version__):
+                raise ImportError(f'built against torch {h.TORCH}, this is {torch.__version__}')
+        except ImportError as e:
+            warnings.warn(f'statequant_amd: no native call path ({e}); calls take some 17 us of Python each.  Build it with '
+                          '`python -m statequant_amd.csrc.build`', stacklevel=3)
+            _host = _PythonOnly()
+            return _host
         addr = lambda f: C.cast(f, C.c_void_p).value                            # noqa: E731
-        _sqhost.init(addr(L.sq_gdn_step), addr(L.sq_kda_step), addr(L.sq_mamba2_step), addr(L.sq_gga_step),
-                     addr(L.sq_pack_vk), addr(L.sq_read))
-        _host = _sqhost
+        h.init(addr(L.sq_gdn_step), addr(L.sq_kda_step), addr(L.sq_mamba2_step), addr(L.sq_gga_step),
+               addr(L.sq_pack_vk), addr(L.sq_read))
+        _host = h
     return _host
 
 

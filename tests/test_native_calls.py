@@ -1,7 +1,9 @@
 """The native call path of the step / hand-over wrappers (csrc/sq_host.cpp) against the Python one: same bytes for the
 calls it takes, None -- and therefore the Python path's own answer -- for every other call."""
 import copy
+import sys
 import time
+import types
 
 import pytest
 import torch
@@ -53,6 +55,37 @@ def test_cpu_tensors_and_wrong_objects_are_declined():
         h.gdn_step(st, V)
     with pytest.raises(RuntimeError, match='GPU'):
         lay.step(V, idx, x, x, out, out, 1.0, g=out[..., 0], beta=out[..., 0])
+
+
+@pytest.mark.parametrize('other', ['missing', 'of another torch'])
+def test_without_a_native_call_path_every_call_goes_the_python_way(other, monkeypatch):
+    """The library needs no torch headers; the extension in front of it does.  Where it is missing or was built against
+    another torch, nothing of it is called (its functions would raise here) and the Python path does every call."""
+    import statequant_amd
+    module = None if other == 'missing' else types.SimpleNamespace(TORCH='0.0')
+    monkeypatch.setitem(sys.modules, 'statequant_amd._sqhost', module)
+    monkeypatch.setattr(statequant_amd, '_sqhost', module, raising=False)
+    if module is None:
+        monkeypatch.delattr(statequant_amd, '_sqhost')
+    monkeypatch.setattr(_hip, '_host', None)
+    lay = SlotLayout(sq.Quantizer(8, 'k', 32), 4, 2, 64, 64)
+    V = lay.views(lay.alloc(3, 'cpu'))
+    lay._conv = lay._lay = lay._layout_struct()
+    idx, x = torch.ones(1, dtype=torch.int32), torch.randn(1, 4, 64, 64)
+    with pytest.warns(UserWarning, match='no native call path'):
+        lay.write(V, idx, x)
+    assert torch.allclose(lay.read(V, idx), x, atol=0.05)
+    q, out = torch.zeros(1, 2, 64), torch.zeros(1, 4, 64)
+    with pytest.raises(RuntimeError, match='GPU'):
+        lay.step(V, idx, q, q, out, out, 1.0, g=out[..., 0], beta=out[..., 0])
+    assert _hip.host().gdn_step(*range(12)) is None
+
+
+def test_the_extension_is_rebuilt_for_another_torch(monkeypatch):
+    from statequant_amd.csrc import build
+    stamp = build._host_stamp()
+    monkeypatch.setattr(torch, '__version__', '0.0')
+    assert build._host_stamp() != stamp
 
 
 def test_a_declined_call_costs_little():
