@@ -101,32 +101,24 @@ def _tile(c):
             + (', true>' if axv else '>'))
 
 
-# Run-time conditions of the workgroup-per-key-head kernels, per family (part of the generated dispatch unit).
-QUAD_OK = {'gdn': [
-    '// q, k per key head (or ungrouped keys), rows that 16-byte vector loads can address',
+# Run-time conditions of the workgroup kernels, per family (part of the generated dispatch unit): vectors and rows of codes
+# that 16-byte accesses can address.  (The C ABI asks int4 states for 8-byte alignment only: those that have no more go to
+# the one-wavefront kernels, which read 8 bytes a lane.)
+QUAD_OK = [
+    'static bool rows16(const void* ptr, uint32_t stride, int dt) {',
+    '    return reinterpret_cast<uintptr_t>(ptr) % 16 == 0 && (uint64_t(stride) * (dt == 0 ? 4 : 2)) % 16 == 0;',
+    '}',
+    'static bool codes16(const StatePtrs& st) { return reinterpret_cast<uintptr_t>(st.S) % 16 == 0 && st.sS % 16 == 0; }',
+    '// q, k per key head (or ungrouped keys)',
     'static bool gdn_quad_ok(const GdnParams& p) {',
-    '    if (!p.qk_per_key_head && p.gqa > 1) return false;',
-    '    auto ok = [](const void* ptr, uint32_t stride, int dt) {',
-    '        return reinterpret_cast<uintptr_t>(ptr) % 16 == 0 && (uint64_t(stride) * (dt == 0 ? 4 : 2)) % 16 == 0;',
-    '    };',
-    '    return ok(p.q, p.s_q, p.q_dt) && ok(p.k, p.s_k, p.k_dt);',
-    '}'],
-    'mamba2': [
-    '// B, C rows that 16-byte vector loads can address',
+    '    return (p.qk_per_key_head || p.gqa == 1) && codes16(p.st) && rows16(p.q, p.s_q, p.q_dt) && rows16(p.k, p.s_k, p.k_dt);',
+    '}',
     'static bool mamba2_quad_ok(const Mamba2Params& p) {',
-    '    auto ok = [](const void* ptr, uint32_t stride, int dt) {',
-    '        return reinterpret_cast<uintptr_t>(ptr) % 16 == 0 && (uint64_t(stride) * (dt == 0 ? 4 : 2)) % 16 == 0;',
-    '    };',
-    '    return ok(p.B, p.s_B, p.B_dt) && ok(p.C, p.s_C, p.C_dt);',
-    '}'],
-    'kda': [
-    '// q, k, g rows that 16-byte vector loads can address',
+    '    return codes16(p.st) && rows16(p.B, p.s_B, p.B_dt) && rows16(p.C, p.s_C, p.C_dt);',
+    '}',
     'static bool kda_quad_ok(const KdaParams& p) {',
-    '    auto ok = [](const void* ptr, uint32_t stride, int dt) {',
-    '        return reinterpret_cast<uintptr_t>(ptr) % 16 == 0 && (uint64_t(stride) * (dt == 0 ? 4 : 2)) % 16 == 0;',
-    '    };',
-    '    return ok(p.q, p.s_q, p.q_dt) && ok(p.k, p.s_k, p.k_dt) && ok(p.g, p.s_g, p.g_dt);',
-    '}']}
+    '    return codes16(p.st) && rows16(p.q, p.s_q, p.q_dt) && rows16(p.k, p.s_k, p.k_dt) && rows16(p.g, p.s_g, p.g_dt);',
+    '}']
 
 
 def quad_variants(fam, c):
@@ -274,13 +266,12 @@ def generate():
          '    g_ghmax.store(ghmax > 0 ? ghmax : 64);',
          '    g_lds_pad.store(lds_pad > 0 ? lds_pad : 0);',
          '}',
-         'int quad_lds_pad() { return g_lds_pad.load(std::memory_order_relaxed); }']
+         'int quad_lds_pad() { return g_lds_pad.load(std::memory_order_relaxed); }', *QUAD_OK]
     for fam, rows in CASES.items():
         P = PARAMS[fam]
         d.append(f'template <class T, int SPEC> int launch_{fam}(const {P}&, hipStream_t);')
         if fam in QUAD_FAMILIES:
             d.append(f'template <class T, int NB, int GH, int WPE, int SPEC> int launch_{fam}_quad(const {P}&, hipStream_t);')
-            d += QUAD_OK[fam]
         d.append(f'int dispatch_{fam}(const {P}& p, hipStream_t stream, bool run) {{')
         d.append('    const int spec = (run && !g_no_spec.load(std::memory_order_relaxed)) ? serving_case(p) : 0;')
         if fam in QUAD_FAMILIES:

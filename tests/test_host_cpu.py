@@ -398,3 +398,46 @@ def test_build_lint_of_the_hand_placed_scalar_wait():
     # a compiler-placed wait does not count: only the assembly statement's own does
     compiler_wait = good.replace('\t;;#ASMSTART\n\ts_waitcnt lgkmcnt(0)\n\t;;#ASMEND\n', '\ts_waitcnt lgkmcnt(0)\n')
     assert lint_counter_loads(compiler_wait) != []
+
+
+def test_workgroup_kernels_ask_for_16_byte_rows_of_codes(tmp_path):
+    """The workgroup kernels move rows of codes 16 bytes at a time; the C ABI takes int4 states aligned to 8.  The
+    dispatch conditions, compiled for the host: a state, a stride or an operand that 16-byte accesses cannot address is
+    left to the one-wavefront kernels."""
+    import shutil
+    import subprocess
+    from statequant_amd.csrc import build
+    if not shutil.which('g++'):
+        pytest.skip('no host compiler')
+    rocm = os.environ.get('ROCM_PATH', '/opt/rocm')
+    src = tmp_path / 'ok.cpp'
+    src.write_text('#include "sq_params.h"\n#include <stdio.h>\nnamespace sq {\n' + '\n'.join(build.QUAD_OK) + r"""
+template <class P, class F> void forms(const char* name, P p, F&& ok) {
+    auto at = [](uintptr_t a) { return reinterpret_cast<uint8_t*>(a); };
+    for (int stride : {4096, 4104}) for (int base : {0, 8}) {
+        p.st.S = at(4096 + base); p.st.sS = stride;
+        printf("%s %d %d %d\n", name, stride % 16, base, int(ok(p)));
+    }
+}
+}
+int main() {
+    using namespace sq;
+    const void* x = reinterpret_cast<const void*>(uintptr_t(1 << 20));
+    GdnParams g{}; g.qk_per_key_head = 1; g.gqa = 2; g.q = g.k = x; g.s_q = g.s_k = 128; g.q_dt = g.k_dt = 1;
+    forms("gdn", g, gdn_quad_ok);
+    KdaParams k{}; k.q = k.k = k.g = x; k.s_q = k.s_k = k.s_g = 128; k.q_dt = k.k_dt = 1; k.g_dt = 0;
+    forms("kda", k, kda_quad_ok);
+    Mamba2Params m{}; m.B = m.C = x; m.s_B = m.s_C = 128; m.B_dt = m.C_dt = 1;
+    forms("mamba2", m, mamba2_quad_ok);
+    k.st.S = reinterpret_cast<uint8_t*>(uintptr_t(4096)); k.st.sS = 4096; k.s_g = 3;
+    printf("operand 0 0 %d\n", int(kda_quad_ok(k)));
+}
+""")
+    exe = str(tmp_path / 'ok')
+    r = subprocess.run(['g++', '-std=c++17', '-D__HIP_PLATFORM_AMD__=1', '-I' + build.HERE, '-I' + os.path.join(rocm, 'include'),
+                        str(src), '-o', exe], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    got = subprocess.run([exe], capture_output=True, text=True, check=True).stdout.split('\n')[:-1]
+    want = [f'{fam} {stride} {base} {int(stride == 0 and base == 0)}'
+            for fam in ('gdn', 'kda', 'mamba2') for stride in (0, 8) for base in (0, 8)] + ['operand 0 0 0']
+    assert got == want, got
