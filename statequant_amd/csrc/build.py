@@ -85,8 +85,8 @@ def specs_of(fam, c, quad):
     """SPEC values an instance is built for: the workgroup-per-key-head kernels for every case they serve, the
     one-wavefront kernels for the cases that have no such kernel."""
     bits, dk, dv, group, qbuf, mmax, axv = c
-    if not (qbuf and mmax == 8) or (not quad and quad_variants(fam, c)):
-        return (0,)
+    if not (qbuf and mmax == 8) or (not quad and quad_variants(fam, c) and not (fam == 'kda' and dk == 64)):
+        return (0,)                                          # (KDA, d_k 64: the one-wavefront kernel serves launches of many heads)
     if not quad and fam != 'kda':
         # measured on the one-wavefront kernels: KDA int4 g32 40.0 -> 38.9 us, GDN value-axis int4 36.3 -> 35.1, but
         # value-axis int8 45.2 -> 48.4 and Mamba2 d_state 256 41.9 -> 48.1 (their register allocation tips over)
@@ -124,8 +124,9 @@ QUAD_OK = [
 def quad_variants(fam, c):
     """[(row blocks per wavefront, value heads per workgroup, wavefronts per SIMD the register allocation aims for,
     serving case, heads per launch it is for -- 0: any)], small launches' first, then widest head group first, of the
-    workgroup kernels (sq_quad.cuh) for a case; empty where only the one-wavefront kernels (sq_tile.cuh) serve it: value-axis groups other than 32 rows, the fp32 state, d_v that is no
-    multiple of 32 (Mamba2: 16), d_k above 128, more than four scale groups per row, states beyond 64 KB."""
+    workgroup kernels (sq_quad.cuh) for a case; empty where only the one-wavefront kernels (sq_tile.cuh) serve it:
+    value-axis groups other than 32 rows, the fp32 state, d_v that is no multiple of 32 (Mamba2: 16), d_k above 128, more
+    than four scale groups per row, states beyond 64 KB."""
     bits, dk, dv, group, qbuf, mmax, axv = c
     if fam not in QUAD_FAMILIES or bits not in (4, 8, 16) or (axv and group != 32):
         return []
@@ -136,6 +137,8 @@ def quad_variants(fam, c):
         return []
     if not axv and not flt and -(-dk // group) > 4:
         return []
+    if fam == 'gdn' and (dk, dv, bits, axv) == (64, 64, 8, 1) and mmax > 8:      # (32 heads, workgroup / one wavefront) 16
+        return []                                        # sequences 9.7 / 8.8 us per launch, 100: 15.2 / 14.6, 250: 23.7 / 23.4
     nrb = -(-dv // 32)                                       # the last one may be half empty (Mamba2)
     # row blocks per wavefront: one for the bf16 state, whose blocks are 8 KB each (a head of 128 x 128 on two wavefronts
     # leaves eight per compute unit)
@@ -193,14 +196,53 @@ SMALL_LAUNCH = {('gdn', 128, 128, 0): 2048, ('gdn', 128, 128, 1): 3072, ('gdn', 
 GROUP_HEADS = 5120
 
 
-def group_limit(fam, c):
-    """Whether a case's workgroup kernels serve launches below GROUP_HEADS heads only."""
+def group_when(fam, c):
+    """The condition (C++, on `heads` of the launch and whether it has a dispatch order) under which a case's workgroup
+    kernels serve; '' always.  What ends their lead is a launch with enough heads to fill the chip several times over:
+    then a head costs its instructions and its LDS, not its length.  A dispatch order ends it earlier: the one-wavefront
+    kernel's folding heads live three times as long as the others, and placed well they no longer decide when the launch
+    ends.  Figures: us per launch, workgroup / one wavefront, sequences out of step."""
     bits, dk, dv, group, qbuf, mmax, axv = c
-    if bits == 16 or (bits == 4 and axv):
-        return False
+    flt, usual = bits == 16, qbuf and mmax == 8
+    when = []
     if fam == 'mamba2':
-        return dv % 32 != 0
-    return dk == 96 and (fam == 'gdn' or (bits == 4 and not axv))
+        if dv % 32 and not flt:
+            # d_state 96, int4 (96 heads): 32 sequences 15.6 / 15.9, 40: 20.2 / 19.0
+            when.append(f'heads < {3328 if (bits, dk, mmax) == (4, 96, 8) else GROUP_HEADS}')
+        if flt and (dk, mmax) == (96, 8):                    # 64 sequences 33.7 / 34.3, 96 in order 47.3 / 43.1
+            when.append('(!p.order || heads < 8192)')
+    elif dk == 96 and not flt and (bits == 8 or not axv) and (fam == 'gdn' or (bits == 4 and not axv)):
+        when.append(f'heads < {GROUP_HEADS}')
+        if fam == 'gdn' and dv == 96 and not axv and mmax == 8:
+            # three wavefronts a head (20 heads, int4 g64): 160 sequences in order 16.2 / 16.9, 192: 18.5 / 17.4, bf16
+            # buffer 128: 14.7 / 15.2, 160: 17.0 / 16.0; 190, not in order, 20.6 / 21.6
+            when.append(f'(!p.order || heads < {3520 if qbuf else 2880})')
+    elif fam == 'gdn' and flt and (dk, dv) == (96, 192) and not usual:
+        # two workgroups per compute unit (30 heads, 16-token buffer): 64 sequences in order 45.9 / 58.2, 96: 64.4 / 61.3,
+        # 128: 80.6 / 64.8; 130, not in order, 81.3 / 87.5
+        when.append('(!p.order || heads < 2560)')
+    elif fam == 'kda' and dk == 64:
+        # one or two wavefronts a head: little to deal out.  64 x 64 (32 heads) int4 g64 128 sequences in order 11.3 / 11.8,
+        # 160: 13.5 / 12.7, 16-token buffer 96: 11.6 / 12.2, 128: 13.5 / 12.8, int8 15.0 / 13.7.  64 x 32 int4 g64 1
+        # sequence 4.9 / 4.6, 8: 5.4 / 5.4, 16-token buffer 8: 6.2 / 6.2, 16: 6.9 / 7.1; bf16 state 100, not in order, 11.1 /
+        # 11.7, 128 in order 11.7 / 11.1; 16-token bf16 buffer 64: 8.5 / 9.7, 130, not in order, int8 13.2 / 13.1, value-axis
+        # 14.4 / 13.1
+        if dv == 32 and not (flt and mmax > 8):
+            when.append(f'heads >= {256 if mmax <= 8 else 384}')
+        if not flt and mmax > 8:
+            when.append('heads < 4096' if dv == 32 and not qbuf else '(!p.order || heads < 4096)')
+        elif dv == 32 and mmax <= 8 and (flt or (bits == 8 and axv)):
+            when.append('(!p.order || heads < 4096)')
+        elif not flt and dv == 64:
+            when.append('(!p.order || heads < 5120)')
+    elif fam == 'kda' and (dk, dv, bits, group, axv) == (128, 128, 8, 32, 0) and qbuf and mmax > 8:
+        # 132 registers (32 heads): 96 sequences in order 27.4 / 29.4, 128: 34.5 / 32.7; 130, not in order, 37.7 / 44.8
+        when.append('(!p.order || heads < 4096)')
+    if axv and (dk, dv) == (64, 64) and fam != 'kda' and not usual:
+        # one wavefront a head in both, and here the front end's barriers are what is left: GDN int8, bf16 buffer, 16
+        # sequences 8.7 / 8.1, 64: 10.7 / 11.2; Mamba2 (64 heads) 8: 7.3 / 6.8, 16: 8.3 / 8.6
+        when.append('heads >= 1024')
+    return ' && '.join(when)
 
 
 def _quad_name(fam, c, v):
@@ -277,6 +319,7 @@ def generate():
         if fam in QUAD_FAMILIES:
             d.append(f'    const bool quad = !g_no_quad.load(std::memory_order_relaxed) && (!run || {fam}_quad_ok(p));')
             d.append('    const int ghmax = g_ghmax.load(std::memory_order_relaxed);')
+            d.append('    const int64_t heads = int64_t(p.rows) * p.hv;')
         # smallest sufficient buffer bound first
         for c in sorted(rows, key=lambda c: c[5]):
             bits, dk, dv, group, qbuf, mmax, axv = c
@@ -284,9 +327,8 @@ def generate():
                     f'&& p.qbuf == {qbuf} && p.m <= {mmax}')
             for v in quad_variants(fam, c):
                 want = f'spec == {v[3]} && ' if v[3] else ''             # the general instance takes whatever is left
-                limit = v[4] or (GROUP_HEADS if group_limit(fam, c) else 0)
-                few = f'(!run || int64_t(p.rows) * p.hv < {limit}) && ' if limit else ''
-                d.append(f'    if (quad && {want}{few}p.gqa % {v[1]} == 0 && {v[1]} <= ghmax && {cond}) return run ? {_quad_name(fam, c, v)}(p, stream) : 0;')
+                size = f'heads < {v[4]} && ' if v[4] else f'{group_when(fam, c)} && ' if group_when(fam, c) else ''
+                d.append(f'    if (quad && {want}{size}p.gqa % {v[1]} == 0 && {v[1]} <= ghmax && {cond}) return run ? {_quad_name(fam, c, v)}(p, stream) : 0;')
             for sp in specs_of(fam, c, False):
                 want = f'spec == {sp} && ' if sp else ''
                 d.append(f'    if ({want}{cond}) return run ? launch_{fam}<{_tile(c)}, {sp}>(p, stream) : 0;')

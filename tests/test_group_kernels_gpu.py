@@ -65,24 +65,22 @@ def _token(family, gen, rows, shape):
                 beta=torch.sigmoid(r(rows, hv)))
 
 
-def _step(family, lay, V, idx, t, out, model):
+def _step(family, lay, V, idx, t, out, model, order=None):
     if family == 'mamba2':
-        lay.step(V, idx, t['x'], t['dt'], t['B'], t['C'], out, *model)
+        lay.step(V, idx, t['x'], t['dt'], t['B'], t['C'], out, *model, order=order)
     elif family == 'kda':
-        lay.step(V, idx, t['q'], t['k'], t['v'], t['g'], t['beta'], out)
+        lay.step(V, idx, t['q'], t['k'], t['v'], t['g'], t['beta'], out, order=order)
     else:
-        lay.step(V, idx, t['q'], t['k'], t['v'], out, lay.DK ** -0.5, g=t['g'], beta=t['beta'])
+        lay.step(V, idx, t['q'], t['k'], t['v'], out, lay.DK ** -0.5, g=t['g'], beta=t['beta'], order=order)
 
 
-@pytest.mark.parametrize('family,fmt,shape,m,bb', CASES)
-def test_group_kernel_matches_the_one_wavefront_kernel(family, fmt, shape, m, bb):
+def _compare(family, fmt, shape, m, bb, idx):
     hv, hk, dk, dv = shape
     lay = _layout(family, fmt, shape, m, bb)
     gen = torch.Generator().manual_seed(5)
-    rows = 7
-    idx = torch.tensor([3, 1, 0, 9, 4, -1, 6], dtype=torch.int32, device=DEV)
+    rows = idx.shape[0]
     live = idx > 0
-    blob = lay.alloc(10, DEV)
+    blob = lay.alloc(int(idx.max()) + 1, DEV)
     V = lay.views(blob)
     S0 = torch.randn(rows, hv, dv, dk, generator=gen).to(DEV) * 0.4
     S0[0] = 0.0                                                     # a fresh sequence: its first fold is the exact one
@@ -129,6 +127,61 @@ def test_group_kernel_matches_the_one_wavefront_kernel(family, fmt, shape, m, bb
     # bf16 steps are 2^-8 of a value; the two sums of up to 17 terms differ by some 2^-23 of it, and by more where they cancel
     assert off <= (2e-3 if lay.bits == 16 else 1e-4) * codes and scales_off <= 1e-4 * scales + 2, (off, codes, scales_off, scales)
     assert flips <= 1e-4 * entries + 2 * max(dk, dv), (flips, entries)
+
+
+@pytest.mark.parametrize('family,fmt,shape,m,bb', CASES)
+def test_group_kernel_matches_the_one_wavefront_kernel(family, fmt, shape, m, bb):
+    _compare(family, fmt, shape, m, bb, torch.tensor([3, 1, 0, 9, 4, -1, 6], dtype=torch.int32, device=DEV))
+
+
+@pytest.mark.parametrize('family,fmt,shape,m,bb,rows', [
+    ('gdn', (8, 'v', 32), (32, 16, 64, 64), 8, 16, 34), ('gdn', (4, 'v', 32), (32, 16, 64, 64), 16, 8, 34),
+    ('mamba2', (8, 'v', 32), (64, 8, 64, 64), 16, 16, 18), ('mamba2', (4, 'v', 32), (64, 8, 64, 64), 4, 16, 18),
+    ('kda', (8, 'k', 32), (32, 32, 64, 32), 4, 8, 10), ('kda', (8, 'v', 32), (32, 32, 64, 32), 2, 16, 10),
+    ('kda', (4, 'k', 64), (32, 32, 64, 32), 16, 8, 14), ('kda', 'bf16', (32, 32, 64, 32), 8, 8, 10)])
+def test_group_kernels_that_serve_larger_launches_only(family, fmt, shape, m, bb, rows):
+    idx = torch.randperm(rows, generator=torch.Generator().manual_seed(1)).to(torch.int32).to(DEV)      # one padding row
+    _compare(family, fmt, shape, m, bb, idx)
+
+
+@pytest.mark.parametrize('family,fmt,shape,m,bb,rows', [
+    ('kda', (4, 'k', 64), (32, 32, 64, 64), 2, 8, 160), ('kda', (8, 'v', 32), (32, 32, 64, 64), 16, 16, 128),
+    ('kda', (8, 'k', 32), (32, 32, 64, 32), 16, 8, 128), ('kda', (8, 'k', 32), (32, 32, 128, 128), 16, 8, 128),
+    ('kda', 'bf16', (32, 32, 64, 32), 2, 8, 128),
+    ('gdn', (4, 'k', 64), (20, 20, 96, 96), 4, 8, 176), ('gdn', 'bf16', (30, 30, 96, 192), 2, 16, 88),
+    ('mamba2', 'bf16', (96, 8, 96, 80), 2, 8, 88)])
+def test_a_dispatch_order_that_changes_the_kernel(family, fmt, shape, m, bb, rows):
+    """Launches of so many heads that a dispatch order moves them to the one-wavefront kernel (bounds as above)."""
+    hv, hk, dk, dv = shape
+    lay = _layout(family, fmt, shape, m, bb)
+    gen = torch.Generator().manual_seed(8)
+    blobs = [lay.alloc(rows + 1, DEV) for _ in range(2)]
+    V = [lay.views(b) for b in blobs]
+    idx = torch.arange(1, rows + 1, dtype=torch.int32, device=DEV)
+    order = torch.randperm(rows, generator=gen).to(torch.int32).to(DEV)
+    S0 = torch.randn(8, hv, dv, dk, generator=gen).to(DEV) * 0.4
+    lay.write(V[0], idx, S0.repeat(rows // 8, 1, 1, 1))
+    r = lambda *s: torch.randn(*s, generator=gen).to(DEV)          # noqa: E731
+    model = (-torch.exp(r(hv)), r(hv), r(hv)) if family == 'mamba2' else None
+    for step in range(m + 1):
+        blobs[1].copy_(blobs[0])
+        t = _token(family, gen, rows, shape)
+        outs = [torch.zeros(rows, hv, dv, device=DEV) for _ in range(2)]
+        for W, o, ordered in zip(V, outs, (None, order)):
+            _step(family, lay, W, idx, t, o, model, order=ordered)
+        assert ((outs[0] - outs[1]).abs().max() / outs[0].abs().max()).item() <= 1e-5, step
+        assert torch.equal(V[0]['NPTR'], V[1]['NPTR'])
+        # this token's entry of the buffer: a value one step off moves its whole row of the state by that step times the
+        # key -- more than a code step where the row's value was near zero -- and a key or a scale that differs, the head
+        off = lambda name: (V[0][name] != V[1][name])[1:].flatten(2).any(2)        # noqa: E731
+        heads = off('KB').repeat_interleave(hv // hk, 1)
+        if 'UBS' in V[0]:
+            heads |= off('UBS') | off('KBS').repeat_interleave(hv // hk, 1)
+        rows_off = (V[0]['UB'] != V[1]['UB'])[1:].any(2) | heads[..., None]
+        assert rows_off.float().mean().item() <= 1e-3
+        A, B = (W['S'][1:][~rows_off].cpu() for W in V)
+        mism, far, n = code_diff(A, B, lay.bits)
+        assert far == 0 and mism <= (2e-3 if lay.bits == 16 else 1e-4) * n
 
 
 @pytest.mark.parametrize('family,fmt,shape,rows', [
