@@ -123,7 +123,7 @@ QUAD_OK = [
 
 def quad_variants(fam, c):
     """[(row blocks per wavefront, value heads per workgroup, wavefronts per SIMD the register allocation aims for,
-    serving case, heads per launch it is for -- 0: any)], small launches' first, then widest head group first, of the
+    serving case, condition on the launch -- '': any)], small launches' first, then widest head group first, of the
     workgroup kernels (sq_quad.cuh) for a case; empty where only the one-wavefront kernels (sq_tile.cuh) serve it:
     value-axis groups other than 32 rows, the fp32 state, d_v that is no multiple of 32 (Mamba2: 16), d_k above 128, more
     than four scale groups per row, states beyond 64 KB."""
@@ -167,22 +167,31 @@ def quad_variants(fam, c):
         wpe = max(1, min(6 if mmax <= 8 and not axv else 5, -(-wgs * nw // 4)))
         # the serving cases compiled in (SPEC of the kernels) for the default buffer: int8, 8 tokens
         for spec in SPECS[fam] if (qbuf and mmax == 8) else (0,):
-            out.append((nb, gh, wpe, spec, 0))
-    small = SMALL_LAUNCH.get((fam, dk, dv, axv)) if not flt and qbuf and mmax == 8 else None
-    if small:                                            # the one-head entries again, a row block per wavefront
-        out = [(1, 1, 6 if not axv else 5, spec, small) for spec in SPECS[fam]] + out
+            out.append((nb, gh, wpe, spec, ''))
+    if small_when(fam, c):                               # the one-head entries again, a row block per wavefront
+        out = [(1, 1, 6 if not axv else 5, spec, small_when(fam, c)) for spec in SPECS[fam]] + out
     return out
 
 
-# Launches below so many heads take one row block per wavefront and one head per workgroup: twice the wavefronts on up to
+# Launches that satisfy this take one row block per wavefront and one head per workgroup: twice the wavefronts on up to
 # four times the compute units, so that a head's life -- which is all such a launch consists of, the fold's four half
 # blocks in sequence above all -- gets shorter.  (One block per wavefront with two heads per workgroup gains nothing:
-# the wavefronts then share the SIMDs they had.)  us per launch, two blocks and two heads / this, sequences out of step:
-# GDN 128 x 128 (32 heads) int8 g32 1 sequence 5.22 / 4.77, 16: 9.8 / 8.0, 56: 15.4 / 14.8, 64: 14.3 / 14.7; int4 g64 16:
-# 9.4 / 7.7, 56: 13.7 / 13.4, 64: 12.2 / 13.3; value-axis int4 1: 6.2 / 5.3, 16: 12.4 / 9.1, 64: 15.0 / 14.0, 100: 24.0 /
-# 23.3; 96 x 192 int4 g64 (30 heads) 8: 7.8 / 6.9, 24: 12.3 / 11.8, 28: 12.6 / 13.9; Mamba2 128 x 64 (128 heads) int8 g128
-# 1: 5.07 / 4.54, 6: 7.16 / 7.09, 8: 7.89 / 8.01.
-SMALL_LAUNCH = {('gdn', 128, 128, 0): 2048, ('gdn', 128, 128, 1): 3072, ('gdn', 96, 192, 0): 768, ('mamba2', 128, 64, 0): 768}
+# the wavefronts then share the SIMDs they had.)  The dispatch order moves the line where a head's fold is the longest, on
+# value-axis states: in order the folding heads no longer end the launch, and the shorter fold is worth less.  us per
+# launch, two blocks and two heads / this, sequences out of step, 16 layers captured:
+# GDN 128 x 128 (32 heads) int8 g32 1 sequence 5.26 / 4.79, 16: 9.9 / 8.1, 56: 15.4 / 14.6, 64: 16.1 / 16.4, in order 14.4 /
+# 15.0; int4 g64 16: 9.5 / 7.8, 56: 13.7 / 13.3, 64: 14.4 / 15.1, in order 12.5 / 13.4.  Value-axis int4 16: 12.4 / 9.2, 96:
+# 23.3 / 22.2, 104: 22.4 / 22.6, in order 80: 17.2 / 16.8, 96: 18.6 / 19.0; int8 16: 12.7 / 9.3, 128: 29.7 / 28.5, 192: 36.9 /
+# 36.5, 256: 45.8 / 46.0, in order 80: 18.7 / 17.6, 96: 19.9 / 19.9, 104: 20.7 / 20.8.  96 x 192 int4 g64 (30 heads) 8: 7.9 /
+# 7.0, 24: 12.3 / 12.0, 26: 12.9 / 12.9, 28: 12.6 / 13.6.  Mamba2 128 x 64 (128 heads) int8 g128 1: 5.04 / 4.65, 5: 6.67 / 6.57, 8:
+# 8.00 / 7.91, 12: 10.0 / 10.2.  The other shapes and buffers that have two blocks or several heads in a workgroup were not
+# built this way: nothing is known about them.
+def small_when(fam, c):
+    bits, dk, dv, group, qbuf, mmax, axv = c
+    if bits == 16 or not qbuf or mmax > 8:
+        return ''
+    return {('gdn', 128, 128, 0): 'heads < 2048', ('gdn', 128, 128, 1): f'heads < (p.order ? 3072 : {3328 if bits == 4 else 6144})',
+            ('gdn', 96, 192, 0): 'heads < 768', ('mamba2', 128, 64, 0): 'heads < 768'}.get((fam, dk, dv, axv), '')
 
 
 # Heads per launch from which the one-wavefront kernel serves these cases again.  Their workgroups waste something -- lanes
@@ -327,7 +336,8 @@ def generate():
                     f'&& p.qbuf == {qbuf} && p.m <= {mmax}')
             for v in quad_variants(fam, c):
                 want = f'spec == {v[3]} && ' if v[3] else ''             # the general instance takes whatever is left
-                size = f'heads < {v[4]} && ' if v[4] else f'{group_when(fam, c)} && ' if group_when(fam, c) else ''
+                size = v[4] or group_when(fam, c)
+                size = f'{size} && ' if size else ''
                 d.append(f'    if (quad && {want}{size}p.gqa % {v[1]} == 0 && {v[1]} <= ghmax && {cond}) return run ? {_quad_name(fam, c, v)}(p, stream) : 0;')
             for sp in specs_of(fam, c, False):
                 want = f'spec == {sp} && ' if sp else ''

@@ -149,7 +149,9 @@ def test_group_kernels_that_serve_larger_launches_only(family, fmt, shape, m, bb
     ('kda', (8, 'k', 32), (32, 32, 64, 32), 16, 8, 128), ('kda', (8, 'k', 32), (32, 32, 128, 128), 16, 8, 128),
     ('kda', 'bf16', (32, 32, 64, 32), 2, 8, 128),
     ('gdn', (4, 'k', 64), (20, 20, 96, 96), 4, 8, 176), ('gdn', 'bf16', (30, 30, 96, 192), 2, 16, 88),
-    ('mamba2', 'bf16', (96, 8, 96, 80), 2, 8, 88)])
+    ('mamba2', 'bf16', (96, 8, 96, 80), 2, 8, 88),
+    # ... or from one row block per wavefront to two
+    ('gdn', (4, 'v', 32), (32, 16, 128, 128), 4, 8, 96), ('gdn', (8, 'v', 32), (32, 16, 128, 128), 8, 8, 104)])
 def test_a_dispatch_order_that_changes_the_kernel(family, fmt, shape, m, bb, rows):
     """Launches of so many heads that a dispatch order moves them to the one-wavefront kernel (bounds as above)."""
     hv, hk, dk, dv = shape
@@ -191,7 +193,8 @@ def test_a_dispatch_order_that_changes_the_kernel(family, fmt, shape, m, bb, row
     # one / two row blocks per wavefront
     ('gdn', (8, 'k', 32), (32, 16, 128, 128), 64), ('gdn', (4, 'k', 64), (32, 16, 128, 128), 64),
     ('gdn', (8, 'k', 128), (32, 8, 128, 128), 64), ('gdn', (4, 'v', 32), (32, 16, 128, 128), 96),
-    ('gdn', (8, 'v', 32), (24, 24, 128, 128), 128), ('gdn', (8, 'k', 64), (30, 30, 96, 192), 26),
+    ('gdn', (8, 'v', 32), (24, 24, 128, 128), 128), ('gdn', (4, 'v', 32), (32, 16, 128, 128), 104),
+    ('gdn', (8, 'v', 32), (32, 16, 128, 128), 192), ('gdn', (8, 'k', 64), (30, 30, 96, 192), 26),
     ('mamba2', (8, 'k', 128), (128, 8, 128, 64), 6), ('mamba2', (4, 'k', 32), (96, 8, 128, 64), 8)])
 def test_launches_either_side_of_a_head_count_agree(family, fmt, shape, rows):
     """A launch at the number of heads where another kernel takes over, and the same launch one sequence shorter (bounds
