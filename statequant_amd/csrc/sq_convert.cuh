@@ -180,7 +180,11 @@ int launch_pack(const PackParams& p, hipStream_t stream) {
 // Column split of the output pass: a lane takes NCH chunks of 4 columns, chunk t = columns 4 LPR t + 4 cg .. + 3, so
 // that the LPR lanes of a row write 16 LPR consecutive bytes with every store instruction (whole 128-byte lines for
 // d_k = 128) -- with 16 consecutive columns per lane each store would scatter 16-byte pieces 64 bytes apart.
-template <int BITS, int DK, int GROUP, bool QBUF, bool KDA, bool AXV>
+// AHEAD: the first pass's stored rows are requested before anything that waits for the fill counter -- for launches of few
+// wavefronts, which a memory round trip less shortens (6 sequences as above: 7.0 -> 6.2 us per launch).  Full launches hide
+// that round trip behind each other and do better with the 10 to 40 registers the early rows take (one wavefront per SIMD
+// more; 256 sequences of GDN 128 x 128 int4 with 16 tokens: 212 us ahead, 194 not).
+template <int BITS, int DK, int GROUP, bool QBUF, bool KDA, bool AXV, bool AHEAD>
 __global__ __launch_bounds__(WAVE) void read_kernel(const ReadParams p, uint32_t part_rows) {
     using T = RowTile<BITS, DK, GROUP, QBUF, AXV>;
     constexpr int NCH = CPL / 4;
@@ -215,9 +219,7 @@ __global__ __launch_bounds__(WAVE) void read_kernel(const ReadParams p, uint32_t
 
     constexpr int RR = 2;                                         // rows per pass over the buffered keys
     constexpr int CW = BITS == 32 ? 4 : BITS == 16 ? 2 : 1;       // words of a 4-column chunk
-    // a pass's stored rows and scales as loaded; the first pass's are requested before anything that waits for the fill
-    // counter (6 sequences as above: 7.0 -> 6.2 us per launch)
-    uint32_t cw[RR][NCH][CW];
+    uint32_t cw[RR][NCH][CW];                                     // a pass's stored rows and scales as loaded
     uint2 sw[RR][NCH];
     auto request = [&](uint32_t r0) {
 #pragma unroll
@@ -247,8 +249,10 @@ __global__ __launch_bounds__(WAVE) void read_kernel(const ReadParams p, uint32_t
             }
         }
     };
-    request(r_begin);
-    asm volatile("" ::: "memory");
+    if constexpr (AHEAD) {
+        request(r_begin);
+        asm volatile("" ::: "memory");
+    }
 
     const int n = *field(p.st.NPTR, seq, p.st.sN, 0u) & (m - 1);     // the first head's copy, as the reference reads it
     // keys of the live slots, times their decay ratio (slot = row group + RG x pass, 16 consecutive columns per lane)
@@ -288,7 +292,7 @@ __global__ __launch_bounds__(WAVE) void read_kernel(const ReadParams p, uint32_t
     for (uint32_t r0 = r_begin; r0 < r_end; r0 += RR * T::RG) {
         uint32_t row[RR], rc[RR];
         float acc[RR][NCH][4];
-        if (r0 != r_begin) request(r0);
+        if (!AHEAD || r0 != r_begin) request(r0);
 #pragma unroll
         for (int k = 0; k < RR; ++k) {
             row[k] = r0 + k * T::RG + l.rg;
@@ -357,8 +361,11 @@ int launch_read(const ReadParams& p, hipStream_t stream) {
     const uint32_t heads = uint32_t(p.rows) * uint32_t(p.hv);
     const RowSplit sp = split_rows(heads, p.dv, 2 * RowTile<BITS, DK, GROUP, QBUF, AXV>::RG);
     const size_t lds = size_t(p.m) * (DK + sp.rows) * sizeof(float);
-    hipLaunchKernelGGL((read_kernel<BITS, DK, GROUP, QBUF, KDA, AXV>), dim3(heads, sp.parts), dim3(WAVE), lds, stream, p,
-                       sp.rows);
+    const dim3 grid(heads, sp.parts);
+    if (sp.parts > 1)
+        hipLaunchKernelGGL((read_kernel<BITS, DK, GROUP, QBUF, KDA, AXV, true>), grid, dim3(WAVE), lds, stream, p, sp.rows);
+    else
+        hipLaunchKernelGGL((read_kernel<BITS, DK, GROUP, QBUF, KDA, AXV, false>), grid, dim3(WAVE), lds, stream, p, sp.rows);
     return int(hipGetLastError());
 }
 
