@@ -31,7 +31,7 @@ from statequant_amd.kernels import _hip  # noqa: E402
 
 MARKS_KDA = ['entry', 'slot known, token loads issued', 'fill count here, every load issued',
              'vectors, scales, buffered values staged', 'keys and decays here, coefficients done', 'state pass done',
-             'outputs stored', 'appended', 'folded (full buffer), counters advanced']
+             'outputs stored', 'appended, counter advanced', 'folded (a full buffer)']
 MARKS = ['entry', 'item known (leading arguments here)', 'slot known, token loads issued', 'row blocks issued',
          'fill counter issued', 'fill count here, buffer loads issued', 'roles done, all loads landed in LDS',
          'first barrier passed', 'state pass done', 'buffer dot products done', 'second barrier passed',
@@ -44,8 +44,9 @@ def timeline(workload, step, dev, m=8):
     fam, lay, views, idx = bench.build(workload, m, dev)
     inputs, extra = bench.make_inputs(fam, lay, slots, layers, m, dev)
     out = torch.zeros(slots, hv, dv, device=dev, dtype=torch.bfloat16)
-    waves = 4                                                # GDN: two value heads x two wavefronts; KDA: four per head
-    nwg = slots * hv // 2 if fam == 'gdn' else slots * hv
+    # four wavefronts a workgroup: GDN codes two value heads of two, the bf16 state and KDA one head of four
+    waves = 4
+    nwg = slots * hv // 2 if fam == 'gdn' and bits < 16 else slots * hv
     buf = torch.zeros(nwg * waves * 16, dtype=torch.int64, device=dev)
 
     def run(s, upto):
@@ -66,9 +67,8 @@ def timeline(workload, step, dev, m=8):
     torch.cuda.synchronize()
     t = buf.cpu().numpy().reshape(nwg, waves, 16)[:, :, :15].astype(np.float64)
     if not (t[:, :, 0] > 0).all():
-        sys.exit(f'profile_timeline.py: {workload} did not run on an instrumented kernel (gdn_quad_kernel serves '
-                 'Gated DeltaNet int4 / int8 states with key-axis groups, two value heads per key head; '
-                 'kda_quad_kernel int4 / int8 KDA states)')
+        sys.exit(f'profile_timeline.py: {workload} did not run on an instrumented kernel (gdn_quad_kernel and '
+                 'kda_quad_kernel at 128 x 128 with 256 slots)')
     return t, nwg, fam
 
 

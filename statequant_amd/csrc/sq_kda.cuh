@@ -11,7 +11,6 @@
 #pragma once
 #include "sq_tile.cuh"
 #include "sq_params.h"
-#include "sq_timeline.cuh"
 
 namespace sq {
 
@@ -23,8 +22,7 @@ __device__ __forceinline__ float kda_exp(float x) { return __builtin_amdgcn_exp2
 template <class T, int SPEC>
 __global__ __launch_bounds__(WAVE, 4)
 void kda_step_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict__ order, int per_xcd,
-                     int hv, int hv_shift, SQ_TL_PARAM const KdaParams args) {
-    SQ_MARK(0);                                                   // entry
+                     int hv, int hv_shift, const KdaParams args) {
     KdaParams p = args;
     assume_serving_case<SPEC>(p);                            // SPEC: see sq_params.h
     using L = LdsPlan<T, 3, 2>;                                   // q, k (normalised), G_n
@@ -78,7 +76,6 @@ void kda_step_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
         for (int r = l.lane; r < DV; r += WAVE) store_f(outp, p.out_dt, r, 0.0f);
         return;
     }
-    SQ_MARK(1);                                                   // slot known, the token's loads issued
     const uint32_t seq = slot;
 
     uint8_t* Sh = field(p.st.S, seq, p.st.sS, h * (DV * T::ROW_BYTES));
@@ -124,7 +121,6 @@ void kda_step_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
         for (int k = 0; k < CPL / 4; ++k) gbp[t][k] = g4[k];
     }
 
-    SQ_MARK(2);                                                   // fill count here, every load issued
 
     // ---- prep: q, k normalised, the running decay per channel ----
     const bool full = n == m - 1;
@@ -168,7 +164,6 @@ void kda_step_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
 #pragma unroll
     for (int i = 0; i < T::MMAX; ++i) ubs[i] = T::QBUF ? lane_bcast(f16_to_f32(ubs_raw), i) : 1.0f;
     wave_sync();
-    SQ_MARK(3);                                                   // vectors, scales, buffered values here and staged
 
     // ---- buffer coefficients with the per-channel decay ratio folded into the buffered key ----
     float cqk[2][T::MMAX];
@@ -211,12 +206,10 @@ void kda_step_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
         }
     }
 
-    SQ_MARK(4);                                                   // buffered keys and decays here, coefficients done
 
     // ---- state pass against A*q, A*k ----
     float own[2][T::NOWN];
     state_pass<T, 2>(lane_base, win, lds_b, lds_xs, lds_sc, lds_a, lds_own, l, xa, own);
-    SQ_MARK(5);                                                   // state pass done (all codes here)
 
     float u[T::NOWN], amax = 0.0f;
 #pragma unroll
@@ -235,7 +228,6 @@ void kda_step_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
         amax = fmaxf(amax, fabsf(u[t]));
     }
 
-    SQ_MARK(6);                                                   // outputs stored
     // ---- append: decay vector, delta value, key ----
     float us = 1.0f, ks = 1.0f;
     if constexpr (T::QBUF) {
@@ -254,7 +246,6 @@ void kda_step_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
         if (e < DK) GBh[n * DK + e] = gn[t];
     }
 
-    SQ_MARK(7);                                                   // appended
     // the running decay: stored here unless the buffer is full (then it restarts at zero, stored behind the fold), so
     // that it does not have to stay in registers across the fold
     if (!full) {
@@ -308,18 +299,12 @@ void kda_step_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
 
     // ---- advance (the running decay of a full buffer is stored at the end of the fold) ----
     if (l.lane == 0) *np = full ? 0 : n + 1;
-    SQ_MARK(8);                                                   // folded (a full buffer), counters advanced
 }
 
 template <class T, int SPEC>
 int launch_kda(const KdaParams& p, hipStream_t stream) {
-#ifdef SQ_TIMELINE
-    hipLaunchKernelGGL((kda_step_kernel<T, SPEC>), dim3(p.rows * p.hv), dim3(WAVE), 0, stream, p.idx, p.order, p.per_xcd,
-                       p.hv, p.hv_shift, sq_timeline_buffer().p, sq_timeline_buffer().cap, p);
-#else
     hipLaunchKernelGGL((kda_step_kernel<T, SPEC>), dim3(p.rows * p.hv), dim3(WAVE), 0, stream, p.idx, p.order, p.per_xcd,
                        p.hv, p.hv_shift, p);
-#endif
     return int(hipGetLastError());
 }
 

@@ -1,4 +1,4 @@
-// KDA packed decode step, one workgroup per (batch row, head): every wavefront owns NB 32-row blocks of the head's state
+// KDA packed decode step, one workgroup per (batch row, head): every wavefront owns one 32-row block of the head's state
 // (int4 / int8 codes, key-axis groups or value-axis groups of one row block, or bf16; geometry and building blocks in
 // sq_quad.cuh).
 //
@@ -7,13 +7,13 @@
 //   c_x[i] = sum_j k_i[j] exp(G_n[j] - G_i[j]) x[j];   u = beta (v - S0^T (A k) - sum_i c_k[i] u_i);
 //   o = S0^T (A q) + sum_i c_q[i] u_i + (k.q) u;   fold: S = S0 diag(A) + sum_i u_i (exp(G_n - G_i) k_i)^T
 // KDA has no grouped keys, so a head is a workgroup.  What its one-wavefront kernel does in sequence is dealt out:
-//   issue            every wavefront: its row blocks, scales, its rows of v and of the buffered values, its share of the
+//   issue            every wavefront: its row block, scales, its rows of v and of the buffered values, its share of the
 //                    buffered keys with their decays; one wavefront each q and k, both with g and the running decay
 //   roles            q / k normalised, A q / A k as digit planes; G_n and A for all                       [barrier]
-//   per wavefront    its row blocks' read-outs; c_q, c_k of its share of the slots                        [barrier]
+//   per wavefront    its row block's read-outs; c_q, c_k of its share of the slots                        [barrier]
 //                    buffer term, u, o of its rows; max |u|; one wavefront each: the key, the decays      [barrier]
-//                    append;  with a full buffer: fold of its row blocks out of LDS (one read of the codes)
-// One row block per wavefront (NB = 1, four wavefronts for d_v 128): two per wavefront measured the same at 128
+//                    append;  with a full buffer: fold of its row block out of LDS (one read of the codes)
+// One row block per wavefront (four wavefronts for d_v 128): two per wavefront measured the same at 128
 // sequences and 3 % faster at 256 (int4), but a third slower at 16 and slower everywhere on int8.
 // us per launch, one wavefront per head -> this (32 heads of 128 x 128, sequences out of step): int4 g32 1 sequence
 // 6.7 -> 4.5, 16: 16.7 -> 7.8, 128: 25.5 -> 20.6, 256: 36.6 -> 35.8; int8 g32 1: 7.8 -> 4.6, 256: 59.0 -> 43.4;
@@ -27,8 +27,8 @@ namespace sq {
 
 template <class T, class Q>
 struct KdaLoads {
-    uint16_t sc[Q::NB][T::NG];             // scales of rows (block bi, lane % 32)
-    uint32_t scv[Q::NB];                   // value-axis groups: the block's scales of columns NE lane ..
+    uint16_t sc[T::NG];                    // scales of row lane % 32 of the block
+    uint32_t scv;                          // value-axis groups: the block's scales of columns NE lane ..
     Raw4<T::QBUF> uraw[Q::UT], kraw[Q::KT];
     float4 gb[Q::KT];                      // cumulative decays beside kraw
     uint16_t kbs[Q::KT], ubs;
@@ -37,10 +37,10 @@ struct KdaLoads {
     float gc[Q::NE];
 };
 
-template <class T, int NB>
+template <class T>
 struct KdaLds {
-    using Q = Quad<T, NB, 1>;
-    using B = QuadLds<T, NB, 1, 2, 2>;                               // read-out vectors: q, k (normalised)
+    using Q = Quad<T, 1, 1>;
+    using B = QuadLds<T, 1, 1, 2, 2>;                                // read-out vectors: q, k (normalised)
     static constexpr int GN = B::BYTES;                              // [DKP] G_n
     static constexpr int CM = GN + Q::DKP * 4;                       // [DKP] A = exp(G_n)
     static constexpr int XA = CM + Q::DKP * 4;                       // [2][DKP] A q, A k (value-axis groups: planes per block)
@@ -50,18 +50,19 @@ struct KdaLds {
 
 // SPEC = 1: the serving case compiled in -- bf16 q / k / v / out, fp32 g and beta, a power-of-two
 // head count where d_k is one too.
-template <class T, int NB, int WPE, int SPEC>
-__global__ __launch_bounds__((Quad<T, NB, 1>::THREADS), WPE)
-void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict__ order, int per_xcd, int hv, int hv_shift,
-                     const uint8_t* codes, uint32_t codes_stride, const int32_t* counters, uint32_t counters_stride,
-                     uint32_t start_ramp, SQ_TL_PARAM const KdaParams p) {
+template <class T, int WPE, int SPEC>
+__global__ __launch_bounds__((Quad<T, 1, 1>::THREADS), WPE)
+void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict__ order, const uint8_t* codes,
+                     const int32_t* counters, int per_xcd, int hv, int hv_shift, uint32_t codes_stride,
+                     uint32_t counters_stride, SQ_TL_PARAM const KdaParams p) {
+    // (the leading arguments without gaps between them: 13 of the 14 words that are in registers when a wavefront starts)
     SQ_MARK(0);                                                   // entry
     constexpr bool FIX = SPEC > 0;
     const int q_dt = FIX ? int(BF16) : p.q_dt, k_dt = FIX ? int(BF16) : p.k_dt, v_dt = FIX ? int(BF16) : p.v_dt;
     const int out_dt = FIX ? int(BF16) : p.out_dt, g_dt = FIX ? int(F32) : p.g_dt, beta_dt = FIX ? int(F32) : p.beta_dt;
-    using Q = Quad<T, NB, 1>;
-    using L = QuadLds<T, NB, 1, 2, 2>;
-    using K = KdaLds<T, NB>;
+    using Q = Quad<T, 1, 1>;
+    using L = QuadLds<T, 1, 1, 2, 2>;
+    using K = KdaLds<T>;
     constexpr int DK = T::DK, DV = T::DV, NW = Q::NW, MM = T::MMAX, NE = Q::NE, NG = T::NG, DKP = Q::DKP;
     constexpr int RQ = 1 % NW, RK = 3 % NW, RX = 2 % NW, RG = 0;  // which wavefront plays which shared role
     __shared__ __attribute__((aligned(16))) uint8_t lds[K::BYTES];
@@ -83,14 +84,13 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
     const int m = p.m;
     const uint32_t um = m;
-    uint8_t* my_codes = lds + L::CODES + w * NB * Q::BLK;
+    uint8_t* blk = lds + L::CODES + w * Q::BLK;                   // this wavefront's row block
 
     const TileId tid = tile_id_lead<(FIX && heads_pow2(T::DK))>(order, per_xcd, hv, hv_shift);
     const uint32_t b = tid.b, h = tid.h;
     const int32_t slot = idx ? idx[b] : int32_t(b);
     const int n32 = lane & 31, kb = lane >> 5;
-    // the row of the head this lane finishes after the pass (NB = 2: the wavefront's halves take a block each)
-    const int row = (w * NB + (NB == 2 ? kb : 0)) * T::MR + n32;
+    const int row = w * T::MR + n32;                              // the row of the head this lane finishes after the pass
 
     KdaLoads<T, Q> F;
     const int vl = Q::vec_lane(lane);                             // whose elements of a d_k vector this lane loads
@@ -115,8 +115,7 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
         for (int t = 0; t < NE; ++t) F.gc[t] = gch[NE * vl + t];
     }
     // ... then the row blocks, straight into their LDS image, and the fill counter (a scalar load; sq_quad.cuh) ...
-    quad_start_wait<Q, WPE>(start_ramp);
-    quad_dma_blocks<Q, NB>(field(codes, seq, codes_stride, h * (DV * T::ROW_BYTES)) + w * NB * Q::GBLK, my_codes, lane);
+    quad_dma_blocks<Q, 1>(field(codes, seq, codes_stride, h * (DV * T::ROW_BYTES)) + w * Q::GBLK, blk, lane);
     F.np = quad_dma_counter(field(counters, seq, counters_stride, h));
     __builtin_amdgcn_sched_barrier(0);
     // ... and the rest of the slot: scales and -- once the fill counter is here -- the live part of the decode buffer
@@ -128,14 +127,11 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     buf.KBS = field(p.st.KBS, seq, p.st.sKBS, h * um);
     buf.UBS = field(p.st.UBS, seq, p.st.sUBS, h * um);
     float* const GBh = field(p.st.GB, seq, p.st.sGB, h * um * DK);
+    if constexpr (T::AXV) {
+        F.scv = quad_load_colscales<NE>(SCh + w * DK, vl);
+    } else if constexpr (!T::FLT) {
 #pragma unroll
-    for (int bi = 0; bi < NB; ++bi) {
-        if constexpr (T::AXV) {
-            F.scv[bi] = quad_load_colscales<NE>(SCh + (w * NB + bi) * DK, vl);
-        } else if constexpr (!T::FLT) {
-#pragma unroll
-            for (int g = 0; g < NG; ++g) F.sc[bi][g] = stream_load(SCh + uint32_t(((w * NB + bi) * T::MR + n32) * NG + g));
-        }
+        for (int g = 0; g < NG; ++g) F.sc[g] = stream_load(SCh + uint32_t(row * NG + g));
     }
     quad_dma_counter_wait(F.np);
     const uint32_t nfill = uint32_t(F.np & (m - 1));
@@ -190,15 +186,12 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     // ---- the loads land ----
     const int n = F.np & (m - 1);
     const bool full = n == m - 1;
-    uint16_t scw[NB][NG];
+    uint16_t scw[NG];
+    if constexpr (!T::AXV && !T::FLT) {
 #pragma unroll
-    for (int bi = 0; bi < NB; ++bi) {
-        if constexpr (!T::AXV && !T::FLT) {
-#pragma unroll
-            for (int g = 0; g < NG; ++g) {
-                scw[bi][g] = F.sc[bi][g];
-                if (kb == 0) lds_sc[((w * NB + bi) * T::MR + n32) * NG + g] = F.sc[bi][g];
-            }
+        for (int g = 0; g < NG; ++g) {
+            scw[g] = F.sc[g];
+            if (kb == 0) lds_sc[row * NG + g] = F.sc[g];
         }
     }
 #pragma unroll
@@ -261,38 +254,24 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     // ---- state pass against A q, A k ----
     float sq, sk;
     {
-        float own[NB];
+        float own;
         if constexpr (T::AXV) {
-#pragma unroll
-            for (int bi = 0; bi < NB; ++bi)
-                own[bi] = quad_block_pass_v<Q, T, 2>(my_codes + bi * Q::BLK, lds_xa, F.scv[bi], lds_pl + w * L::PL_BYTES,
-                                                     lds_xs + w * (L::XS_BYTES / 4), lane);
+            own = quad_block_pass_v<Q, T, 2>(blk, lds_xa, F.scv, lds_pl + w * L::PL_BYTES, lds_xs + w * (L::XS_BYTES / 4), lane);
         } else if constexpr (T::FLT) {
-#pragma unroll
-            for (int bi = 0; bi < NB; ++bi) own[bi] = quad_block_pass_f<Q, T, 2>(my_codes + bi * Q::BLK, lds_xa, lane);
+            own = quad_block_pass_f<Q, T, 2>(blk, lds_xa, lane);
         } else {
             v4i aop[Q::NKS];
             quad_fetch_planes<Q, T, 2>(lds_pl, lane, aop);
-            float xs[NG];
+            float xs[NG], sc[NG];
 #pragma unroll
             for (int g = 0; g < NG; ++g) xs[g] = lds_xs[kb * NG + g];
 #pragma unroll
-            for (int bi = 0; bi < NB; ++bi) {
-                float sc[NG];
-#pragma unroll
-                for (int g = 0; g < NG; ++g) sc[g] = f16_to_f32(scw[bi][g]);
-                own[bi] = quad_block_pass<Q, T>(my_codes + bi * Q::BLK, aop, xs, sc, lane);
-            }
+            for (int g = 0; g < NG; ++g) sc[g] = f16_to_f32(scw[g]);
+            own = quad_block_pass<Q, T>(blk, aop, xs, sc, lane);
         }
-        if constexpr (NB == 2) {                         // lane (n, kb) takes over row n of block kb: both sums
-            const auto r = __builtin_amdgcn_permlane32_swap(as_u32(own[0]), as_u32(own[1]), false, false);
-            sq = as_f32(r[0]);
-            sk = as_f32(r[1]);
-        } else {
-            const Pair qk = pair32(own[0]);
-            sq = qk.lo;
-            sk = qk.hi;
-        }
+        const Pair qk = pair32(own);
+        sq = qk.lo;
+        sk = qk.hi;
     }
     SQ_MARK(5);                                                   // state pass done
     lds_barrier();
@@ -361,7 +340,7 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     }
     const float u = beta * (raw_to_f(F.vr, v_dt) - acck);
     const float o = __builtin_fmaf(kq, u, accq);
-    if (NB == 2 || kb == 0) store_f(outp, out_dt, row, o);
+    if (kb == 0) store_f(outp, out_dt, row, o);
     SQ_MARK(6);                                                   // outputs stored
     float us = 1.0f;
     if constexpr (T::QBUF) {
@@ -375,7 +354,7 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
         us = fp16_scale(amax, 127.0f);
         if (w == RG && lane == 0) { buf.UBS[n] = f32_to_f16(us); lds_ubsf[n] = us; }
     }
-    if (NB == 2 || kb == 0) {
+    if (kb == 0) {
         if constexpr (T::QBUF) {
             const int8_t c = int8_t(int(round_buf(u, us)));
             reinterpret_cast<int8_t*>(buf.UB)[n * DV + row] = c;
@@ -401,25 +380,19 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
                 return sl < m ? kv : 0.0f;
             };
             auto cm = [&](int col) { return lds_cm[col]; };
+            uint16_t* old = reinterpret_cast<uint16_t*>(lds_pl + w * L::PL_BYTES);      // the planes are done with
+            quad_store_colscales<NE>(old, lf, F.scv);
+            wave_sync();
+            float dop[MT];
 #pragma unroll
-            for (int bi = 0; bi < NB; ++bi) {
-                uint8_t* blk = my_codes + bi * Q::BLK;
-                const int grp = w * NB + bi;
-                uint16_t* old = reinterpret_cast<uint16_t*>(lds_pl + w * L::PL_BYTES);      // the planes are done with
-                quad_store_colscales<NE>(old, lf, F.scv[bi]);
-                wave_sync();
-                float dop[MT];
-#pragma unroll
-                for (int t = 0; t < MT; ++t) {
-                    const int sl = 2 * t + fkb;
-                    const int sc_ = sl < m ? sl : 0;
-                    float uv_ = lds_raw<T::QBUF>(lds_ubr, sc_ * DV + grp * T::MR + fj);
-                    if constexpr (T::QBUF) uv_ = uv_ * lds_ubsf[sc_];
-                    dop[t] = sl < m ? uv_ : 0.0f;
-                }
-                quad_fold_block_v<Q, T>(blk, key, dop, cm, false, old, SCh + grp * DK, lf);
-                quad_store_block<Q>(Sh + grp * Q::GBLK, blk, lf);
+            for (int t = 0; t < MT; ++t) {
+                const int sl = 2 * t + fkb;
+                const int sc_ = sl < m ? sl : 0;
+                float uv_ = lds_raw<T::QBUF>(lds_ubr, sc_ * DV + w * T::MR + fj);
+                if constexpr (T::QBUF) uv_ = uv_ * lds_ubsf[sc_];
+                dop[t] = sl < m ? uv_ : 0.0f;
             }
+            quad_fold_block_v<Q, T>(blk, key, dop, cm, false, old, SCh + w * DK, lf);
         } else {
             constexpr int MT4 = (MM + 3) / 4, CL = DKP / 4;
             const int fn = lf & 15, fq = lf >> 4;
@@ -427,46 +400,42 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
             FoldKeys<T, true> kop;
             quad_fold_keys_f32<T>(lds_kd, m, lf, kop);
 #pragma unroll
-            for (int bi = 0; bi < NB; ++bi) {
-                uint8_t* blk = my_codes + bi * Q::BLK;
+            for (int hf = 0; hf < 2; ++hf) {
+                const int frow = w * T::MR + 16 * hf + fn;
+                float bop[MT4];
 #pragma unroll
-                for (int hf = 0; hf < 2; ++hf) {
-                    const int frow = (w * NB + bi) * T::MR + 16 * hf + fn;
-                    float bop[MT4];
-#pragma unroll
-                    for (int t = 0; t < MT4; ++t) {
-                        const int sl = 4 * t + fq;
-                        const int sc_ = sl < m ? sl : 0;
-                        float uv_ = lds_raw<T::QBUF>(lds_ubr, sc_ * DV + frow);
-                        if constexpr (T::QBUF) uv_ = uv_ * lds_ubsf[sc_];
-                        bop[t] = sl < m ? uv_ : 0.0f;
-                    }
-                    if constexpr (T::FLT)
-                        quad_fold_half_f<Q, T, true>(blk, hf, kop, bop, 1.0f, lf, lds_cm);
-                    else
-                        quad_fold_half<Q, T, true>(blk, hf, kop, bop, 1.0f, f16_to_f32(lds_sc[frow * NG + fg]),
-                                               SCh + frow * NG + fg, lf, lds_cm);
+                for (int t = 0; t < MT4; ++t) {
+                    const int sl = 4 * t + fq;
+                    const int sc_ = sl < m ? sl : 0;
+                    float uv_ = lds_raw<T::QBUF>(lds_ubr, sc_ * DV + frow);
+                    if constexpr (T::QBUF) uv_ = uv_ * lds_ubsf[sc_];
+                    bop[t] = sl < m ? uv_ : 0.0f;
                 }
-                wave_sync();
-                quad_store_block<Q>(Sh + (w * NB + bi) * Q::GBLK, blk, lf);
+                if constexpr (T::FLT)
+                    quad_fold_half_f<Q, T, true>(blk, hf, kop, bop, 1.0f, lf, lds_cm);
+                else
+                    quad_fold_half<Q, T, true>(blk, hf, kop, bop, 1.0f, f16_to_f32(lds_sc[frow * NG + fg]),
+                                               SCh + frow * NG + fg, lf, lds_cm);
             }
+            wave_sync();
         }
+        quad_store_block<Q>(Sh + w * Q::GBLK, blk, lf);
     }
     SQ_MARK(8);                                                   // folded (a full buffer)
 }
 
 template <class T, int NB, int GH, int WPE, int SPEC>
 int launch_kda_quad(const KdaParams& p, hipStream_t stream) {
-    static_assert(GH == 1, "no grouped keys");
+    static_assert(NB == 1 && GH == 1, "a row block per wavefront; no grouped keys");
     const uint32_t grid = uint32_t(p.rows) * uint32_t(p.hv);
-    using Q = Quad<T, NB, 1>;
+    using Q = Quad<T, 1, 1>;
 #ifdef SQ_TIMELINE
     const SqTimelineBuf tl = sq_timeline_buffer();
-    hipLaunchKernelGGL((kda_quad_kernel<T, NB, WPE, SPEC>), dim3(grid), dim3(Q::THREADS), quad_lds_pad(), stream, p.idx,
-                       p.order, p.per_xcd, p.hv, p.hv_shift, p.st.S, p.st.sS, p.st.NPTR, p.st.sN, 0u, tl.p, tl.cap, p);
+    hipLaunchKernelGGL((kda_quad_kernel<T, WPE, SPEC>), dim3(grid), dim3(Q::THREADS), quad_lds_pad(), stream, p.idx, p.order,
+                       p.st.S, p.st.NPTR, p.per_xcd, p.hv, p.hv_shift, p.st.sS, p.st.sN, tl.p, tl.cap, p);
 #else
-    hipLaunchKernelGGL((kda_quad_kernel<T, NB, WPE, SPEC>), dim3(grid), dim3(Q::THREADS), quad_lds_pad(), stream, p.idx,
-                       p.order, p.per_xcd, p.hv, p.hv_shift, p.st.S, p.st.sS, p.st.NPTR, p.st.sN, 0u, p);
+    hipLaunchKernelGGL((kda_quad_kernel<T, WPE, SPEC>), dim3(grid), dim3(Q::THREADS), quad_lds_pad(), stream, p.idx, p.order,
+                       p.st.S, p.st.NPTR, p.per_xcd, p.hv, p.hv_shift, p.st.sS, p.st.sN, p);
 #endif
     return int(hipGetLastError());
 }

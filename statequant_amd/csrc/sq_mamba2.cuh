@@ -32,7 +32,7 @@ void mamba2_step_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
     float* lds_u = reinterpret_cast<float*>(lds + L::FU);
 
     const LaneId l = lane_id<T>();
-    const TileId tid = tile_id_lead<(SPEC > 0 && heads_pow2(T::DK))>(order, per_xcd, hv, hv_shift);   // from the leading arguments
+    const TileId tid = tile_id_lead<SPEC == 1>(order, per_xcd, hv, hv_shift);   // from the leading arguments
     const uint32_t b = tid.b, h = tid.h, hk = p.gqa_shift >= 0 ? tid.h >> p.gqa_shift : tid.h / p.gqa;
     const int gqa = p.gqa;
     const int m = p.m;

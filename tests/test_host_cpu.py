@@ -220,9 +220,10 @@ def test_timeline_marks_stay_out_of_the_product_library():
     assert "libsqhip_timeline.so" in src and "build_timeline" in src
     marks = open(os.path.join(root, 'statequant_amd', 'csrc', 'sq_timeline.cuh')).read()
     assert marks.count('#ifdef SQ_TIMELINE') == 1 and '#define SQ_MARK(k) do { } while (0)' in marks
-    for name in ('sq_gdn_quad.cuh', 'sq_kda.cuh'):                     # the marked kernels
+    for name in ('sq_gdn_quad.cuh', 'sq_kda_quad.cuh'):                     # the marked kernels
         kern = open(os.path.join(root, 'statequant_amd', 'csrc', name)).read()
-        assert '#include "sq_timeline.cuh"' in kern and 'SQ_MARK(0)' in kern and '#ifdef SQ_TIMELINE' in kern
+        assert ('#include "sq_timeline.cuh"' in kern or '#include "sq_gdn_quad.cuh"' in kern) and 'SQ_MARK(0)' in kern
+        assert '#ifdef SQ_TIMELINE' in kern
     if not torch.cuda.is_available():
         r = subprocess.run([sys.executable, os.path.join(root, 'profile_timeline.py')], capture_output=True, text=True)
         assert r.returncode != 0 and ('is missing' in r.stderr or 'no GPU visible' in r.stderr), r.stderr
@@ -237,8 +238,9 @@ def test_timeline_marks_stay_out_of_the_product_library():
                 f.write('#include "%s"\n#include "%s"\nnamespace sq {\n'
                         'template int launch_gdn_quad<Tile<8, 128, 128, 128, true, 8>, 2, 2, 4, 1>(const GdnParams&, '
                         'hipStream_t);\n'
-                        'template int launch_kda<Tile<4, 128, 128, 32, true, 8>, 1>(const KdaParams&, hipStream_t);\n}\n'
-                        % (os.path.join(csrc, 'sq_gdn_quad.cuh'), os.path.join(csrc, 'sq_kda.cuh')))
+                        'template int launch_kda_quad<Tile<4, 128, 128, 32, true, 8>, 1, 1, 6, 1>(const KdaParams&, '
+                        'hipStream_t);\n}\n'
+                        % (os.path.join(csrc, 'sq_gdn_quad.cuh'), os.path.join(csrc, 'sq_kda_quad.cuh')))
             r = subprocess.run(['hipcc', *build.HIPCC_FLAGS, '-DSQ_TIMELINE', '--cuda-device-only', '-c', unit, '-o',
                                 os.path.join(d, 'one.o')], capture_output=True, text=True)
             assert r.returncode == 0, r.stderr[-2000:]
