@@ -170,7 +170,7 @@ def _stepped_twice(step, blobs):
     assert torch.equal(blobs[0], blobs[1])
 
 
-@pytest.mark.parametrize('fmt', [(8, 'k', 128), (4, 'k', 32), (4, 'k', 64), (4, 'v', 32), 'bf16'])      # the last two: one wavefront per tile
+@pytest.mark.parametrize('fmt', [(8, 'k', 128), (4, 'k', 32), (4, 'k', 64), (4, 'v', 32), 'bf16'])
 @pytest.mark.parametrize('gated', [False, True])
 def test_gdn_serving_case_instances_match_the_general_one(fmt, gated):
     """bf16 q / k / v / out with fp32 g, beta -- or the gate formed in the kernel from bf16 a, b and fp32 A_log, dt_bias

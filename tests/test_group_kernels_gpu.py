@@ -248,3 +248,57 @@ def test_int4_states_aligned_to_8_bytes(family, fmt, shape):
         assert far == 0 and mism <= 1e-4 * n
         for name in V[0]:                                           # a tie that went the other way is not carried on
             V[1][name].copy_(V[0][name])
+
+
+@pytest.mark.parametrize('family,fmt,shape,rows,form', [
+    # GDN: g and beta, or the gate in the kernel; head counts that are powers of two and not, one and two row blocks per
+    # wavefront, the one-wavefront kernel of launches of many 96-wide heads
+    ('gdn', (8, 'k', 32), (32, 16, 128, 128), 5, 'gate'), ('gdn', (8, 'k', 128), (32, 16, 128, 128), 70, 'plain'),
+    ('gdn', (4, 'k', 64), (32, 16, 128, 128), 70, 'gate'), ('gdn', (4, 'v', 32), (32, 16, 128, 128), 5, 'gate'),
+    ('gdn', (8, 'v', 32), (32, 16, 128, 128), 200, 'plain'), ('gdn', 'bf16', (32, 16, 128, 128), 5, 'gate'),
+    ('gdn', (4, 'k', 64), (30, 30, 96, 192), 5, 'gate'), ('gdn', (8, 'k', 32), (30, 30, 96, 192), 40, 'plain'),
+    ('gdn', 'bf16', (30, 30, 96, 192), 5, 'plain'), ('gdn', (4, 'k', 64), (40, 40, 96, 96), 130, 'gate'),
+    # KDA: fp32 g and beta
+    ('kda', (4, 'k', 32), (32, 32, 128, 128), 5, 'plain'), ('kda', (8, 'v', 32), (32, 32, 128, 128), 5, 'plain'),
+    ('kda', (4, 'k', 32), (20, 20, 96, 96), 5, 'plain'), ('kda', 'bf16', (20, 20, 96, 96), 5, 'plain'),
+    ('kda', (8, 'k', 32), (32, 32, 64, 32), 5, 'plain'), ('kda', (8, 'k', 32), (32, 32, 64, 32), 10, 'plain'),
+    # Mamba2: dt of either type, head counts that are powers of two and not
+    ('mamba2', (8, 'k', 128), (128, 8, 128, 64), 5, 'bf16 dt'), ('mamba2', (8, 'k', 128), (128, 8, 128, 64), 9, 'fp32 dt'),
+    ('mamba2', (4, 'k', 64), (112, 8, 128, 64), 9, 'bf16 dt'), ('mamba2', (4, 'v', 32), (96, 8, 128, 64), 5, 'fp32 dt'),
+    ('mamba2', (8, 'k', 128), (96, 8, 128, 80), 5, 'bf16 dt'), ('mamba2', 'bf16', (96, 8, 128, 80), 5, 'bf16 dt')])
+def test_serving_case_instances_leave_the_bytes_of_the_general_one(family, fmt, shape, rows, form):
+    """The tokens as serving layers hand them over (bf16, fp32 gates) through the instances with that compiled in and
+    through the general one, two fold periods of sequences out of step, a padding row: the same bytes throughout."""
+    hv, hk, dk, dv = shape
+    lay = _layout(family, fmt, shape, 8, 8)
+    gen = torch.Generator(device=DEV).manual_seed(9)
+    r = lambda *s: torch.randn(*s, device=DEV, generator=gen)      # noqa: E731
+    blobs = [lay.alloc(rows, DEV) for _ in range(2)]
+    V = [lay.views(b) for b in blobs]
+    idx = torch.randperm(rows, device=DEV, generator=gen).to(torch.int32)
+    lay.write(V[0], idx, r(rows, hv, dv, dk) * 0.4)
+    blobs[1].copy_(blobs[0])
+    for step in range(17):
+        if step in (3, 6):
+            for W in V:
+                lay.write(W, idx[:rows // 2], torch.ones(rows // 2, hv, dv, dk, device=DEV) * 0.1)
+        x = r(rows, 2 * hk * dk + hv * dv).bfloat16()
+        q, k, v = (x[:, lo:hi].unflatten(1, (h, d)) for lo, hi, h, d in (
+            (0, hk * dk, hk, dk), (hk * dk, 2 * hk * dk, hk, dk), (2 * hk * dk, 2 * hk * dk + hv * dv, hv, dv)))
+        g = -torch.nn.functional.softplus(r(rows, hv, dk) if family == 'kda' else r(rows, hv))
+        beta, raw, model = torch.sigmoid(r(rows, hv)), r(rows, hv).bfloat16(), (r(hv) * 0.3, r(hv) * 0.3, r(hv))
+        outs = [torch.full((rows, hv, dv), 3.0, device=DEV, dtype=torch.bfloat16) for _ in range(2)]
+        for i, (W, out) in enumerate(zip(V, outs)):
+            _hip.select_instances(no_specialised=i == 1)
+            try:
+                if family == 'mamba2':
+                    lay.step(W, idx, v, raw if form == 'bf16 dt' else raw.float(), q, k, out, -torch.exp(model[0]), *model[1:])
+                elif family == 'kda':
+                    lay.step(W, idx, q, k, v, g, beta, out)
+                elif form == 'gate':
+                    lay.step(W, idx, q, k, v, out, dk ** -0.5, gate=(raw, raw.flip(0), *model[:2]))
+                else:
+                    lay.step(W, idx, q, k, v, out, dk ** -0.5, g=g, beta=beta)
+            finally:
+                _hip.select_instances()
+        assert torch.equal(outs[0], outs[1]) and torch.equal(blobs[0], blobs[1]), step
