@@ -46,7 +46,9 @@ SHADER_SETS = {
 
 
 def rocprof(args, bench_args, workdir, timeout=240):
-    """One rocprofv3 run of bench.py; returns (command as text, directory with the csv output)."""
+    """One rocprofv3 run of bench.py; returns (command as text, directory with the csv output, how many of the step's
+    launches belong to its warm-up and timed steps -- None: all; the default line measures sequences out of step behind
+    them)."""
     out = tempfile.mkdtemp(prefix='prof_', dir=workdir)
     cmd = ['rocprofv3', *args, '--output-format', 'csv', '-d', out, '-o', 'p', '--',
            'python3', os.path.join(ROOT, 'bench.py'), *bench_args]
@@ -55,7 +57,9 @@ def rocprof(args, bench_args, workdir, timeout=240):
     if r.returncode:
         sys.exit(f'{" ".join(cmd)}\nexit {r.returncode}\n{r.stdout[-2000:]}\n{r.stderr[-2000:]}')
     shown = ['rocprofv3', *args, '--output-format', 'csv', '-d', '<dir>', '-o', 'p', '--', 'python3', 'bench.py', *bench_args]
-    return ' '.join(shown), out
+    line = [x for x in r.stdout.split('\n') if x.startswith('{')]
+    res = json.loads(line[-1]) if line else {}
+    return ' '.join(shown), out, (res['steps'] + res['warmup']) * LAYERS if 'out_of_step' in res else None
 
 
 def read_csv(d, suffix):
@@ -69,11 +73,13 @@ def kind_of(i):
     return 'fold' if (i // LAYERS) % M == M - 1 else 'plain'
 
 
-def counters(d, pick):
-    """{(counter, kind): average per dispatch} over the dispatches whose kernel name `pick` accepts, in dispatch
+def counters(d, pick, first=None):
+    """{(counter, kind): average per dispatch} over the (first) dispatches whose kernel name `pick` accepts, in dispatch
     order; kind = fold / plain by the step of the period a dispatch belongs to ('all' for a calibration run)."""
     rows = [r for r in read_csv(d, 'counter_collection.csv') if pick(r['Kernel_Name'])]
-    ids = sorted({int(r['Dispatch_Id']) for r in rows})
+    ids = sorted({int(r['Dispatch_Id']) for r in rows})[:first]
+    kept = set(ids)
+    rows = [r for r in rows if int(r['Dispatch_Id']) in kept]
     pos = {x: i for i, x in enumerate(ids)}
     acc = collections.defaultdict(lambda: [0.0, 0])
     name = rows[0]['Kernel_Name'] if rows else ''
@@ -115,9 +121,10 @@ def main():
     kernel = ''
 
     if 'trace' in sets:
-        cmd, d = rocprof(['--kernel-trace', '--stats'], targs, work, timeout=600)
+        cmd, d, first = rocprof(['--kernel-trace', '--stats'], targs, work, timeout=600)
         rows = [r for r in read_csv(d, 'kernel_trace.csv') if is_step(r['Kernel_Name'])]
         rows.sort(key=lambda r: int(r['Start_Timestamp']))
+        rows = rows[:first]
         dur = [(int(r['End_Timestamp']) - int(r['Start_Timestamp'])) / 1e3 for r in rows]
         kernel = rows[0]['Kernel_Name']
         by = collections.defaultdict(list)
@@ -145,13 +152,13 @@ def main():
         lines.append('== HBM traffic ==')
         factor, per = {}, {}
         for c, known in (('FETCH_SIZE', 'bytes_read'), ('WRITE_SIZE', 'bytes_written')):
-            cmd_c, d = rocprof(['--pmc', c], ['--calibrate-copy'], work)
+            cmd_c, d, _ = rocprof(['--pmc', c], ['--calibrate-copy'], work)
             cal, ncal, kcal = counters(d, lambda n: 'copy' in n.lower())
             shutil.rmtree(d, ignore_errors=True)
             kib = cal[(c, 'all')]
             factor[c] = (1 << 30) / 1024 / kib                      # the copy moves 1 GiB each way per dispatch
-            cmd_w, d = rocprof(['--pmc', c], bargs, work)
-            val, n, kernel = counters(d, is_step)
+            cmd_w, d, first = rocprof(['--pmc', c], bargs, work)
+            val, n, kernel = counters(d, is_step, first)
             shutil.rmtree(d, ignore_errors=True)
             per[c] = {k: val[(c, k)] * 1024 * factor[c] for k in ('plain', 'fold', 'all')}
             lines += [cmd_c, f'  {kcal[:60]}: {ncal} copies of 1 GiB, {c} {kib:.1f} KiB per dispatch -> factor {factor[c]:.3f}',
@@ -179,8 +186,8 @@ def main():
     if 'shader' in sets:
         lines.append('== shader counters, average per dispatch ==')
         for name, cs in SHADER_SETS.items():
-            cmd, d = rocprof(['--pmc', *cs], bargs, work)
-            val, n, kernel = counters(d, is_step)
+            cmd, d, first = rocprof(['--pmc', *cs], bargs, work)
+            val, n, kernel = counters(d, is_step, first)
             shutil.rmtree(d, ignore_errors=True)
             lines += [cmd, f'  {"counter":28s} {"plain step":>16s} {"fold step":>16s}']
             for c in cs:
