@@ -146,8 +146,8 @@ def quad_variants(fam, c):
     be = 1 if qbuf else 2
     out = []
     for gh in QUAD_FAMILIES[fam]:
-        if dv % 32 and gh > 1:                               # d_v 80: a head a workgroup (96 heads, int8 g32, 128 sequences:
-            continue                                         # 42.3 us per launch, two heads 53.5, four 44.5)
+        if dv % 32 and gh > 1:                               # d_v 80: a head a workgroup (96 heads, int8 g32; us per launch
+            continue                                         # with one, two, four: 1 sequence 5.6, 5.8, 6.4, 48: 24.8, 31.8, 25.5)
         nw = gh * nrb // nb
         if nw > 16:
             continue

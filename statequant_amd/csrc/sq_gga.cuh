@@ -512,7 +512,8 @@ struct GgaLds {
 // Four wavefronts per SIMD (128 registers, 11 of them spilled): the launch of 32 sequences x 32 heads of 128 x 128 then
 // runs in one round of workgroups.  us per launch there, mixed widths: 44.0 with values and quotients side by side (225
 // registers, two wavefronts per SIMD) -> 34.6 at three -> 32.4 at four; 4151 -> 3415 vector instructions per wavefront,
-// which is 23 us of issue.
+// which is 23 us of issue.  At 256 sequences 287 -> 187, although the spilled registers then reach memory (188 -> 283 MB
+// per launch: 1.5 TB/s, far from a bound).
 template <class T>
 __global__ __launch_bounds__(GGA_THREADS, 4) void gga_step_kernel(const GgaParams p) {
     constexpr int CT = T::CT, CO = T::CO, RPT = T::RPT, DK = T::DK, DV = T::DV, NE = T::NE, NV = T::NV;

@@ -2,9 +2,9 @@
 // decode step (or state hand-over) without an interpreted instruction in between.
 //
 // What it is for: a decode step calls the library once per layer, and reading some twenty tensors' pointers, strides and
-// dtypes through Python took 17.5 us per call -- four times as long as the kernel itself runs for one sequence, so small
-// batches waited for the host.  24 GDN layers, int8: 1 sequence 430 -> 155 us, 13 sequences (int4) 433 -> 198; six KDA
-// layers in lockstep 103 -> 36 (5.4 to 6.5 us of each call is the kernel itself).
+// dtypes through Python took 16 to 19 us per call -- four times as long as the kernel itself runs for one sequence, so small
+// batches waited for the host.  Host time of a call: GDN step on slots, gates from a, b 18.9 -> 6 to 7 us, KDA step on plain
+// tensors 16.5 -> 3.8; a layer of one GDN sequence, int8, launched so 18.1 -> 6 (its kernel alone 4.8, in a graph).
 //
 // Every function here takes exactly the calls that the Python code around it accepts in its ordinary form -- plain dense
 // tensors on one GPU, the documented shapes -- and answers None to anything else (another tensor class, a tensor under a
