@@ -37,6 +37,9 @@ constexpr int GGA_THREADS = 256;
 constexpr int GGA_WAVES = GGA_THREADS / WAVE;
 constexpr int GGA_MMAX = 8;
 constexpr int GGA_GROUP = 32;
+// the slot's second counter: the ring index of the oldest pair, and above it -- while a step runs -- the heads that have
+// read the counters
+constexpr uint32_t GGA_RING = 0xFFFF, GGA_TICKET = 0x10000;
 
 template <int DK_, int DV_>
 struct GgaTile {
@@ -202,24 +205,29 @@ struct GgaCode {
     }
 };
 
-// Head state of width B at S -> the thread's x[s][e] (reference: `_load_head`, _gga_triton.py:131-143).
-template <class T, int B>
-__device__ __forceinline__ void gga_load_head(const uint8_t* S, const GgaThread& t, float (&x)[T::RPT][T::CT]) {
+// Head state of width B at S -> the thread's x[s][e] (reference: `_load_head`, _gga_triton.py:131-143).  `between` runs
+// when the loads are out and before any of them is used: what else is to be requested.
+template <class T, int B, class F>
+__device__ __forceinline__ void gga_load_head(const uint8_t* S, const GgaThread& t, float (&x)[T::RPT][T::CT], F&& between) {
     constexpr int CT = T::CT, RPT = T::RPT, DK = T::DK, DV = T::DV;
     if constexpr (B == 16) {
         const uint16_t* H = reinterpret_cast<const uint16_t*>(S);
+        uint2 v[RPT][CT / 4];
 #pragma unroll
-        for (int s = 0; s < RPT; ++s) {
-            const int i = s * 16 + t.tr;
+        for (int s = 0; s < RPT; ++s)
 #pragma unroll
-            for (int e4 = 0; e4 < CT; e4 += 4) {
-                const uint2 v = *reinterpret_cast<const uint2*>(H + i * DV + t.tc * CT + e4);
-                x[s][e4 + 0] = f16_to_f32(uint16_t(v.x));
-                x[s][e4 + 1] = f16_to_f32(uint16_t(v.x >> 16));
-                x[s][e4 + 2] = f16_to_f32(uint16_t(v.y));
-                x[s][e4 + 3] = f16_to_f32(uint16_t(v.y >> 16));
+            for (int e4 = 0; e4 < CT / 4; ++e4)
+                v[s][e4] = *reinterpret_cast<const uint2*>(H + (s * 16 + t.tr) * DV + t.tc * CT + 4 * e4);
+        between();
+#pragma unroll
+        for (int s = 0; s < RPT; ++s)
+#pragma unroll
+            for (int e4 = 0; e4 < CT / 4; ++e4) {
+                x[s][4 * e4 + 0] = f16_to_f32(uint16_t(v[s][e4].x));
+                x[s][4 * e4 + 1] = f16_to_f32(uint16_t(v[s][e4].x >> 16));
+                x[s][4 * e4 + 2] = f16_to_f32(uint16_t(v[s][e4].y));
+                x[s][4 * e4 + 3] = f16_to_f32(uint16_t(v[s][e4].y >> 16));
             }
-        }
     } else {
         constexpr int NB = CT * B / 8;
         constexpr int RB = DV * B / 8;                                     // bytes of a row of codes
@@ -233,20 +241,19 @@ __device__ __forceinline__ void gga_load_head(const uint8_t* S, const GgaThread&
             raw[s] = gga_load_bytes<NB>(S + i * RB + t.tc * NB);
             rr[s] = B == 2 ? R[i * T::NG + (t.tc * CT) / GGA_GROUP] : R[i];
         }
-        float c[CT];                                                       // column factors, over the code's scale
-        {
-            uint32_t cw[CT / 2];
-            if constexpr (CT == 8) {
-                const uint4 v = *reinterpret_cast<const uint4*>(C + t.tc * CT);
-                cw[0] = v.x; cw[1] = v.y; cw[2] = v.z; cw[3] = v.w;
-            } else {
-                const uint2 v = *reinterpret_cast<const uint2*>(C + t.tc * CT);
-                cw[0] = v.x; cw[1] = v.y;
-            }
-#pragma unroll
-            for (int e = 0; e < CT; ++e)
-                c[e] = f16_to_f32(uint16_t(cw[e / 2] >> (16 * (e % 2)))) * (1.0f / float(1u << GgaCode<B>::up(e)));
+        uint32_t cw[CT / 2];
+        if constexpr (CT == 8) {
+            const uint4 v = *reinterpret_cast<const uint4*>(C + t.tc * CT);
+            cw[0] = v.x; cw[1] = v.y; cw[2] = v.z; cw[3] = v.w;
+        } else {
+            const uint2 v = *reinterpret_cast<const uint2*>(C + t.tc * CT);
+            cw[0] = v.x; cw[1] = v.y;
         }
+        between();
+        float c[CT];                                                       // column factors, over the code's scale
+#pragma unroll
+        for (int e = 0; e < CT; ++e)
+            c[e] = f16_to_f32(uint16_t(cw[e / 2] >> (16 * (e % 2)))) * (1.0f / float(1u << GgaCode<B>::up(e)));
 #pragma unroll
         for (int s = 0; s < RPT; ++s) {
             const float r = f16_to_f32(rr[s]);
@@ -440,13 +447,14 @@ __device__ __forceinline__ void gga_fit_store(uint8_t* S, float (&x)[T::RPT][T::
     }
 }
 
-template <class T>
-__device__ __forceinline__ void gga_load_any(const uint8_t* S, int bits, const GgaThread& t, float (&x)[T::RPT][T::CT]) {
-    if (bits == 16) gga_load_head<T, 16>(S, t, x);
-    else if (bits == 8) gga_load_head<T, 8>(S, t, x);
-    else if (bits == 6) gga_load_head<T, 6>(S, t, x);
-    else if (bits == 4) gga_load_head<T, 4>(S, t, x);
-    else gga_load_head<T, 2>(S, t, x);
+template <class T, class F>
+__device__ __forceinline__ void gga_load_any(const uint8_t* S, int bits, const GgaThread& t, float (&x)[T::RPT][T::CT],
+                                             F&& between) {
+    if (bits == 16) gga_load_head<T, 16>(S, t, x, between);
+    else if (bits == 8) gga_load_head<T, 8>(S, t, x, between);
+    else if (bits == 6) gga_load_head<T, 6>(S, t, x, between);
+    else if (bits == 4) gga_load_head<T, 4>(S, t, x, between);
+    else gga_load_head<T, 2>(S, t, x, between);
 }
 template <class T>
 __device__ __forceinline__ void gga_store_any(uint8_t* S, int bits, float (&x)[T::RPT][T::CT], const float* w,
@@ -509,44 +517,49 @@ struct GgaLds {
     GgaFitLds<T> fit;
 };
 
-// Four wavefronts per SIMD (128 registers, 11 of them spilled): the launch of 32 sequences x 32 heads of 128 x 128 then
-// runs in one round of workgroups.  us per launch there, mixed widths: 44.0 with values and quotients side by side (225
-// registers, two wavefronts per SIMD) -> 34.6 at three -> 32.4 at four; 4151 -> 3415 vector instructions per wavefront,
-// which is 23 us of issue.  At 256 sequences 287 -> 187, although the spilled registers then reach memory (188 -> 283 MB
-// per launch: 1.5 TB/s, far from a bound).
-template <class T>
-__global__ __launch_bounds__(GGA_THREADS, 4) void gga_step_kernel(const GgaParams p) {
+// Four wavefronts per SIMD (128 registers, some spilled): the launch of 32 sequences x 32 heads of 128 x 128 then runs in
+// one round of workgroups.  us per launch there, mixed widths: 44.0 with values and quotients side by side (225 registers,
+// two wavefronts per SIMD) -> 34.6 at three -> 32.4 at four.  In one round every workgroup loads, computes and stores at
+// the same time as all others, so what stands in front of the first value and behind the last one is paid in full: with
+// the serving case's types compiled in (SPEC, as in the other families; some 200 branches on them were in the way), the
+// leading arguments in registers, the state requested ahead of the counters and of the window that waits for them, the
+// new pair queued ahead of the fit and the counters advanced in the same launch (a ticket, below) a layer takes 30.2 us
+// where the step and a launch for the counters took 33.7.
+template <class T, int SPEC>
+__global__ __launch_bounds__(GGA_THREADS, 4)
+void gga_step_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict__ offs, const int32_t* __restrict__ widths,
+                     uint8_t* blob, uint64_t slot_stride, const GgaParams p0) {
+    // (the leading arguments, copies of fields of the block, are in registers when a wavefront starts)
+    GgaParams p = p0;
+    assume_serving_case<SPEC>(p);
     constexpr int CT = T::CT, CO = T::CO, RPT = T::RPT, DK = T::DK, DV = T::DV, NE = T::NE, NV = T::NV;
     __shared__ __attribute__((aligned(16))) GgaLds<T> L;
     const GgaThread t = gga_thread();
     // head-major order: workgroups that run together work on the same head, hence on the same width, and share the
     // instructions of one of the five width paths (each path is ~40 KB of straight-line code)
-    const uint32_t h = blockIdx.x / uint32_t(p.rows), b = blockIdx.x - h * uint32_t(p.rows);
+    const uint32_t h = blockIdx.y, b = blockIdx.x;
     const uint32_t bh = b * uint32_t(p.hv) + h;
-    const uint32_t hk = h / uint32_t(p.gqa);
+    const uint32_t hk = p.gqa_shift >= 0 ? h >> p.gqa_shift : h / uint32_t(p.gqa);
+    const int32_t seq = idx[b];
+    const int bits = widths[h];
+    const int32_t off = offs[h];
     void* const outp = advance(p.out, p.out_dt, uint64_t(bh) * DV);
-    const int32_t seq = p.idx[b];
     if (seq <= 0) {
         if (t.tid < DV) store_f(outp, p.out_dt, t.tid, 0.0f);
         return;
     }
-    uint8_t* const base = p.blob + uint64_t(seq) * p.slot_stride;
-    const int bits = p.bits[h];
-    uint8_t* const S = base + p.offs[h];
+    uint8_t* const base = blob + uint64_t(seq) * slot_stride;
+    uint8_t* const S = base + off;
     const bool window = p.pw && bits != 16;
     const int m = p.m;
-    int n = 0, hd = 0;
-    if (window) {
-        n = reinterpret_cast<const int32_t*>(base)[0];
-        hd = reinterpret_cast<const int32_t*>(base)[1];
-        n = n < 0 ? 0 : n > m ? m : n;
-        hd = hd < 0 ? 0 : hd >= m ? m - 1 : hd;
-    }
     uint8_t* const qb = base + p.qoff + uint64_t(h) * p.qsz;
     uint8_t* const PP = qb;
     uint8_t* const VP = qb + m * DK;
     float* const PS = reinterpret_cast<float*>(qb + m * (DK + DV));
     float* const VS = PS + m;
+    // the slot's counters: scalar loads (left to the compiler, vector loads: the same words are written further down)
+    const auto* const ct = (const __attribute__((address_space(4))) int32_t*)(base);
+    int n = ct[0], hd = ct[1];
 
     // ---- q, k of the key head (every wavefront on its own: lane l holds elements l NE .. l NE + NE - 1), gates ----
     const void* qp = advance(p.q, p.q_dt, uint64_t(b) * p.s_q + hk * DK);
@@ -563,7 +576,6 @@ __global__ __launch_bounds__(GGA_THREADS, 4) void gga_step_kernel(const GgaParam
     const uint32_t dbr = load_raw_uniform(p.dt_bias, p.dt_bias_dt, h);
     // the lane's kept columns of v and of the queued right factors (for the output), and all its columns of the write
     // that enters the state: the oldest pair of a full window, v itself without a window
-    const bool full = window && n == m, enters = full || !window;
     const void* vp = advance(p.v, p.v_dt, uint64_t(b) * p.s_v + h * DV);
     const int c0 = t.tc * CT, oc = c0 + t.own * CO;
     uint32_t vo[CO], v0q[CT / 4];
@@ -571,23 +583,30 @@ __global__ __launch_bounds__(GGA_THREADS, 4) void gga_step_kernel(const GgaParam
     for (int e = 0; e < CO; ++e) vo[e] = load_raw(vp, p.v_dt, oc + e);
     uint32_t vq[GGA_MMAX];
     float vsl = 0.0f;                                   // lane oi: the scale of the oi-th oldest right factor
-    if (window) {
-        if (t.lane < n) vsl = VS[hd + t.lane < m ? hd + t.lane : hd + t.lane - m];
-#pragma unroll
-        for (int oi = 0; oi < GGA_MMAX; ++oi) {
-            const int jj = hd + oi < m ? hd + oi : hd + oi - m;
-            const bool live = oi < n;
-            if constexpr (CO == 2) vq[oi] = live ? *reinterpret_cast<const uint16_t*>(VP + jj * DV + oc) : 0u;
-            else vq[oi] = live ? VP[jj * DV + oc] : 0u;
-        }
-        if (full) {
-#pragma unroll
-            for (int w4 = 0; w4 < CT / 4; ++w4) v0q[w4] = reinterpret_cast<const uint32_t*>(VP + hd * DV + c0)[w4];
-        }
-    }
-
     float x[RPT][CT];
-    gga_load_any<T>(S, bits, t, x);
+    // the state goes out ahead of the window, whose addresses wait for the counters
+    gga_load_any<T>(S, bits, t, x, [&] {
+        asm volatile("" : "+s"(n), "+s"(hd) :: "memory");           // read here, never again: see the ticket below
+        n = n < 0 ? 0 : n > m ? m : n;
+        hd &= GGA_RING;                                              // (the ticket above it may be counting already)
+        hd = hd >= m ? m - 1 : hd;
+        if (!window) n = hd = 0;
+        if (window) {
+            if (t.lane < n) vsl = VS[hd + t.lane < m ? hd + t.lane : hd + t.lane - m];
+#pragma unroll
+            for (int oi = 0; oi < GGA_MMAX; ++oi) {      // entries beyond the queue: any of the ring, not used below
+                int jj = hd + oi < m ? hd + oi : hd + oi - m;
+                jj = jj < m ? jj : 0;
+                if constexpr (CO == 2) vq[oi] = *reinterpret_cast<const uint16_t*>(VP + jj * DV + oc);
+                else vq[oi] = VP[jj * DV + oc];
+            }
+            if (n == m) {
+#pragma unroll
+                for (int w4 = 0; w4 < CT / 4; ++w4) v0q[w4] = reinterpret_cast<const uint32_t*>(VP + hd * DV + c0)[w4];
+            }
+        }
+    });
+    const bool full = window && n == m, enters = full || !window;
 
     float qe[NE], ke[NE], ssq = 0.0f, ssk = 0.0f;
 #pragma unroll
@@ -660,6 +679,15 @@ __global__ __launch_bounds__(GGA_THREADS, 4) void gga_step_kernel(const GgaParam
         }
     }
     __syncthreads();
+    // ---- a ticket for the slot's counters: every head of the slot reads them, the last one to have done so advances them.
+    // The tickets are counted in the upper half of the ring index (whose value is below 16; zero between steps), so the
+    // slot's bytes are what a launch of its own behind every step left there.  This head's reads have returned (their
+    // values are in registers) before its ticket goes out, so no head reads what the last one writes; the writes are seen
+    // by the next launch.
+    uint32_t ticket = 0;
+    if (p.pw && t.tid == 0)
+        ticket = __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(base) + 1, GGA_TICKET, __ATOMIC_RELAXED,
+                                        __HIP_MEMORY_SCOPE_AGENT);
 
     // ---- k^T O and q^T O; the output: q^T O_pre = a (q^T O - (beta k . q) k^T O), the queued pairs oldest first, and
     //      this token's write -- for the lane's kept columns ----
@@ -729,14 +757,10 @@ __global__ __launch_bounds__(GGA_THREADS, 4) void gga_step_kernel(const GgaParam
         }
     }
 
-    // ---- re-fit and re-pack in place ----
-    gga_store_any<T>(S, bits, x, p.w + h * DK, L.fit);
-
     // ---- queue (R(beta k), R(v)).  A full window's new pair replaces the oldest one, whose right factor every
     // wavefront has read for the merge: the barrier puts the store behind all of those reads (each wavefront used its
     // copy before it got here).
     if (window) {
-        const GgaThread t = gga_thread();
         __syncthreads();
         const int jn = n == m ? hd : hd + n < m ? hd + n : hd + n - m;
         if (t.wave == 0) {
@@ -756,19 +780,17 @@ __global__ __launch_bounds__(GGA_THREADS, 4) void gga_step_kernel(const GgaParam
             if (t.lane == 0) VS[jn] = sc;
         }
     }
-}
 
-// Counters of the stepped slots, after the step (all heads of a slot read them): reference `_gga_advance`.
-template <class T>
-__global__ void gga_advance_kernel(uint8_t* blob, uint64_t slot_stride, const int32_t* idx, int rows, int m) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= rows) return;
-    const int32_t seq = idx[b];
-    if (seq <= 0) return;
-    int32_t* ct = reinterpret_cast<int32_t*>(blob + uint64_t(seq) * slot_stride);
-    const int n = ct[0], hd = ct[1];
-    ct[0] = n + 1 < m ? n + 1 : m;
-    ct[1] = n == m ? (hd + 1) % m : hd;
+    // ---- re-fit and re-pack in place ----
+    gga_store_any<T>(S, bits, x, p.w + h * DK, L.fit);
+
+    // ---- the last head's: the counters of the slot, advanced (reference `_gga_advance`) ----
+    if (p.pw && t.tid == 0 && ticket / GGA_TICKET == uint32_t(p.hv) - 1) {
+        int32_t* const ct = reinterpret_cast<int32_t*>(base);
+        const int n0 = ct[0], hd0 = int(ticket & GGA_RING);
+        ct[0] = n0 + 1 < m ? n0 + 1 : m;
+        __hip_atomic_store(ct + 1, n0 == m ? (hd0 + 1) % m : hd0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
 }
 
 // Fit + pack canonical states X [rows, hv, d_k, d_v] fp32 into slots idx; zero the counters (reference `_gga_store`).
@@ -812,7 +834,7 @@ __global__ __launch_bounds__(GGA_THREADS, 2) void gga_load_kernel(const GgaParam
     float* Y = p.Y + uint64_t(bh) * (DK * DV);
     float x[RPT][CT];
     if (seq > 0) {
-        gga_load_any<T>(p.blob + uint64_t(seq) * p.slot_stride + p.offs[h], p.bits[h], t, x);
+        gga_load_any<T>(p.blob + uint64_t(seq) * p.slot_stride + p.offs[h], p.bits[h], t, x, [] {});
     } else {
 #pragma unroll
         for (int s = 0; s < RPT; ++s)
@@ -827,15 +849,19 @@ __global__ __launch_bounds__(GGA_THREADS, 2) void gga_load_kernel(const GgaParam
                 make_float4(x[s][e4], x[s][e4 + 1], x[s][e4 + 2], x[s][e4 + 3]);
 }
 
-// op: 0 step (+ advance), 1 store, 2 load
+// op: 0 step, 1 store, 2 load
 template <class T>
 int launch_gga(const GgaParams& p, int op, hipStream_t stream) {
     const dim3 grid(p.rows * p.hv), block(GGA_THREADS);
     if (op == 0) {
-        hipLaunchKernelGGL(gga_step_kernel<T>, grid, block, 0, stream, p);
-        if (p.pw)
-            hipLaunchKernelGGL(gga_advance_kernel<T>, dim3((p.rows + 63) / 64), dim3(64), 0, stream, p.blob, p.slot_stride,
-                               p.idx, p.rows, p.m);
+        const dim3 tiles(p.rows, p.hv);
+        const int spec = serving_case(p);
+        if (spec == 2) hipLaunchKernelGGL((gga_step_kernel<T, 2>), tiles, block, 0, stream, p.idx, p.offs, p.bits, p.blob,
+                               p.slot_stride, p);
+        else if (spec == 1) hipLaunchKernelGGL((gga_step_kernel<T, 1>), tiles, block, 0, stream, p.idx, p.offs, p.bits, p.blob,
+                               p.slot_stride, p);
+        else hipLaunchKernelGGL((gga_step_kernel<T, 0>), tiles, block, 0, stream, p.idx, p.offs, p.bits, p.blob,
+                               p.slot_stride, p);
     } else if (op == 1) {
         hipLaunchKernelGGL(gga_store_kernel<T>, grid, block, 0, stream, p);
     } else {

@@ -104,7 +104,7 @@ struct GgaParams {
     const int32_t* offs;                          // [hv] byte offset of each head in the slot
     const int32_t* bits;                          // [hv] width of each head: 2, 4, 6, 8 or 16 (fp16 pivot)
     const float* w;                               // [hv, dk] row impact factors of the fit
-    int hv, hk, gqa, dk, dv, m, pw;
+    int hv, hk, gqa, gqa_shift, dk, dv, m, pw;    // gqa_shift: log2 of gqa where it is a power of two, else -1
     uint32_t qoff, qsz;                           // windows: at qoff + h * qsz
     const void *q, *k, *v;
     uint32_t s_q, s_k, s_v;
@@ -146,8 +146,22 @@ inline int serving_case(const Mamba2Params& p) {
     return (p.A_dt == 0 && p.D_dt == 0 && p.dt_bias_dt == 0) 
                ? (p.hv_shift >= 0 && p.gqa_shift >= 0 ? 1 : 2) : 0;
 }
+inline int serving_case(const GgaParams& p) {             // as for GDN; any head count
+    if (p.q_dt != 1 || p.k_dt != 1 || p.v_dt != 1 || p.out_dt != 1) return 0;
+    if (!p.gate) return (p.a_dt == 0 && p.bt_dt == 0) ? 1 : 0;
+    return (p.a_dt == 1 && p.bt_dt == 1 && p.A_log_dt == 0 && p.dt_bias_dt == 0) ? 2 : 0;
+}
 template <int SPEC>
 __device__ __forceinline__ void assume_serving_case(GdnParams& p) {
+    if constexpr (SPEC > 0) {
+        p.q_dt = p.k_dt = p.v_dt = p.out_dt = 1;
+        p.a_dt = p.bt_dt = SPEC == 1 ? 0 : 1;
+        p.A_log_dt = p.dt_bias_dt = 0;
+        p.gate = SPEC == 2;
+    }
+}
+template <int SPEC>
+__device__ __forceinline__ void assume_serving_case(GgaParams& p) {
     if constexpr (SPEC > 0) {
         p.q_dt = p.k_dt = p.v_dt = p.out_dt = 1;
         p.a_dt = p.bt_dt = SPEC == 1 ? 0 : 1;

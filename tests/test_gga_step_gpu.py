@@ -1,0 +1,66 @@
+"""The mixed-width step's one launch: the slot's counters, which its last head advances, and the instances with the serving
+case's types compiled in against the general one."""
+import pytest
+import torch
+
+from statequant_amd.kernels.gga import GGAPacked, GGAPlan
+
+pytestmark = pytest.mark.gpu
+DEV = 'cuda'
+
+
+def _case(hv, hk, d, m, rows, seed=0, pw=True):
+    gen = torch.Generator().manual_seed(seed)
+    widths = torch.tensor(([2, 4, 6, 8, 16] * hv)[:hv])
+    lay = GGAPacked(GGAPlan({0: (widths, torch.rand(hv, d, generator=gen) + 0.5)}), hv, hk, d, d, pw=pw, m=m)
+    views = lay.views(lay.alloc(rows + 3, DEV))
+    idx = (torch.randperm(rows + 2, generator=gen)[:rows] + 1).to(torch.int32).to(DEV)
+    lay.write(views, idx, (torch.randn(rows, hv, d, d, generator=gen) * 0.3).to(DEV), layer=0)
+    return lay.prepare(DEV), views, idx, gen
+
+
+def _token(gen, rows, hv, hk, d):
+    r = lambda *s: torch.randn(*s, generator=gen).bfloat16().to(DEV)         # noqa: E731
+    return r(rows, hk, d), r(rows, hk, d), r(rows, hv, d), r(rows, hv), r(rows, hv)
+
+
+@pytest.mark.parametrize('hv, hk, d, m, rows', [(1, 1, 64, 1, 1), (3, 3, 64, 8, 5), (5, 5, 128, 3, 2), (32, 16, 64, 8, 40)])
+def test_counters_advance_once_a_step(hv, hk, d, m, rows):
+    lay, views, idx, gen = _case(hv, hk, d, m, rows)
+    blob = views['blob']
+    blob[:, 8:16] = 0xA5                                                     # not the step's to write
+    idx[rows // 2] = 0 if rows > 1 else idx[0]                               # padding
+    live = idx[idx > 0].long()
+    A, bias = torch.randn(hv, generator=gen).to(DEV) * 0.3, torch.randn(hv, generator=gen).to(DEV) * 0.3
+    out = torch.zeros(rows, hv, d, dtype=torch.bfloat16, device=DEV)
+    want = torch.zeros(blob.shape[0], 2, dtype=torch.int32)
+    for t in range(2 * m + 3):
+        q, k, v, a, b = _token(gen, rows, hv, hk, d)
+        lay.step(views, idx, q, k, v, out, d ** -0.5, gate=(a, b, A, bias), layer=0)
+        for s in live.tolist():
+            n, head = want[s].tolist()
+            want[s] = torch.tensor([min(n + 1, m), (head + 1) % m if n == m else head])
+        assert torch.equal(blob[:, :8].cpu().view(torch.int32), want), t
+        assert (blob[:, 8:16] == 0xA5).all()
+
+
+@pytest.mark.parametrize('gate', [True, False])
+@pytest.mark.parametrize('hv, hk, d, pw', [(5, 5, 64, True), (8, 4, 128, True), (6, 2, 128, False)])
+def test_serving_instances_equal_the_general_one(gate, hv, hk, d, pw):
+    rows = 3
+    lay, views, idx, gen = _case(hv, hk, d, 8, rows, pw=pw)
+    twin = lay.views(views['blob'].clone())
+    A, bias = torch.randn(hv, generator=gen).to(DEV) * 0.3, torch.randn(hv, generator=gen).to(DEV) * 0.3
+    o16 = torch.zeros(rows, hv, d, dtype=torch.bfloat16, device=DEV)
+    o32 = torch.zeros(rows, hv, d, device=DEV)
+    for t in range(11):
+        q, k, v, a, b = _token(gen, rows, hv, hk, d)
+        if gate:
+            one, two = dict(gate=(a, b, A, bias)), dict(gate=(a.float(), b.float(), A, bias))
+        else:
+            g, beta = -torch.nn.functional.softplus(a.float()), torch.sigmoid(b.float())
+            one = two = dict(g=g, beta=beta)
+        lay.step(views, idx, q, k, v, o16, d ** -0.5, layer=0, **one)
+        lay.step(twin, idx, q.float(), k.float(), v.float(), o32, d ** -0.5, layer=0, **two)      # fp32: the general instance
+        assert torch.equal(o16, o32.bfloat16()), t
+        assert torch.equal(views['blob'], twin['blob']), t
