@@ -33,6 +33,15 @@ HIPCC_FLAGS = ['--offload-arch=' + ARCH, '-O3', '-std=c++17', '-fPIC', '-ffp-con
                # scalar kernel arguments ahead of a parameter struct arrive in registers (no load at wave start)
                '-mllvm', '-amdgpu-kernarg-preload-count=16']
 
+# The mixed-width step holds a row of eight columns in eight registers: vectorized by the compiler they become tuples that
+# have to sit side by side, and the kernel spills twice as much.
+UNIT_FLAGS = {'inst_gga_': ['-fno-slp-vectorize']}
+
+
+def _flags(src):
+    base = os.path.basename(src)
+    return HIPCC_FLAGS + [f for prefix, flags in UNIT_FLAGS.items() if base.startswith(prefix) for f in flags]
+
 
 def _cases():
     """family -> [(bits, dk, dv, group, qbuf, mmax, axv)].  Shapes: Qwen3.5 GDN 128x128, small test heads 64x64,
@@ -402,7 +411,7 @@ def _unit_hash(src, seen=None):
         text = open(path).read()
         seen[path] = text
         todo += [os.path.normpath(os.path.join(os.path.dirname(path), inc)) for inc in _INCLUDE.findall(text)]
-    h = hashlib.sha256(' '.join(HIPCC_FLAGS).encode())
+    h = hashlib.sha256(' '.join(_flags(src)).encode())
     for path in sorted(seen):
         h.update(path.encode())
         h.update(seen[path].encode())
@@ -465,7 +474,7 @@ def _compile(src, force=False):
     if not force and os.path.exists(obj) and os.path.exists(tag) and open(tag).read() == want:
         return obj
     lint = base.startswith(tuple(f'inst_{fam}q_' for fam in QUAD_FAMILIES))
-    cmd = ['hipcc', *HIPCC_FLAGS, *(['--save-temps=obj'] if lint else []), '-c', src, '-o', obj]
+    cmd = ['hipcc', *_flags(src), *(['--save-temps=obj'] if lint else []), '-c', src, '-o', obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode:
         raise RuntimeError(f'{" ".join(cmd)}\n{r.stdout}\n{r.stderr}')
@@ -554,7 +563,7 @@ def resources(pattern='', jobs=None):
     units = [u for u in generate() if not u.endswith(('dispatch.hip', 'sq_api.hip'))]
 
     def one(src):
-        cmd = ['hipcc', *HIPCC_FLAGS, '--cuda-device-only', '-Rpass-analysis=kernel-resource-usage', '-c', src,
+        cmd = ['hipcc', *_flags(src), '--cuda-device-only', '-Rpass-analysis=kernel-resource-usage', '-c', src,
                '-o', os.devnull]
         r = subprocess.run(cmd, capture_output=True, text=True)
         rows, cur = [], None

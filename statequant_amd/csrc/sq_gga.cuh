@@ -275,6 +275,16 @@ struct GgaFitLds {
 constexpr float GGA_MAGIC = 12582912.0f;               // 1.5 2^23 (even: ties go to even): adding it rounds to an integer, left
                                                        // in the low mantissa bits
 
+// The fit needs the IEEE quotients' roundings -- a code, a column's fp16 factor -- not the quotients, and products with the
+// reciprocals nearly always round alike.  With u = 2^-24: RN(1 / r), RN(1 / c) and each product add at most u, IEEE x / r
+// and (x / r) / c at most u each, so a product raised and lowered by 8 u (GGA_ABOVE, GGA_BELOW: a rounding or two less)
+// encloses the quotient with 2 u to spare.  Where both ends round to the same number that is the quotient's; where they
+// do not, the lanes' values are divided (a row step of 512 values: one in 20 at 8 bits, one in 350 at 4).  Not meant for
+// overflows: from GGA_FAST_MAX on everything is divided.  6 instructions a code instead of 9 and 8, 1.5 a value instead of
+// 4 for the column maxima: some 600 of a wavefront's 3400, 30.2 -> 27.4 us for 32 sequences x 32 heads of 128 x 128, the same
+// bits stored.  (Leaving the clamp out where no code can need it measured 29.1: another order of the compiler's.)
+constexpr float GGA_ABOVE = 1.0f + 0x1p-21f, GGA_BELOW = 1.0f - 0x1p-21f, GGA_FAST_MAX = 1e30f;
+
 // A row's factor from its mean |x| a: {r, 1 / r, w^2}.  The division and the square root are IEEE.
 __device__ __forceinline__ float4 gga_row_factor(float a, float w) {
     const float r = gga_half(sqrtf(fmaxf(a, 1e-20f) / w));
@@ -283,9 +293,9 @@ __device__ __forceinline__ float4 gga_row_factor(float a, float w) {
 
 // STEP's dual-axis fit of the thread block's tile x at width B, packed at S (reference: `_store_head` ->
 // `_fit_parts`): row factors r = half(sqrt(max(mean_j |x|, 1e-20) / w)), column factors c = half(max_i |x / r| /
-// qmax), codes, one w^2-weighted least-squares refit of c with the codes fixed, codes again.  Divisions and the
-// square root are IEEE, as in torch (quotients are exact half-integers often enough -- one 8-bit head in eight -- that
-// rounding y times a reciprocal would store other codes).  `w` = the head's row weights.
+// qmax), codes, one w^2-weighted least-squares refit of c with the codes fixed, codes again.  Codes and factors are
+// those of IEEE divisions, as in torch (quotients are exact half-integers often enough -- one 8-bit head in eight -- that
+// rounding y times a reciprocal would store other codes); the square root is IEEE.  `w` = the head's row weights.
 template <class T, int B>
 __device__ __forceinline__ void gga_fit_store(uint8_t* S, float (&x)[T::RPT][T::CT], const float* w,
                                               GgaFitLds<T>& L, const GgaThread& t) {
@@ -347,41 +357,96 @@ __device__ __forceinline__ void gga_fit_store(uint8_t* S, float (&x)[T::RPT][T::
             __syncthreads();
         }
         // ---- the columns' first factors, from the quotients y by the row factors ----
-        float cmax[1][CT], cm[1][CO];
+        // max_i (|y| / qmax) = (max_i |y|) / qmax: division is monotonic
+        auto factor = [&](float m) { return gga_half(gga_div(m, QMAX, 1.0f / QMAX)); };
+        float c[CO];
+        bool exactly;                                       // infinities among the values: every quotient by division
+        {
+            float cmax[1][CT], cm[1][CO];
 #pragma unroll
-        for (int e = 0; e < CT; ++e) cmax[0][e] = 0.0f;
+            for (int e = 0; e < CT; ++e) cmax[0][e] = 0.0f;
 #pragma unroll
-        for (int s = 0; s < RPT; ++s) {
-            const float2 f = *reinterpret_cast<const float2*>(&L.row[grp][s * 16 + t.tr]);
+            for (int s = 0; s < RPT; s += 2) {
+                const float rc0 = L.row[grp][s * 16 + t.tr].y, rc1 = L.row[grp][(s + 1) * 16 + t.tr].y;
 #pragma unroll
-            for (int e = 0; e < CT; ++e) cmax[0][e] = fmaxf(cmax[0][e], fabsf(gga_div(x[s][e], f.x, f.y)));
-            __builtin_amdgcn_sched_barrier(0);
+                for (int e = 0; e < CT; ++e)
+                    cmax[0][e] = fmaxf(fmaxf(cmax[0][e], fabsf(x[s][e] * rc0)), fabsf(x[s + 1][e] * rc1));
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            gga_col_reduce<T, 1, true>(cmax, cm);
+            bool sure = true, tame = true;
+#pragma unroll
+            for (int e = 0; e < CO; ++e) {
+                c[e] = factor(cm[0][e] * GGA_ABOVE);
+                sure = sure && c[e] == factor(cm[0][e] * GGA_BELOW);
+                tame = tame && cm[0][e] < GGA_FAST_MAX;
+            }
+            exactly = __builtin_amdgcn_ballot_w64(!tame) != 0;
+            if (__builtin_expect(exactly || __builtin_amdgcn_ballot_w64(!sure) != 0, 0)) {
+#pragma unroll
+                for (int e = 0; e < CT; ++e) cmax[0][e] = 0.0f;
+#pragma unroll
+                for (int s = 0; s < RPT; ++s) {
+                    float2 f = *reinterpret_cast<const float2*>(&L.row[grp][s * 16 + t.tr]);
+                    asm volatile("" : "+v"(f.y));
+#pragma unroll
+                    for (int e = 0; e < CT; ++e) cmax[0][e] = fmaxf(cmax[0][e], fabsf(gga_div(x[s][e], f.x, f.y)));
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                gga_col_reduce<T, 1, true>(cmax, cm);
+#pragma unroll
+                for (int e = 0; e < CO; ++e) c[e] = factor(cm[0][e]);
+            }
         }
-        gga_col_reduce<T, 1, true>(cmax, cm);
-        // what a code is formed with, per column: its factor and the reciprocal; two bits: twice the factor
-        float c[CO], k[CT], crc[CT];
+        // what a code is formed with, per column: the reciprocal of its factor, a margin up and down; two bits: twice the
+        // factor
+        float k[B == 2 ? CT : 1], above[B == 2 ? 1 : CT], below[B == 2 ? 1 : CT];
         auto against = [&]() {
             float f[CO];
+            if constexpr (B == 2) {
 #pragma unroll
-            for (int e = 0; e < CO; ++e) f[e] = B == 2 ? 2.0f * c[e] : c[e];
-            gga_col_gather<T>(f, k);
-            if constexpr (B != 2) {
+                for (int e = 0; e < CO; ++e) f[e] = 2.0f * c[e];
+                gga_col_gather<T>(f, k);
+            } else {
+                float rc[CT];
 #pragma unroll
                 for (int e = 0; e < CO; ++e) f[e] = gga_rcp_f16(c[e]);
-                gga_col_gather<T>(f, crc);
+                gga_col_gather<T>(f, rc);
+#pragma unroll
+                for (int e = 0; e < CT; ++e) {
+                    above[e] = rc[e] * GGA_ABOVE;
+                    below[e] = rc[e] * GGA_BELOW;
+                }
             }
         };
-        // rint(y / c), clamped, as GGA_MAGIC + z, of value v in a row of factors {r, 1 / r}
-        auto code = [&](float v, const float4& f, int e) {
-            return __builtin_amdgcn_fmed3f(gga_div(gga_div(v, f.x, f.y), k[e], crc[e]) + GGA_MAGIC, GGA_MAGIC - QMAX,
-                                           GGA_MAGIC + QMAX);
+        // rint(y / c), clamped, as GGA_MAGIC + z, of the row step's values in a row of factors {r, 1 / r}
+        auto codes = [&](const float (&v)[CT], const float4& f, float (&z)[CT]) {
+            float fy = f.y;
+            asm volatile("" : "+v"(fy));                    // products of an earlier pass over the tile are formed again, not kept
+            uint32_t differ = 0;
+#pragma unroll
+            for (int e = 0; e < CT; ++e) {
+                const float y = v[e] * fy;
+                const float up = __builtin_fmaf(y, above[e], GGA_MAGIC), down = __builtin_fmaf(y, below[e], GGA_MAGIC);
+                differ |= as_u32(up) ^ as_u32(down);
+                z[e] = __builtin_amdgcn_fmed3f(up, GGA_MAGIC - QMAX, GGA_MAGIC + QMAX);
+            }
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(differ != 0 || exactly) != 0, 0)) {
+                float g[CO], cc[CT], rc[CT];
+                asm volatile("" : "+v"(fy));
+#pragma unroll
+                for (int e = 0; e < CO; ++e) g[e] = gga_rcp_f16(c[e]);
+                gga_col_gather<T>(c, cc);
+                gga_col_gather<T>(g, rc);
+#pragma unroll
+                for (int e = 0; e < CT; ++e)
+                    z[e] = __builtin_amdgcn_fmed3f(gga_div(gga_div(v[e], f.x, fy), cc[e], rc[e]) + GGA_MAGIC,
+                                                   GGA_MAGIC - QMAX, GGA_MAGIC + QMAX);
+            }
         };
         // two bits: |z| is 3 where y / c >= 2, which -- rounded quotients or not -- is exactly where |x| >= r 2 c: the
         // product of two fp16 numbers is exact, and the next float below it is further off than the quotients' rounding
         auto big = [&](float v, const float4& f, int e) { return fabsf(v) >= f.x * k[e]; };
-#pragma unroll
-        for (int e = 0; e < CO; ++e)                        // max_i (|y| / qmax) = (max_i |y|) / qmax: division is monotonic
-            c[e] = gga_half(gga_div(cm[0][e], QMAX, 1.0f / QMAX));
         against();
         // ---- codes, and the least-squares column factors for them ----
         float nd[2][CT], so[2][CO];
@@ -390,18 +455,21 @@ __device__ __forceinline__ void gga_fit_store(uint8_t* S, float (&x)[T::RPT][T::
 #pragma unroll
         for (int s = 0; s < RPT; ++s) {
             const float4 f = L.row[grp][s * 16 + t.tr];
+            float z[CT];
+            if constexpr (B != 2) codes(x[s], f, z);
+            const float off = -GGA_MAGIC * f.x;             // exact, and so is r z = r (MAGIC + z) - r MAGIC
 #pragma unroll
             for (int e = 0; e < CT; ++e) {
-                float z;
+                float vv;
                 if constexpr (B == 2) {
                     const float mag = big(x[s][e], f, e) ? 3.0f : 1.0f;
-                    z = x[s][e] >= 0.0f ? mag : -mag;
+                    vv = f.x * (x[s][e] >= 0.0f ? mag : -mag);
                 } else {
-                    z = code(x[s][e], f, e) - GGA_MAGIC;
+                    vv = __builtin_fmaf(f.x, z[e], off);
                 }
-                const float vv = f.x * z;
                 nd[0][e] = __builtin_fmaf(f.z * vv, x[s][e], nd[0][e]);
                 nd[1][e] = __builtin_fmaf(f.z, vv * vv, nd[1][e]);
+                asm volatile("" : "+v"(nd[0][e]), "+v"(nd[1][e]));      // (here, not behind the last row step's branch)
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -416,6 +484,8 @@ __device__ __forceinline__ void gga_fit_store(uint8_t* S, float (&x)[T::RPT][T::
             constexpr int WB = B == 6 ? 4 : 32 / B;         // codes per word (six bits: 24 of its bits)
             constexpr int WORDS = (CT + WB - 1) / WB;
             const float4 f = L.row[grp][s * 16 + t.tr];
+            float z[CT];
+            if constexpr (B != 2) codes(x[s], f, z);
             uint64_t bits = 0;
 #pragma unroll
             for (int d = WORDS - 1; d >= 0; --d) {
@@ -429,7 +499,7 @@ __device__ __forceinline__ void gga_fit_store(uint8_t* S, float (&x)[T::RPT][T::
                         const bool b3 = big(x[s][e], f, e);
                         u = x[s][e] >= 0.0f ? (b3 ? 3u : 2u) : (b3 ? 0u : 1u);
                     } else {                                // z on top of constant bits, which add up to a constant
-                        u = as_u32(code(x[s][e], f, e));
+                        u = as_u32(z[e]);
                         magic = (magic << B) + (0x4B400000u - uint32_t(gga_qmax(B)));
                     }
                     acc = (acc << B) + u;

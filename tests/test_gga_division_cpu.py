@@ -138,3 +138,33 @@ def test_scale_is_rounded_twice_as_the_reference_does():
             assert rn16_of_f32(s32) == rn16_of_f32(rn32(x / d))         # what the kernel computes == the reference
             single += rn16_of_f32(r * rc + q) != rn16_of_f32(s32)       # one rounding of the unrounded sum instead
     assert single > 0                                                   # the fused form would differ on some of these
+
+
+def test_raised_and_lowered_products_enclose_the_quotients():
+    """The fit takes codes and column factors from products with the reciprocals where a product raised and one lowered by
+    8 x 2^-24 round alike (statequant_amd/csrc/sq_gga.cuh: GGA_ABOVE, GGA_BELOW).  That is right if the two enclose the
+    IEEE quotients: (x / r) / c against fma(x rc_r, rc_c (1 +- 2^-21), magic), max |x / r| against max |x rc_r| (1 +- 2^-21)."""
+    rng = np.random.default_rng(5)
+    above, below = 1 + Fraction(1, 2 ** 21), 1 - Fraction(1, 2 ** 21)
+    ds = fp16_divisors()
+    same = total = 0
+    for r, c in zip(rng.choice(ds[3000:], 500), rng.choice(ds[3000:], 500)):
+        r, c = fr(r), fr(c)
+        rr, rc = rn32(1 / r), rn32(1 / c)
+        up, down = rn32(rc * above), rn32(rc * below)
+        xs = [fr(np.float32(v)) for v in rng.uniform(0.01, 127.4, 4) * float(r * c)]
+        for k in (0, 1, 6, 30, 126):                                    # quotients within a few ulp of a tie
+            base = rn32(Fraction(2 * k + 1, 2) * r * c)
+            xs += [base + j * ulp_of(base) for j in (-9, -4, -1, 0, 1, 4, 9)]
+        for x in xs:
+            y = rn32(x * rr)
+            quotient = rn32(x / r)
+            assert rn32(y * below) <= quotient <= rn32(y * above)
+            z = rn32(quotient / c)
+            assert y * down <= z <= y * up
+            lo, hi = round(y * down), round(y * up)                     # ties to even, as adding the magic number
+            total += 1
+            if lo == hi:
+                same += 1
+                assert round(z) == lo
+    assert 0.3 < same / total < 0.9, (same, total)                      # both outcomes are covered
