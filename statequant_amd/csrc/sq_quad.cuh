@@ -186,7 +186,9 @@ __device__ __forceinline__ Pair pair16(float v) {
     const auto r = __builtin_amdgcn_permlane16_swap(as_u32(v), as_u32(v), false, false);
     return Pair{as_f32(r[0]), as_f32(r[1])};
 }
-// Sum / maximum over aligned blocks of N lanes, N a power of two up to 64; every lane of a block gets the result.
+// Sum / maximum over aligned blocks of N lanes, N a power of two up to 64; every lane of a block gets the result.  The
+// maximum is of numbers that are not negative (a NaN is dropped, as fmaxf drops it): their bits compare as integers, which
+// saves the quieting instruction that the compiler puts in front of both operands of an fmaxf across lanes.
 template <int N>
 __device__ __forceinline__ float lanes_sum(float v) {
     v = block_sum<(N < 16 ? N : 16)>(v);
@@ -194,11 +196,24 @@ __device__ __forceinline__ float lanes_sum(float v) {
     if constexpr (N >= 64) { const Pair p = pair32(v); v = p.lo + p.hi; }
     return v;
 }
+__device__ __forceinline__ uint32_t umax(uint32_t a, uint32_t b) { return a > b ? a : b; }
+__device__ __forceinline__ float max16(float v) {           // of lanes 16 apart, of numbers that are neither negative nor NaN
+    const auto r = __builtin_amdgcn_permlane16_swap(as_u32(v), as_u32(v), false, false);
+    return as_f32(umax(r[0], r[1]));
+}
+__device__ __forceinline__ float max32(float v) {           // 32 apart
+    const auto r = __builtin_amdgcn_permlane32_swap(as_u32(v), as_u32(v), false, false);
+    return as_f32(umax(r[0], r[1]));
+}
 template <int N>
 __device__ __forceinline__ float lanes_max(float v) {
-    v = block_max<(N < 16 ? N : 16)>(v);
-    if constexpr (N >= 32) { const Pair p = pair16(v); v = fmaxf(p.lo, p.hi); }
-    if constexpr (N >= 64) { const Pair p = pair32(v); v = fmaxf(p.lo, p.hi); }
+    v = fmaxf(v, 0.0f);
+    if constexpr (N >= 2) v = as_f32(umax(as_u32(v), as_u32(partner<0>(v))));
+    if constexpr (N >= 4) v = as_f32(umax(as_u32(v), as_u32(partner<1>(v))));
+    if constexpr (N >= 8) v = as_f32(umax(as_u32(v), as_u32(partner<2>(v))));
+    if constexpr (N >= 16) v = as_f32(umax(as_u32(v), as_u32(partner<3>(v))));
+    if constexpr (N >= 32) v = max16(v);
+    if constexpr (N >= 64) v = max32(v);
     return v;
 }
 
@@ -455,18 +470,22 @@ __device__ __forceinline__ float ubyte_fma(uint32_t w, float s, float o) {
 // S = cmul S0 + sum_i du_i (x) kx_i over the m buffer slots, four slots per matrix-core issue in slot order
 // (v_mfma_f32_16x16x4_f32, fp32), re-quantized into the block's LDS image and its scales (reference:
 // _fused_triton.py:278-394 `_fold_head`).  Half a row block at a time: lane (n, q) -- n = lane % 16 the row of the
-// half, q = lane / 16 -- owns the quarter q of row n, CL = d_k / 4 consecutive columns, as CL / 4 accumulator tiles
+// half, q = lane / 16 -- owns the quarter q of row n, CL = d_k / 4 consecutive columns, as NT = CL / 4 accumulator tiles
 // of 4 columns: the instruction leaves result rows 4 q + b of result column n in lane (n, q), and the keys are fed
-// so that result row 4 q' + b of tile ct is state column q' CL + 4 ct + b.  A lane's codes are whole 16-byte (8-byte)
-// pieces of the LDS image, a scale group lies in 1, 2 or 4 lanes of a row (lanes 16 or 32 apart), and a 128-column
-// row needs 32 accumulator registers.
+// so that result row 4 q' + b of tile ct is state column q' CL + NT b + ct -- the NT columns that a lane feeds are then
+// consecutive, one LDS read for each slot instead of NT of single bytes (int4 g64, 13 sequences out of
+// step: 7.8 -> 7.6 us per launch; 256: 27.4 -> 27.1).
+// (int8 codes with one scale per row enter the accumulators four consecutive columns at a time: q' CL + 4 ct + b.  So do
+// fp32 keys, which as 16-byte reads had the compiler spill in kernels of 80 registers.)
+// A lane's codes are whole 16-byte (8-byte) pieces of the LDS image, a scale group lies in 1, 2 or 4 lanes of a row
+// (lanes 16 or 32 apart), and a 128-column row needs 32 accumulator registers.
 //   lds_kbr / kbsf   buffered keys, raw, and their scales (slot m - 1: this token's, as stored)
 //   bop[t]           the lane's folded values: slot 4 t + q, row n (decay ratio x stored value)
 //   cmul             the decay of the old state over the buffer
 typedef float v4f __attribute__((ext_vector_type(4)));
 
 // The folded keys as the matrix core's first operand, once per wavefront (they are the same for every half block):
-// key(ct, t) = kx_{4 t + q}[column (n / 4) CL + 4 ct + n % 4] for lane (n, q); 0 for slots >= m.  Held as fp32, or --
+// key(ct, t) = kx_{4 t + q}[column NT n + ct] for lane (n, q) (RUNS; else (n / 4) CL + 4 ct + n % 4); 0 for slots >= m.  Held as fp32, or --
 // int4 states with the int8 buffer, whose kernels run at 80 registers where 16 more long-lived ones made the compiler
 // shuffle and spill -- as the raw bytes (biased to unsigned, four per register) with the slot's scale, expanded where
 // they are used: (byte - 128) x scale in one conversion and one fma, the same number as the product it replaces.
@@ -474,6 +493,10 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 template <class T, bool F32 = false>
 struct FoldKeys {
     static constexpr int MT4 = (T::MMAX + 3) / 4, DKP = pow2_ceil(T::DK), NT = DKP / 16;
+    static constexpr bool RUNS = !F32 && (T::BITS != 8 || T::NG != 1);
+    // where a lane's column c is: accumulator tile, element
+    static constexpr int tile(int c) { return RUNS ? c % NT : c / 4; }
+    static constexpr int elem(int c) { return RUNS ? c / NT : c % 4; }
     static constexpr bool PACKED = !F32 && T::BITS == 4 && T::QBUF && NT % 4 == 0;
     float f[PACKED ? 1 : NT][PACKED ? 1 : MT4];
     uint32_t raw[PACKED ? MT4 : 1][PACKED ? NT / 4 : 1];
@@ -490,23 +513,40 @@ __device__ __forceinline__ void quad_fold_keys(const uint8_t* lds_kbr, const flo
                                                FoldKeys<T>& kop) {
     constexpr int MT4 = (T::MMAX + 3) / 4, DKP = pow2_ceil(T::DK), CL = DKP / 4, NT = CL / 4;
     const int n = lane & 15, q = lane >> 4;
-    const int kcol = (n >> 2) * CL + (n & 3);
 #pragma unroll
     for (int t = 0; t < MT4; ++t) {
         const int slot = 4 * t + q;
         const int sl = slot < m ? slot : 0;
         const float ks = T::QBUF ? lds_kbsf[sl] : 1.0f;
-        if constexpr (FoldKeys<T>::PACKED) {
-#pragma unroll
-            for (int c4 = 0; c4 < NT / 4; ++c4) {
-                uint32_t w = 0;
-#pragma unroll
-                for (int b = 0; b < 4; ++b) w |= uint32_t(lds_kbr[sl * DKP + kcol + 4 * (4 * c4 + b)]) << (8 * b);
-                kop.raw[t][c4] = w ^ 0x80808080u;
+        if constexpr (FoldKeys<T>::RUNS) {
+            constexpr int NW = NT * T::BE / 4;                // words of the lane's NT keys
+            uint32_t w[NW];
+            const uint8_t* at = lds_kbr + (sl * DKP + NT * n) * T::BE;
+            if constexpr (NW == 4) {
+                const v4u x = *reinterpret_cast<const v4u*>(at);
+                w[0] = x.x; w[1] = x.y; w[2] = x.z; w[3] = x.w;
+            } else if constexpr (NW == 2) {
+                const v2u x = *reinterpret_cast<const v2u*>(at);
+                w[0] = x.x; w[1] = x.y;
+            } else {
+                static_assert(NW == 1, "4 or 8 keys of 1 or 2 bytes");
+                w[0] = *reinterpret_cast<const uint32_t*>(at);
             }
-            kop.ks[t] = slot < m ? ks : 0.0f;                 // a slot beyond m contributes nothing
-            kop.off[t] = -128.0f * kop.ks[t];
+            if constexpr (FoldKeys<T>::PACKED) {
+#pragma unroll
+                for (int c4 = 0; c4 < NW; ++c4) kop.raw[t][c4] = w[c4] ^ 0x80808080u;
+                kop.ks[t] = slot < m ? ks : 0.0f;             // a slot beyond m contributes nothing
+                kop.off[t] = -128.0f * kop.ks[t];
+            } else {
+#pragma unroll
+                for (int ct = 0; ct < NT; ++ct) {
+                    const float kv = T::QBUF ? s8_to_f(w[ct / 4], ct % 4) * ks
+                                             : as_f32(ct % 2 ? w[ct / 2] & 0xFFFF0000u : w[ct / 2] << 16);
+                    kop.f[ct][t] = slot < m ? kv : 0.0f;
+                }
+            }
         } else {
+            const int kcol = (n >> 2) * CL + (n & 3);
 #pragma unroll
             for (int ct = 0; ct < NT; ++ct) {
                 float kv = lds_raw<T::QBUF>(lds_kbr, sl * DKP + kcol + 4 * ct);
@@ -573,6 +613,9 @@ __device__ __forceinline__ void quad_fold_half(uint8_t* blk, int hf, const FoldK
     const float sm = COLVEC ? s : s * cmul;
     const float off = -128.0f * sm;
     v4f acc[NT];
+    using K = FoldKeys<T, COLVEC>;                           // the lane's column c
+    auto set = [&](int c, float v) { acc[K::tile(c)][K::elem(c)] = v; };
+    auto get = [&](int c) { return acc[K::tile(c)][K::elem(c)]; };
     // int8 with one scale group per row: the whole half block is folded in units of the row's old scale x decay
     // (S / sm = code + sum_i (du_i / sm) kx_i), so the codes need neither conversion nor multiplication on the vector
     // ALU -- they enter the accumulators through the matrix core: each byte, biased to unsigned, becomes the fp16
@@ -614,29 +657,29 @@ __device__ __forceinline__ void quad_fold_half(uint8_t* blk, int hf, const FoldK
 #pragma unroll
         for (int d = 0; d < NW32; ++d) {
             const uint32_t u = w[d] ^ 0x80808080u;
-            acc[d][0] = ubyte_fma<0>(u, sm, off); acc[d][1] = ubyte_fma<1>(u, sm, off);
-            acc[d][2] = ubyte_fma<2>(u, sm, off); acc[d][3] = ubyte_fma<3>(u, sm, off);
+            set(4 * d, ubyte_fma<0>(u, sm, off)); set(4 * d + 1, ubyte_fma<1>(u, sm, off));
+            set(4 * d + 2, ubyte_fma<2>(u, sm, off)); set(4 * d + 3, ubyte_fma<3>(u, sm, off));
         }
     } else {
         // a stored nibble is code + 8: moved to the high half of a byte it reads 16 code + 128 as an unsigned byte
 #pragma unroll
         for (int d = 0; d < NW32; ++d) {                     // word d: columns 8 d .. 8 d + 7
             const uint32_t lo = (w[d] << 4) & 0xF0F0F0F0u, hi = w[d] & 0xF0F0F0F0u;
-            acc[2 * d][0] = ubyte_fma<0>(lo, sm, off); acc[2 * d][1] = ubyte_fma<0>(hi, sm, off);
-            acc[2 * d][2] = ubyte_fma<1>(lo, sm, off); acc[2 * d][3] = ubyte_fma<1>(hi, sm, off);
-            acc[2 * d + 1][0] = ubyte_fma<2>(lo, sm, off); acc[2 * d + 1][1] = ubyte_fma<2>(hi, sm, off);
-            acc[2 * d + 1][2] = ubyte_fma<3>(lo, sm, off); acc[2 * d + 1][3] = ubyte_fma<3>(hi, sm, off);
+            set(8 * d, ubyte_fma<0>(lo, sm, off)); set(8 * d + 1, ubyte_fma<0>(hi, sm, off));
+            set(8 * d + 2, ubyte_fma<1>(lo, sm, off)); set(8 * d + 3, ubyte_fma<1>(hi, sm, off));
+            set(8 * d + 4, ubyte_fma<2>(lo, sm, off)); set(8 * d + 5, ubyte_fma<2>(hi, sm, off));
+            set(8 * d + 6, ubyte_fma<3>(lo, sm, off)); set(8 * d + 7, ubyte_fma<3>(hi, sm, off));
         }
     }
     if constexpr (COLVEC) {
 #pragma unroll
-        for (int ct = 0; ct < NT; ++ct) {
-            const float4 c = *reinterpret_cast<const float4*>(lds_cm + q * CL + 4 * ct);
-            acc[ct][0] = acc[ct][0] * c.x; acc[ct][1] = acc[ct][1] * c.y;
-            acc[ct][2] = acc[ct][2] * c.z; acc[ct][3] = acc[ct][3] * c.w;
+        for (int c4 = 0; c4 < CL; c4 += 4) {
+            const float4 c = *reinterpret_cast<const float4*>(lds_cm + q * CL + c4);
+            set(c4, get(c4) * c.x); set(c4 + 1, get(c4 + 1) * c.y);
+            set(c4 + 2, get(c4 + 2) * c.z); set(c4 + 3, get(c4 + 3) * c.w);
         }
     }
-    // the m rank-1 updates: first operand = keys (result row i = 4 q' + b <-> column q' CL + 4 ct + b), second = values
+    // the m rank-1 updates: first operand = keys (result rows <-> columns as `FoldKeys::col`), second = values
     float bv[MT4];
     {
         // units are this kernel's own device (no reference quantity): an estimate plus one Newton step is plenty
@@ -658,8 +701,8 @@ __device__ __forceinline__ void quad_fold_half(uint8_t* blk, int hf, const FoldK
         mx = fmaxf(fmaxf(mx, fabsf(acc[ct][2])), fabsf(acc[ct][3]));
     }
     if (!inside) mx = 0.0f;
-    if constexpr (LPG >= 2) { const Pair pm = pair16(mx); mx = fmaxf(pm.lo, pm.hi); }
-    if constexpr (LPG >= 4) { const Pair pm = pair32(mx); mx = fmaxf(pm.lo, pm.hi); }
+    if constexpr (LPG >= 2) mx = max16(mx);
+    if constexpr (LPG >= 4) mx = max32(mx);
     const float sc = fp16_scale(UNITS ? mx * unit : mx, T::QMAX);
     const Divisor dsc = scale_divisor(sc);                   // sc is an fp16 value: the correctly rounded reciprocal
     const float rs = UNITS ? unit * dsc.rc : dsc.rc;         // (exact mode: unit is a power of two, both stay exact)
@@ -674,7 +717,7 @@ __device__ __forceinline__ void quad_fold_half(uint8_t* blk, int hf, const FoldK
             for (int c = 0; c < CL / 16; ++c) {              // 16 columns per call
                 float a16[CPL];
 #pragma unroll
-                for (int e = 0; e < CPL; ++e) a16[e] = acc[4 * c + e / 4][e % 4];
+                for (int e = 0; e < CPL; ++e) a16[e] = get(16 * c + e);
                 const RawRow<T::BITS> r = quantize_row<T::BITS, CLAMP, EXACT>(a16, rs, ds);
                 if constexpr (T::BITS == 8) *reinterpret_cast<uint4*>(blk + (c == 0 ? at : at1)) = r.v;
                 else *reinterpret_cast<uint2*>(blk + at + 8 * c) = r.v;      // 16 columns = half a chunk
@@ -682,7 +725,7 @@ __device__ __forceinline__ void quad_fold_half(uint8_t* blk, int hf, const FoldK
         } else {
             float a16[CPL];
 #pragma unroll
-            for (int e = 0; e < CPL; ++e) a16[e] = acc[e / 4][e % 4];
+            for (int e = 0; e < CPL; ++e) a16[e] = get(e);
             const RawRow<T::BITS> r = quantize_row<T::BITS, CLAMP, EXACT>(a16, rs, ds);
             *reinterpret_cast<uint2*>(blk + at) = r.v;
         }
@@ -702,6 +745,7 @@ __device__ __forceinline__ void quad_fold_half_f(uint8_t* blk, int hf, const Fol
     constexpr int CHUNKS = CL / 8;                           // 16-byte chunks (8 columns, two tiles) per lane
     static_assert(T::DK % CL == 0, "a quarter is inside d_k or outside");
     const int n = lane & 15, q = lane >> 4;
+    using K = FoldKeys<T, COLVEC>;
     v4f acc[NT];
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) {
@@ -714,8 +758,9 @@ __device__ __forceinline__ void quad_fold_half_f(uint8_t* blk, int hf, const Fol
                 const float2 f = *reinterpret_cast<const float2*>(lds_cm + q * CL + 8 * c + 2 * d);
                 f0 = f.x; f1 = f.y;
             }
-            acc[2 * c + d / 2][2 * (d % 2)] = as_f32(w[d] << 16) * f0;
-            acc[2 * c + d / 2][2 * (d % 2) + 1] = as_f32(w[d] & 0xFFFF0000u) * f1;
+            const int e = 8 * c + 2 * d;                     // of the lane's columns
+            acc[K::tile(e)][K::elem(e)] = as_f32(w[d] << 16) * f0;
+            acc[K::tile(e + 1)][K::elem(e + 1)] = as_f32(w[d] & 0xFFFF0000u) * f1;
         }
     }
     static_for<NT>([&](auto ct) {
@@ -729,8 +774,9 @@ __device__ __forceinline__ void quad_fold_half_f(uint8_t* blk, int hf, const Fol
         v4u o;
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
-            const v4f a = acc[2 * c + d / 2];
-            o[d] = uint32_t(f32_to_bf16(a[2 * (d % 2)])) | (uint32_t(f32_to_bf16(a[2 * (d % 2) + 1])) << 16);
+            const int e = 8 * c + 2 * d;
+            o[d] = uint32_t(f32_to_bf16(acc[K::tile(e)][K::elem(e)])) |
+                   (uint32_t(f32_to_bf16(acc[K::tile(e + 1)][K::elem(e + 1)])) << 16);
         }
         *reinterpret_cast<v4u*>(blk + swz<Q>(16 * hf + n, q * CHUNKS + c)) = o;
     }
@@ -844,8 +890,7 @@ __device__ __forceinline__ void quad_fold_block_v(uint8_t* blk, KeyF&& key, cons
         float mx = 0.0f;
 #pragma unroll
         for (int e = 0; e < CPL; e += 2) mx = fmaxf(fmaxf(mx, fabsf(acc[e])), fabsf(acc[e + 1]));
-        const Pair pm = pair32(mx);
-        const float sc = fp16_scale(fmaxf(pm.lo, pm.hi), T::QMAX);
+        const float sc = fp16_scale(max32(mx), T::QMAX);
         const Divisor d = scale_divisor(sc);
         if (kb == 0) sc_out[col] = f32_to_f16(sc);
         // codes, four rows to a word: byte b of word a is row 8 a + 4 kb + b of the lane's column
