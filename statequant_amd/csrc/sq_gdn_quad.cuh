@@ -75,14 +75,13 @@ struct GdnLoads {
 // a, b and fp32 A_log, dt_bias.  SPEC = 0 reads all of it from the arguments.
 template <class T, int NB, int GH, int WPE, int SPEC>
 __global__ __launch_bounds__((Quad<T, NB, GH>::THREADS), WPE)
-void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict__ order, int per_xcd, int hv, int hv_shift,
-                     const uint8_t* codes,
-                     uint32_t codes_stride, const int32_t* counters, uint32_t counters_stride, uint32_t start_ramp,
-                     SQ_TL_PARAM const GdnParams p) {
+void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict__ order, const uint8_t* codes,
+                     const int32_t* counters, int per_xcd, int hv, int hv_shift, uint32_t codes_stride,
+                     uint32_t counters_stride, uint32_t start_ramp, SQ_TL_PARAM const GdnParams p) {
     SQ_MARK(0);                                                   // entry
     // the leading arguments (copies of fields of `p`) are what the slot index load, the fill counter and the row blocks
     // need: as separate scalar arguments they are preloaded into registers at wave launch, so those requests go out
-    // without waiting for the argument block
+    // without waiting for the argument block (14 words without a gap: as many as arrive that way)
     constexpr bool FIX = SPEC > 0, POW2 = FIX && heads_pow2(T::DK);
     const int q_dt = FIX ? int(BF16) : p.q_dt, k_dt = FIX ? int(BF16) : p.k_dt, v_dt = FIX ? int(BF16) : p.v_dt;
     const int out_dt = FIX ? int(BF16) : p.out_dt;
@@ -127,6 +126,16 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
         if (order) tid.b = order[tid.b];            // the caller's dispatch order: position -> batch row
         SQ_MARK(1);                                               // item known (the leading arguments are here)
         slot = idx ? idx[tid.b] : tid.b;
+        // what the requests below need of the argument block, in one go with the slot index (where the head counts are no
+        // powers of two the compiler fetches it piece by piece, a wait for each)
+        if constexpr (!POW2) {
+            asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.a), "s"(p.bt), "s"(p.A_log), "s"(p.dt_bias), "s"(p.s_q),
+                         "s"(p.s_k), "s"(p.s_v), "s"(p.s_a), "s"(p.s_bt), "s"(p.gqa), "s"(p.gqa_shift), "s"(p.m),
+                         "s"(p.out), "s"(p.hv));
+            asm volatile("" ::"s"(p.st.SC), "s"(p.st.KB), "s"(p.st.KBS), "s"(p.st.UB), "s"(p.st.UBS), "s"(p.st.GB),
+                         "s"(p.st.GCUR), "s"(p.st.sSC), "s"(p.st.sKB), "s"(p.st.sKBS), "s"(p.st.sUB), "s"(p.st.sUBS),
+                         "s"(p.st.sGB), "s"(p.st.sGC));
+        }
         tid.hk = (POW2 || p.gqa_shift >= 0) ? tid.h >> p.gqa_shift : tid.h / p.gqa;
     }
     const int lane = lane0;
@@ -251,6 +260,9 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
         if (w == RK) role_vector(F.xr, k_dt, 1.0f, 1);
     }
     if (wh == 0) {                                   // this head's gates and decays
+        // (opened here: the compiler would convert bf16 gates where they are requested, ahead of the row blocks, and have
+        // this wavefront wait there for one after the other)
+        asm volatile("" : "+v"(F.g0), "+v"(F.g1));
         float g, beta;
         if (gate) {
             const float x = raw_to_f(F.g0, a_dt) + raw_to_f(F.g3, dt_bias_dt);
@@ -591,11 +603,11 @@ int launch_gdn_quad(const GdnParams& p0, hipStream_t stream) {
 #ifdef SQ_TIMELINE
     const SqTimelineBuf tl = sq_timeline_buffer();
     hipLaunchKernelGGL((gdn_quad_kernel<T, NB, GH, WPE, SPEC>), dim3(grid), dim3(Quad<T, NB, GH>::THREADS),
-                       quad_lds_pad(), stream, p.idx, p.order, p.per_xcd, p.hv, p.hv_shift, p.st.S, p.st.sS, p.st.NPTR, p.st.sN, stag,
+                       quad_lds_pad(), stream, p.idx, p.order, p.st.S, p.st.NPTR, p.per_xcd, p.hv, p.hv_shift, p.st.sS, p.st.sN, stag,
                        tl.p, tl.cap, p);
 #else
     hipLaunchKernelGGL((gdn_quad_kernel<T, NB, GH, WPE, SPEC>), dim3(grid), dim3(Quad<T, NB, GH>::THREADS),
-                       quad_lds_pad(), stream, p.idx, p.order, p.per_xcd, p.hv, p.hv_shift, p.st.S, p.st.sS, p.st.NPTR, p.st.sN, stag, p);
+                       quad_lds_pad(), stream, p.idx, p.order, p.st.S, p.st.NPTR, p.per_xcd, p.hv, p.hv_shift, p.st.sS, p.st.sN, stag, p);
 #endif
     return int(hipGetLastError());
 }

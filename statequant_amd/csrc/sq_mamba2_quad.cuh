@@ -31,10 +31,9 @@ struct Mamba2Loads {
 // per launch against SPEC 0), 2: others.  SPEC = 0 reads all of it from the arguments.
 template <class T, int NB, int GH, int WPE, int SPEC>
 __global__ __launch_bounds__((Quad<T, NB, GH>::THREADS), WPE)
-void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict__ order, int per_xcd, int hv, int hv_shift,
-                     const uint8_t* codes,
-                        uint32_t codes_stride, const int32_t* counters, uint32_t counters_stride, uint32_t start_ramp,
-                        const Mamba2Params p) {
+void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict__ order, const uint8_t* codes,
+                        const int32_t* counters, int per_xcd, int hv, int hv_shift, uint32_t codes_stride,
+                        uint32_t counters_stride, uint32_t start_ramp, const Mamba2Params p) {
     constexpr bool FIX = SPEC > 0, POW2 = SPEC == 1;
     const int x_dt = FIX ? int(BF16) : p.x_dt, B_dt = FIX ? int(BF16) : p.B_dt, C_dt = FIX ? int(BF16) : p.C_dt;
     const int out_dt = FIX ? int(BF16) : p.out_dt, dt_dt = p.dt_dt, A_dt = FIX ? int(F32) : p.A_dt;
@@ -501,7 +500,7 @@ int launch_mamba2_quad(const Mamba2Params& p0, hipStream_t stream) {
     p.per_xcd = (p.per_xcd % GH == 0) ? p.per_xcd / GH : 0;          // dealing over head groups
     const uint32_t grid = uint32_t(p.rows) * uint32_t(p.hv / GH);
     hipLaunchKernelGGL((mamba2_quad_kernel<T, NB, GH, WPE, SPEC>), dim3(grid), dim3(Quad<T, NB, GH>::THREADS),
-                       quad_lds_pad(), stream, p.idx, p.order, p.per_xcd, p.hv, p.hv_shift, p.st.S, p.st.sS, p.st.NPTR, p.st.sN,
+                       quad_lds_pad(), stream, p.idx, p.order, p.st.S, p.st.NPTR, p.per_xcd, p.hv, p.hv_shift, p.st.sS, p.st.sN,
                        quad_start_ramp<Quad<T, NB, GH>, WPE>(grid, 24), p);
     return int(hipGetLastError());
 }
