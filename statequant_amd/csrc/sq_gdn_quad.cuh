@@ -242,9 +242,9 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
             xe[t] = Q::vec_live(lane) ? vec_elem<NE>(raw, dt, t) : 0.0f;
             ss = __builtin_fmaf(xe[t], xe[t], ss);
         }
-        const float nrm = sqrtf(lanes_sum<WAVE>(ss) + 1e-6f);
+        const Quotient nrm(sqrtf(lanes_sum<WAVE>(ss) + 1e-6f));
 #pragma unroll
-        for (int t = 0; t < NE; ++t) xe[t] = xe[t] / nrm * post;
+        for (int t = 0; t < NE; ++t) xe[t] = nrm.of(xe[t]) * post;
         if constexpr (NE == 1) lds_xn[v * DKP + lane] = xe[0];
         else if constexpr (NE == 2) *reinterpret_cast<float2*>(lds_xn + v * DKP + 2 * lane) = make_float2(xe[0], xe[1]);
         else *reinterpret_cast<float4*>(lds_xn + v * DKP + 4 * lane) = make_float4(xe[0], xe[1], xe[2], xe[3]);
@@ -377,13 +377,17 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
 #pragma unroll
                 for (int c = 0; c < 4; ++c) kf[c] = kf[c] * s;
             }
+            float pr[2];                             // both sums side by side, then both stores
 #pragma unroll
             for (int v = 0; v < 2; ++v) {
-                float pr = kf[0] * x[v][0];
+                pr[v] = kf[0] * x[v][0];
 #pragma unroll
-                for (int c = 1; c < 4; ++c) pr = __builtin_fmaf(kf[c], x[v][c], pr);
-                pr = lanes_sum<Q::LPS>(pr);
-                if (lane % Q::LPS == 0 && i < MM) lds_dots[v * MM + i] = pr;
+                for (int c = 1; c < 4; ++c) pr[v] = __builtin_fmaf(kf[c], x[v][c], pr[v]);
+            }
+            lanes_sum2<Q::LPS>(pr);
+            if (lane % Q::LPS == 0 && i < MM) {
+                lds_dots[i] = pr[0];
+                lds_dots[MM + i] = pr[1];
             }
         }
     }
@@ -395,6 +399,10 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
         kqp = lanes_sum<WAVE>(kqp);
         if (lane == 0) lds_gsc[0] = kqp;
     }
+    // a slot's decay times its value scale, lane i: what its coefficients need besides the dot products
+    const int li = lane < m ? lane : 0;
+    float slot_f = expf(gcur - lds_gbf[li]);
+    if constexpr (T::QBUF) slot_f = slot_f * lds_ubsf[li];
     SQ_MARK(9);                                                   // buffer dot products done
     lds_barrier();                                   // the raw keys of slot n may be overwritten from here on
     SQ_MARK(10);                                                  // second barrier passed
@@ -444,16 +452,8 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     const float kq = lds_gsc[0];
     // coefficients of the head's slots, lane i: c_x[i] = exp(gcur - G_i) (K_i . x), times the slot's value scale;
     // dead slots (i >= n) may hold anything: select, never multiply
-    const int li = lane < m ? lane : 0;
-    float cq, ck;
-    {
-        const float dec = expf(gcur - lds_gbf[li]);
-        const float dq = lds_dots[li], dk_ = lds_dots[MM + li];
-        const float us_i = T::QBUF ? lds_ubsf[li] : 1.0f;
-        const bool alive = lane < n;
-        cq = alive ? (T::QBUF ? (dec * dq) * us_i : dec * dq) : 0.0f;
-        ck = alive ? (T::QBUF ? (dec * dk_) * us_i : dec * dk_) : 0.0f;
-    }
+    const bool alive = lane < n;
+    const float cq = alive ? slot_f * lds_dots[li] : 0.0f, ck = alive ? slot_f * lds_dots[MM + li] : 0.0f;
     // every slot's value is fetched up front (one wait for all of them), dead slots then add c = 0 times a finite
     // int8 value, or are skipped (bf16 values of a dead slot may be NaNs)
     float uv[MM];

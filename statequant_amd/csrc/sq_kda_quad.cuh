@@ -166,10 +166,10 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
             xe[t] = Q::vec_live(lane) ? vec_elem<NE>(raw, dt, t) : 0.0f;
             ss = __builtin_fmaf(xe[t], xe[t], ss);
         }
-        const float nrm = sqrtf(lanes_sum<WAVE>(ss) + 1e-6f);
+        const Quotient nrm(sqrtf(lanes_sum<WAVE>(ss) + 1e-6f));
 #pragma unroll
         for (int t = 0; t < NE; ++t) {
-            xe[t] = xe[t] / nrm * post;
+            xe[t] = nrm.of(xe[t]) * post;
             const float gn = F.gc[t] + vec_elem<NE>(F.gr, g_dt, t);
             const float A = kda_exp(gn);
             xa[t] = A * xe[t];
@@ -234,13 +234,17 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
                 kf[c] = alive ? kf[c] * kda_exp(gn[c] - gi[c]) : 0.0f;
             }
             if (full && i < n) *reinterpret_cast<float4*>(lds_kd + i * DKP + c4) = make_float4(kf[0], kf[1], kf[2], kf[3]);
+            float pr[2];                             // both sums side by side, then both stores
 #pragma unroll
             for (int v = 0; v < 2; ++v) {
-                float pr = kf[0] * x[v][0];
+                pr[v] = kf[0] * x[v][0];
 #pragma unroll
-                for (int c = 1; c < 4; ++c) pr = __builtin_fmaf(kf[c], x[v][c], pr);
-                pr = lanes_sum<Q::LPS>(pr);
-                if (lane % Q::LPS == 0 && i < MM) lds_dots[v * MM + i] = pr;
+                for (int c = 1; c < 4; ++c) pr[v] = __builtin_fmaf(kf[c], x[v][c], pr[v]);
+            }
+            lanes_sum2<Q::LPS>(pr);
+            if (lane % Q::LPS == 0 && i < MM) {
+                lds_dots[i] = pr[0];
+                lds_dots[MM + i] = pr[1];
             }
         }
     }

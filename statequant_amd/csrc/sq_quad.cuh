@@ -176,6 +176,9 @@ __device__ __forceinline__ constexpr int op_colbase(int ks, int kb) {
     return T::BITS == 8 ? 32 * ks + 16 * kb : 32 * (2 * (ks / 2) + kb) + 16 * (ks % 2);
 }
 
+// The slot behind the six of the first 16-column piece, zeros (several groups: pieces of eight slots).
+constexpr int ZERO_PLANE = 6 * 16;
+
 // Both values of a lane pair 16 / 32 lanes apart, in both lanes: {lower lane's, upper lane's}.
 struct Pair { float lo, hi; };
 __device__ __forceinline__ Pair pair32(float v) {
@@ -195,6 +198,18 @@ __device__ __forceinline__ float lanes_sum(float v) {
     if constexpr (N >= 32) { const Pair p = pair16(v); v = p.lo + p.hi; }
     if constexpr (N >= 64) { const Pair p = pair32(v); v = p.lo + p.hi; }
     return v;
+}
+// Two sums at a time: a lane's cross-lane add waits two cycles for the one before it, which the other's fill.
+template <int N>
+__device__ __forceinline__ void lanes_sum2(float (&v)[2]) {
+    auto step = [&](auto lvl) {
+        const float a = partner<decltype(lvl)::value>(v[0]), b = partner<decltype(lvl)::value>(v[1]);
+        v[0] = v[0] + a;
+        v[1] = v[1] + b;
+    };
+    static_for<(N < 2 ? 0 : N < 4 ? 1 : N < 8 ? 2 : N < 16 ? 3 : 4)>(step);
+    if constexpr (N >= 32) { const Pair p = pair16(v[0]), q = pair16(v[1]); v[0] = p.lo + p.hi; v[1] = q.lo + q.hi; }
+    if constexpr (N >= 64) { const Pair p = pair32(v[0]), q = pair32(v[1]); v[0] = p.lo + p.hi; v[1] = q.lo + q.hi; }
 }
 __device__ __forceinline__ uint32_t umax(uint32_t a, uint32_t b) { return a > b ? a : b; }
 __device__ __forceinline__ float max16(float v) {           // of lanes 16 apart, of numbers that are neither negative nor NaN
@@ -253,22 +268,23 @@ __device__ __forceinline__ void quad_stage_planes(const float (&xe)[NE], int v, 
             at[32] = uint8_t(d[t] >> 16);
         }
     }
+    if (T::NG > 1 && v == 0 && lane == 0) *reinterpret_cast<uint4*>(lds_pl + ZERO_PLANE) = make_uint4(0, 0, 0, 0);
     if (e0 % T::KGROUP == 0 && (!Q::PADK || e0 < T::DK)) lds_xs[v * T::NG + e0 / T::KGROUP] = __builtin_ldexpf(1.0f, ex - 22 - (T::BITS == 4 ? 4 : 0));
 }
 
 // The digit planes as the matrix core's first operand, per k-step: lane (i, kb) carries result row i = 8 g + 4 v + d,
-// i.e. digit d of vector v -- on the k-steps whose columns belong to scale group g, zero elsewhere (and zero in the
-// unused rows), so that ONE accumulation over all k-steps leaves every group's sums in its own result rows.
+// i.e. digit d of vector v -- on the k-steps whose columns belong to scale group g, zero elsewhere (read from a slot of
+// zeros), so that ONE accumulation over all k-steps leaves every group's sums in its own result rows.  The result rows that
+// nobody reads (d = 3, no such vector or group) carry whatever their lanes read.
 template <class Q, class T, int NV>
 __device__ __forceinline__ void quad_fetch_planes(const uint8_t* lds_pl, int lane, v4i (&aop)[Q::NKS]) {
     const int i = lane & 31, kb = lane >> 5;
     const int g = i >> 3, v = (i >> 2) & 1, d = i & 3;
-    const bool used = d < 3 && g < T::NG && v < NV;
+    const int mine = (kb * Q::PLS + 3 * (v < NV ? v : 0) + (d < 3 ? d : 0)) * 16;
 #pragma unroll
     for (int ks = 0; ks < Q::NKS; ++ks) {
-        const v4i x = *reinterpret_cast<const v4i*>(lds_pl + ((ks * 2 + kb) * Q::PLS + 3 * (v < NV ? v : 0) + (d < 3 ? d : 0)) * 16);
-        const bool mine = used && (kb == 0 ? op_colbase<T>(ks, 0) : op_colbase<T>(ks, 1)) / T::KGROUP == g;
-        aop[ks] = mine ? x : v4i{0, 0, 0, 0};
+        const int group = (kb == 0 ? op_colbase<T>(ks, 0) : op_colbase<T>(ks, 1)) / T::KGROUP;
+        aop[ks] = *reinterpret_cast<const v4i*>(lds_pl + (T::NG == 1 || group == g ? ks * 2 * Q::PLS * 16 + mine : ZERO_PLANE));
     }
 }
 

@@ -211,9 +211,9 @@ __device__ __forceinline__ v4i operand(const RawRow<BITS>& r) {
     if constexpr (BITS == 8) {
         return v4i{int(r.v.x), int(r.v.y), int(r.v.z), int(r.v.w)};
     } else {
-        const uint32_t w0 = r.v.x ^ 0x88888888u, w1 = r.v.y ^ 0x88888888u;
-        return v4i{int((w0 << 4) & 0xF0F0F0F0u), int(w0 & 0xF0F0F0F0u), int((w1 << 4) & 0xF0F0F0F0u),
-                   int(w1 & 0xF0F0F0F0u)};
+        // (mask, then flip: one three-operand instruction)
+        auto high = [](uint32_t w) { return int((w & 0xF0F0F0F0u) ^ 0x80808080u); };
+        return v4i{high(r.v.x << 4), high(r.v.x), high(r.v.y << 4), high(r.v.y)};
     }
 }
 
