@@ -151,8 +151,7 @@ __global__ __launch_bounds__(WAVE) void pack_f_kernel(const PackParams p, uint32
         const float4 f = *reinterpret_cast<const float4*>(src + e);
         if constexpr (BITS == 16)
             *reinterpret_cast<uint2*>(Sh + 2 * e) =
-                make_uint2(uint32_t(f32_to_bf16(f.x)) | (uint32_t(f32_to_bf16(f.y)) << 16),
-                           uint32_t(f32_to_bf16(f.z)) | (uint32_t(f32_to_bf16(f.w)) << 16));
+                make_uint2(f32_to_bf16x2(f.x, f.y), f32_to_bf16x2(f.z, f.w));
         else
             *reinterpret_cast<float4*>(Sh + 4 * e) = f;
     }

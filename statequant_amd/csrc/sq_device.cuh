@@ -40,11 +40,13 @@ __device__ __forceinline__ float as_f32(uint32_t u) { return __builtin_bit_cast(
 __device__ __forceinline__ uint32_t as_u32(float f) { return __builtin_bit_cast(uint32_t, f); }
 
 __device__ __forceinline__ float bf16_to_f32(uint16_t h) { return as_f32(uint32_t(h) << 16); }
-__device__ __forceinline__ uint16_t f32_to_bf16(float f) {      // round to nearest even, quiet NaNs (as torch)
-    uint32_t u = as_u32(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return uint16_t((u >> 16) | 0x40u);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return uint16_t(u >> 16);
+__device__ __forceinline__ uint16_t f32_to_bf16(float f) {      // round to nearest even, quiet NaNs (as torch): one
+    return __builtin_bit_cast(uint16_t, __bf16(f));              // instruction of this machine (v_cvt_pk_bf16_f32)
+}
+__device__ __forceinline__ uint32_t f32_to_bf16x2(float lo, float hi) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){lo, hi}, b2));
 }
 __device__ __forceinline__ float f16_to_f32(uint16_t h) { return float(__builtin_bit_cast(_Float16, h)); }
 __device__ __forceinline__ uint16_t f32_to_f16(float f) { return __builtin_bit_cast(uint16_t, _Float16(f)); }
@@ -187,6 +189,14 @@ __device__ __forceinline__ float block_max(float v) {
     if constexpr (N >= 8) v = fmaxf(v, partner<2>(v));
     if constexpr (N >= 16) v = fmaxf(v, partner<3>(v));
     return v;
+}
+// acc + c x, rounded once, with the c of lane I of every 16 lanes for all of them.  (In assembly: the compiler leaves the
+// broadcast an instruction of its own.  The idle cycles in front are for a c that was written just before.)
+template <int I>
+__device__ __forceinline__ float fma_row_bcast(float c, float x, float acc) {
+    static_assert(I < 16, "a lane of a row");
+    asm("s_nop 1\n\tv_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(c), "v"(x), "n"(I));
+    return acc;
 }
 __device__ __forceinline__ float lane_bcast(float v, int lane) {
     return as_f32(uint32_t(__builtin_amdgcn_readlane(int(as_u32(v)), lane)));

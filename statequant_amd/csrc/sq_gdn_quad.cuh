@@ -399,16 +399,8 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
         kqp = lanes_sum<WAVE>(kqp);
         if (lane == 0) lds_gsc[0] = kqp;
     }
-    // a slot's decay times its value scale, lane i: what its coefficients need besides the dot products
-    const int li = lane < m ? lane : 0;
-    float slot_f = expf(gcur - lds_gbf[li]);
-    if constexpr (T::QBUF) slot_f = slot_f * lds_ubsf[li];
-    SQ_MARK(9);                                                   // buffer dot products done
-    lds_barrier();                                   // the raw keys of slot n may be overwritten from here on
-    SQ_MARK(10);                                                  // second barrier passed
-
     // ---- the buffered key of this token: the rounded k, for this workgroup's folds and (first head group of
-    //      the key head only) for the slot ----
+    //      the key head only) for the slot; whoever still reads slot n discards what it reads ----
     if (w == RX) {
         float kxe[NE], kmax = 0.0f;
 #pragma unroll
@@ -447,25 +439,35 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
         }
     }
 
+    // a slot's decay times its value scale, lane i of every 16: what its coefficients need besides the dot products
+    const int ls = lane & 15, li = ls < m ? ls : 0;
+    float slot_f = expf(gcur - lds_gbf[li]);
+    if constexpr (T::QBUF) slot_f = slot_f * lds_ubsf[li];
+    SQ_MARK(9);                                                   // buffer dot products done
+    lds_barrier();
+    SQ_MARK(10);                                                  // second barrier passed
+
     // ---- this wavefront's rows: buffer term, u, o ----
     const float beta = lds_scal[0], alpha = lds_scal[1], a = lds_scal[2], gnew = lds_scal[3];
     const float kq = lds_gsc[0];
-    // coefficients of the head's slots, lane i: c_x[i] = exp(gcur - G_i) (K_i . x), times the slot's value scale;
+    // coefficients of the head's slots, lane i of every 16: c_x[i] = exp(gcur - G_i) (K_i . x), times the slot's value scale;
     // dead slots (i >= n) may hold anything: select, never multiply
-    const bool alive = lane < n;
-    const float cq = alive ? slot_f * lds_dots[li] : 0.0f, ck = alive ? slot_f * lds_dots[MM + li] : 0.0f;
+    const bool alive = ls < n;
+    float cq = lds_dots[li], ck = lds_dots[MM + li];
     // every slot's value is fetched up front (one wait for all of them), dead slots then add c = 0 times a finite
     // int8 value, or are skipped (bf16 values of a dead slot may be NaNs)
     float uv[MM];
 #pragma unroll
-    for (int i = 0; i < MM; ++i) uv[i] = lds_raw<T::QBUF>(lds_ubr, (i < m ? i : 0) * DV + row);
+    for (int i = 0; i < MM; ++i) uv[i] = lds_raw<T::QBUF>(lds_ubr, i * DV + row);
+    asm volatile("" : "+v"(cq), "+v"(ck));           // (read with the others, not each behind a branch on `alive`)
+    cq = alive ? slot_f * cq : 0.0f;
+    ck = alive ? slot_f * ck : 0.0f;
     float accq = alpha * sq, acck = alpha * sk;
-#pragma unroll
-    for (int i = 0; i < MM; ++i) {
+    static_for<MM>([&](auto i) {
         const float u_i = T::QBUF ? uv[i] : (i < n ? uv[i] : 0.0f);
-        accq = __builtin_fmaf(u_i, lane_bcast(cq, i), accq);
-        acck = __builtin_fmaf(u_i, lane_bcast(ck, i), acck);
-    }
+        accq = fma_row_bcast<decltype(i)::value>(cq, u_i, accq);
+        acck = fma_row_bcast<decltype(i)::value>(ck, u_i, acck);
+    });
     const float vt = raw_to_f(vr, v_dt);
     const float u = beta * __builtin_fmaf(-a, acck, vt);
     const float o = __builtin_fmaf(kq, u, a * accq);
@@ -480,7 +482,7 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
             if (lane == 0) lds_red[w] = amax;
             lds_barrier();
 #pragma unroll
-            for (int ww = 0; ww < NWH; ++ww) amax = fmaxf(amax, lds_red[hl * NWH + ww]);
+            for (int ww = 0; ww < NWH; ++ww) amax = as_f32(umax(as_u32(amax), as_u32(lds_red[hl * NWH + ww])));
         }
 #ifdef SQ_TIMELINE
         asm volatile("" ::"v"(amax));

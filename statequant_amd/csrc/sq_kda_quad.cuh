@@ -324,25 +324,22 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     }
     // ---- this wavefront's rows: buffer term, u, o ----
     const float kq = lds_scal[0], beta = raw_to_f(F.beta, beta_dt);
-    float cq, ck;
-    {
-        const int li = lane < m ? lane : 0;
-        const float us_i = T::QBUF ? lds_ubsf[li] : 1.0f;
-        const float dq = lds_dots[li], dk_ = lds_dots[MM + li];
-        const bool alive = lane < n;
-        cq = alive ? (T::QBUF ? dq * us_i : dq) : 0.0f;
-        ck = alive ? (T::QBUF ? dk_ * us_i : dk_) : 0.0f;
-    }
+    const int ls = lane & 15, li = ls < m ? ls : 0;      // lane i of every 16: the coefficients of slot i
+    const float us_i = T::QBUF ? lds_ubsf[li] : 1.0f;
+    const bool alive = ls < n;
+    float cq = lds_dots[li], ck = lds_dots[MM + li];
     float uv[MM];
 #pragma unroll
-    for (int i = 0; i < MM; ++i) uv[i] = lds_raw<T::QBUF>(lds_ubr, (i < m ? i : 0) * DV + row);
+    for (int i = 0; i < MM; ++i) uv[i] = lds_raw<T::QBUF>(lds_ubr, i * DV + row);
+    asm volatile("" : "+v"(cq), "+v"(ck));               // (read with the others, not each behind a branch on `alive`)
+    cq = alive ? (T::QBUF ? cq * us_i : cq) : 0.0f;
+    ck = alive ? (T::QBUF ? ck * us_i : ck) : 0.0f;
     float accq = sq, acck = sk;
-#pragma unroll
-    for (int i = 0; i < MM; ++i) {
+    static_for<MM>([&](auto i) {
         const float u_i = T::QBUF ? uv[i] : (i < n ? uv[i] : 0.0f);
-        accq = __builtin_fmaf(u_i, lane_bcast(cq, i), accq);
-        acck = __builtin_fmaf(u_i, lane_bcast(ck, i), acck);
-    }
+        accq = fma_row_bcast<decltype(i)::value>(cq, u_i, accq);
+        acck = fma_row_bcast<decltype(i)::value>(ck, u_i, acck);
+    });
     const float u = beta * (raw_to_f(F.vr, v_dt) - acck);
     const float o = __builtin_fmaf(kq, u, accq);
     if (kb == 0) store_f(outp, out_dt, row, o);
@@ -354,7 +351,7 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
             if (lane == 0) lds_red[w] = amax;
             lds_barrier();
 #pragma unroll
-            for (int ww = 0; ww < NW; ++ww) amax = fmaxf(amax, lds_red[ww]);
+            for (int ww = 0; ww < NW; ++ww) amax = as_f32(umax(as_u32(amax), as_u32(lds_red[ww])));
         }
         us = fp16_scale(amax, 127.0f);
         if (w == RG && lane == 0) { buf.UBS[n] = f32_to_f16(us); lds_ubsf[n] = us; }

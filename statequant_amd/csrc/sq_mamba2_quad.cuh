@@ -308,10 +308,8 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
         bcp = lanes_sum<WAVE>(bcp);
         if (lane == 0) lds_gsc[0] = bcp;
     }
-    lds_barrier();                                       // the raw keys of slot n may be overwritten from here on
-
     // ---- the buffered key of this token: the rounded B, for this workgroup's folds and (first head group of the
-    //      B / C group only) for the slot ----
+    //      B / C group only) for the slot; whoever still reads slot n discards what it reads ----
     if (w == RX) {
         float kxe[NE], kmax = 0.0f;
 #pragma unroll
@@ -350,30 +348,36 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
         }
     }
 
-    // ---- this wavefront's rows: buffer term, u, y ----
-    const float dt = lds_scal[0], alpha = lds_scal[1], a = lds_scal[2], gnew = lds_scal[3], dd = lds_scal[4];
-    const float bc = lds_gsc[0];
-    // coefficients of the head's slots, lane i: c[i] = exp(gcur - G_i) (B_i . C), times the slot's value scale; dead
-    // slots (i >= n) may hold anything: select, never multiply
-    const int li = lane < m ? lane : 0;
-    float cq;
-    {
-        const float dec = expf(gcur - lds_gbf[li]);
-        const float dq = lds_dots[li];
-        const float us_i = T::QBUF ? lds_ubsf[li] : 1.0f;
-        cq = lane < n ? (T::QBUF ? (dec * dq) * us_i : dec * dq) : 0.0f;
+    // a slot's decay times its value scale, lane i of every 16: what its coefficients need besides the dot products
+    const int ls = lane & 15, li = ls < m ? ls : 0;
+    float slot_f = expf(gcur - lds_gbf[li]);
+    if constexpr (T::QBUF) slot_f = slot_f * lds_ubsf[li];
+    // this token's write, u = dt x, and its largest magnitude in the head: known ahead of the state's sums
+    const float xt = raw_to_f(vr, x_dt);
+    const float u = rlive ? lds_scal[0] * xt : 0.0f;
+    float amax = 0.0f;
+    if constexpr (T::QBUF) {
+        amax = lanes_max<WAVE>(fabsf(u));
+        if (NWH > 1 && lane == 0) lds_red[w] = amax;
     }
+    lds_barrier();
+
+    // ---- this wavefront's rows: buffer term, u, y ----
+    const float alpha = lds_scal[1], a = lds_scal[2], gnew = lds_scal[3], dd = lds_scal[4];
+    const float bc = lds_gsc[0];
+    // coefficients of the head's slots, lane i of every 16: c[i] = exp(gcur - G_i) (B_i . C), times the slot's value scale; dead
+    // slots (i >= n) may hold anything: select, never multiply
+    float cq = lds_dots[li];
     float uv[MM];
 #pragma unroll
-    for (int i = 0; i < MM; ++i) uv[i] = lds_raw<T::QBUF>(lds_ubr, (i < m ? i : 0) * DV + row);
+    for (int i = 0; i < MM; ++i) uv[i] = lds_raw<T::QBUF>(lds_ubr, i * DV + row);
+    asm volatile("" : "+v"(cq));                         // (read with the others, not behind a branch)
+    cq = ls < n ? slot_f * cq : 0.0f;
     float accq = alpha * sq;
-#pragma unroll
-    for (int i = 0; i < MM; ++i) {
+    static_for<MM>([&](auto i) {
         const float u_i = T::QBUF ? uv[i] : (i < n ? uv[i] : 0.0f);
-        accq = __builtin_fmaf(u_i, lane_bcast(cq, i), accq);
-    }
-    const float xt = raw_to_f(vr, x_dt);
-    const float u = rlive ? dt * xt : 0.0f;
+        accq = fma_row_bcast<decltype(i)::value>(cq, u_i, accq);
+    });
     float y = __builtin_fmaf(bc, u, a * accq);
     if (p.has_D) y = __builtin_fmaf(dd, xt, y);
     if (rlive && (NB == 2 || kb == 0)) store_f(outp, out_dt, row, y);
@@ -381,12 +385,9 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
     // ---- append ----
     float us = 1.0f;
     if constexpr (T::QBUF) {
-        float amax = lanes_max<WAVE>(fabsf(u));
         if constexpr (NWH > 1) {
-            if (lane == 0) lds_red[w] = amax;
-            lds_barrier();
 #pragma unroll
-            for (int ww = 0; ww < NWH; ++ww) amax = fmaxf(amax, lds_red[hl * NWH + ww]);
+            for (int ww = 0; ww < NWH; ++ww) amax = as_f32(umax(as_u32(amax), as_u32(lds_red[hl * NWH + ww])));
         }
         us = fp16_scale(amax, 127.0f);
         if (wh == 0 && lane == 0) { UBSp[n] = f32_to_f16(us); lds_ubsf[n] = us; }

@@ -791,8 +791,7 @@ __device__ __forceinline__ void quad_fold_half_f(uint8_t* blk, int hf, const Fol
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
             const int e = 8 * c + 2 * d;
-            o[d] = uint32_t(f32_to_bf16(acc[K::tile(e)][K::elem(e)])) |
-                   (uint32_t(f32_to_bf16(acc[K::tile(e + 1)][K::elem(e + 1)])) << 16);
+            o[d] = f32_to_bf16x2(acc[K::tile(e)][K::elem(e)], acc[K::tile(e + 1)][K::elem(e + 1)]);
         }
         *reinterpret_cast<v4u*>(blk + swz<Q>(16 * hf + n, q * CHUNKS + c)) = o;
     }

@@ -838,7 +838,7 @@ __device__ __forceinline__ void float_fold(const float* lds_k, const float* lds_
                 uint32_t q[4];
 #pragma unroll
                 for (int d = 0; d < 4; ++d)
-                    q[d] = uint32_t(f32_to_bf16(acc[2 * d])) | (uint32_t(f32_to_bf16(acc[2 * d + 1])) << 16);
+                    q[d] = f32_to_bf16x2(acc[2 * d], acc[2 * d + 1]);
                 o = make_uint4(q[0], q[1], q[2], q[3]);
             } else {
                 o = make_uint4(as_u32(acc[0]), as_u32(acc[1]), as_u32(acc[2]), as_u32(acc[3]));
