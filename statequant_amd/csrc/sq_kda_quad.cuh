@@ -29,7 +29,7 @@ namespace sq {
 template <class T, class Q>
 struct KdaLoads {
     uint16_t sc[T::NG];                    // scales of row lane % 32 of the block
-    uint32_t scv;                          // value-axis groups: the block's scales of columns NE lane ..
+    ColScales<T> scv;                      // value-axis groups: the block's scales of the lane's columns
     Raw4<T::QBUF> uraw[Q::UT], kraw[Q::KT];
     float4 gb[Q::KT];                      // cumulative decays beside kraw
     uint16_t kbs[Q::KT], ubs;
@@ -129,7 +129,7 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     buf.UBS = field(p.st.UBS, seq, p.st.sUBS, h * um);
     float* const GBh = field(p.st.GB, seq, p.st.sGB, h * um * DK);
     if constexpr (T::AXV) {
-        F.scv = quad_load_colscales<NE>(SCh + w * DK, vl);
+        F.scv.load(SCh + w * DK, lane);
     } else if constexpr (!T::FLT) {
 #pragma unroll
         for (int g = 0; g < NG; ++g) F.sc[g] = stream_load(SCh + uint32_t(row * NG + g));
@@ -161,6 +161,9 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     // ---- roles: q and k normalised, times A the read-out vectors of the stored state; G_n, A ----
     auto role_vector = [&](const uint32_t (&raw)[NE], int dt, float post, int v) {
         float xe[NE], xa[NE], ss = 0.0f;
+        // (opened here: both roles add the decays, and the compiler would have all wavefronts do it, and wait for them, first)
+#pragma unroll
+        for (int t = 0; t < NE; ++t) asm volatile("" : "+v"(F.gr[t]), "+v"(F.gc[t]));
 #pragma unroll
         for (int t = 0; t < NE; ++t) {
             xe[t] = Q::vec_live(lane) ? vec_elem<NE>(raw, dt, t) : 0.0f;
@@ -377,13 +380,14 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
         if constexpr (T::AXV) {
             constexpr int MT = (MM + 1) / 2;
             const int fj = lf & 31, fkb = lf >> 5;
-            auto key = [&](int sl, int col) {
+            auto key = [&](int t, int col) {
+                const int sl = 2 * t + fkb;
                 const float kv = lds_kd[(sl < m ? sl : 0) * DKP + col];
                 return sl < m ? kv : 0.0f;
             };
             auto cm = [&](int col) { return lds_cm[col]; };
             uint16_t* old = reinterpret_cast<uint16_t*>(lds_pl + w * L::PL_BYTES);      // the planes are done with
-            quad_store_colscales<NE>(old, lf, F.scv);
+            F.scv.store(old, lf);
             wave_sync();
             float dop[MT];
 #pragma unroll

@@ -18,7 +18,7 @@ namespace sq {
 template <class T, class Q>
 struct Mamba2Loads {
     uint16_t sc[Q::NB][T::NG];             // scales of rows (block bi, lane % 32)
-    uint32_t scv[Q::NB];                   // value-axis groups: the block's scales of columns NE lane ..
+    ColScales<T> scv[Q::NB];               // value-axis groups: the block's scales of the lane's columns
     Raw4<T::QBUF> uraw[Q::UT], kraw[Q::KT];
     uint16_t kbs[Q::KT], ubs;
     float gbl, gcur;
@@ -134,7 +134,7 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
 #pragma unroll
     for (int bi = 0; bi < NB; ++bi) {
         if constexpr (T::AXV) {
-            F.scv[bi] = quad_load_colscales<NE>(SCh + (wh * NB + bi) * DK, vl);
+            F.scv[bi].load(SCh + (wh * NB + bi) * DK, lane);
         } else if constexpr (!T::FLT) {
 #pragma unroll
             for (int g = 0; g < NG; ++g) F.sc[bi][g] = stream_load(SCh + uint32_t((T::RAGV ? row : (wh * NB + bi) * T::MR + n32) * NG + g));
@@ -426,18 +426,23 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
                 const int sl = 2 * t + fkb;
                 decf[t] = sl < m - 1 ? expf(gnew - lds_gbf[sl < m - 1 ? sl : 0]) : 1.0f;
             }
-            auto key = [&](int sl, int col) {
-                const int sc_ = sl < m ? sl : 0;
-                float kv = lds_raw<T::QBUF>(lds_kbr, sc_ * DKP + col);
-                if constexpr (T::QBUF) kv = kv * lds_kbsf[sc_];
-                return sl < m ? kv : 0.0f;
+            float ksf[MT];                           // ... their key scales; 0 for slots that do not exist
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                const int sl = 2 * t + fkb;
+                ksf[t] = T::QBUF && sl < m ? lds_kbsf[sl] : 0.0f;
+            }
+            auto key = [&](int t, int col) {
+                const int sl = 2 * t + fkb;
+                const float kv = lds_raw<T::QBUF>(lds_kbr, (T::QBUF || sl < m ? sl : 0) * DKP + col);
+                return T::QBUF ? kv * ksf[t] : sl < m ? kv : 0.0f;
             };
 #pragma unroll
             for (int bi = 0; bi < NB; ++bi) {
                 uint8_t* blk = my_codes + bi * Q::BLK;
                 const int grp = wh * NB + bi;
                 uint16_t* old = reinterpret_cast<uint16_t*>(lds_pl + w * L::PL_BYTES);      // the planes are done with
-                quad_store_colscales<NE>(old, lf, F.scv[bi]);
+                F.scv[bi].store(old, lf);
                 wave_sync();
                 float dop[MT];
 #pragma unroll

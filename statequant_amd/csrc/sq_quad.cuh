@@ -807,33 +807,71 @@ __device__ __forceinline__ void quad_fold_half_f(uint8_t* blk, int hf, const Fol
 // int4 1 sequence 9.9 -> 6.0, 16: 19.3 -> 10.5, 100: 32.0 -> 23.0, 256: 37.7 -> 32.3; int8 1: 9.3 -> 5.7,
 // 32: 20.8 -> 14.5, 256: 44.6 -> 38.1; Mamba2 (128 heads of 128 x 64) int4 16: 15.4 -> 13.9.
 // ---------------------------------------------------------------------------------------------------------------
-// A lane's scales of one row block: columns NE lane .. (the columns it holds of a read-out vector), NE fp16 numbers.
-template <int NE>
-__device__ __forceinline__ uint32_t quad_load_colscales(const uint16_t* sc, int lane) {
-    if constexpr (NE == 1) return stream_load(sc + lane);
-    else return stream_load(reinterpret_cast<const uint32_t*>(sc) + lane);
-}
-template <int NE>
-__device__ __forceinline__ void quad_store_colscales(uint16_t* lds_sc, int lane, uint32_t s) {
-    if constexpr (NE == 1) lds_sc[lane] = uint16_t(s);
-    else reinterpret_cast<uint32_t*>(lds_sc)[lane] = s;
+// A lane's columns of one row block: the four that share a word of the matrix operand -- int8: 4 j .. 4 j + 3, j = lane %
+// 32; int4: of every eight columns the even or the odd ones (see `operand`).  Their scales as loaded: four fp16 numbers,
+// int4: the eight of both lanes.
+template <class T>
+struct ColScales {
+    static constexpr int LANES = pow2_ceil(T::DK) / 4, LIVE = T::DK / 4;     // lanes with columns, with columns inside d_k
+    typename std::conditional<T::BITS == 4, v4u, v2u>::type w;
+    __device__ __forceinline__ static int index(int lane) { return (lane & 31) < LANES ? lane & 31 : 0; }
+    __device__ __forceinline__ static int column(int t, int lane) {          // the t-th of the lane's four
+        const int j = index(lane);
+        return T::BITS == 4 ? 8 * (j / 2) + j % 2 + 2 * t : 4 * j + t;
+    }
+    __device__ __forceinline__ void load(const uint16_t* sc, int lane) {
+        const int j = index(lane) < LIVE ? index(lane) : LIVE - 1;
+        if constexpr (T::BITS == 4) w = stream_load(reinterpret_cast<const v4u*>(sc) + j / 2);
+        else w = stream_load(reinterpret_cast<const v2u*>(sc) + j);
+    }
+    __device__ __forceinline__ float scale(int t, int lane) const {
+        if constexpr (T::BITS == 4) return f16_to_f32(uint16_t(w[t] >> (16 * (index(lane) % 2))));
+        else return f16_to_f32(uint16_t(w[t / 2] >> (16 * (t % 2))));
+    }
+    __device__ __forceinline__ void store(uint16_t* lds_sc, int lane) const {
+        if (lane >= LIVE) return;
+        if constexpr (T::BITS == 8) reinterpret_cast<v2u*>(lds_sc)[lane] = w;
+        else if (lane % 2 == 0) reinterpret_cast<v4u*>(lds_sc)[lane / 2] = w;
+    }
+};
+// Digit planes (as `quad_stage_planes`) of the read-out vectors `lds_x` [NV][DKP] times a row block's column scales, both
+// vectors at once: half a wavefront each, four columns a lane, so that a lane's digits of one plane are a word.
+template <class Q, class T, int NV>
+__device__ __forceinline__ void quad_stage_planes_v(const float* lds_x, const ColScales<T>& sc, int lane, uint8_t* lds_pl,
+                                                    float* lds_xs) {
+    using C = ColScales<T>;
+    const int j = C::index(lane), v = NV == 2 ? lane >> 5 : 0;
+    const bool mine = (C::LANES == 32 || (lane & 31) < C::LANES) && (NV == 2 || lane < 32);
+    float xe[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        xe[t] = lds_x[v * Q::DKP + C::column(t, lane)] * sc.scale(t, lane);
+        if (C::LIVE < C::LANES) xe[t] = j < C::LIVE ? xe[t] : 0.0f;
+    }
+    const float mx = fmaxf(fmaxf(fabsf(xe[0]), fabsf(xe[1])), fmaxf(fabsf(xe[2]), fabsf(xe[3])));
+    int ex = __builtin_amdgcn_frexp_expf(lanes_max<C::LANES>(mx));
+    ex = ex < -100 ? -100 : ex;
+    const float up = __builtin_ldexpf(1.0f, 22 - ex);
+    uint32_t d[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) d[t] = (as_u32(__builtin_fmaf(xe[t], up, 12582912.0f)) + 0x408080u) ^ 0x808080u;
+    const uint32_t a = __builtin_amdgcn_perm(d[1], d[0], 0x05010400u), b = __builtin_amdgcn_perm(d[3], d[2], 0x05010400u);
+    const uint32_t p = __builtin_amdgcn_perm(d[1], d[0], 0x0c0c0602u), q = __builtin_amdgcn_perm(d[3], d[2], 0x0c0c0602u);
+    if (mine) {
+        uint8_t* at = lds_pl + plane_addr<Q, T>(16 * (j / 4), 3 * v) + 4 * (j % 4);
+        *reinterpret_cast<uint32_t*>(at) = __builtin_amdgcn_perm(b, a, 0x05040100u);
+        *reinterpret_cast<uint32_t*>(at + 16) = __builtin_amdgcn_perm(b, a, 0x07060302u);
+        *reinterpret_cast<uint32_t*>(at + 32) = __builtin_amdgcn_perm(q, p, 0x05040100u);
+        if (j == 0) lds_xs[v] = __builtin_ldexpf(1.0f, ex - 22 - (T::BITS == 4 ? 4 : 0));
+    }
 }
 // The row sums of one block: the scales belong to (block, column), so they ride on the read-out vectors (x'_k = x_k
 // s_k, `lds_x` [NV][DKP] fp32) and the digit planes are rebuilt per block, in this wavefront's own plane set.  Lane
 // (n, kb) returns (S0 x_kb)[row n of the block].
 template <class Q, class T, int NV>
-__device__ __forceinline__ float quad_block_pass_v(const uint8_t* blk, const float* lds_x, uint32_t colscales,
+__device__ __forceinline__ float quad_block_pass_v(const uint8_t* blk, const float* lds_x, const ColScales<T>& sc,
                                                    uint8_t* lds_pl, float* lds_xs, int lane) {
-    constexpr int NE = Q::NE;
-    static_assert(NE <= 2, "two fp16 scales per lane");
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-        float xe[NE];
-#pragma unroll
-        for (int t = 0; t < NE; ++t)
-            xe[t] = Q::vec_live(lane) ? lds_x[v * Q::DKP + NE * lane + t] * f16_to_f32(uint16_t(colscales >> (16 * t))) : 0.0f;
-        quad_stage_planes<Q, T, NE>(xe, v, lane, lds_pl, lds_xs);
-    }
+    quad_stage_planes_v<Q, T, NV>(lds_x, sc, lane, lds_pl, lds_xs);
     wave_sync();
     v4i aop[Q::NKS];
     quad_fetch_planes<Q, T, NV>(lds_pl, lane, aop);
@@ -859,7 +897,7 @@ __device__ __forceinline__ uint32_t pack_low_bytes(uint32_t a, uint32_t b, uint3
 // The new codes go back to rows across lanes through the matrix core too and enter LDS in words: written byte by byte
 // from the column shape (16 one-byte stores per column step, each with its own address) the fold took half again as
 // long (int4, 100 sequences 27.8 -> 23.0 us per launch with this).
-//   key(slot, col)  the folded key's element as fp32 (0 for slots >= m)
+//   key(t, col)     element col of the lane's folded key, slot 2 t + kb, as fp32 (0 for slots >= m)
 //   dop[t]          the lane's folded value: slot 2 t + kb, row j of the block
 //   cm(col)         the factor on the old state's column
 //   sc_old / sc_out the block's old scales (LDS) / where the new ones go (memory), [DK]
@@ -892,7 +930,7 @@ __device__ __forceinline__ void quad_fold_block_v(uint8_t* blk, KeyF&& key, cons
         const RawRow<T::BITS> r = load_row<T::BITS>(blk + swz<Q>(j, piece * LB / 16) + (piece * LB) % 16);
         float kop[MT];
 #pragma unroll
-        for (int t = 0; t < MT; ++t) kop[t] = key(2 * t + kb, col);
+        for (int t = 0; t < MT; ++t) kop[t] = key(t, col);
         const v16i ci = __builtin_amdgcn_mfma_i32_32x32x32_i8(operand<T::BITS>(r), ident, v16i{0}, 0, 0, 0);
         // exact quotients where the old state is empty or undecayed, as in `fold_tile_v`
         const bool exact = __builtin_amdgcn_ballot_w64(frozen || so <= 1) != 0;
@@ -940,9 +978,8 @@ __device__ __forceinline__ void quad_fold_block_v(uint8_t* blk, KeyF&& key, cons
                                                               v16i{0}, 0, 0, 0);
         wave_sync();                                         // every lane has its codes of these columns
 #pragma unroll
-        for (int a = 0; a < 4; ++a) {
-            const int byte = (32 * cs + 8 * a + 4 * kb) * T::BITS / 8;
-            uint8_t* at = blk + swz<Q>(j, byte / 16) + byte % 16;
+        for (int a = 0; a < 4; ++a) {                        // columns 32 cs + 8 a + 4 kb ..: one chunk, int8: two
+            uint8_t* at = T::BITS == 8 ? blk + swz<Q>(j, 2 * cs + a / 2) + 8 * (a % 2) + 4 * kb : blk + swz<Q>(j, cs) + 4 * a + 2 * kb;
             if constexpr (T::BITS == 8)
                 *reinterpret_cast<uint32_t*>(at) = pack_low_bytes(uint32_t(co[4 * a]), uint32_t(co[4 * a + 1]),
                                                                   uint32_t(co[4 * a + 2]), uint32_t(co[4 * a + 3]));
