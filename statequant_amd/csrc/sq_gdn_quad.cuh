@@ -235,8 +235,11 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     SQ_MARK(5);                                                   // fill count here, buffer loads issued
 
     // ---- shared roles (their inputs were issued first) ----
-    auto role_vector = [&](const uint32_t (&raw)[NE], int dt, float post, int v) {
+    auto role_vector = [&](uint32_t (&raw)[NE], int dt, float post, int v) {
         float xe[NE], ss = 0.0f;
+        // (opened here, as the gates below: what both roles begin with the compiler has all wavefronts do, and wait for, first)
+#pragma unroll
+        for (int t = 0; t < NE; ++t) asm volatile("" : "+v"(raw[t]));
 #pragma unroll
         for (int t = 0; t < NE; ++t) {
             xe[t] = Q::vec_live(lane) ? vec_elem<NE>(raw, dt, t) : 0.0f;
@@ -298,12 +301,12 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
 #pragma unroll
     for (int t = 0; t < Q::UT; ++t) {
         const int i = lane / Q::LU + Q::SU * t;
-        if (i < m) store_raw4<T::QBUF>(lds_ubr + (i * DV + wh * Q::RW + 4 * (lane % Q::LU)) * T::BE, F.uraw[t]);
+        if (Q::SU * Q::UT == MM || i < MM) store_raw4<T::QBUF>(lds_ubr + (i * DV + wh * Q::RW + 4 * (lane % Q::LU)) * T::BE, F.uraw[t]);
     }
 #pragma unroll
     for (int t = 0; t < Q::KT; ++t) {
         const int i = Q::SPP * (NW * t + w) + lane / Q::LPS;
-        if (i < m) {
+        if (Q::SPP * NW * Q::KT == MM || i < MM) {
             store_raw4<T::QBUF>(lds_kbr + (i * DKP + 4 * (lane % Q::LPS)) * T::BE, F.kraw[t]);
             if (T::QBUF && lane % Q::LPS == 0) lds_kbsf[i] = f16_to_f32(F.kbs[t]);
         }
@@ -369,7 +372,7 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
 #pragma unroll
         for (int t = 0; t < Q::KT; ++t) {
             const int i = Q::SPP * (NW * t + w) + lane / Q::LPS;
-            const int ic = i < m ? i : m - 1;
+            const int ic = Q::SPP * NW * Q::KT == MM ? i : i < m ? i : m - 1;      // (a slot that does not exist: discarded)
             float kf[4];
             decode_raw4<T::QBUF>(load_raw4<T::QBUF>(lds_kbr + (ic * DKP + 4 * (lane % Q::LPS)) * T::BE), kf);
             if constexpr (T::QBUF) {
@@ -439,10 +442,9 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
         }
     }
 
-    // a slot's decay times its value scale, lane i of every 16: what its coefficients need besides the dot products
+    // a slot's decay and value scale, lane i of every 16: what its coefficients need besides the dot products
     const int ls = lane & 15, li = ls < m ? ls : 0;
-    float slot_f = expf(gcur - lds_gbf[li]);
-    if constexpr (T::QBUF) slot_f = slot_f * lds_ubsf[li];
+    const float dec_i = expf(gcur - lds_gbf[li]), us_i = T::QBUF ? lds_ubsf[li] : 1.0f;
     SQ_MARK(9);                                                   // buffer dot products done
     lds_barrier();
     SQ_MARK(10);                                                  // second barrier passed
@@ -460,8 +462,8 @@ void gdn_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
 #pragma unroll
     for (int i = 0; i < MM; ++i) uv[i] = lds_raw<T::QBUF>(lds_ubr, i * DV + row);
     asm volatile("" : "+v"(cq), "+v"(ck));           // (read with the others, not each behind a branch on `alive`)
-    cq = alive ? slot_f * cq : 0.0f;
-    ck = alive ? slot_f * ck : 0.0f;
+    cq = alive ? (T::QBUF ? (dec_i * cq) * us_i : dec_i * cq) : 0.0f;
+    ck = alive ? (T::QBUF ? (dec_i * ck) * us_i : dec_i * ck) : 0.0f;
     float accq = alpha * sq, acck = alpha * sk;
     static_for<MM>([&](auto i) {
         const float u_i = T::QBUF ? uv[i] : (i < n ? uv[i] : 0.0f);

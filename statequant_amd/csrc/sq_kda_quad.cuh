@@ -201,7 +201,7 @@ void kda_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
 #pragma unroll
     for (int t = 0; t < Q::UT; ++t) {
         const int i = lane / Q::LU + Q::SU * t;
-        if (i < m) store_raw4<T::QBUF>(lds_ubr + (i * DV + w * Q::RW + 4 * (lane % Q::LU)) * T::BE, F.uraw[t]);
+        if (Q::SU * Q::UT == MM || i < MM) store_raw4<T::QBUF>(lds_ubr + (i * DV + w * Q::RW + 4 * (lane % Q::LU)) * T::BE, F.uraw[t]);
     }
     if (w == RG && T::QBUF && lane < m) lds_ubsf[lane] = f16_to_f32(F.ubs);
     quad_dma_landed();                                             // the row blocks are in LDS

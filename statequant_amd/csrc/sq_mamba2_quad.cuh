@@ -172,8 +172,11 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
     __builtin_amdgcn_sched_barrier(0);
 
     // ---- shared roles: C (planes + fp32 copy), B (fp32 copy) ----
-    auto role_vector = [&](const uint32_t (&raw)[NE], int dt, int v) {
+    auto role_vector = [&](uint32_t (&raw)[NE], int dt, int v) {
         float xe[NE];
+        // (opened here: what both roles begin with the compiler has all wavefronts do, and wait for, first)
+#pragma unroll
+        for (int t = 0; t < NE; ++t) asm volatile("" : "+v"(raw[t]));
 #pragma unroll
         for (int t = 0; t < NE; ++t) xe[t] = Q::vec_live(lane) ? vec_elem<NE>(raw, dt, t) : 0.0f;
         if constexpr (NE == 1) lds_xn[v * DKP + lane] = xe[0];
@@ -224,12 +227,12 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
 #pragma unroll
     for (int t = 0; t < Q::UT; ++t) {
         const int i = lane / Q::LU + Q::SU * t;
-        if (i < m) store_raw4<T::QBUF>(lds_ubr + (i * DV + wh * Q::RW + ucol) * T::BE, F.uraw[t]);
+        if (Q::SU * Q::UT == MM || i < MM) store_raw4<T::QBUF>(lds_ubr + (i * DV + wh * Q::RW + ucol) * T::BE, F.uraw[t]);
     }
 #pragma unroll
     for (int t = 0; t < Q::KT; ++t) {
         const int i = Q::SPP * (NW * t + w) + lane / Q::LPS;
-        if (i < m) {
+        if (Q::SPP * NW * Q::KT == MM || i < MM) {
             store_raw4<T::QBUF>(lds_kbr + (i * DKP + 4 * (lane % Q::LPS)) * T::BE, F.kraw[t]);
             if (T::QBUF && lane % Q::LPS == 0) lds_kbsf[i] = f16_to_f32(F.kbs[t]);
         }
@@ -285,7 +288,7 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
 #pragma unroll
         for (int t = 0; t < Q::KT; ++t) {
             const int i = Q::SPP * (NW * t + w) + lane / Q::LPS;
-            const int ic = i < m ? i : m - 1;
+            const int ic = Q::SPP * NW * Q::KT == MM ? i : i < m ? i : m - 1;      // (a slot that does not exist: discarded)
             float kf[4];
             decode_raw4<T::QBUF>(load_raw4<T::QBUF>(lds_kbr + (ic * DKP + 4 * (lane % Q::LPS)) * T::BE), kf);
             if constexpr (T::QBUF) {
@@ -348,10 +351,9 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
         }
     }
 
-    // a slot's decay times its value scale, lane i of every 16: what its coefficients need besides the dot products
+    // a slot's decay and value scale, lane i of every 16: what its coefficients need besides the dot products
     const int ls = lane & 15, li = ls < m ? ls : 0;
-    float slot_f = expf(gcur - lds_gbf[li]);
-    if constexpr (T::QBUF) slot_f = slot_f * lds_ubsf[li];
+    const float dec_i = expf(gcur - lds_gbf[li]), us_i = T::QBUF ? lds_ubsf[li] : 1.0f;
     // this token's write, u = dt x, and its largest magnitude in the head: known ahead of the state's sums
     const float xt = raw_to_f(vr, x_dt);
     const float u = rlive ? lds_scal[0] * xt : 0.0f;
@@ -372,7 +374,7 @@ void mamba2_quad_kernel(const int32_t* __restrict__ idx, const int32_t* __restri
 #pragma unroll
     for (int i = 0; i < MM; ++i) uv[i] = lds_raw<T::QBUF>(lds_ubr, i * DV + row);
     asm volatile("" : "+v"(cq));                         // (read with the others, not behind a branch)
-    cq = ls < n ? slot_f * cq : 0.0f;
+    cq = ls < n ? (T::QBUF ? (dec_i * cq) * us_i : dec_i * cq) : 0.0f;
     float accq = alpha * sq;
     static_for<MM>([&](auto i) {
         const float u_i = T::QBUF ? uv[i] : (i < n ? uv[i] : 0.0f);

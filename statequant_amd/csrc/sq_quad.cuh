@@ -747,7 +747,7 @@ __device__ __forceinline__ void quad_fold_half(uint8_t* blk, int hf, const FoldK
         }
     };
     if (exact) requantize(std::true_type{}, std::true_type{});
-    else if (__builtin_amdgcn_ballot_w64(sc < 6.103515625e-05f) != 0) requantize(std::true_type{}, std::false_type{});
+    else if (__builtin_amdgcn_ballot_w64(inside && sc < 6.103515625e-05f) != 0) requantize(std::true_type{}, std::false_type{});
     else requantize(std::false_type{}, std::false_type{});
 }
 
