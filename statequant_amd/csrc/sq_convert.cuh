@@ -47,33 +47,47 @@ __device__ __forceinline__ void reset_counters(const PackParams& p, uint32_t seq
             *field(p.GCUR, seq, p.sGC, h * uint32_t(p.gcur_per_head) + e) = 0.0f;
 }
 
+// The leading arguments (copies of fields of the block; `src0` its src) are in registers when a wavefront starts, so the
+// slot index and the rows to be packed, whose addresses need nothing of a slot, are requested at once, and the argument
+// block arrives behind them.
+#define SQ_PACK_LEAD                                                                                                 \
+    const int32_t *__restrict__ idx, const float *__restrict__ src0, uint32_t s_src, uint32_t hv, uint32_t dv, uint32_t part_rows
+#define SQ_PACK_ARGS p.idx, p.src, p.s_src, uint32_t(p.hv), uint32_t(p.dv), sp.rows
 template <int BITS, int DK, int GROUP>
-__global__ __launch_bounds__(WAVE) void pack_kernel(const PackParams p, uint32_t part_rows) {
+__global__ __launch_bounds__(WAVE) void pack_kernel(SQ_PACK_LEAD, const PackParams p) {
     using T = RowTile<BITS, DK, GROUP, true>;
     const LaneId l = lane_id<T>();
-    const uint32_t b = blockIdx.x / uint32_t(p.hv), h = blockIdx.x - b * uint32_t(p.hv);
-    const int32_t slot = p.idx ? p.idx[b] : int32_t(b);
-    if (p.idx && slot <= 0) return;
-    const uint32_t seq = slot, dv = p.dv;
-    const float* src = p.src + (uint64_t(b) * p.s_src + uint64_t(h) * dv * DK);
-    uint8_t* Sh = field(p.S, seq, p.sS, h * (dv * T::ROW_BYTES));
-    uint16_t* SCh = field(p.SC, seq, p.sSC, h * (dv * T::NG));
+    const uint32_t b = blockIdx.x / hv, h = blockIdx.x - b * hv;
+    const int32_t slot = idx ? idx[b] : int32_t(b);
+    const float* src = src0 + (uint64_t(b) * s_src + uint64_t(h) * dv * DK);
+    const uint32_t r_begin = blockIdx.y * part_rows, r_end = min(dv, r_begin + part_rows);
     const bool live = l.cg < T::LPR;
     const int cc = live ? l.cg : T::LPR - 1;
+    float4 f[CPL / 4];
+    auto request = [&](uint32_t r0) {
+        const uint32_t row = r0 + l.rg;
+        const float4* s4 = reinterpret_cast<const float4*>(src + (row < dv ? row : dv - 1) * DK + cc * CPL);
+#pragma unroll
+        for (int t = 0; t < CPL / 4; ++t) f[t] = s4[t];
+    };
+    request(r_begin);                                        // (of a padding row as well: it has a row in src)
+    asm volatile("" ::: "memory");
+    if (idx && slot <= 0) return;
+    const uint32_t seq = slot;
+    uint8_t* Sh = field(p.S, seq, p.sS, h * (dv * T::ROW_BYTES));
+    uint16_t* SCh = field(p.SC, seq, p.sSC, h * (dv * T::NG));
     int gi = (l.cg * CPL) / GROUP;
     const bool has_group = gi < T::NG;
     gi = has_group ? gi : T::NG - 1;
     const bool lead = live && (l.cg % T::LPG) == 0 && has_group;
-    const uint32_t r_begin = blockIdx.y * part_rows, r_end = min(dv, r_begin + part_rows);
     for (uint32_t r0 = r_begin; r0 < r_end; r0 += T::RG) {
         const uint32_t row = r0 + l.rg;
         const bool in = row < dv;
-        const float4* s4 = reinterpret_cast<const float4*>(src + (in ? row : dv - 1) * DK + cc * CPL);
+        if (r0 != r_begin) request(r0);
         float x[CPL];
 #pragma unroll
         for (int t = 0; t < CPL / 4; ++t) {
-            const float4 f = s4[t];
-            x[4 * t] = f.x; x[4 * t + 1] = f.y; x[4 * t + 2] = f.z; x[4 * t + 3] = f.w;
+            x[4 * t] = f[t].x; x[4 * t + 1] = f[t].y; x[4 * t + 2] = f[t].z; x[4 * t + 3] = f[t].w;
         }
         float amax = 0.0f;
 #pragma unroll
@@ -93,25 +107,30 @@ __global__ __launch_bounds__(WAVE) void pack_kernel(const PackParams p, uint32_t
 // Value-axis groups of G rows (fold.py:139-146): scales [dv / G][DK].  A lane owns columns 2 lane, 2 lane + 1 and
 // walks the G rows of a group twice (absmax, then codes) with the group's 2 G values in registers.
 template <int BITS, int DK, int G>
-__global__ __launch_bounds__(WAVE) void pack_v_kernel(const PackParams p, uint32_t part_rows) {
+__global__ __launch_bounds__(WAVE) void pack_v_kernel(SQ_PACK_LEAD, const PackParams p) {
     constexpr float QMAX = float((1 << (BITS - 1)) - 1);
     constexpr int ROW_BYTES = DK * BITS / 8;
     static_assert(DK % 2 == 0 && DK <= 2 * WAVE, "two columns per lane");
     const int lane = threadIdx.x;
-    const uint32_t b = blockIdx.x / uint32_t(p.hv), h = blockIdx.x - b * uint32_t(p.hv);
-    const int32_t slot = p.idx ? p.idx[b] : int32_t(b);
-    if (p.idx && slot <= 0) return;
-    const uint32_t seq = slot, dv = p.dv;
-    const float* src = p.src + (uint64_t(b) * p.s_src + uint64_t(h) * dv * DK);
-    uint8_t* Sh = field(p.S, seq, p.sS, h * (dv * ROW_BYTES));
-    uint16_t* SCh = field(p.SC, seq, p.sSC, h * ((dv / G) * DK));
+    const uint32_t b = blockIdx.x / hv, h = blockIdx.x - b * hv;
+    const int32_t slot = idx ? idx[b] : int32_t(b);
+    const float* src = src0 + (uint64_t(b) * s_src + uint64_t(h) * dv * DK);
     const bool live = 2 * lane < DK;
     const int c0 = live ? 2 * lane : DK - 2;
     const uint32_t r_begin = blockIdx.y * part_rows, r_end = min(dv, r_begin + part_rows);
-    for (uint32_t r0 = r_begin; r0 < r_end; r0 += G) {
-        float2 x[G];
+    float2 x[G];
+    auto request = [&](uint32_t r0) {
 #pragma unroll
         for (int r = 0; r < G; ++r) x[r] = *reinterpret_cast<const float2*>(src + (r0 + r) * DK + c0);
+    };
+    request(r_begin);
+    asm volatile("" ::: "memory");
+    if (idx && slot <= 0) return;
+    const uint32_t seq = slot;
+    uint8_t* Sh = field(p.S, seq, p.sS, h * (dv * ROW_BYTES));
+    uint16_t* SCh = field(p.SC, seq, p.sSC, h * ((dv / G) * DK));
+    for (uint32_t r0 = r_begin; r0 < r_end; r0 += G) {
+        if (r0 != r_begin) request(r0);
         float a0 = 0.0f, a1 = 0.0f;
 #pragma unroll
         for (int r = 0; r < G; ++r) { a0 = fmaxf(a0, fabsf(x[r].x)); a1 = fmaxf(a1, fabsf(x[r].y)); }
@@ -137,14 +156,14 @@ __global__ __launch_bounds__(WAVE) void pack_v_kernel(const PackParams p, uint32
 
 // The unquantized state: a cast to bf16 (round to nearest even) or a copy (fp32), [dv][DK] per head.
 template <int BITS, int DK>
-__global__ __launch_bounds__(WAVE) void pack_f_kernel(const PackParams p, uint32_t part_rows) {
+__global__ __launch_bounds__(WAVE) void pack_f_kernel(SQ_PACK_LEAD, const PackParams p) {
     static_assert(DK % 4 == 0, "four columns per lane and step");
     const int lane = threadIdx.x;
-    const uint32_t b = blockIdx.x / uint32_t(p.hv), h = blockIdx.x - b * uint32_t(p.hv);
-    const int32_t slot = p.idx ? p.idx[b] : int32_t(b);
-    if (p.idx && slot <= 0) return;
-    const uint32_t seq = slot, n = p.dv * DK;
-    const float* src = p.src + (uint64_t(b) * p.s_src + uint64_t(h) * n);
+    const uint32_t b = blockIdx.x / hv, h = blockIdx.x - b * hv;
+    const int32_t slot = idx ? idx[b] : int32_t(b);
+    if (idx && slot <= 0) return;
+    const uint32_t seq = slot, n = dv * DK;
+    const float* src = src0 + (uint64_t(b) * s_src + uint64_t(h) * n);
     uint8_t* Sh = field(p.S, seq, p.sS, h * (n * (BITS / 8)));
     const uint32_t e_begin = blockIdx.y * part_rows * DK, e_end = min(n, e_begin + part_rows * DK);
     for (uint32_t e = e_begin + 4 * lane; e < e_end; e += 4 * WAVE) {
@@ -164,16 +183,18 @@ int launch_pack(const PackParams& p, hipStream_t stream) {
     const uint32_t heads = uint32_t(p.rows) * uint32_t(p.hv);
     if constexpr (BITS >= 16) {
         const RowSplit sp = split_rows(heads, p.dv, 8);
-        hipLaunchKernelGGL((pack_f_kernel<BITS, DK>), dim3(heads, sp.parts), dim3(WAVE), 0, stream, p, sp.rows);
+        hipLaunchKernelGGL((pack_f_kernel<BITS, DK>), dim3(heads, sp.parts), dim3(WAVE), 0, stream, SQ_PACK_ARGS, p);
     } else if constexpr (AXV) {
         const RowSplit sp = split_rows(heads, p.dv, GROUP);
-        hipLaunchKernelGGL((pack_v_kernel<BITS, DK, GROUP>), dim3(heads, sp.parts), dim3(WAVE), 0, stream, p, sp.rows);
+        hipLaunchKernelGGL((pack_v_kernel<BITS, DK, GROUP>), dim3(heads, sp.parts), dim3(WAVE), 0, stream, SQ_PACK_ARGS, p);
     } else {
         const RowSplit sp = split_rows(heads, p.dv, RowTile<BITS, DK, GROUP, true>::RG);
-        hipLaunchKernelGGL((pack_kernel<BITS, DK, GROUP>), dim3(heads, sp.parts), dim3(WAVE), 0, stream, p, sp.rows);
+        hipLaunchKernelGGL((pack_kernel<BITS, DK, GROUP>), dim3(heads, sp.parts), dim3(WAVE), 0, stream, SQ_PACK_ARGS, p);
     }
     return int(hipGetLastError());
 }
+#undef SQ_PACK_LEAD
+#undef SQ_PACK_ARGS
 
 // LDS (dynamic): keys x decay ratio [m][DK] fp32, values [m][rows of the part] fp32.
 // Column split of the output pass: a lane takes NCH chunks of 4 columns, chunk t = columns 4 LPR t + 4 cg .. + 3, so
@@ -184,22 +205,23 @@ int launch_pack(const PackParams& p, hipStream_t stream) {
 // that round trip behind each other and do better with the 10 to 40 registers the early rows take (one wavefront per SIMD
 // more; 256 sequences of GDN 128 x 128 int4 with 16 tokens: 212 us ahead, 194 not).
 template <int BITS, int DK, int GROUP, bool QBUF, bool KDA, bool AXV, bool AHEAD>
-__global__ __launch_bounds__(WAVE) void read_kernel(const ReadParams p, uint32_t part_rows) {
+__global__ __launch_bounds__(WAVE) void read_kernel(const int32_t* __restrict__ idx, uint32_t hv, uint32_t dv, uint32_t part_rows,
+                                                    const ReadParams p) {
     using T = RowTile<BITS, DK, GROUP, QBUF, AXV>;
     constexpr int NCH = CPL / 4;
     constexpr int CSTEP = 4 * T::LPR;                             // columns between a lane's chunks
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int m = p.m;
-    const uint32_t um = m, dv = p.dv;
+    const uint32_t um = m;
     float* lds_k = reinterpret_cast<float*>(lds);
     float* lds_u = lds_k + m * DK;
     const LaneId l = lane_id<T>();
-    const uint32_t b = blockIdx.x / uint32_t(p.hv), h = blockIdx.x - b * uint32_t(p.hv);
+    const uint32_t b = blockIdx.x / hv, h = blockIdx.x - b * hv;
+    const int32_t slot = idx ? idx[b] : int32_t(b);
     const uint32_t hk = h / uint32_t(p.gqa);
     float* out = p.out + (uint64_t(b) * p.s_out + uint64_t(h) * dv * DK);
     const uint32_t r_begin = blockIdx.y * part_rows, r_end = min(dv, r_begin + part_rows), nrows = r_end - r_begin;
-    const int32_t slot = p.idx ? p.idx[b] : int32_t(b);
-    if (p.idx && slot <= 0) {                                      // padding row: a zero state, nothing of a slot read
+    if (idx && slot <= 0) {                                        // padding row: a zero state, nothing of a slot read
         float4* o4 = reinterpret_cast<float4*>(out + r_begin * DK);
         for (uint32_t e = l.lane; e < nrows * DK / 4; e += WAVE) o4[e] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         return;
@@ -248,44 +270,77 @@ __global__ __launch_bounds__(WAVE) void read_kernel(const ReadParams p, uint32_t
             }
         }
     };
-    if constexpr (AHEAD) {
+    // a pass of the keys (slot = row group + RG x pass, 16 consecutive columns per lane) with its scale and decays, and
+    // values of the part's rows, slot-major; `last`: the slots there are
+    KPiece<QBUF> kp;
+    uint16_t kbs;
+    float gi[KDA ? CPL : 1];
+    auto request_keys = [&](int i0, int last) {
+        const int i = i0 + l.rg, ic = i < last ? i : last - 1;
+        kp = load_kpiece<T>(KB, ic, last, l);
+        kbs = QBUF ? KBS[ic] : uint16_t(0);
+#pragma unroll
+        for (int t = 0; t < (KDA ? CPL : 1); ++t) gi[t] = KDA ? GBh[ic * DK + cc * CPL + t] : GBh[ic];
+    };
+    constexpr int UA = AHEAD ? 2 : 0;                             // values of the part requested early, per lane
+    uint32_t uw[UA + 1];
+    uint16_t ubs[UA + 1];
+    auto request_value = [&](uint32_t e, uint32_t& w, uint16_t& s) {
+        const uint32_t i = e / nrows, at = i * dv + r_begin + (e - i * nrows);
+        w = QBUF ? uint32_t(UB[at]) : uint32_t(reinterpret_cast<const uint16_t*>(UB)[at]);
+        s = QBUF ? UBS[i] : uint16_t(0);
+    };
+    float gc[KDA ? CPL : 1];
+    auto request_decay = [&]() {
+#pragma unroll
+        for (int t = 0; t < (KDA ? CPL : 1); ++t) gc[t] = KDA ? gch[cc * CPL + t] : gch[0];
+    };
+    const int* const counter = field(p.st.NPTR, seq, p.st.sN, 0u);   // the first head's copy, as the reference reads it
+    int n = 0;
+    if constexpr (AHEAD) {                                        // everything before anything is used
+        n = *counter;
+        request_keys(0, m);
+        request_decay();
+#pragma unroll
+        for (int j = 0; j < UA; ++j) request_value(min(uint32_t(l.lane + j * WAVE), um * nrows - 1), uw[j], ubs[j]);
         request(r_begin);
         asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    } else {
+        n = *counter;
+        request_decay();
     }
-
-    const int n = *field(p.st.NPTR, seq, p.st.sN, 0u) & (m - 1);     // the first head's copy, as the reference reads it
-    // keys of the live slots, times their decay ratio (slot = row group + RG x pass, 16 consecutive columns per lane)
+    n &= m - 1;
+    // keys of the live slots, times their decay ratio
     for (int i0 = 0; i0 < n; i0 += T::RG) {
         const int i = i0 + l.rg;
-        const int ic = i < n ? i : n - 1;
-        const KPiece<QBUF> kp = load_kpiece<T>(KB, ic, n, l);
-        const float ks = QBUF ? f16_to_f32(KBS[ic]) : 1.0f;
+        if (!AHEAD || i0 != 0) request_keys(i0, n);
         float kb[CPL];
-        decode_kpiece<T>(kp, ks, l, kb);
+        decode_kpiece<T>(kp, QBUF ? f16_to_f32(kbs) : 1.0f, l, kb);
 #pragma unroll
-        for (int t = 0; t < CPL; ++t) {
-            const float gi = KDA ? GBh[ic * DK + cc * CPL + t] : GBh[ic];
-            const float gc = KDA ? gch[cc * CPL + t] : gch[0];
-            kb[t] = kb[t] * expf(gc - gi);
-        }
+        for (int t = 0; t < CPL; ++t) kb[t] = kb[t] * expf(gc[KDA ? t : 0] - gi[KDA ? t : 0]);
         if (i < n && live) {
             float4* d4 = reinterpret_cast<float4*>(lds_k + i * DK + l.cg * CPL);
 #pragma unroll
             for (int c = 0; c < CPL / 4; ++c) d4[c] = make_float4(kb[4 * c], kb[4 * c + 1], kb[4 * c + 2], kb[4 * c + 3]);
         }
     }
-    for (uint32_t e = l.lane; e < uint32_t(n) * nrows; e += WAVE) {
-        const uint32_t i = e / nrows, at = i * dv + r_begin + (e - i * nrows);
-        float u;
-        if constexpr (QBUF) u = float(reinterpret_cast<const int8_t*>(UB)[at]) * f16_to_f32(UBS[i]);
-        else u = bf16_to_f32(reinterpret_cast<const uint16_t*>(UB)[at]);
-        lds_u[e] = u;
+    auto stage_value = [&](uint32_t e, uint32_t w, uint16_t s) {
+        if constexpr (QBUF) lds_u[e] = float(int8_t(w)) * f16_to_f32(s);
+        else lds_u[e] = bf16_to_f32(uint16_t(w));
+    };
+#pragma unroll
+    for (int j = 0; j < UA; ++j)
+        if (l.lane + j * WAVE < uint32_t(n) * nrows) stage_value(l.lane + j * WAVE, uw[j], ubs[j]);
+    for (uint32_t e = l.lane + UA * WAVE; e < uint32_t(n) * nrows; e += WAVE) {
+        request_value(e, uw[UA], ubs[UA]);
+        stage_value(e, uw[UA], ubs[UA]);
     }
     float alpha_p[NCH][4];                                        // a_n at this lane's columns
 #pragma unroll
     for (int t = 0; t < NCH; ++t)
 #pragma unroll
-        for (int c = 0; c < 4; ++c) alpha_p[t][c] = expf(KDA ? gch[t * CSTEP + 4 * cc + c] : gch[0]);
+        for (int c = 0; c < 4; ++c) alpha_p[t][c] = expf(KDA ? gch[t * CSTEP + 4 * cc + c] : gc[0]);
     __syncthreads();
 
     for (uint32_t r0 = r_begin; r0 < r_end; r0 += RR * T::RG) {
@@ -362,9 +417,11 @@ int launch_read(const ReadParams& p, hipStream_t stream) {
     const size_t lds = size_t(p.m) * (DK + sp.rows) * sizeof(float);
     const dim3 grid(heads, sp.parts);
     if (sp.parts > 1)
-        hipLaunchKernelGGL((read_kernel<BITS, DK, GROUP, QBUF, KDA, AXV, true>), grid, dim3(WAVE), lds, stream, p, sp.rows);
+        hipLaunchKernelGGL((read_kernel<BITS, DK, GROUP, QBUF, KDA, AXV, true>), grid, dim3(WAVE), lds, stream, p.idx,
+                           uint32_t(p.hv), uint32_t(p.dv), sp.rows, p);
     else
-        hipLaunchKernelGGL((read_kernel<BITS, DK, GROUP, QBUF, KDA, AXV, false>), grid, dim3(WAVE), lds, stream, p, sp.rows);
+        hipLaunchKernelGGL((read_kernel<BITS, DK, GROUP, QBUF, KDA, AXV, false>), grid, dim3(WAVE), lds, stream, p.idx,
+                           uint32_t(p.hv), uint32_t(p.dv), sp.rows, p);
     return int(hipGetLastError());
 }
 
