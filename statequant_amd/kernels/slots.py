@@ -134,6 +134,10 @@ class SlotLayout:
     def views(self, blob):
         """uint8 [num_slots, >= nbytes] (inner stride 1, slot stride and base 16-byte aligned) ->
         {field: typed view [num_slots, *shape]} (slots.py:108-117)."""
+        if blob.is_cuda and (self._lay is not None or self._conv is not None):       # in native code
+            views = _hip.host().views(blob, self.fields, self.nbytes)
+            if views is not None:
+                return views
         assert blob.dtype == torch.uint8 and blob.dim() == 2 and blob.shape[1] >= self.nbytes, blob.shape
         assert blob.stride(1) == 1 and blob.stride(0) % _ALIGN == 0 and blob.data_ptr() % _ALIGN == 0
         n = blob.shape[0]

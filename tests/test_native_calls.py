@@ -229,3 +229,30 @@ def test_calls_out_of_the_ordinary_are_declined():
         assert h.gdn_step(*{**base, 'beta': t}.values()) is None
         return t
     torch.vmap(under_vmap)(torch.rand(2, rows, 4, device=dev))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('fmt', [(4, 'k', 32), (8, 'v', 32), None])
+def test_views_cut_natively_are_the_views_the_python_code_cuts(fmt, monkeypatch):
+    """Same geometry, dtype, memory and base, for a blob of its own, a part of one and one with wider slots; what the
+    Python code refuses stays refused."""
+    for family in ('gdn', 'kda', 'mamba2'):
+        lay = _slot_case(family, fmt, False, 3, torch.Generator(device='cuda').manual_seed(1), 'cuda')[0]
+        big = torch.zeros(9, lay.nbytes + 32, dtype=torch.uint8, device='cuda')
+        lay._layout_struct()
+        for blob in (lay.alloc(5), big, big[2:7], big[:, 16:], big[::2], lay.alloc(1)):
+            got = _hip.host().views(blob, lay.fields, lay.nbytes)
+            with monkeypatch.context() as m:
+                m.setattr(_hip, '_host', _Declines())
+                want = lay.views(blob)
+            assert list(got) == list(want) == list(lay.fields)
+            for k in want:
+                a, b = got[k], want[k]
+                assert (a.shape, a.stride(), a.dtype, a.data_ptr(), a.storage_offset()) == \
+                    (b.shape, b.stride(), b.dtype, b.data_ptr(), b.storage_offset())
+                assert (a._version, a._base.shape, a._base.dtype) == (b._version, b._base.shape, b._base.dtype)
+        for blob in (big[:, 8:], big[:, :lay.nbytes - 16], big.t(), big.view(torch.int8), big[0], lay.alloc(2, 'cpu')):
+            assert _hip.host().views(blob, lay.fields, lay.nbytes) is None
+        for blob in (big[:, 8:], big[:, :lay.nbytes - 16]):
+            with pytest.raises(AssertionError):
+                lay.views(blob)
