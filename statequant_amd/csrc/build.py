@@ -185,32 +185,33 @@ def quad_variants(fam, c):
 # Launches that satisfy this take one row block per wavefront and one head per workgroup: twice the wavefronts on up to
 # four times the compute units, so that a head's life -- which is all such a launch consists of, the fold's four half
 # blocks in sequence above all -- gets shorter.  (One block per wavefront with two heads per workgroup gains nothing:
-# the wavefronts then share the SIMDs they had.)  The dispatch order moves the line where a head's fold is the longest, on
-# value-axis states: in order the folding heads no longer end the launch, and the shorter fold is worth less.  us per
-# launch, two blocks and two heads / this, sequences out of step, 16 layers captured:
-# GDN 128 x 128 (32 heads) int8 g32 1 sequence 5.26 / 4.79, 16: 9.9 / 8.1, 56: 15.4 / 14.6, 64: 16.1 / 16.4, in order 14.4 /
-# 15.0; int4 g64 16: 9.5 / 7.8, 56: 13.7 / 13.3, 64: 14.4 / 15.1, in order 12.5 / 13.4.  Value-axis int4 16: 12.4 / 9.2, 96:
-# 23.3 / 22.2, 104: 22.4 / 22.6, in order 80: 17.2 / 16.8, 96: 18.6 / 19.0; int8 16: 12.7 / 9.3, 128: 29.7 / 28.5, 192: 36.9 /
-# 36.5, 256: 45.8 / 46.0, in order 80: 18.7 / 17.6, 96: 19.9 / 19.9, 104: 20.7 / 20.8.  96 x 192 int4 g64 (30 heads) 8: 7.9 /
-# 7.0, 24: 12.3 / 12.0, 26: 12.9 / 12.9, 28: 12.6 / 13.6.  Mamba2 128 x 64 (128 heads) int8 g128 1: 5.04 / 4.65, 5: 6.67 / 6.57, 8:
-# 8.00 / 7.91, 12: 10.0 / 10.2.  The other shapes and buffers that have two blocks or several heads in a workgroup were not
-# built this way: nothing is known about them.
+# the wavefronts then share the SIMDs they had.)  With a dispatch order the folding heads no longer end the launch, so the
+# shorter fold is worth less and the line lies earlier -- but for int4 with key-axis groups, where the launch without an
+# order has a second, nearly empty round of workgroups from 72 sequences on.  us per launch, two blocks and two heads / this,
+# sequences out of step, 16 layers captured:
+# GDN 128 x 128 (32 heads) int4 g64 32 sequences 9.93 / 8.15, 60: 12.85 / 12.37, 66: 13.65 / 13.37, 76: 14.45 / 14.47, 90: 15.4 /
+# 16.3; in order 64: 11.18 / 10.88, 80: 13.1 / 12.6, 96: 14.9 / 14.3, 104: 15.0 / 15.0, 112: 15.6 / 15.8, 128: 16.3 / 17.3; int8
+# g32 32: 11.0 / 9.6, 66: 16.2 / 15.8, 76: 17.9 / 17.2, 90: 19.5 / 18.8, in order 64: 13.7 / 13.4, 72: 14.4 / 14.5, 80: 15.0 /
+# 15.6 (g128 alike).  Value-axis int4 60: 15.5 / 13.7, 100: 20.8 / 19.4, 150: 25.7 / 25.0, 190: 29.0 / 28.7, 220: 32.4 / 33.4, in
+# order 96: 16.2 / 15.3, 128: 18.8 / 18.4, 136: 19.0 / 19.3, 160: 20.8 / 21.8; int8 130: 26.6 / 24.8, 190: 33.2 / 31.1, 250: 40.6 /
+# 39.9, in order 80: 16.3 / 15.4, 120: 20.1 / 20.1, 128: 20.4 / 21.4.  96 x 192 int4 g64 (30 heads) 16: 9.6 / 8.5, 25: 11.7 / 11.4,
+# 26: 11.8 / 11.9, 28: 11.4 / 12.4.  Mamba2 128 x 64 (128 heads) int8 g128 3: 6.0 / 5.8, 10: 8.7 / 8.2, 12: 9.66 / 9.67, 13: 9.6 /
+# 9.5; int4 g64 10: 8.2 / 7.6, 18: 10.1 / 9.8, 20: 10.0 / 10.5.  The other shapes and buffers that have two blocks or several
+# heads in a workgroup were not built this way: nothing is known about them.
 def small_when(fam, c):
     bits, dk, dv, group, qbuf, mmax, axv = c
     if bits == 16 or not qbuf or mmax > 8:
         return ''
-    return {('gdn', 128, 128, 0): 'heads < 2048', ('gdn', 128, 128, 1): f'heads < (p.order ? 3072 : {3328 if bits == 4 else 6144})',
-            ('gdn', 96, 192, 0): 'heads < 768', ('mamba2', 128, 64, 0): 'heads < 768'}.get((fam, dk, dv, axv), '')
+    return {('gdn', 128, 128, 0): f'heads < (p.order ? {3456 if bits == 4 else 2176} : {2304 if bits == 4 else 3072})',
+            ('gdn', 128, 128, 1): f'heads < (p.order ? {4224 if bits == 4 else 3968} : {6400 if bits == 4 else 8192})',
+            ('gdn', 96, 192, 0): 'heads < 768',
+            ('mamba2', 128, 64, 0): f'heads < {2432 if bits == 4 else 1696}'}.get((fam, dk, dv, axv), '')
 
 
-# Heads per launch from which the one-wavefront kernel serves these cases again.  Their workgroups waste something -- lanes
-# and LDS on the columns between 96 and 128, a half empty row block (d_v 80) -- which does not matter while a launch is
-# short of wavefronts and does once it has several rounds of them.  us per launch, workgroup / one wavefront, sequences out
-# of step, just below and above: 96 x 192 (30 heads) int4 g64 128 sequences 25.1 / 27.7, 256 40.9 / 39.2; int8 g128 27.6 /
-# 30.3, 48.1 / 46.9; int8 value-axis 31.0 / 34.6, 192 sequences 43.2 / 42.1; KDA 96 x 96 (20 heads) int4 g32 192 sequences
-# 19.7 / 21.4, 256 24.0 / 23.5; Mamba2 128 x 80 (96 heads) int4 g64 48 sequences 23.3 / 25.5, 64 24.3 / 22.0, int8 g128
-# 24.2 / 27.1, 25.5 / 24.5.  Not for int4 value-axis groups (256 sequences 49.5 / 50.6), KDA's other formats (int8 g32 256
-# sequences 25.3 / 32.2) and the bf16 state (96 x 192, 128 sequences 52.1 / 62.1; Mamba2 128 x 80, 64: 36.8 / 38.7).
+# Heads per launch from which the one-wavefront kernel serves these cases again where nothing below has a line of its own: the
+# buffers of 16 tokens or bf16, and int8 value-axis groups of 96 x 96.  Their workgroups waste something -- lanes and LDS on
+# the columns between 96 and 128, a half empty row block (d_v 80) -- which does not matter while a launch is short of
+# wavefronts and may once it has several rounds of them.
 GROUP_HEADS = 5120
 
 
@@ -225,33 +226,46 @@ def group_when(fam, c):
     when = []
     if fam == 'mamba2':
         if dv % 32 and not flt:
-            # d_state 96, int4 (96 heads): 32 sequences 15.6 / 15.9, 40: 20.2 / 19.0
-            when.append(f'heads < {3328 if (bits, dk, mmax) == (4, 96, 8) else GROUP_HEADS}')
+            # a half empty row block.  128 x 80 (96 heads) int4 g64 48 sequences 22.0 / 25.3, 100: 35.3 / 36.4, 150: 49.8 / 48.0, in
+            # order 64: 22.0 / 21.3, 80: 25.7 / 23.7; int8 g128 52: 22.9 / 26.7, 100: 37.2 / 40.3, 190: 60.9 / 66.4, in order 64: 23.2 /
+            # 23.8, 72: 26.2 / 25.8 (g32 24.0 / 25.0, 26.7 / 26.5).  d_state 96, int4 32: 15.3 / 16.6, 40: 18.2 / 18.0, 56: 23.1 / 24.3,
+            # 100: 35.7 / 33.8, in order 64: 22.3 / 19.7; int8 48: 22.4 / 24.7, 100: 36.7 / 37.3, in order 64: 23.1 / 22.1
+            lines = {(4, 128): 'heads < (p.order ? 5120 : 11520)', (8, 128): '(!p.order || heads < 6656)',
+                     (4, 96): 'heads < (p.order ? 3328 : 6144)', (8, 96): f'(!p.order || heads < {GROUP_HEADS})'}
+            plain = usual and not axv and (bits, dk) in lines
+            when.append(lines[bits, dk] if plain else f'heads < {3328 if (bits, dk, mmax) == (4, 96, 8) else GROUP_HEADS}')
         if flt and (dk, mmax) == (96, 8):                    # 64 sequences 33.7 / 34.3, 96 in order 47.3 / 43.1
             when.append('(!p.order || heads < 8192)')
     elif dk == 96 and not flt and (bits == 8 or not axv) and (fam == 'gdn' or (bits == 4 and not axv)):
-        when.append(f'heads < {GROUP_HEADS}')
+        # a quarter of the lanes and of LDS on padded columns.  96 x 192 (30 heads) int4 g64 130 sequences 26.9 / 37.0, 250: 40.0 /
+        # 50.4, in order 160: 25.1 / 29.5, 256: 36.9 / 39.0, 400: 53.7 / 54.7; int8 g128 in order 160: 29.6 / 33.0, 400: 64.1 / 73.1,
+        # value-axis 256: 45.1 / 53.7.  96 x 96 (20 heads) KDA int4 g32 in order 160: 15.4 / 19.4, 400: 29.0 / 31.6, 390: 30.9 / 38.2;
+        # GDN, three wavefronts a head, int4 g64 190: 19.5 / 21.5, 250: 23.1 / 26.1, in order 176: 15.9 / 16.3, 192: 16.9 / 16.8, 256:
+        # 20.5 / 19.4, int8 g32 in order 192: 18.2 / 19.3, 256: 21.9 / 22.0
+        if not usual or (axv and dv != 192):
+            when.append(f'heads < {GROUP_HEADS}')
+        elif fam == 'gdn' and dv == 192 and bits == 4:
+            when.append('(!p.order || heads < 12288)')
         if fam == 'gdn' and dv == 96 and not axv and mmax == 8:
-            # three wavefronts a head (20 heads, int4 g64): 160 sequences in order 16.2 / 16.9, 192: 18.5 / 17.4, bf16
-            # buffer 128: 14.7 / 15.2, 160: 17.0 / 16.0; 190, not in order, 20.6 / 21.6
-            when.append(f'(!p.order || heads < {3520 if qbuf else 2880})')
+            # (bf16 buffer 128: 14.7 / 15.2, 160: 17.0 / 16.0)
+            when.append(f'(!p.order || heads < {2880 if not qbuf else 3680 if bits == 4 else 5120})')
     elif fam == 'gdn' and flt and (dk, dv) == (96, 192) and not usual:
         # two workgroups per compute unit (30 heads, 16-token buffer): 64 sequences in order 45.9 / 58.2, 96: 64.4 / 61.3,
         # 128: 80.6 / 64.8; 130, not in order, 81.3 / 87.5
         when.append('(!p.order || heads < 2560)')
     elif fam == 'kda' and dk == 64:
-        # one or two wavefronts a head: little to deal out.  64 x 64 (32 heads) int4 g64 128 sequences in order 11.3 / 11.8,
-        # 160: 13.5 / 12.7, 16-token buffer 96: 11.6 / 12.2, 128: 13.5 / 12.8, int8 15.0 / 13.7.  64 x 32 int4 g64 1
-        # sequence 4.9 / 4.6, 8: 5.4 / 5.4, 16-token buffer 8: 6.2 / 6.2, 16: 6.9 / 7.1; bf16 state 100, not in order, 11.1 /
-        # 11.7, 128 in order 11.7 / 11.1; 16-token bf16 buffer 64: 8.5 / 9.7, 130, not in order, int8 13.2 / 13.1, value-axis
-        # 14.4 / 13.1
+        # one or two wavefronts a head: little to deal out.  64 x 64 (32 heads) int4 g64 in order 128 sequences 9.6 / 10.8, 160:
+        # 11.5 / 11.8, 256: 15.5 / 16.3, int8 g32 17.0 / 19.2; 16-token buffer int4 96: 11.6 / 12.2, 128: 13.5 / 12.8, int8 15.0 /
+        # 13.7.  64 x 32 int4 g64 1 sequence 4.9 / 4.6, 8: 5.4 / 5.4, 16-token buffer 8: 6.2 / 6.2, 16: 6.9 / 7.1; bf16 state 100,
+        # not in order, 11.1 / 11.7, 128 in order 11.7 / 11.1; 16-token bf16 buffer 64: 8.5 / 9.7, 130, not in order, int8 13.2 /
+        # 13.1, value-axis 14.4 / 13.1
         if dv == 32 and not (flt and mmax > 8):
             when.append(f'heads >= {256 if mmax <= 8 else 384}')
         if not flt and mmax > 8:
             when.append('heads < 4096' if dv == 32 and not qbuf else '(!p.order || heads < 4096)')
         elif dv == 32 and mmax <= 8 and (flt or (bits == 8 and axv)):
             when.append('(!p.order || heads < 4096)')
-        elif not flt and dv == 64:
+        elif not flt and dv == 64 and (axv or not usual):
             when.append('(!p.order || heads < 5120)')
     elif fam == 'kda' and (dk, dv, bits, group, axv) == (128, 128, 8, 32, 0) and qbuf and mmax > 8:
         # 132 registers (32 heads): 96 sequences in order 27.4 / 29.4, 128: 34.5 / 32.7; 130, not in order, 37.7 / 44.8

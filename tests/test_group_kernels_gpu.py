@@ -151,7 +151,10 @@ def test_group_kernels_that_serve_larger_launches_only(family, fmt, shape, m, bb
     ('gdn', (4, 'k', 64), (20, 20, 96, 96), 4, 8, 176), ('gdn', 'bf16', (30, 30, 96, 192), 2, 16, 88),
     ('mamba2', 'bf16', (96, 8, 96, 80), 2, 8, 88),
     # ... or from one row block per wavefront to two
-    ('gdn', (4, 'v', 32), (32, 16, 128, 128), 4, 8, 96), ('gdn', (8, 'v', 32), (32, 16, 128, 128), 8, 8, 104)])
+    ('gdn', (4, 'v', 32), (32, 16, 128, 128), 4, 8, 96), ('gdn', (8, 'v', 32), (32, 16, 128, 128), 8, 8, 104),
+    ('gdn', (4, 'v', 32), (32, 16, 128, 128), 4, 8, 136), ('gdn', (8, 'k', 32), (32, 16, 128, 128), 2, 8, 72),
+    ('gdn', (4, 'k', 64), (32, 16, 128, 128), 4, 8, 88), ('gdn', (4, 'k', 64), (20, 20, 96, 96), 4, 8, 184),
+    ('mamba2', (8, 'k', 128), (96, 8, 128, 80), 4, 8, 72), ('mamba2', (4, 'k', 64), (96, 8, 128, 80), 2, 8, 56)])
 def test_a_dispatch_order_that_changes_the_kernel(family, fmt, shape, m, bb, rows):
     """Launches of so many heads that a dispatch order moves them to the one-wavefront kernel (bounds as above)."""
     hv, hk, dk, dv = shape
@@ -195,7 +198,12 @@ def test_a_dispatch_order_that_changes_the_kernel(family, fmt, shape, m, bb, row
     ('gdn', (8, 'k', 128), (32, 8, 128, 128), 64), ('gdn', (4, 'v', 32), (32, 16, 128, 128), 96),
     ('gdn', (8, 'v', 32), (24, 24, 128, 128), 128), ('gdn', (4, 'v', 32), (32, 16, 128, 128), 104),
     ('gdn', (8, 'v', 32), (32, 16, 128, 128), 192), ('gdn', (8, 'k', 64), (30, 30, 96, 192), 26),
-    ('mamba2', (8, 'k', 128), (128, 8, 128, 64), 6), ('mamba2', (4, 'k', 32), (96, 8, 128, 64), 8)])
+    ('mamba2', (8, 'k', 128), (128, 8, 128, 64), 6), ('mamba2', (4, 'k', 32), (96, 8, 128, 64), 8),
+    ('gdn', (4, 'k', 64), (32, 16, 128, 128), 72), ('gdn', (8, 'k', 32), (32, 16, 128, 128), 96),
+    ('gdn', (4, 'v', 32), (32, 16, 128, 128), 200), ('gdn', (8, 'v', 32), (32, 16, 128, 128), 256),
+    ('mamba2', (8, 'k', 128), (128, 8, 128, 64), 14), ('mamba2', (4, 'k', 32), (128, 8, 128, 64), 19),
+    # workgroup / one-wavefront kernel again
+    ('mamba2', (4, 'k', 64), (96, 8, 128, 80), 120), ('mamba2', (4, 'k', 32), (96, 8, 96, 80), 64)])
 def test_launches_either_side_of_a_head_count_agree(family, fmt, shape, rows):
     """A launch at the number of heads where another kernel takes over, and the same launch one sequence shorter (bounds
     as above)."""
