@@ -49,7 +49,7 @@ __device__ __forceinline__ void reset_counters(const PackParams& p, uint32_t seq
 
 // The leading arguments (copies of fields of the block; `src0` its src) are in registers when a wavefront starts, so the
 // slot index and the rows to be packed, whose addresses need nothing of a slot, are requested at once, and the argument
-// block arrives behind them.
+// block arrives behind them (6 sequences as above: 4.47 -> 4.29 us per launch; 64: 43.3 -> 42.7).
 #define SQ_PACK_LEAD                                                                                                 \
     const int32_t *__restrict__ idx, const float *__restrict__ src0, uint32_t s_src, uint32_t hv, uint32_t dv, uint32_t part_rows
 #define SQ_PACK_ARGS p.idx, p.src, p.s_src, uint32_t(p.hv), uint32_t(p.dv), sp.rows
@@ -200,8 +200,10 @@ int launch_pack(const PackParams& p, hipStream_t stream) {
 // Column split of the output pass: a lane takes NCH chunks of 4 columns, chunk t = columns 4 LPR t + 4 cg .. + 3, so
 // that the LPR lanes of a row write 16 LPR consecutive bytes with every store instruction (whole 128-byte lines for
 // d_k = 128) -- with 16 consecutive columns per lane each store would scatter 16-byte pieces 64 bytes apart.
-// AHEAD: the first pass's stored rows are requested before anything that waits for the fill counter -- for launches of few
-// wavefronts, which a memory round trip less shortens (6 sequences as above: 7.0 -> 6.2 us per launch).  Full launches hide
+// AHEAD: the fill counter, the keys, the part's values, the decays and the first pass's stored rows are requested together --
+// every slot of the buffer exists, what lies beyond the live ones is left unused -- for launches of few wavefronts, which
+// every memory round trip less shortens (6 sequences as above, us per launch: 7.0, with the rows ahead of the counter 6.4, with
+// the buffer beside it 6.1; 64 sequences 35.3 -> 34.5 with the latter).  Full launches hide
 // that round trip behind each other and do better with the 10 to 40 registers the early rows take (one wavefront per SIMD
 // more; 256 sequences of GDN 128 x 128 int4 with 16 tokens: 212 us ahead, 194 not).
 template <int BITS, int DK, int GROUP, bool QBUF, bool KDA, bool AXV, bool AHEAD>
