@@ -8,7 +8,8 @@ kernels' ``x / scale``), checked in exact rational arithmetic on the CPU: with f
     an IEEE division (torch's, the reference's ``div_rn``) returns -- also for x chosen to sit next to the rounding
     ties of the code grid, and for the divisors 3, 7, 31, 127 (qmax).
 
-So the kernel's codes are those of true divisions, which the GPU tests can only show statistically.
+So the kernel's codes are those of true divisions, which the GPU tests can only show statistically.  (The workgroup
+kernels' l2 norm, ``Quotient``, divides by numbers of 24 bits: there the quotient is the IEEE one but for rare last bits.)
 """
 from fractions import Fraction
 
@@ -168,3 +169,30 @@ def test_raised_and_lowered_products_enclose_the_quotients():
                 same += 1
                 assert round(z) == lo
     assert 0.3 < same / total < 0.9, (same, total)                      # both outcomes are covered
+
+
+def test_quotients_by_a_norm_are_within_a_last_bit_of_the_ieee_ones():
+    """``Quotient`` (the l2 norm of q and k in the workgroup kernels): the same steps for a divisor of 24 bits, whose
+    reciprocal may come out an ulp off from an estimate within one.  The quotient is then the IEEE one or its neighbour:
+    the remainder x - q d is exact, and r rc corrects q to within 2^-23 of an ulp before the one rounding."""
+    rng = np.random.default_rng(9)
+    off = total = 0
+    for _ in range(1200):
+        v = rng.standard_normal(8) * 10.0 ** rng.uniform(-3, 3)
+        x16 = (v.astype(np.float32).view(np.uint32) & 0xFFFF0000).view(np.float32)             # bf16 numbers
+        d = fr(np.float32(np.sqrt(np.float32((x16.astype(np.float64) ** 2).sum() * rng.uniform(1, 16) + 1e-6))))
+        near = rn32(1 / d)
+        u = ulp_of(near)
+        for r0 in (near - u, near, near + u):
+            rc = fma32(fma32(-d, r0, Fraction(1)), r0, r0)
+            assert abs(rc - near) <= u
+            for x in x16:
+                x = fr(x)
+                if x == 0:
+                    continue
+                q = rn32(x * rc)
+                got, want = fma32(fma32(-q, d, x), rc, q), rn32(x / d)
+                assert abs(got - want) <= ulp_of(want)
+                off += got != want
+                total += 1
+    assert total > 25000 and off <= 3, (off, total)

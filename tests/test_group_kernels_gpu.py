@@ -310,3 +310,35 @@ def test_serving_case_instances_leave_the_bytes_of_the_general_one(family, fmt, 
             finally:
                 _hip.select_instances()
         assert torch.equal(outs[0], outs[1]) and torch.equal(blobs[0], blobs[1]), step
+
+
+@pytest.mark.parametrize('huge', ['q', 'k'])
+@pytest.mark.parametrize('family,fmt,shape', [('gdn', (8, 'k', 128), (2, 2, 128, 128)), ('gdn', (4, 'v', 32), (4, 2, 64, 64)),
+                                              ('gdn', 'bf16', (2, 1, 96, 96)), ('kda', (4, 'k', 32), (2, 2, 128, 128))])
+def test_a_norm_that_overflows_leaves_a_vector_of_zeros(family, fmt, shape, huge):
+    """q or k whose sum of squares is an infinity in fp32: divided by it, its finite entries are 0, in both kinds."""
+    hv, hk, dk, dv = shape
+    lay = _layout(family, fmt, shape, 8, 8)
+    gen = torch.Generator().manual_seed(11)
+    idx = torch.tensor([2, 1], dtype=torch.int32, device=DEV)
+    blob = lay.alloc(3, DEV)
+    lay.write(lay.views(blob), idx, torch.randn(2, hv, dv, dk, generator=gen).to(DEV))
+    t = _token(family, gen, 2, shape)
+    big = torch.randn(hk, dk, generator=gen).to(DEV) * 1e37
+    big[0, 0] = 3e38
+    t[huge][1] = big
+    twin, outs = blob.clone(), []
+    for group in (True, False):
+        out = torch.full((2, hv, dv), 3.0, device=DEV)
+        V = lay.views(blob if group else twin)
+        _hip.select_instances(no_group_kernel=not group)
+        try:
+            _step(family, lay, V, idx, t, out, None)
+        finally:
+            _hip.select_instances()
+        if huge == 'q':
+            assert (out[1] == 0).all() and (out[0] != 0).any()
+        else:
+            assert (V['KB'][1, :, 0] == 0).all()                     # the key of the row's slot, as buffered
+        outs.append(out)
+    assert (outs[0] - outs[1]).abs().max() <= 1e-5 * outs[1].abs().max()
