@@ -152,7 +152,7 @@ typedef struct sq_mamba2_args {
  * src [rows, hv, dv, dk] value-major fp32, row stride s_src in elements; codes / scales as in sq_state.
  * Uses lay.bits, axis_k, group, hv, dk, dv.  GCUR / NPTR may be NULL (left alone); nptr_copies = counter copies per sequence that are zeroed (the slot
  * layout keeps max(hv, 4), slots.py:13-15; 0 means hv); gcur_per_head = 1 (GDN, Mamba2)
- * or dk (KDA).  Rows with idx[b] <= 0 are skipped (src has a row for them all the same). */
+ * or dk (KDA).  Rows with idx[b] <= 0 are skipped: src is not read there. */
 typedef struct sq_pack_args {
     sq_layout lay;
     int32_t rows;

@@ -48,8 +48,9 @@ __device__ __forceinline__ void reset_counters(const PackParams& p, uint32_t seq
 }
 
 // The leading arguments (copies of fields of the block; `src0` its src) are in registers when a wavefront starts, so the
-// slot index and the rows to be packed, whose addresses need nothing of a slot, are requested at once, and the argument
-// block arrives behind them (6 sequences as above: 4.47 -> 4.29 us per launch; 64: 43.3 -> 42.7).
+// slot index and, behind it, the rows to be packed are requested ahead of the argument block (6 sequences as above: 4.47 ->
+// 4.29 us per launch; 64: 43.3 -> 42.7).  Not ahead of the slot index, though the rows' addresses need nothing of a slot: a
+// padding row is skipped and need not have a row in src.
 #define SQ_PACK_LEAD                                                                                                 \
     const int32_t *__restrict__ idx, const float *__restrict__ src0, uint32_t s_src, uint32_t hv, uint32_t dv, uint32_t part_rows
 #define SQ_PACK_ARGS p.idx, p.src, p.s_src, uint32_t(p.hv), uint32_t(p.dv), sp.rows
@@ -70,9 +71,9 @@ __global__ __launch_bounds__(WAVE) void pack_kernel(SQ_PACK_LEAD, const PackPara
 #pragma unroll
         for (int t = 0; t < CPL / 4; ++t) f[t] = s4[t];
     };
-    request(r_begin);                                        // (of a padding row as well: it has a row in src)
-    asm volatile("" ::: "memory");
     if (idx && slot <= 0) return;
+    request(r_begin);
+    asm volatile("" ::: "memory");
     const uint32_t seq = slot;
     uint8_t* Sh = field(p.S, seq, p.sS, h * (dv * T::ROW_BYTES));
     uint16_t* SCh = field(p.SC, seq, p.sSC, h * (dv * T::NG));
@@ -123,9 +124,9 @@ __global__ __launch_bounds__(WAVE) void pack_v_kernel(SQ_PACK_LEAD, const PackPa
 #pragma unroll
         for (int r = 0; r < G; ++r) x[r] = *reinterpret_cast<const float2*>(src + (r0 + r) * DK + c0);
     };
+    if (idx && slot <= 0) return;
     request(r_begin);
     asm volatile("" ::: "memory");
-    if (idx && slot <= 0) return;
     const uint32_t seq = slot;
     uint8_t* Sh = field(p.S, seq, p.sS, h * (dv * ROW_BYTES));
     uint16_t* SCh = field(p.SC, seq, p.sSC, h * ((dv / G) * DK));

@@ -443,3 +443,35 @@ int main() {
     want = [f'{fam} {stride} {base} {int(stride == 0 and base == 0)}'
             for fam in ('gdn', 'kda', 'mamba2') for stride in (0, 8) for base in (0, 8)] + ['operand 0 0 0']
     assert got == want, got
+
+
+def _loads_behind_the_skip(body):
+    """Whether a pack kernel's assembly branches on the slot index (`s_cmp_lt_i32 .., 1`, a conditional branch) before its
+    first vector load."""
+    first = re.search(r'^\s(?:global|buffer|flat)_load', body, re.M)
+    assert first, body[:500]
+    return bool(re.search(r's_cmp_lt_i32 s\d+, 1\n(?:.*\n)*?\ts_cbranch', body[:first.start()]))
+
+
+def test_pack_kernels_read_no_row_of_a_padding_row(tmp_path):
+    """``sq_pack_vk`` skips rows with idx[b] <= 0, which need not have a row in src: in the compiled kernels the branch on the
+    slot index comes before the first request for rows.  (Read from the device assembly: a row that is not there is no
+    test case for a GPU.)"""
+    import shutil
+    import subprocess
+    from statequant_amd.csrc import build
+    if not shutil.which('hipcc'):
+        pytest.skip('no hipcc')
+    src, asm = tmp_path / 'pack.hip', tmp_path / 'pack.s'
+    kinds = ['8, 128, 32, false', '4, 96, 32, false', '4, 64, 32, true', '8, 128, 32, true', '16, 128, 128, false']
+    src.write_text(f'#include "{build.HERE}/sq_convert.cuh"\nnamespace sq {{\n'
+                   + ''.join(f'template int launch_pack<{k}>(const PackParams&, hipStream_t);\n' for k in kinds) + '}\n')
+    r = subprocess.run(['hipcc', *build.HIPCC_FLAGS, '--cuda-device-only', '-S', str(src), '-o', str(asm)],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    bodies = re.findall(r'^(_ZN2sq\d+pack_(?:v_|f_)?kernel\w+):.*\n((?:.*\n)*?)\ts_endpgm', asm.read_text(), re.M)
+    assert len(bodies) == len(kinds)
+    for name, body in bodies:
+        assert _loads_behind_the_skip(body), name
+        load = re.search(r'^\s(?:global|buffer|flat)_load.*\n', body, re.M)[0]
+        assert not _loads_behind_the_skip(load + body), name          # the check sees a load in front
