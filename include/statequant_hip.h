@@ -178,7 +178,8 @@ typedef struct sq_read_args {
 
 /* The mixed-width GGA / STEP slot of one layer (../integrations/vllm_gga.py:185-217 `GGAPacked`; byte layout in
  * _gga_triton.py:3-13).  One blob per slot:
- *   bytes 0..15     int32 n (queued pairs), head (ring index of the oldest pair), 2 unused
+ *   bytes 0..15     int32 n (queued pairs, 0 .. m), head (ring index of the oldest pair, 0 .. m - 1; while a step runs,
+ *                   the bits above its lowest 8 count the heads that have read the two), 2 unused
  *   offs[h]         value head h at its frozen width bits[h]: 16 = fp16 [dk, dv]; 4, 6, 8 = codes [dk, dv*b/8] (u = z +
  *                   qmax, little-endian along dv), row factors fp16 [dk], column factors fp16 [dv]; 2 = codes
  *                   [dk, dv/4] (u = (z+3)/2), row factors fp16 [dk, dv/32], column factors fp16 [dv]
@@ -199,7 +200,10 @@ typedef struct sq_gga_slots {
 /* One decode token per batch row on slots idx[b] (idx required; <= 0: padding).  q, k [rows, hk, dk] (normalised in
  * the kernel, q also times `scale`), v [rows, hv, dv] with row strides in elements; out [rows, hv, dv] contiguous.
  * gate = 1: a, b [rows, hv], A_log, dt_bias [hv] (decay exp(-exp(A_log) softplus(a + dt_bias)), beta = sigmoid(b));
- * gate = 0: g (log decay) and beta [rows, hv].  With pw the slots' counters are advanced by a second small launch. */
+ * gate = 0: g (log decay) and beta [rows, hv].  With pw the slots' counters are advanced by the last head to have read
+ * them: both must be what sq_gga_store and sq_gga_step leave (bits above head's lowest 8 stay, and the counters then
+ * advance at the wrong head, until the slot is stored again).  A slot that several rows of a call name advances its
+ * counters once; which of them steps its state is not defined. */
 typedef struct sq_gga_args {
     sq_gga_slots sl;
     int32_t rows;

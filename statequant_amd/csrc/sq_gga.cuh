@@ -38,8 +38,8 @@ constexpr int GGA_WAVES = GGA_THREADS / WAVE;
 constexpr int GGA_MMAX = 8;
 constexpr int GGA_GROUP = 32;
 // the slot's second counter: the ring index of the oldest pair, and above it -- while a step runs -- the heads that have
-// read the counters
-constexpr uint32_t GGA_RING = 0xFFFF, GGA_TICKET = 0x10000;
+// read the counters, in 24 bits: as many as a launch has workgroups
+constexpr uint32_t GGA_RING = 0xFF, GGA_TICKET = 0x100;
 
 template <int DK_, int DV_>
 struct GgaTile {
@@ -598,7 +598,7 @@ struct GgaLds {
 template <class T, int SPEC>
 __global__ __launch_bounds__(GGA_THREADS, 4)
 void gga_step_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict__ offs, const int32_t* __restrict__ widths,
-                     uint8_t* blob, uint64_t slot_stride, const GgaParams p0) {
+                     uint8_t* blob, uint64_t slot_stride, uint32_t rows, const GgaParams p0) {
     // (the leading arguments, copies of fields of the block, are in registers when a wavefront starts)
     GgaParams p = p0;
     assume_serving_case<SPEC>(p);
@@ -750,10 +750,10 @@ void gga_step_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     }
     __syncthreads();
     // ---- a ticket for the slot's counters: every head of the slot reads them, the last one to have done so advances them.
-    // The tickets are counted in the upper half of the ring index (whose value is below 16; zero between steps), so the
-    // slot's bytes are what a launch of its own behind every step left there.  This head's reads have returned (their
-    // values are in registers) before its ticket goes out, so no head reads what the last one writes; the writes are seen
-    // by the next launch.
+    // The tickets are counted above the ring index (whose value is below 16; zero between steps), so the slot's bytes are
+    // what a launch of its own behind every step left there.  This head's reads have returned (their values are in
+    // registers) before its ticket goes out, so no head reads what the last one writes; the writes are seen by the next
+    // launch.
     uint32_t ticket = 0;
     if (p.pw && t.tid == 0)
         ticket = __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(base) + 1, GGA_TICKET, __ATOMIC_RELAXED,
@@ -854,12 +854,24 @@ void gga_step_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     // ---- re-fit and re-pack in place ----
     gga_store_any<T>(S, bits, x, p.w + h * DK, L.fit);
 
-    // ---- the last head's: the counters of the slot, advanced (reference `_gga_advance`) ----
-    if (p.pw && t.tid == 0 && ticket / GGA_TICKET == uint32_t(p.hv) - 1) {
-        int32_t* const ct = reinterpret_cast<int32_t*>(base);
-        const int n0 = ct[0], hd0 = int(ticket & GGA_RING);
-        ct[0] = n0 + 1 < m ? n0 + 1 : m;
-        __hip_atomic_store(ct + 1, n0 == m ? (hd0 + 1) % m : hd0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // ---- the last head's: the counters of the slot, advanced (reference `_gga_advance`).  The last one is the last of all
+    // rows that name the slot; who could be it counts them (in the tail of one workgroup a slot: 27.5 -> 27.65 us for 32
+    // sequences, 146.9 -> 147.8 for 256; counted ahead of the tickets by everybody 27.9 and 152.9).  A launch that names a
+    // slot twice steps its state in no order that could be relied on, but the counters advance once, and no ticket is left
+    // for the next step. ----
+    if (p.pw && t.tid < WAVE) {
+        const uint32_t drawn = uint32_t(__builtin_amdgcn_readfirstlane(int(ticket))) / GGA_TICKET + 1;
+        if (drawn >= uint32_t(p.hv)) {
+            uint32_t named = 0;
+            for (uint32_t r = 0; r < rows; r += WAVE)
+                named += __builtin_popcountll(__builtin_amdgcn_ballot_w64(r + t.tid < rows && idx[min(r + t.tid, rows - 1)] == seq));
+            if (t.tid == 0 && drawn == named * uint32_t(p.hv)) {
+                int32_t* const ct = reinterpret_cast<int32_t*>(base);
+                const int n0 = ct[0], hd0 = int(ticket & GGA_RING);
+                ct[0] = n0 + 1 < m ? n0 + 1 : m;
+                __hip_atomic_store(ct + 1, n0 == m ? (hd0 + 1) % m : hd0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
     }
 }
 
@@ -927,11 +939,11 @@ int launch_gga(const GgaParams& p, int op, hipStream_t stream) {
         const dim3 tiles(p.rows, p.hv);
         const int spec = serving_case(p);
         if (spec == 2) hipLaunchKernelGGL((gga_step_kernel<T, 2>), tiles, block, 0, stream, p.idx, p.offs, p.bits, p.blob,
-                               p.slot_stride, p);
+                               p.slot_stride, uint32_t(p.rows), p);
         else if (spec == 1) hipLaunchKernelGGL((gga_step_kernel<T, 1>), tiles, block, 0, stream, p.idx, p.offs, p.bits, p.blob,
-                               p.slot_stride, p);
+                               p.slot_stride, uint32_t(p.rows), p);
         else hipLaunchKernelGGL((gga_step_kernel<T, 0>), tiles, block, 0, stream, p.idx, p.offs, p.bits, p.blob,
-                               p.slot_stride, p);
+                               p.slot_stride, uint32_t(p.rows), p);
     } else if (op == 1) {
         hipLaunchKernelGGL(gga_store_kernel<T>, grid, block, 0, stream, p);
     } else {

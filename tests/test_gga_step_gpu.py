@@ -44,6 +44,29 @@ def test_counters_advance_once_a_step(hv, hk, d, m, rows):
         assert (blob[:, 8:16] == 0xA5).all()
 
 
+@pytest.mark.parametrize('hv, hk, rows, twice', [(1, 1, 2, [(0, 1)]), (5, 5, 6, [(0, 2), (1, 4), (1, 5)]),
+                                                 (32, 16, 40, [(3, 39)]), (3, 3, 130, [(0, 64), (0, 129), (70, 71)])])
+def test_a_slot_named_twice_advances_once_and_leaves_nothing_behind(hv, hk, rows, twice):
+    """What such a launch leaves of the state is in no order; the slot's counters move on by one token, and the steps after
+    it, which name every slot once, find them as they should be."""
+    lay, views, idx, gen = _case(hv, hk, 64, 3, rows)
+    blob = views['blob']
+    doubled = idx.clone()
+    for a, b in twice:
+        doubled[b] = idx[a]
+    A, bias = torch.randn(hv, generator=gen).to(DEV) * 0.3, torch.randn(hv, generator=gen).to(DEV) * 0.3
+    out = torch.zeros(rows, hv, 64, dtype=torch.bfloat16, device=DEV)
+    want = torch.zeros(blob.shape[0], 2, dtype=torch.int32)
+    for t in range(9):
+        rows_now = doubled if t in (0, 1, 4) else idx
+        q, k, v, a, b = _token(gen, rows, hv, hk, 64)
+        lay.step(views, rows_now, q, k, v, out, 0.125, gate=(a, b, A, bias), layer=0)
+        for s in set(rows_now.tolist()):
+            n, head = want[s].tolist()
+            want[s] = torch.tensor([min(n + 1, 3), (head + 1) % 3 if n == 3 else head])
+        assert torch.equal(blob[:, :8].cpu().view(torch.int32), want), t
+
+
 @pytest.mark.parametrize('gate', [True, False])
 @pytest.mark.parametrize('hv, hk, d, pw', [(5, 5, 64, True), (8, 4, 128, True), (6, 2, 128, False)])
 def test_serving_instances_equal_the_general_one(gate, hv, hk, d, pw):
