@@ -394,7 +394,6 @@ int sq_gga_step(const sq_gga_args* a, void* stream) {
     if (a->rows == 0) return SQ_OK;
     sq::GgaParams p{};
     SQ_TRY(check_gga_slots(a->sl, who, &p));
-    if (a->sl.hv > 65535) return fail(SQ_E_UNSUPPORTED, "%s: hv %d > 65535", who, a->sl.hv);     // grid.y, tickets of 16 bits
     if (!a->idx || !a->q || !a->k || !a->v || !a->out) return fail(SQ_E_ARG, "%s: null idx / q / k / v / out", who);
     if (!dtype_ok(a->q_dtype) || !dtype_ok(a->k_dtype) || !dtype_ok(a->v_dtype) || !dtype_ok(a->out_dtype))
         return fail(SQ_E_ARG, "%s: bad dtype code", who);

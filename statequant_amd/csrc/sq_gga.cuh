@@ -40,6 +40,7 @@ constexpr int GGA_GROUP = 32;
 // the slot's second counter: the ring index of the oldest pair, and above it -- while a step runs -- the heads that have
 // read the counters, in 24 bits: as many as a launch has workgroups
 constexpr uint32_t GGA_RING = 0xFF, GGA_TICKET = 0x100;
+constexpr int GGA_GRID_Y = 65535;                       // heads along the second dimension of a launch
 
 template <int DK_, int DV_>
 struct GgaTile {
@@ -598,7 +599,7 @@ struct GgaLds {
 template <class T, int SPEC>
 __global__ __launch_bounds__(GGA_THREADS, 4)
 void gga_step_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict__ offs, const int32_t* __restrict__ widths,
-                     uint8_t* blob, uint64_t slot_stride, uint32_t rows, const GgaParams p0) {
+                     uint8_t* blob, uint64_t slot_stride, uint32_t rows, uint32_t head0, const GgaParams p0) {
     // (the leading arguments, copies of fields of the block, are in registers when a wavefront starts)
     GgaParams p = p0;
     assume_serving_case<SPEC>(p);
@@ -607,7 +608,7 @@ void gga_step_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     const GgaThread t = gga_thread();
     // head-major order: workgroups that run together work on the same head, hence on the same width, and share the
     // instructions of one of the five width paths (each path is ~40 KB of straight-line code)
-    const uint32_t h = blockIdx.y, b = blockIdx.x;
+    const uint32_t h = head0 + blockIdx.y, b = blockIdx.x;
     const uint32_t bh = b * uint32_t(p.hv) + h;
     const uint32_t hk = p.gqa_shift >= 0 ? h >> p.gqa_shift : h / uint32_t(p.gqa);
     const int32_t seq = idx[b];
@@ -936,14 +937,17 @@ template <class T>
 int launch_gga(const GgaParams& p, int op, hipStream_t stream) {
     const dim3 grid(p.rows * p.hv), block(GGA_THREADS);
     if (op == 0) {
-        const dim3 tiles(p.rows, p.hv);
         const int spec = serving_case(p);
-        if (spec == 2) hipLaunchKernelGGL((gga_step_kernel<T, 2>), tiles, block, 0, stream, p.idx, p.offs, p.bits, p.blob,
-                               p.slot_stride, uint32_t(p.rows), p);
-        else if (spec == 1) hipLaunchKernelGGL((gga_step_kernel<T, 1>), tiles, block, 0, stream, p.idx, p.offs, p.bits, p.blob,
-                               p.slot_stride, uint32_t(p.rows), p);
-        else hipLaunchKernelGGL((gga_step_kernel<T, 0>), tiles, block, 0, stream, p.idx, p.offs, p.bits, p.blob,
-                               p.slot_stride, uint32_t(p.rows), p);
+        for (int h0 = 0; h0 < p.hv; h0 += GGA_GRID_Y) {                   // (one launch but for 65 536 heads and more)
+            const dim3 tiles(p.rows, p.hv - h0 < GGA_GRID_Y ? p.hv - h0 : GGA_GRID_Y);
+#define SQ_GGA_STEP(SPEC)                                                                                                \
+            hipLaunchKernelGGL((gga_step_kernel<T, SPEC>), tiles, block, 0, stream, p.idx, p.offs, p.bits, p.blob,       \
+                               p.slot_stride, uint32_t(p.rows), uint32_t(h0), p)
+            if (spec == 2) SQ_GGA_STEP(2);
+            else if (spec == 1) SQ_GGA_STEP(1);
+            else SQ_GGA_STEP(0);
+#undef SQ_GGA_STEP
+        }
     } else if (op == 1) {
         hipLaunchKernelGGL(gga_store_kernel<T>, grid, block, 0, stream, p);
     } else {

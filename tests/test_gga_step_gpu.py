@@ -67,6 +67,36 @@ def test_a_slot_named_twice_advances_once_and_leaves_nothing_behind(hv, hk, rows
         assert torch.equal(blob[:, :8].cpu().view(torch.int32), want), t
 
 
+def test_more_heads_than_a_launch_dimension_takes():
+    """65 601 heads of one slot: those on either side of the launch's dimensions step like the same heads in a small slot."""
+    hv, d, picked = 65601, 64, [0, 32767, 32768, 65535, 65536, 65600]
+    gen = torch.Generator(device=DEV).manual_seed(4)
+    w = torch.rand(hv, d, device=DEV, generator=gen).cpu() + 0.5
+    widths = torch.full((hv,), 2)
+    widths[picked] = torch.tensor([4, 2, 8, 6, 2, 16])
+    S = torch.randn(1, hv, d, d, device=DEV, generator=gen) * 0.3
+    r = lambda *s: torch.randn(*s, device=DEV, generator=gen).bfloat16()         # noqa: E731
+    tokens = [(r(1, 1, d), r(1, 1, d), r(1, hv, d), r(1, hv), r(1, hv)) for _ in range(4)]
+    A, bias = torch.randn(hv, device=DEV, generator=gen) * 0.3, torch.randn(hv, device=DEV, generator=gen) * 0.3
+    idx = torch.ones(1, dtype=torch.int32, device=DEV)
+
+    def outputs(sel):
+        lay = GGAPacked(GGAPlan({0: (widths[sel], w[sel])}), len(sel), 1, d, d, pw=True, m=3)
+        views = lay.views(lay.alloc(2, DEV))
+        lay.write(views, idx, S[:, sel], layer=0)
+        outs = []
+        for q, k, v, a, b in tokens:
+            o = torch.zeros(1, len(sel), d, dtype=torch.bfloat16, device=DEV)
+            outs.append(lay.step(views, idx, q, k, v[:, sel].contiguous(), o, 0.125, layer=0,
+                                 gate=(a[:, sel].contiguous(), b[:, sel].contiguous(), A[sel], bias[sel])))
+        return torch.stack(outs), views['blob'][1, :8].view(torch.int32).tolist()
+
+    many, counters = outputs(list(range(hv)))
+    few, want = outputs(picked)
+    assert counters == want == [3, 1]
+    assert torch.equal(many[:, :, picked], few)
+
+
 @pytest.mark.parametrize('gate', [True, False])
 @pytest.mark.parametrize('hv, hk, d, pw', [(5, 5, 64, True), (8, 4, 128, True), (6, 2, 128, False)])
 def test_serving_instances_equal_the_general_one(gate, hv, hk, d, pw):
