@@ -184,73 +184,90 @@ def quad_variants(fam, c):
     return out
 
 
+# Where a line lies for launches without a dispatch order.  A lockstep state (no slot indices: `p.idx` null) folds all its heads
+# on the same step or none: no head is a straggler then, and the variants that shorten a fold are worth less.  Slots without
+# an order are mostly out of step (an engine orders batches of 64 and more where their count allows it), but may be in
+# lockstep too, which no argument tells: their line is where what the one gains is what the other loses.
+#
 # Launches that satisfy this take one row block per wavefront and one head per workgroup: twice the wavefronts on up to
 # four times the compute units, so that a head's life -- which is all such a launch consists of, the fold's four half
 # blocks in sequence above all -- gets shorter.  (One block per wavefront with two heads per workgroup gains nothing:
-# the wavefronts then share the SIMDs they had.)  With a dispatch order the folding heads no longer end the launch, so the
-# shorter fold is worth less and the line lies earlier -- but for int4 with key-axis groups, where the launch without an
-# order has a second, nearly empty round of workgroups from 72 sequences on.  us per launch, two blocks and two heads / this,
-# sequences out of step, 16 layers captured:
-# GDN 128 x 128 (32 heads) int4 g64 32 sequences 9.93 / 8.15, 60: 12.85 / 12.37, 66: 13.65 / 13.37, 76: 14.45 / 14.47, 90: 15.4 /
-# 16.3; in order 64: 11.18 / 10.88, 80: 13.1 / 12.6, 96: 14.9 / 14.3, 104: 15.0 / 15.0, 112: 15.6 / 15.8, 128: 16.3 / 17.3; int8
-# g32 32: 11.0 / 9.6, 66: 16.2 / 15.8, 76: 17.9 / 17.2, 90: 19.5 / 18.8, in order 64: 13.7 / 13.4, 72: 14.4 / 14.5, 80: 15.0 /
-# 15.6 (g128 alike).  Value-axis int4 60: 15.5 / 13.7, 100: 20.8 / 19.4, 150: 25.7 / 25.0, 190: 29.0 / 28.7, 220: 32.4 / 33.4, in
-# order 96: 16.2 / 15.3, 128: 18.8 / 18.4, 136: 19.0 / 19.3, 160: 20.8 / 21.8; int8 130: 26.6 / 24.8, 190: 33.2 / 31.1, 250: 40.6 /
-# 39.9, in order 80: 16.3 / 15.4, 120: 20.1 / 20.1, 128: 20.4 / 21.4.  96 x 192 int4 g64 (30 heads) 16: 9.6 / 8.5, 25: 11.7 / 11.4,
-# 26: 11.8 / 11.9, 28: 11.4 / 12.4.  Mamba2 128 x 64 (128 heads) int8 g128 3: 6.0 / 5.8, 10: 8.7 / 8.2, 12: 9.66 / 9.67, 13: 9.6 /
-# 9.5; int4 g64 10: 8.2 / 7.6, 18: 10.1 / 9.8, 20: 10.0 / 10.5.  The other shapes and buffers that have two blocks or several
-# heads in a workgroup were not built this way: nothing is known about them.
+# the wavefronts then share the SIMDs they had.)  us per launch, two blocks and two heads / this, 16 layers captured, sequences
+# out of step; in lockstep (ls); in order:
+# GDN 128 x 128 (32 heads on 16 key heads) int4 g64 60 sequences 13.3 / 12.8, 64: 13.0 / 12.8 (ls 9.2 / 10.3), 71: 14.1 / 14.0 (10.3
+# / 11.1), in order 64: 11.6 / 11.2, 96: 15.1 / 14.3, 104: 15.1 / 15.0, 112: 15.6 / 15.8; int8 g32 60: 15.6 / 15.2, 64, one full
+# round of pairs: 15.1 / 15.3 (11.7 / 12.5), 66: 15.9 / 15.9 (12.9 / 13.0), 72: 16.6 / 16.1 (13.4 / 13.5), 90: 19.3 / 18.7 (15.1 / 15.6; g128
+# 14.7 / 15.1), in order 64: 13.7 / 13.3, 72: 14.2 / 14.4.  Value-axis int4 104: 20.7 / 19.3 (14.0 / 15.0), 108: 22.5 / 21.7 (15.3 /
+# 16.8), 128: 22.7 / 22.0 (16.2 / 17.9), 190: 28.7 / 29.1, in order 104: 16.2 / 15.9, 128: 17.7 / 17.9, 136: 19.0 / 19.3; int8 190:
+# 33.6 / 31.5 (26.8 / 27.2), 200: 34.9 / 33.1 (28.2 / 28.1), 250: 40.7 / 39.4 (34.0 / 35.1), in order 120: 19.9 / 19.7, 128: 20.4 /
+# 21.4.  Ungrouped heads (16 on 16), where the other side has one head a workgroup too, int4 128: 15.1 / 13.4 (10.2 / 10.5), 140:
+# 16.1 / 14.1 (11.3 / 11.1), in order 208: 16.3 / 15.1; int8 136: 18.9 / 15.9 (14.5 / 13.2), 190: 22.5 / 19.7; value-axis int4 250:
+# 25.4 / 21.9 (17.5 / 17.6), int8 256: 28.8 / 24.2 (22.0 / 20.3).  48 on 16 int4 44: 15.7 / 15.0 (11.3 / 12.7), int8 60: 22.7 /
+# 20.6 (17.5 / 17.4).  96 x 192 int4 g64 (30 heads) 25: 11.4 / 11.0 (7.9 / 8.1), 26: 11.8 / 11.9, 40: 13.1 / 16.4, in order 64: 14.2 /
+# 17.7, 128: 21.5 / 31.9; int8 g128 40: 14.2 / 17.0, in order 64: 16.2 / 18.6.  Mamba2 128 x 64 (128 heads) int8 g128 8: 7.7 / 7.5 (5.6
+# / 5.8), 10: 9.4 / 8.7 (6.7 / 6.5), 12: 9.0 / 9.0 (6.8 / 7.1), 13: 9.8 / 9.7 (7.0 / 7.3); int4 g64 10: 8.9 / 8.1 (6.0 / 6.0), 14: 9.2 /
+# 9.2 (6.2 / 6.8), 18: 10.5 / 10.1 (7.2 / 7.6); 112 heads 14: 9.9 / 9.2 (6.4 / 6.9).  The other shapes and buffers that have two
+# blocks or several heads in a workgroup were not built this way: nothing is known about them.
 def small_when(fam, c):
     bits, dk, dv, group, qbuf, mmax, axv = c
     if bits == 16 or not qbuf or mmax > 8:
         return ''
-    return {('gdn', 128, 128, 0): f'heads < (p.order ? {3456 if bits == 4 else 2176} : {2304 if bits == 4 else 3072})',
-            ('gdn', 128, 128, 1): f'heads < (p.order ? {4224 if bits == 4 else 3968} : {6400 if bits == 4 else 8192})',
+    gdn4 = 'heads < (p.order ? 3456 : p.gqa == 1 ? 2304 : 2048)'
+    gdn8 = '(p.order ? heads < 2176 : p.gqa == 1 ? heads < 3072 : heads < 2048 || (p.idx && heads > 2048 && heads < 3072))'
+    gdn4v = 'heads < (p.order ? 4224 : p.gqa == 1 ? 6400 : 3328)'
+    gdn8v = 'heads < (p.order ? 3968 : p.idx || p.gqa == 1 ? 8192 : 6144)'
+    return {('gdn', 128, 128, 0): gdn4 if bits == 4 else gdn8, ('gdn', 128, 128, 1): gdn4v if bits == 4 else gdn8v,
             ('gdn', 96, 192, 0): 'heads < 768',
-            ('mamba2', 128, 64, 0): f'heads < {2432 if bits == 4 else 1696}'}.get((fam, dk, dv, axv), '')
+            ('mamba2', 128, 64, 0): f'heads < (p.idx ? {2432 if bits == 4 else 1664} : 768)'}.get((fam, dk, dv, axv), '')
 
 
 # Heads per launch from which the one-wavefront kernel serves these cases again where nothing below has a line of its own: the
-# buffers of 16 tokens or bf16, and int8 value-axis groups of 96 x 96.  Their workgroups waste something -- lanes and LDS on
+# buffers of 16 tokens or bf16, int8 value-axis groups of 96 x 96, and some lockstep states.  Their workgroups waste something -- lanes and LDS on
 # the columns between 96 and 128, a half empty row block (d_v 80) -- which does not matter while a launch is short of
 # wavefronts and may once it has several rounds of them.
 GROUP_HEADS = 5120
 
 
 def group_when(fam, c):
-    """The condition (C++, on `heads` of the launch and whether it has a dispatch order) under which a case's workgroup
-    kernels serve; '' always.  What ends their lead is a launch with enough heads to fill the chip several times over:
+    """The condition (C++, on `heads` of the launch and whether it has slot indices and a dispatch order) under which a case's
+    workgroup kernels serve; '' always.  What ends their lead is a launch with enough heads to fill the chip several times over:
     then a head costs its instructions and its LDS, not its length.  A dispatch order ends it earlier: the one-wavefront
     kernel's folding heads live three times as long as the others, and placed well they no longer decide when the launch
-    ends.  Figures: us per launch, workgroup / one wavefront, sequences out of step."""
+    ends.  Figures: us per launch, workgroup / one wavefront, sequences out of step (ls: in lockstep)."""
     bits, dk, dv, group, qbuf, mmax, axv = c
     flt, usual = bits == 16, qbuf and mmax == 8
     when = []
     if fam == 'mamba2':
         if dv % 32 and not flt:
-            # a half empty row block.  128 x 80 (96 heads) int4 g64 48 sequences 22.0 / 25.3, 100: 35.3 / 36.4, 150: 49.8 / 48.0, in
-            # order 64: 22.0 / 21.3, 80: 25.7 / 23.7; int8 g128 52: 22.9 / 26.7, 100: 37.2 / 40.3, 190: 60.9 / 66.4, in order 64: 23.2 /
-            # 23.8, 72: 26.2 / 25.8 (g32 24.0 / 25.0, 26.7 / 26.5).  d_state 96, int4 32: 15.3 / 16.6, 40: 18.2 / 18.0, 56: 23.1 / 24.3,
-            # 100: 35.7 / 33.8, in order 64: 22.3 / 19.7; int8 48: 22.4 / 24.7, 100: 36.7 / 37.3, in order 64: 23.1 / 22.1
-            lines = {(4, 128): 'heads < (p.order ? 5120 : 11520)', (8, 128): '(!p.order || heads < 6656)',
-                     (4, 96): 'heads < (p.order ? 3328 : 6144)', (8, 96): f'(!p.order || heads < {GROUP_HEADS})'}
+            # a half empty row block.  128 x 80 (96 heads) int4 g64 52 sequences 22.3 / 24.7 (ls 17.6 / 17.3), 64: 24.8 / 27.7 (20.5 /
+            # 19.2), 76: 27.2 / 29.4 (23.5 / 21.8), 80: 29.3 / 31.3 (24.4 / 22.1), 120: 39.8 / 39.9 (34.0 / 30.2), in order 64: 21.7 / 21.1;
+            # int8 g128 52: 23.5 / 26.7 (18.8 / 19.3), 64: 26.2 / 29.5 (21.7 / 21.6), 128: 44.4 / 47.9 (38.3 / 36.9), 250: 78.5 / 82.3
+            # (71.6 / 68.4), 400: 120.0 / 124.5 (112.0 / 107.4), in order 64: 23.0 / 23.7 (g32 128: 46.0 / 51.0, ls 40.5 / 39.3).
+            # d_state 96, int4 34: 16.7 / 18.1 (13.2 / 12.8), 40: 18.7 / 18.7 (14.8 / 13.1), 64: 25.1 / 25.3 (20.9 / 18.3), in order 22.1 /
+            # 19.7; int8 50: 22.1 / 24.0 (18.0 / 17.6), 72: 27.4 / 29.5 (23.9 / 22.0), 80: 30.5 / 31.8 (25.9 / 23.7), 150: 49.5 / 48.9, 250:
+            # 75.9 / 70.9 (68.4 / 60.8), in order 64: 22.4 / 21.7
+            lines = {(4, 128): 'heads < (p.idx && !p.order ? 7424 : 5120)', (8, 128): 'heads < (p.order ? 6656 : p.idx ? 38400 : 5120)',
+                     (4, 96): 'heads < 3328', (8, 96): 'heads < (p.idx && !p.order ? 7040 : 5120)'}
             plain = usual and not axv and (bits, dk) in lines
             when.append(lines[bits, dk] if plain else f'heads < {3328 if (bits, dk, mmax) == (4, 96, 8) else GROUP_HEADS}')
         if flt and (dk, mmax) == (96, 8):                    # 64 sequences 33.7 / 34.3, 96 in order 47.3 / 43.1
             when.append('(!p.order || heads < 8192)')
     elif dk == 96 and not flt and (bits == 8 or not axv) and (fam == 'gdn' or (bits == 4 and not axv)):
-        # a quarter of the lanes and of LDS on padded columns.  96 x 192 (30 heads) int4 g64 130 sequences 26.9 / 37.0, 250: 40.0 /
-        # 50.4, in order 160: 25.1 / 29.5, 256: 36.9 / 39.0, 400: 53.7 / 54.7; int8 g128 in order 160: 29.6 / 33.0, 400: 64.1 / 73.1,
-        # value-axis 256: 45.1 / 53.7.  96 x 96 (20 heads) KDA int4 g32 in order 160: 15.4 / 19.4, 400: 29.0 / 31.6, 390: 30.9 / 38.2;
-        # GDN, three wavefronts a head, int4 g64 190: 19.5 / 21.5, 250: 23.1 / 26.1, in order 176: 15.9 / 16.3, 192: 16.9 / 16.8, 256:
-        # 20.5 / 19.4, int8 g32 in order 192: 18.2 / 19.3, 256: 21.9 / 22.0
+        # a quarter of the lanes and of LDS on padded columns.  96 x 192 (30 heads) int4 g64 170 sequences 31.1 / 41.6 (ls 25.3 /
+        # 27.5), 400: 60.1 / 69.5 (51.2 / 53.9), in order 256: 35.7 / 38.7, 400: 51.9 / 54.7; int8 g128 256: 48.8 / 58.6 (42.3 / 44.5), in
+        # order 43.3 / 48.3, value-axis 50.1 / 67.0 (44.6 / 51.5), 44.8 / 53.2.  96 x 96 (20 heads) KDA int4 g32 200: 20.3 / 25.5 (17.1
+        # / 18.0), 390: 30.7 / 37.6 (27.9 / 30.9), in order 256: 21.0 / 23.7, 400: 29.0 / 31.6; GDN, three wavefronts a head, int4 g64 160:
+        # 18.0 / 20.1 (14.3 / 14.2), 256: 23.7 / 26.2 (19.9 / 18.6), 300: 26.6 / 28.5 (22.5 / 20.3), 400: 32.0 / 32.4 (28.1 / 24.5), in
+        # order 160: 15.0 / 16.4, 192: 16.9 / 17.2, 256: 20.5 / 19.7; int8 g32 256: 24.8 / 28.6 (21.1 / 21.3), 400: 33.9 / 37.1 (30.1 /
+        # 28.8), in order 256: 21.8 / 22.2, 400: 30.8 / 30.2
         if not usual or (axv and dv != 192):
             when.append(f'heads < {GROUP_HEADS}')
         elif fam == 'gdn' and dv == 192 and bits == 4:
             when.append('(!p.order || heads < 12288)')
-        if fam == 'gdn' and dv == 96 and not axv and mmax == 8:
-            # (bf16 buffer 128: 14.7 / 15.2, 160: 17.0 / 16.0)
-            when.append(f'(!p.order || heads < {2880 if not qbuf else 3680 if bits == 4 else 5120})')
+        elif fam == 'gdn' and dv == 96:
+            when.append('heads < (p.order ? 3680 : p.idx ? 5760 : 5120)' if bits == 4 else '(heads < 5120 || (p.idx && !p.order))')
+        if fam == 'gdn' and dv == 96 and not axv and mmax == 8 and not qbuf:
+            when.append('(!p.order || heads < 2880)')        # bf16 buffer 128: 14.7 / 15.2, 160: 17.0 / 16.0
     elif fam == 'gdn' and flt and (dk, dv) == (96, 192) and not usual:
         # two workgroups per compute unit (30 heads, 16-token buffer): 64 sequences in order 45.9 / 58.2, 96: 64.4 / 61.3,
         # 128: 80.6 / 64.8; 130, not in order, 81.3 / 87.5

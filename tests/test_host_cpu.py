@@ -475,3 +475,52 @@ def test_pack_kernels_read_no_row_of_a_padding_row(tmp_path):
         assert _loads_behind_the_skip(body), name
         load = re.search(r'^\s(?:global|buffer|flat)_load.*\n', body, re.M)[0]
         assert not _loads_behind_the_skip(load + body), name          # the check sees a load in front
+
+
+def test_lines_between_kernel_variants(tmp_path):
+    """Which variant a launch gets, by the generated conditions compiled for the host: lockstep states (no slot indices) stay
+    with what serves launches whose heads all fold at once, and every line between variants of launches without an order has
+    an upper end where the other variant was measured to be faster."""
+    import shutil
+    import subprocess
+    from statequant_amd.csrc import build
+    if not shutil.which('g++'):
+        pytest.skip('no host compiler')
+    Q4, Q8 = (4, 128, 128, 64, 1, 8, 0), (8, 128, 128, 128, 1, 8, 0)
+    V4, V8 = (4, 128, 128, 32, 1, 8, 1), (8, 128, 128, 32, 1, 8, 1)
+    M4, M8, N4, N8 = (4, 128, 80, 64, 1, 8, 0), (8, 128, 80, 128, 1, 8, 0), (4, 96, 80, 32, 1, 8, 0), (8, 96, 80, 32, 1, 8, 0)
+    small, group = build.small_when, build.group_when
+    # (rule, family, case, grouping, heads of one sequence): sequences -> whether the rule holds, per form of the call
+    table = [
+        (small, 'gdn', Q4, 2, 32, dict(state={63: 1, 64: 0, 71: 0}, slots={63: 1, 64: 0, 71: 0}, order={64: 1, 104: 1, 112: 0})),
+        (small, 'gdn', Q4, 1, 16, dict(state={128: 1, 143: 1, 144: 0}, slots={140: 1, 144: 0}, order={208: 1, 216: 0})),
+        (small, 'gdn', Q8, 2, 32, dict(state={63: 1, 64: 0, 72: 0}, slots={63: 1, 64: 0, 65: 1, 95: 1, 96: 0}, order={64: 1, 72: 0})),
+        (small, 'gdn', Q8, 1, 16, dict(state={128: 1, 190: 1}, slots={128: 1, 190: 1, 192: 0}, order={128: 1, 136: 0})),
+        (small, 'gdn', V4, 2, 32, dict(state={103: 1, 104: 0}, slots={103: 1, 104: 0, 190: 0}, order={128: 1, 136: 0})),
+        (small, 'gdn', V4, 1, 16, dict(state={250: 1}, slots={250: 1}, order={256: 1})),
+        (small, 'gdn', V8, 2, 32, dict(state={191: 1, 192: 0}, slots={255: 1, 256: 0}, order={120: 1, 128: 0})),
+        (small, 'mamba2', (8, 128, 64, 128, 1, 8, 0), 16, 128, dict(state={5: 1, 6: 0}, slots={12: 1, 13: 0})),
+        (small, 'mamba2', (4, 128, 64, 64, 1, 8, 0), 16, 128, dict(state={5: 1, 6: 0}, slots={18: 1, 19: 0})),
+        (group, 'mamba2', M4, 12, 96, dict(state={53: 1, 54: 0}, slots={76: 1, 78: 0}, order={48: 1, 64: 0})),
+        (group, 'mamba2', M8, 12, 96, dict(state={53: 1, 54: 0, 128: 0}, slots={128: 1, 399: 1, 400: 0}, order={64: 1, 72: 0})),
+        (group, 'mamba2', N4, 12, 96, dict(state={34: 1, 35: 0}, slots={34: 1, 35: 0, 52: 0}, order={64: 0})),
+        (group, 'mamba2', N8, 12, 96, dict(state={53: 1, 54: 0}, slots={73: 1, 74: 0, 250: 0}, order={64: 0})),
+        (group, 'gdn', (4, 96, 96, 64, 1, 8, 0), 1, 20, dict(state={255: 1, 256: 0}, slots={256: 1, 288: 0}, order={176: 1, 184: 0})),
+        (group, 'gdn', (8, 96, 96, 32, 1, 8, 0), 1, 20, dict(state={255: 1, 256: 0}, slots={400: 1}, order={248: 1, 256: 0})),
+        (group, 'gdn', (4, 96, 192, 64, 1, 8, 0), 1, 30, dict(state={256: 1, 400: 1}, slots={256: 1, 400: 1}, order={400: 1, 416: 0})),
+    ]
+    calls, want = [], []
+    for rule, fam, case, gqa, hv, forms in table:
+        for form, rows in forms.items():
+            for r, holds in rows.items():
+                calls.append(f'    show({{{int(form != "state")}, {int(form == "order")}, {gqa}}}, {r * hv}, '
+                             f'[](P p, int64_t heads) {{ return bool({rule(fam, case)}); }});')
+                want.append(f'{holds}')
+    src, exe = tmp_path / 'lines.cpp', str(tmp_path / 'lines')
+    src.write_text('#include <stdint.h>\n#include <stdio.h>\nstruct P { int idx, order, gqa; };\n'
+                   'template <class F> void show(P p, int64_t heads, F&& f) { printf("%d\\n", int(f(p, heads))); }\n'
+                   'int main() {\n' + '\n'.join(calls) + '\n}\n')
+    r = subprocess.run(['g++', '-std=c++17', str(src), '-o', exe], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    got = subprocess.run([exe], capture_output=True, text=True, check=True).stdout.split()
+    assert got == want, [c for c, g, w in zip(calls, got, want) if g != w]
