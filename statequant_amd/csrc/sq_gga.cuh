@@ -863,8 +863,8 @@ void gga_step_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     if (p.pw && t.tid < WAVE) {
         const uint32_t drawn = uint32_t(__builtin_amdgcn_readfirstlane(int(ticket))) / GGA_TICKET + 1;
         if (drawn >= uint32_t(p.hv)) {
-            uint32_t named = 0;
-            for (uint32_t r = 0; r < rows; r += WAVE)
+            uint32_t named = rows == 1;
+            for (uint32_t r = 0; rows > 1 && r < rows; r += WAVE)
                 named += __builtin_popcountll(__builtin_amdgcn_ballot_w64(r + t.tid < rows && idx[min(r + t.tid, rows - 1)] == seq));
             if (t.tid == 0 && drawn == named * uint32_t(p.hv)) {
                 int32_t* const ct = reinterpret_cast<int32_t*>(base);
