@@ -184,10 +184,11 @@ def quad_variants(fam, c):
     return out
 
 
-# Where a line lies for launches without a dispatch order.  A lockstep state (no slot indices: `p.idx` null) folds all its heads
-# on the same step or none: no head is a straggler then, and the variants that shorten a fold are worth less.  Slots without
-# an order are mostly out of step (an engine orders batches of 64 and more where their count allows it), but may be in
-# lockstep too, which no argument tells: their line is where what the one gains is what the other loses.
+# Where a line lies for launches without a dispatch order.  Such a launch is a batch out of step or one in lockstep, whose
+# heads fold all on the same step: no head is a straggler then, and the variants that shorten a fold are worth less.  From 64
+# sequences on a serving engine orders a batch that is out of step where its count allows it, so there the line is where a
+# batch in lockstep begins to lose; below, it is where what a batch out of step gains is what one in lockstep loses (a lockstep
+# state, which is one for sure, has no slot indices: `p.idx` null).
 #
 # Launches that satisfy this take one row block per wavefront and one head per workgroup: twice the wavefronts on up to
 # four times the compute units, so that a head's life -- which is all such a launch consists of, the fold's four half
@@ -213,24 +214,24 @@ def small_when(fam, c):
     if bits == 16 or not qbuf or mmax > 8:
         return ''
     gdn4 = 'heads < (p.order ? 3456 : p.gqa == 1 ? 2304 : 2048)'
-    gdn8 = '(p.order ? heads < 2176 : p.gqa == 1 ? heads < 3072 : heads < 2048 || (p.idx && heads > 2048 && heads < 3072))'
+    gdn8 = '(p.order ? heads < 2176 : p.gqa == 1 ? heads < 3072 : heads < 2560 && heads != 2048)'
     gdn4v = 'heads < (p.order ? 4224 : p.gqa == 1 ? 6400 : 3328)'
-    gdn8v = 'heads < (p.order ? 3968 : p.idx || p.gqa == 1 ? 8192 : 6144)'
+    gdn8v = 'heads < (p.order ? 3968 : p.gqa == 1 ? 8192 : 6912)'
     return {('gdn', 128, 128, 0): gdn4 if bits == 4 else gdn8, ('gdn', 128, 128, 1): gdn4v if bits == 4 else gdn8v,
             ('gdn', 96, 192, 0): 'heads < 768',
             ('mamba2', 128, 64, 0): f'heads < (p.idx ? {2432 if bits == 4 else 1664} : 768)'}.get((fam, dk, dv, axv), '')
 
 
-# Heads per launch from which the one-wavefront kernel serves these cases again where nothing below has a line of its own: the
-# buffers of 16 tokens or bf16, int8 value-axis groups of 96 x 96, and some lockstep states.  Their workgroups waste something -- lanes and LDS on
-# the columns between 96 and 128, a half empty row block (d_v 80) -- which does not matter while a launch is short of
-# wavefronts and may once it has several rounds of them.
+# Heads per launch from which the one-wavefront kernel serves these cases again where nothing below has a line of its own:
+# the buffers of 16 tokens or bf16, int8 value-axis groups of 96 x 96, and launches without an order whose lockstep batches
+# lose from about there on.  Their workgroups waste something -- lanes and LDS on the columns between 96 and 128, a half empty
+# row block (d_v 80) -- which does not matter while a launch is short of wavefronts and may once it has several rounds of them.
 GROUP_HEADS = 5120
 
 
 def group_when(fam, c):
-    """The condition (C++, on `heads` of the launch and whether it has slot indices and a dispatch order) under which a case's
-    workgroup kernels serve; '' always.  What ends their lead is a launch with enough heads to fill the chip several times over:
+    """The condition (C++, on `heads` of the launch and whether it has a dispatch order) under which a case's workgroup
+    kernels serve; '' always.  What ends their lead is a launch with enough heads to fill the chip several times over:
     then a head costs its instructions and its LDS, not its length.  A dispatch order ends it earlier: the one-wavefront
     kernel's folding heads live three times as long as the others, and placed well they no longer decide when the launch
     ends.  Figures: us per launch, workgroup / one wavefront, sequences out of step (ls: in lockstep)."""
@@ -246,10 +247,8 @@ def group_when(fam, c):
             # d_state 96, int4 34: 16.7 / 18.1 (13.2 / 12.8), 40: 18.7 / 18.7 (14.8 / 13.1), 64: 25.1 / 25.3 (20.9 / 18.3), in order 22.1 /
             # 19.7; int8 50: 22.1 / 24.0 (18.0 / 17.6), 72: 27.4 / 29.5 (23.9 / 22.0), 80: 30.5 / 31.8 (25.9 / 23.7), 150: 49.5 / 48.9, 250:
             # 75.9 / 70.9 (68.4 / 60.8), in order 64: 22.4 / 21.7
-            lines = {(4, 128): 'heads < (p.idx && !p.order ? 7424 : 5120)', (8, 128): 'heads < (p.order ? 6656 : p.idx ? 38400 : 5120)',
-                     (4, 96): 'heads < 3328', (8, 96): 'heads < (p.idx && !p.order ? 7040 : 5120)'}
-            plain = usual and not axv and (bits, dk) in lines
-            when.append(lines[bits, dk] if plain else f'heads < {3328 if (bits, dk, mmax) == (4, 96, 8) else GROUP_HEADS}')
+            line = {(4, 96): 3328, (8, 128): 6656 if usual and not axv else GROUP_HEADS}.get((bits, dk), GROUP_HEADS)
+            when.append(f'heads < {line if mmax == 8 else GROUP_HEADS}')
         if flt and (dk, mmax) == (96, 8):                    # 64 sequences 33.7 / 34.3, 96 in order 47.3 / 43.1
             when.append('(!p.order || heads < 8192)')
     elif dk == 96 and not flt and (bits == 8 or not axv) and (fam == 'gdn' or (bits == 4 and not axv)):
@@ -265,7 +264,7 @@ def group_when(fam, c):
         elif fam == 'gdn' and dv == 192 and bits == 4:
             when.append('(!p.order || heads < 12288)')
         elif fam == 'gdn' and dv == 96:
-            when.append('heads < (p.order ? 3680 : p.idx ? 5760 : 5120)' if bits == 4 else '(heads < 5120 || (p.idx && !p.order))')
+            when.append(f'heads < (p.order ? 3680 : {GROUP_HEADS})' if bits == 4 else f'heads < (p.order ? {GROUP_HEADS} : 6400)')
         if fam == 'gdn' and dv == 96 and not axv and mmax == 8 and not qbuf:
             when.append('(!p.order || heads < 2880)')        # bf16 buffer 128: 14.7 / 15.2, 160: 17.0 / 16.0
     elif fam == 'gdn' and flt and (dk, dv) == (96, 192) and not usual:

@@ -478,9 +478,8 @@ def test_pack_kernels_read_no_row_of_a_padding_row(tmp_path):
 
 
 def test_lines_between_kernel_variants(tmp_path):
-    """Which variant a launch gets, by the generated conditions compiled for the host: lockstep states (no slot indices) stay
-    with what serves launches whose heads all fold at once, and every line between variants of launches without an order has
-    an upper end where the other variant was measured to be faster."""
+    """Which variant a launch gets, by the generated conditions compiled for the host: launches without a dispatch order, which
+    may be in lockstep, get the variant that serves those no slower, and small lockstep states (no slot indices) keep theirs."""
     import shutil
     import subprocess
     from statequant_amd.csrc import build
@@ -494,19 +493,19 @@ def test_lines_between_kernel_variants(tmp_path):
     table = [
         (small, 'gdn', Q4, 2, 32, dict(state={63: 1, 64: 0, 71: 0}, slots={63: 1, 64: 0, 71: 0}, order={64: 1, 104: 1, 112: 0})),
         (small, 'gdn', Q4, 1, 16, dict(state={128: 1, 143: 1, 144: 0}, slots={140: 1, 144: 0}, order={208: 1, 216: 0})),
-        (small, 'gdn', Q8, 2, 32, dict(state={63: 1, 64: 0, 72: 0}, slots={63: 1, 64: 0, 65: 1, 95: 1, 96: 0}, order={64: 1, 72: 0})),
+        (small, 'gdn', Q8, 2, 32, dict(state={63: 1, 64: 0, 66: 1}, slots={63: 1, 64: 0, 72: 1, 80: 0, 90: 0}, order={64: 1, 72: 0})),
         (small, 'gdn', Q8, 1, 16, dict(state={128: 1, 190: 1}, slots={128: 1, 190: 1, 192: 0}, order={128: 1, 136: 0})),
         (small, 'gdn', V4, 2, 32, dict(state={103: 1, 104: 0}, slots={103: 1, 104: 0, 190: 0}, order={128: 1, 136: 0})),
         (small, 'gdn', V4, 1, 16, dict(state={250: 1}, slots={250: 1}, order={256: 1})),
-        (small, 'gdn', V8, 2, 32, dict(state={191: 1, 192: 0}, slots={255: 1, 256: 0}, order={120: 1, 128: 0})),
+        (small, 'gdn', V8, 2, 32, dict(state={200: 1, 216: 0}, slots={200: 1, 216: 0, 250: 0}, order={120: 1, 128: 0})),
         (small, 'mamba2', (8, 128, 64, 128, 1, 8, 0), 16, 128, dict(state={5: 1, 6: 0}, slots={12: 1, 13: 0})),
         (small, 'mamba2', (4, 128, 64, 64, 1, 8, 0), 16, 128, dict(state={5: 1, 6: 0}, slots={18: 1, 19: 0})),
-        (group, 'mamba2', M4, 12, 96, dict(state={53: 1, 54: 0}, slots={76: 1, 78: 0}, order={48: 1, 64: 0})),
-        (group, 'mamba2', M8, 12, 96, dict(state={53: 1, 54: 0, 128: 0}, slots={128: 1, 399: 1, 400: 0}, order={64: 1, 72: 0})),
+        (group, 'mamba2', M4, 12, 96, dict(state={53: 1, 54: 0}, slots={53: 1, 64: 0, 120: 0}, order={48: 1, 64: 0})),
+        (group, 'mamba2', M8, 12, 96, dict(state={64: 1, 128: 0}, slots={64: 1, 72: 0, 128: 0}, order={64: 1, 72: 0})),
         (group, 'mamba2', N4, 12, 96, dict(state={34: 1, 35: 0}, slots={34: 1, 35: 0, 52: 0}, order={64: 0})),
-        (group, 'mamba2', N8, 12, 96, dict(state={53: 1, 54: 0}, slots={73: 1, 74: 0, 250: 0}, order={64: 0})),
-        (group, 'gdn', (4, 96, 96, 64, 1, 8, 0), 1, 20, dict(state={255: 1, 256: 0}, slots={256: 1, 288: 0}, order={176: 1, 184: 0})),
-        (group, 'gdn', (8, 96, 96, 32, 1, 8, 0), 1, 20, dict(state={255: 1, 256: 0}, slots={400: 1}, order={248: 1, 256: 0})),
+        (group, 'mamba2', N8, 12, 96, dict(state={53: 1, 54: 0}, slots={53: 1, 64: 0, 250: 0}, order={64: 0})),
+        (group, 'gdn', (4, 96, 96, 64, 1, 8, 0), 1, 20, dict(state={255: 1, 256: 0}, slots={255: 1, 256: 0}, order={176: 1, 184: 0})),
+        (group, 'gdn', (8, 96, 96, 32, 1, 8, 0), 1, 20, dict(state={256: 1, 400: 0}, slots={256: 1, 400: 0}, order={248: 1, 256: 0})),
         (group, 'gdn', (4, 96, 192, 64, 1, 8, 0), 1, 30, dict(state={256: 1, 400: 1}, slots={256: 1, 400: 1}, order={400: 1, 416: 0})),
     ]
     calls, want = [], []
