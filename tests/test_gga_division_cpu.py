@@ -147,9 +147,11 @@ def test_raised_and_lowered_products_enclose_the_quotients():
     IEEE quotients: (x / r) / c against fma(x rc_r, rc_c (1 +- 2^-21), magic), max |x / r| against max |x rc_r| (1 +- 2^-21)."""
     rng = np.random.default_rng(5)
     above, below = 1 + Fraction(1, 2 ** 21), 1 - Fraction(1, 2 ** 21)
-    ds = fp16_divisors()
+    ds = fp16_divisors()                                                # from 2^-24, where the fit clamps, subnormals and all
     same = total = 0
-    for r, c in zip(rng.choice(ds[3000:], 500), rng.choice(ds[3000:], 500)):
+    pairs = list(zip(rng.choice(ds, 500), rng.choice(ds, 500))) + [(r, c) for r in (ds[0], ds[1], ds[1022], ds[1023], ds[-1])
+                                                                   for c in (ds[0], ds[2], ds[1022], ds[1024], ds[-1])]
+    for r, c in pairs:
         r, c = fr(r), fr(c)
         rr, rc = rn32(1 / r), rn32(1 / c)
         up, down = rn32(rc * above), rn32(rc * below)

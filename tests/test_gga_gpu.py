@@ -489,3 +489,36 @@ def test_fit_factors_differ_from_the_oracle_only_on_rounding_thresholds(D):
     print(f'\n[gga fit, d={D}] row factors one fp16 step off: {rows_off} of {rows_seen}; column factors (heads with all '
           f'rows equal): {cols_off} of {cols_seen}; heads byte-identical to the oracle: {heads_exact} of {heads}')
     assert rows_off <= 2e-3 * rows_seen and cols_off <= 2e-3 * cols_seen, (rows_off, rows_seen, cols_off, cols_seen)
+
+
+@pytest.mark.parametrize('D', [64, 128])
+def test_fit_of_values_that_are_fitted_by_division_alone(D):
+    """Codes and column factors come from products with reciprocals while those are below 1e30, from divisions beyond: heads of
+    every width with a column of up to 3e37 (its factor is the largest fp16 number, so are its rows'), one with a single such
+    value, and one without, stored and then stepped with nothing written (beta = 0, no decay: the stored values are fitted
+    again).  Bytes as the oracle's, whose divisions are IEEE."""
+    widths = torch.tensor([2, 4, 6, 8] * 3)
+    HV = len(widths)
+    w = torch.ones(HV, D)                                                        # (row sums: magnitudes only)
+    pk = GGAPacked(GGAPlan({0: (widths, w)}), HV, HV, D, D, pw=False)
+    V = pk.views(pk.alloc(3, DEV))
+    g = torch.Generator().manual_seed(23)
+    S = torch.randn(1, HV, D, D, generator=g)
+    S[0, :4, :, 37] = (torch.rand(4, D, generator=g) * 2 + 1) * 1e37 * torch.randn(4, D, generator=g).sign()
+    S[0, 4:8, 11, 5] = 3e37
+    idx = torch.ones(1, dtype=torch.int32, device=DEV)
+    pk.write(V, idx, S.transpose(-1, -2).to(DEV), layer=0)
+    for stage in range(2):
+        rf, c, z, _ = G.fit_parts(S, widths, w)
+        assert ((S / rf).abs().amax((2, 3))[0, :8] > 1e30).all() or stage       # what the kernel looks at
+        blob = V['blob'][1].cpu().numpy()
+        same = 0
+        for h, (b, off) in enumerate(zip(widths.tolist(), pk.tables[0][0])):
+            raw = G.pack_head(rf[0, h, :, ::32] if b == 2 else rf[0, h, :, 0], c[0, h, 0], z[0, h], b)
+            same += np.array_equal(blob[off:off + raw.size], raw)
+        assert same >= HV - 1, (stage, same)                                     # (a factor on an fp16 threshold, as above)
+        S = pk.stored(V, idx, 0).cpu()
+        assert torch.isfinite(S).all()
+        zero = torch.zeros(1, HV, device=DEV)
+        r = torch.randn(1, HV, D, generator=g).to(DEV)
+        pk.step(V, idx, r, r, r, torch.zeros(1, HV, D, device=DEV), 0.1, g=zero, beta=zero, layer=0)
