@@ -24,9 +24,10 @@
 //
 // What bounds the step is the vector ALU: every head is unpacked, updated, fitted and packed at every token (some 20
 // instructions per state value), while its bytes would take a tenth of the time.  So what counts is instructions, and
-// enough wavefronts to hide the serial stretches between them: the fit keeps ONE copy of the tile and divides by the
-// row factors again where it needs the quotients (three instructions a value), which leaves registers for four
-// wavefronts per SIMD where values and quotients side by side left them for two.
+// enough wavefronts to hide the serial stretches between them: the fit keeps ONE copy of the tile and multiplies by the
+// row factors' reciprocals again where it needs the quotients (one instruction a value; divisions only where a rounding
+// could differ, see GGA_ABOVE), which leaves registers for four wavefronts per SIMD where values and quotients side by side
+// left them for two.
 #pragma once
 #include "sq_device.cuh"
 #include "sq_params.h"

@@ -22,8 +22,8 @@
 // chunks alone, the read-out vectors are zero there -- so that every address stays shifts and masks.
 //
 // us per launch, sequences out of step, one wavefront per head -> this: 96 x 192 int4 g64 (30 heads, 64 sequences) 21.8 ->
-// 15.0; bf16 128 x 128 (32 heads, 40 sequences) 31.4 -> 17.0, where the one-wavefront kernel reads the state twice on a
-// fold and has five wavefronts per compute unit to wait with; four workgroups of 38 KB per compute unit are what LDS
+// 14.1; bf16 128 x 128 (32 heads, 40 sequences) 31.4 -> 14.8, where the one-wavefront kernel reads the state twice on a
+// fold and has five wavefronts per compute unit to wait with; four workgroups of 36 KB per compute unit are what LDS
 // admits there.
 #pragma once
 #include <stdlib.h>
@@ -695,7 +695,7 @@ __device__ __forceinline__ void quad_fold_half(uint8_t* blk, int hf, const FoldK
             set(c4 + 2, get(c4 + 2) * c.z); set(c4 + 3, get(c4 + 3) * c.w);
         }
     }
-    // the m rank-1 updates: first operand = keys (result rows <-> columns as `FoldKeys::col`), second = values
+    // the m rank-1 updates: first operand = keys (result rows <-> columns as `FoldKeys::tile` and `elem` say), second = values
     float bv[MT4];
     {
         // units are this kernel's own device (no reference quantity): an estimate plus one Newton step is plenty
