@@ -857,19 +857,21 @@ void gga_step_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict_
     gga_store_any<T>(S, bits, x, p.w + h * DK, L.fit);
 
     // ---- the last head's: the counters of the slot, advanced (reference `_gga_advance`).  The last one is the last of all
-    // rows that name the slot; who could be it counts them (in the tail of one workgroup a slot: 27.5 -> 27.65 us for 32
-    // sequences, 146.9 -> 147.8 for 256; counted ahead of the tickets by everybody 27.9 and 152.9).  A launch that names a
-    // slot twice steps its state in no order that could be relied on, but the counters advance once, and no ticket is left
-    // for the next step. ----
+    // rows that name the slot; who could be it counts them, in the tail of one workgroup a slot, the counter requested with
+    // the indices (against no count at all, 32 sequences 27.87 -> 27.99 us, 6: 15.24 -> 15.40; the counter behind the indices
+    // 28.04; the indices requested by everybody ahead of the fit 27.96 and 15.36, but 16 sequences with g and beta given
+    // 18.57 -> 18.97 instead of 18.62).  A launch that names a slot twice steps its state in no order that could be relied
+    // on, but the counters advance once, and no ticket is left for the next step. ----
     if (p.pw && t.tid < WAVE) {
         const uint32_t drawn = uint32_t(__builtin_amdgcn_readfirstlane(int(ticket))) / GGA_TICKET + 1;
         if (drawn >= uint32_t(p.hv)) {
+            int32_t* const ct = reinterpret_cast<int32_t*>(base);
+            const int n0 = ct[0];
             uint32_t named = rows == 1;
             for (uint32_t r = 0; rows > 1 && r < rows; r += WAVE)
                 named += __builtin_popcountll(__builtin_amdgcn_ballot_w64(r + t.tid < rows && idx[min(r + t.tid, rows - 1)] == seq));
             if (t.tid == 0 && drawn == named * uint32_t(p.hv)) {
-                int32_t* const ct = reinterpret_cast<int32_t*>(base);
-                const int n0 = ct[0], hd0 = int(ticket & GGA_RING);
+                const int hd0 = int(ticket & GGA_RING);
                 ct[0] = n0 + 1 < m ? n0 + 1 : m;
                 __hip_atomic_store(ct + 1, n0 == m ? (hd0 + 1) % m : hd0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
