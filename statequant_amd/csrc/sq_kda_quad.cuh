@@ -16,10 +16,10 @@
 // One row block per wavefront (four wavefronts for d_v 128): two per wavefront measured the same at 128
 // sequences and 3 % faster at 256 (int4), but a third slower at 16 and slower everywhere on int8.
 // us per launch, one wavefront per head -> this (32 heads of 128 x 128, sequences out of step): int4 g32 1 sequence
-// 6.7 -> 4.5, 16: 16.7 -> 7.8, 128: 25.5 -> 20.6, 256: 36.6 -> 35.8 (in lockstep 35.0 -> 35.7, the one figure that lost);
-// int8 g32 1: 7.8 -> 4.6, 256: 59.0 -> 43.4; value-axis int4 128: 33.6 -> 22.1, int8 256: 60.0 -> 45.0.  Bound at small
-// batches by the chain of a head's life, at large ones by the vector ALU (int4, 256 sequences: 420 instructions per
-// wavefront, 987 with a fold; 13.8 M and 32.3 M a launch, where the one-wavefront kernel has 9.1 M and 29.4 M).
+// 7.6 -> 4.2, 16: 17.7 -> 7.4, 128: 30.0 -> 21.8 (in order 18.8), 256: 47.8 -> 36.6 (in order 33.2; in lockstep 35.0 -> 33.7);
+// when it was built, int8 g32 1: 7.8 -> 4.6, 256: 59.0 -> 43.4, value-axis int4 128: 33.6 -> 22.1, int8 256: 60.0 -> 45.0.  Bound at
+// small batches by the chain of a head's life, at large ones by the vector ALU (int4, 256 sequences: 337 instructions per
+// wavefront, 903 with a fold; 11.0 M and 29.6 M a launch, where the one-wavefront kernel has 9.1 M and 29.4 M).
 #pragma once
 #include "sq_gdn_quad.cuh"
 #include "sq_kda.cuh"

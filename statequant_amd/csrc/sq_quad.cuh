@@ -21,8 +21,8 @@
 // padding.  A d_k that is no power of two (96) gets rows as long as the next one's in LDS -- the loads leave the unused
 // chunks alone, the read-out vectors are zero there -- so that every address stays shifts and masks.
 //
-// us per launch, sequences out of step, one wavefront per head -> this: 96 x 192 int4 g64 (30 heads, 64 sequences) 21.8 ->
-// 14.1; bf16 128 x 128 (32 heads, 40 sequences) 31.4 -> 14.8, where the one-wavefront kernel reads the state twice on a
+// us per launch, sequences out of step, one wavefront per head -> this: 96 x 192 int4 g64 (30 heads, 64 sequences) 24.2 ->
+// 16.2 (in order 12.8); bf16 128 x 128 (32 heads, 40 sequences) 25.6 -> 14.7, where the one-wavefront kernel reads the state twice on a
 // fold and has five wavefronts per compute unit to wait with; four workgroups of 36 KB per compute unit are what LDS
 // admits there.
 #pragma once
@@ -804,8 +804,8 @@ __device__ __forceinline__ void quad_fold_half_f(uint8_t* blk, int hf, const Fol
 // wavefront per head is the length of a head's life (bound by latency and by the vector ALU, not by memory, at every
 // batch size: the fold of a head is half of it) -- two wavefronts per head and the front end shared by the heads of a
 // key head.  us per launch with sequences out of step, one wavefront per head -> this (32 / 16 heads of 128 x 128):
-// int4 1 sequence 9.9 -> 6.0, 16: 19.3 -> 10.5, 100: 32.0 -> 23.0, 256: 37.7 -> 32.3; int8 1: 9.3 -> 5.7,
-// 32: 20.8 -> 14.5, 256: 44.6 -> 38.1; Mamba2 (128 heads of 128 x 64) int4 16: 15.4 -> 13.9.
+// int4 1 sequence 9.5 -> 4.3, 16: 22.3 -> 8.3, 100: 31.7 -> 19.3, 256: 50.3 -> 35.5 (in order 27.2); int8 1: 9.0 -> 4.2,
+// 32: 20.5 -> 10.2, 256: 54.3 -> 41.0 (in order 34.8).
 // ---------------------------------------------------------------------------------------------------------------
 // A lane's columns of one row block: the four that share a word of the matrix operand -- int8: 4 j .. 4 j + 3, j = lane %
 // 32; int4: of every eight columns the even or the odd ones (see `operand`).  Their scales as loaded: four fp16 numbers,
